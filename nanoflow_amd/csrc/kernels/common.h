@@ -191,10 +191,15 @@ __device__ __forceinline__ void load16_to_lds_nt(rsrc_t r, uint32_t byte_off, ui
                :: "s"(lds_addr), "v"(byte_off), "s"(r) : "memory", "m0");
 }
 // The same with the LDS address given as a wavefront-uniform base plus a compile-time constant.
-template <int kLdsOffset>
+// kOnce: with the non-temporal hint.
+template <int kLdsOffset, bool kOnce = false>
 __device__ __forceinline__ void load16_to_lds(rsrc_t r, uint32_t byte_off, uint32_t lds_base) {
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds_base), "v"(byte_off), "s"(r), "n"(kLdsOffset) : "memory", "scc", "m0");
+  if constexpr (kOnce)
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                 :: "s"(lds_base), "v"(byte_off), "s"(r), "n"(kLdsOffset) : "memory", "scc", "m0");
+  else
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :: "s"(lds_base), "v"(byte_off), "s"(r), "n"(kLdsOffset) : "memory", "scc", "m0");
 }
 __device__ __forceinline__ short4_t lds_read_tr16(const uint8_t* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)p);

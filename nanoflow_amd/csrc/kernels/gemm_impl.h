@@ -47,20 +47,22 @@ namespace nf {
 
 constexpr int BK = 64;  // K slab (halves); an A-style LDS row is 128 bytes
 
-template <int BM, int BN, int NB>
+// kCap: bytes of LDS the operand ring may take.  80 KB: two workgroups share a CU.
+constexpr int kWholeCu = 144 * 1024, kHalfCu = 80 * 1024;
+template <int BM, int BN, int NB, int kCap = kWholeCu>
 struct GemmSmem {
   static constexpr int a_bytes = BM * 128;
   static constexpr int b_bytes = BN * 128;  // 64 rows x BN*2 bytes, or BN rows x 128 bytes
   static constexpr int stage_bytes = a_bytes + NB * b_bytes;
   // as many stages as fit 144 KB (of the CU's 160 KB), at most 4: the loads of a slab are issued
   // stages-1 slabs before they are needed
-  static constexpr int stages = (144 * 1024) / stage_bytes > 4 ? 4 : (144 * 1024) / stage_bytes;
+  static constexpr int stages = kCap / stage_bytes > 4 ? 4 : kCap / stage_bytes;
   static_assert(stages >= 2, "tile too large for two LDS stages");
   // Tiles with room for two stages only (256 x 256, the 256 x 128 pair: 64 KB per slab) would have to
   // land every load of a slab within the slab before it -- less than a microsecond, which a load
   // that misses the L2 does not make.  They keep the activations in a ring of two stages and give
   // the weights (the operand that streams from HBM) a ring of three: 2 x 32 + 3 x 32 KB = all 160 KB.
-  static constexpr bool split = stages == 2 && 2 * a_bytes + 3 * NB * b_bytes <= 160 * 1024;
+  static constexpr bool split = stages == 2 && 2 * a_bytes + 3 * NB * b_bytes <= (kCap == kWholeCu ? 160 * 1024 : kCap);
   static constexpr int b_ring = 2 * a_bytes;  // split rings: activation stages first, then the weight stages
   static constexpr size_t bytes = split ? (size_t)2 * a_bytes + (size_t)3 * NB * b_bytes : (size_t)stages * stage_bytes;
 };
@@ -165,7 +167,7 @@ __device__ __forceinline__ float swiglu_rounded(float g_acc, float u_acc) {
 // kPartial: the fp32 sums are stored as they are to D taken as float [M][N] (no alpha, beta, C).
 // kGroup (kBCol only): operands of one group of a grouped product -- the weights' row stride is ldb, D's is
 // ldd, and where a_rows is not null row m of A is row a_rows[m] of a matrix of a_total rows.
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kPartial = false, bool kGroup = false>
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kPartial = false, bool kGroup = false, int kCap = kWholeCu>
 __device__ __forceinline__ void gemm_tile(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
@@ -175,7 +177,7 @@ __device__ __forceinline__ void gemm_tile(
   static_assert(!kGroup || (kBCol && !kDual && !kPartial), "grouped products: plain, k-contiguous weights");
   const int ldb = kGroup ? group_ldb : lda, ldd = kGroup ? group_ldd : N;
   constexpr int NB = kDual ? 2 : 1;
-  using SM = GemmSmem<BM, BN, NB>;
+  using SM = GemmSmem<BM, BN, NB, kCap>;
   // four wavefronts (one per SIMD) or eight (two per SIMD, at most 256 registers each)
   constexpr int NW = WM * WN;
   // The MFMA the tile is computed with.  kM16: v_mfma_f32_16x16x32 -- at this part's power cap the
@@ -795,8 +797,8 @@ __global__ __launch_bounds__(256) void gemm_f16_hybrid_kernel(
 // workgroup (tile, share) computes the tile's sums over k in [share * k_per, ...) and stores them
 // as fp32 to P[share][M][N]; splitk_reduce_kernel adds the shares and applies alpha, beta and C.
 // kDual: two weight matrices; the sums of the second go to P1[share][M][N].
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_f16_splitk_kernel(
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, int kCap = kWholeCu>
+__global__ __launch_bounds__(WM * WN * 64, kCap == kHalfCu ? 2 : 1) void gemm_f16_splitk_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, const uint16_t* __restrict__ B1,
     float* __restrict__ P, float* __restrict__ P1, int M, int N, int K, int shares, int k_per, int tiles_m,
     int tiles_n) {
@@ -807,7 +809,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_f16_splitk_kernel(
   const int k0 = share * k_per;
   const int k_len = K - k0 < k_per ? K - k0 : k_per;
   const size_t b_off = kBCol ? (size_t)k0 : (size_t)k0 * N, p_off = (size_t)share * M * N;
-  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, true>(
+  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, true, false, kCap>(
       A + k0, B + b_off, kDual ? B1 + b_off : nullptr,
       kDual ? reinterpret_cast<const uint16_t*>(P1 + p_off) : nullptr, reinterpret_cast<uint16_t*>(P + p_off), M, N,
       k_len, 1.f, 0.f, N, (tile % tiles_m) * BM, (tile / tiles_m) * BN, K);
@@ -851,12 +853,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 }
 
 // kDual: B1 is the second weight matrix, C is not used, D = the SwiGLU output.
-template <class E, int BM, int BN, int WM, int WN, bool kBCol, bool kDual = false>
+template <class E, int BM, int BN, int WM, int WN, bool kBCol, bool kDual = false, int kCap = kWholeCu>
 static int launch_splitk(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N,
                          int K, float alpha, float beta, int ldc, int shares, int k_per, float* P,
                          hipStream_t stream, const uint16_t* B1 = nullptr) {
-  using SM = GemmSmem<BM, BN, kDual ? 2 : 1>;
-  auto kern = gemm_f16_splitk_kernel<typename E::Mul, BM, BN, WM, WN, kDual, kBCol>;
+  using SM = GemmSmem<BM, BN, kDual ? 2 : 1, kCap>;
+  auto kern = gemm_f16_splitk_kernel<typename E::Mul, BM, BN, WM, WN, kDual, kBCol, kCap>;
   float* P1 = kDual ? P + (size_t)shares * M * N : nullptr;
   static bool attr_set = false;  // benign race: the call is idempotent
   if (!attr_set) {
@@ -1098,6 +1100,8 @@ static int dispatch_menu(int index, const uint16_t* A, const uint16_t* B, const 
 
 }  // namespace nf
 
+#include "gemm_rows.h"
+
 using namespace nf;
 
 static int check_gemm_args(const char* who, const void* A, const void* B, const void* D, int M,
@@ -1126,8 +1130,21 @@ static int gemm_entry(const char* who, const uint16_t* A, const uint16_t* B, con
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
   const int ldc = c_is_row ? 0 : N;  // row stride of C: 0 reads the same row for every m
+  if (b_col_major && rows_pay(M, N, K)) return dispatch_rows<E, false>(A, B, C, D, M, N, K, alpha, beta, ldc, s);
   return b_col_major ? dispatch_plain<E, true>(A, B, C, D, M, N, K, alpha, beta, ldc, s)
                      : dispatch_plain<E, false>(A, B, C, D, M, N, K, alpha, beta, ldc, s);
+}
+
+// At most 64 rows, split over K into `shares` (what the workspace holds the sums of); k-contiguous weights in no more of them
+// than their narrower tiles need.
+template <class E>
+static int launch_splitk_64(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
+                            int ldc, int shares, int k_per, float* P, int b_col_major, hipStream_t s) {
+  if (!b_col_major) return launch_splitk<E, 64, 256, 1, 4, false>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
+  int k_narrow = 0;
+  const int narrow = M > 16 ? splitk_plan_narrow(N, K, &k_narrow) : 1;
+  if (narrow > 1 && narrow <= shares) return launch_splitk<E, 64, 64, 2, 2, true, false, kHalfCu>(A, B, C, D, M, N, K, alpha, beta, ldc, narrow, k_narrow, P, s);
+  return launch_splitk<E, 64, 256, 1, 4, true>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
 }
 
 // gemm_entry with a workspace: shapes that profit are split over K through it.
@@ -1136,7 +1153,7 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
                          int M, int N, int K, float alpha, float beta, int b_col_major, void* workspace,
                          size_t workspace_bytes, nf_stream_t stream, bool c_is_row = false) {
   int k_per = 0;
-  const bool shape_ok = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0;
+  const bool shape_ok = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && !(b_col_major && rows_pay(M, N, K));
   int shares = shape_ok ? splitk_plan(M, N, K, &k_per) : 1;
   const bool dense = shares < 2 && shape_ok && (shares = dense_split_plan(M, N, K, &k_per)) > 1;
   if (shares < 2 || !workspace || workspace_bytes < (size_t)shares * M * N * sizeof(float))
@@ -1150,9 +1167,7 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   if (dense)
     return b_col_major ? launch_splitk<E, 256, 256, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
                        : launch_splitk<E, 256, 256, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
-  if (M <= 64)
-    return b_col_major ? launch_splitk<E, 64, 256, 1, 4, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
-                       : launch_splitk<E, 64, 256, 1, 4, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
+  if (M <= 64) return launch_splitk_64<E>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, b_col_major, s);
   if (M > 256 && M <= kTallRows)
     return b_col_major ? launch_splitk<E, 320, 128, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
                        : launch_splitk<E, 320, 128, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
@@ -1172,6 +1187,7 @@ static int dual_entry(const char* who, const uint16_t* A, const uint16_t* Bgate,
   NF_REQUIRE(((uintptr_t)Bup) % 16 == 0, "%s: operands must be 16-byte aligned", who);
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
+  if (rows_pay_dual(M, K, kBCol)) return dispatch_rows_dual<E, kBCol>(A, Bgate, Bup, out, M, N, K, s);
   if (M <= 64)
     return launch_gemm<E, 64, 128, 2, 2, true, kBCol>(A, Bgate, Bup, nullptr, out, M, N, K, 1.f, 0.f, N, s);
   // 257 .. 320 rows against enough column panels to fill the chip: one 320-row tile per panel, so
@@ -1196,7 +1212,7 @@ static int dual_ws_entry(const char* who, const uint16_t* A, const uint16_t* Bga
                          uint16_t* out, int M, int N, int K, void* workspace, size_t workspace_bytes,
                          nf_stream_t stream) {
   int k_per = 0;
-  const int shares = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 ? splitk_plan_dual(M, N, K, &k_per) : 1;
+  const int shares = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && !rows_pay_dual(M, K, kBCol) ? splitk_plan_dual(M, N, K, &k_per) : 1;
   if (shares < 2 || !workspace || workspace_bytes < (size_t)2 * shares * M * N * sizeof(float))
     return dual_entry<E, kBCol>(who, A, Bgate, Bup, out, M, N, K, stream);
   int rc = check_gemm_args(who, A, Bgate, out, M, N, K);

@@ -4,16 +4,26 @@
 
 namespace {
 
-// Tile of a launch that stores fp32 sums, and its split over K: enough shares of at least 128 to give
+// Tile of a launch that stores fp32 sums, and its split over K.  Few rows: whole sums where the kernel of gemm_rows.h pays, else
+// 64 x 64 tiles in as many shares as give every CU a workgroup.  Other launches: enough shares of at least 128 to give
 // every CU a tile while the sums stay within 64 MiB; two shares of 256 x 256 tiles where dense_split_plan
 // says so; else, from 257 rows on, the largest tile that still gives every CU work.
 struct SumPlan {
-  int tile;  // 0: 64x256, 1: 128x128, 2: 256x256
+  int tile;  // 0: 64x256, 1: 128x128, 2: 256x256, 3: gemm_rows.h, 4: 64x64
   int shares, k_per;
 };
 
 SumPlan sum_plan(int M, int N, int K, int max_shares) {
   SumPlan p{M <= 64 ? 0 : 1, 1, (K + BK - 1) / BK * BK};
+  if (rows_pay(M, N, K)) {
+    p.tile = 3;
+    return p;
+  }
+  if (M > 16 && M <= 64) {
+    int k_narrow = 0;
+    const int narrow = splitk_plan_narrow(N, K, &k_narrow);
+    if (narrow > 1 && narrow <= max_shares) return SumPlan{4, narrow, k_narrow};
+  }
   const long long t256 = (long long)((M + 255) / 256) * ((N + 255) / 256);
   if (M > 256 && t256 >= cu_count() / 2) p.tile = 2;
   if (max_shares < 2 || K < 256) return p;
@@ -30,10 +40,10 @@ SumPlan sum_plan(int M, int N, int K, int max_shares) {
   return p;
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int BM, int BN, int WM, int WN, int kCap = kWholeCu>
 int launch_sums(const uint16_t* A, const uint16_t* B, float* P, int M, int N, int K, const SumPlan& p, hipStream_t s) {
-  using SM = GemmSmem<BM, BN, 1>;
-  auto kern = gemm_f16_splitk_kernel<BF16, BM, BN, WM, WN, false, true>;
+  using SM = GemmSmem<BM, BN, 1, kCap>;
+  auto kern = gemm_f16_splitk_kernel<BF16, BM, BN, WM, WN, false, true, kCap>;
   static bool attr_set = false;  // benign race: the call is idempotent
   if (!attr_set) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -97,6 +107,8 @@ int nf_gemm_nk_sums_bf16(const uint16_t* A, const uint16_t* B, float* P, size_t 
              p.shares, M, N, p_bytes);
   NF_REQUIRE((size_t)32 * N * 4 < 0x7fffffffull, "%s: N=%d", who, N);
   hipStream_t s = (hipStream_t)stream;
+  if (p.tile == 3) return dispatch_rows<BF16, true>(A, B, nullptr, reinterpret_cast<uint16_t*>(P), M, N, K, 1.f, 0.f, N, s);
+  if (p.tile == 4) return launch_sums<64, 64, 2, 2, kHalfCu>(A, B, P, M, N, K, p, s);
   if (p.tile == 0) return launch_sums<64, 256, 1, 4>(A, B, P, M, N, K, p, s);
   if (p.tile == 1) return launch_sums<128, 128, 2, 2>(A, B, P, M, N, K, p, s);
   return launch_sums<256, 256, 2, 2>(A, B, P, M, N, K, p, s);

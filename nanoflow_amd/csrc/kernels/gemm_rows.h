@@ -1,0 +1,289 @@
+#pragma once
+// GEMMs of at most 64 rows: the weights are read once and that is the time (a product of 16 x 4096 x 4096 takes 0.2 us of
+// the matrix cores and 4.8 us of HBM), so this kernel is a weight stream with MFMAs beside it.
+//
+// A workgroup owns NT tiles of 16 weight rows (output columns) and AR rows of A over the WHOLE of K; its wavefronts share K
+// out in units of 64, and their sums meet in LDS at the end, where the epilogue follows: no fp32 shares in memory, no second
+// launch.  Every wavefront streams its own units through a ring of its own in LDS (S units, `buffer_load ... lds`), waits for
+// nobody until the end and refills a slot as soon as its fragments are in registers.  An instruction fetches 8 rows of 128
+// bytes: whole lines, with the non-temporal hint, reach 6.3 - 7.0 TB/s where fragments loaded straight into registers
+// (16 rows of 64 bytes) stop at 5.0 (the gate/up pair of 1 x 14336 x 4096: 37 us against 47).  Weights may be [K][N] as well
+// (kBCol false): rows of NT * 32 bytes per k, read back through the transposing LDS read.
+//
+// The sum of an output element is taken in the same order whatever the tile: eight classes of units (unit mod 8), each in the
+// order of k, then the classes one after the other.  A row's result does not depend on how many rows come with it, nor on
+// the weights' layout.
+//
+// Measured against the tiles and the split over K that it replaces (us, one launch after the other on streamed weights):
+//   rows x N x K              before   here         rows x N x K              before   here
+//   1 x 4096 x 4096             14.3    7.4         64 x 4096 x 4096            15.5   12.0
+//   1 x 6144 x 4096             14.5    9.9         64 x 6144 x 4096            17.8   17.0
+//   1 x 4096 x 14336            25.1   19.6         64 x 2048 x 2048            11.1    6.2
+//   1 x 14336 x 4096 (pair)     47.4   37.2         64 x 14336 x 4096           54.4   27.9
+//   16 x 14336 x 4096 (pair)    48.0   38.7         64 x 14336 x 4096 (pair)    61.5   50.4
+//   16 x 128256 x 4096         173    153.5         16 x 14336 x 4096           49.1   21.1
+// (included by gemm_impl.h, between its kernels and its entry functions)
+
+namespace nf {
+
+constexpr int kRowsMax = 64;       // rows of A
+constexpr int kRowsClasses = 8;    // K is summed in this many interleaved classes of units
+
+template <int AR, int NT, int NW, int NB, int S>
+struct RowsSmem {
+  static constexpr int w_bytes = NB * NT * 2048, slot = w_bytes + AR * 128, ring = NW * S * slot;
+  static constexpr int tiles = NB * ((AR + 15) / 16) * NT;                // accumulator tiles of a wavefront
+  static constexpr int pass = (tiles < 8 ? tiles : 8) / NB;               // output tiles whose sums meet at a time
+  static constexpr int bytes = ring > kRowsClasses * pass * NB * 1024 ? ring : kRowsClasses * pass * NB * 1024;
+  static_assert(bytes <= 160 * 1024 && NB * ((AR + 15) / 16) * NT % (pass * NB) == 0, "rows tile");
+};
+
+// AR: rows of A a workgroup takes (8, 16, 32 or 64).  NB: 2 = the gate/up pair.  kSums: D is float, sums as they are.
+template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, bool kSums>
+__global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                                            const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D, int M,
+                                                            int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n) {
+  using SM = RowsSmem<AR, NT, NW, NB, S>;
+  constexpr int MT = (AR + 15) / 16, PAR = kRowsClasses / NW;  // classes per wavefront
+  static_assert(NW * PAR == kRowsClasses && S % PAR == 0, "a ring slot belongs to one class");
+  const int total = tiles_m * tiles_n, logical = xcd_order(blockIdx.x, total);
+  if (logical >= total) return;
+  // the m tiles of a weight panel side by side: the panel is fetched once
+  const int tm = logical % tiles_m, tn = logical / tiles_m, m0 = tm * AR, n0 = tn * NT * 16;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, lq = lane >> 4;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  const uint32_t mine_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * (S * SM::slot));
+  const uint8_t* mine = smem + wave * (S * SM::slot);
+  const rsrc_t a_rsrc = make_rsrc(A, (size_t)M * K * 2);
+  rsrc_t b_rsrc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) b_rsrc[b] = make_rsrc(b ? B1 : B, (size_t)N * K * 2);
+  const int units = (K + 63) / 64;
+
+  // Rows of 128 bytes (A, [N][K] weights): lane -> row lane / 8 of the instruction's 8, position lane % 8, which holds chunk
+  // position ^ ((row >> 1) & 7) of the 16-row tile (an odd instruction has its rows 8..15): fragment reads without conflicts.
+  const int r8 = lane >> 3;
+  const uint32_t kc[2] = {(uint32_t)((lane & 7) ^ (r8 >> 1)) * 16u, (uint32_t)((lane & 7) ^ ((r8 >> 1) | 4)) * 16u};
+  uint32_t a_off[AR / 8], b_off[NT * 2];
+#pragma unroll
+  for (int i = 0; i < AR / 8; ++i) a_off[i] = (uint32_t)(m0 + i * 8 + r8) * (uint32_t)K * 2u + kc[i & 1];
+  // [K][N] weights: 64 k rows of NT * 32 bytes, as they lie; columns from N on belong to the next row and are not stored
+  constexpr int CPR = NT * 2;  // 16-byte chunks of such a row
+#pragma unroll
+  for (int j = 0; j < NT * 2; ++j) {
+    if constexpr (kBCol) b_off[j] = (uint32_t)(n0 + j * 8 + r8) * (uint32_t)K * 2u + kc[j & 1];
+    else b_off[j] = ((uint32_t)((j * 64 + lane) / CPR) * (uint32_t)N + n0 + (j * 64 + lane) % CPR * 8) * 2u;
+  }
+  // Rows past the operands' last ones lie past the end of the buffers and read as zero.
+  auto issue = [&](auto s_c, int u) {
+    constexpr int s = decltype(s_c)::value;
+    const uint32_t kb = (uint32_t)u * 128u;
+    const bool in = u < units;
+    const bool ok[2] = {in && kb + kc[0] < (uint32_t)K * 2u, in && kb + kc[1] < (uint32_t)K * 2u};
+    static_for<NB>([&](auto b_c) {
+      static_for<NT * 2>([&](auto j_c) {
+        constexpr int b = decltype(b_c)::value, j = decltype(j_c)::value, dst = s * SM::slot + (b * NT * 2 + j) * 1024;
+        if constexpr (kBCol) load16_to_lds<dst, true>(b_rsrc[b], ok[j & 1] ? b_off[j] + kb : kOob, mine_lds);
+        else load16_to_lds<dst, (NT >= 4)>(b_rsrc[b], in ? b_off[j] + (uint32_t)u * 64u * (uint32_t)N * 2u : kOob, mine_lds);
+      });
+    });
+    static_for<AR / 8>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      load16_to_lds<s * SM::slot + SM::w_bytes + i * 1024>(a_rsrc, ok[i & 1] ? a_off[i] + kb : kOob, mine_lds);
+    });
+  };
+
+  float4_t acc[PAR][NB][MT][NT];
+#pragma unroll
+  for (int p = 0; p < PAR; ++p)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[p][b][i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const uint32_t f_row = (uint32_t)l16 * 128u, f_swz = (l16 >> 1) & 7;
+  // eight rows of A stand for sixteen: the upper half of the products is not stored
+  const uint32_t a_row = AR == 8 ? (uint32_t)(l16 & 7) * 128u : f_row, a_swz = AR == 8 ? (l16 & 7) >> 1 : f_swz;
+  auto consume = [&](auto s_c) {
+    constexpr int s = decltype(s_c)::value;
+    const uint8_t* slot = mine + s * SM::slot;
+    half8_t w[2][NB][NT], a[2][MT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          if constexpr (kBCol) {
+            w[h][b][j] = *reinterpret_cast<const half8_t*>(slot + (b * NT + j) * 2048 + f_row + (((h * 4 + lq) ^ f_swz) << 4));
+          } else {  // k rows h * 32 + lq * 8 .. + 7, columns j * 16 .. + 15
+            const uint8_t* p = slot + b * NT * 2048 + (h * 32 + lq * 8 + (l16 >> 2)) * (NT * 32) + j * 32 + (l16 & 3) * 8;
+            typedef short short8_t __attribute__((ext_vector_type(8)));
+            const short4_t lo = lds_read_tr16(p), hi = lds_read_tr16(p + 4 * NT * 32);
+            w[h][b][j] = __builtin_bit_cast(half8_t, (short8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+        }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        a[h][i] = *reinterpret_cast<const half8_t*>(slot + SM::w_bytes + i * 2048 + a_row + (((h * 4 + lq) ^ a_swz) << 4));
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments are in registers, the slot may be refilled
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) acc[s % PAR][b][i][j] = E::mfma16(w[h][b][j], a[h][i], acc[s % PAR][b][i][j]);
+  };
+  constexpr int kLoads = SM::slot / 1024, kYounger = kLoads * (S - 1);
+  static_assert(kYounger < 64, "vmcnt range");
+  int u = wave;
+  static_for<S>([&](auto s_c) {
+    issue(s_c, u);
+    u += NW;
+  });
+  for (int done = wave; done < units; done += NW * S) {  // units past the last one read as zero
+    static_for<S>([&](auto s_c) {
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));  // vmcnt(kYounger): the slot has landed
+      __builtin_amdgcn_sched_barrier(0);
+      consume(s_c);
+      issue(s_c, u);
+      u += NW;
+    });
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  __syncthreads();
+
+  // The classes' sums, SM::pass output tiles at a time: [class][tile][matrix][lane].  Lane (l16, lq) of a tile has columns
+  // lq * 4 .. + 3 of row l16; items are handed out along the rows.
+  constexpr int TP = SM::pass;
+  float4_t* red = reinterpret_cast<float4_t*>(smem);
+  static_for<MT * NT / TP>([&](auto g_c) {
+    constexpr int g = decltype(g_c)::value;
+    if (g) __syncthreads();
+    static_for<PAR * TP * NB>([&](auto q_c) {
+      constexpr int q = decltype(q_c)::value, p = q / (TP * NB), t = q / NB % TP, b = q % NB, tt = g * TP + t;
+      red[(((wave + p * NW) * TP + t) * NB + b) * 64 + lane] = acc[p][b][tt / NT][tt % NT];
+    });
+    __syncthreads();
+    for (int it = threadIdx.x; it < TP * 64; it += NW * 64) {
+      const int t = it >> 6, ln = (it & 3) * 16 + ((it >> 2) & 15), tt = g * TP + t;
+      float4_t v[NB];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        v[b] = red[(t * NB + b) * 64 + ln];
+#pragma unroll
+        for (int c = 1; c < kRowsClasses; ++c) v[b] += red[((c * TP + t) * NB + b) * 64 + ln];
+      }
+      const int row = tt / NT * 16 + (ln & 15), m = m0 + row, n = n0 + tt % NT * 16 + (ln >> 4) * 4;
+      if (row >= AR || m >= M || n >= N) continue;
+      if constexpr (kSums) {
+        *reinterpret_cast<float4_t*>(reinterpret_cast<float*>(D) + (size_t)m * N + n) = v[0];
+      } else {
+        float4_t o;
+        if constexpr (NB == 2) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = swiglu_rounded<E>(v[0][e], v[NB - 1][e]);
+        } else {
+          o = v[0] * alpha;
+          if (beta != 0.f) {
+            const u32x2 c = *reinterpret_cast<const u32x2*>(C + (size_t)m * ldc + n);
+            o[0] += beta * E::widen(c.x & 0xffffu);
+            o[1] += beta * E::widen(c.x >> 16);
+            o[2] += beta * E::widen(c.y & 0xffffu);
+            o[3] += beta * E::widen(c.y >> 16);
+          }
+          o = E::finish(o);
+        }
+        *reinterpret_cast<u32x2*>(D + (size_t)m * N + n) = u32x2{E::pack2(o[0], o[1]), E::pack2(o[2], o[3])};
+      }
+    }
+  });
+}
+
+template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, bool kSums>
+static int launch_rows(const uint16_t* A, const uint16_t* B, const uint16_t* B1, const uint16_t* C, uint16_t* D, int M, int N, int K,
+                       float alpha, float beta, int ldc, hipStream_t stream) {
+  using SM = RowsSmem<AR, NT, NW, NB, S>;
+  auto kern = gemm_rows_kernel<E, AR, NT, NW, NB, S, kBCol, kSums>;
+  static bool attr_set = false;  // benign race: the call is idempotent
+  if (!attr_set) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SM::bytes);
+    if (e != hipSuccess) {
+      set_error("gemm: cannot reserve %d bytes of LDS: %s", SM::bytes, hipGetErrorString(e));
+      return NF_ERR_RUNTIME;
+    }
+    attr_set = true;
+  }
+  const int tiles_m = (M + AR - 1) / AR, tiles_n = (N + NT * 16 - 1) / (NT * 16);
+  kern<<<(tiles_m * tiles_n + 7) / 8 * 8, NW * 64, SM::bytes, stream>>>(A, B, B1, C, D, M, N, K, alpha, beta, ldc, tiles_m, tiles_n);
+  return check_launch("gemm (few rows) launch");
+}
+
+// Which launches run here: at most 64 rows against k-contiguous weights with K >= 1536 (three units a class; below, the plain tile
+// is as good).  Every workgroup reads its rows of A over all of K, so from 17 rows on that traffic counts: a long
+// contraction against a narrow N is better off split over K between workgroups (64 x 4096 x 14336: 26.4 us against 37.5;
+// 64 x 8192 x 8192: even at 31), and from 33 rows on more workgroups than CUs re-read A once too often (64 x 128256 x 4096: 215
+// us against 181 on 64 x 256 tiles).
+static bool rows_pay(int M, int N, int K) {
+  if (M <= 0 || M > kRowsMax || K < 3 * kRowsClasses * 64) return false;
+  if (M <= 16) return true;
+  if (K > 4096 && N < 8192) return false;
+  return M <= 32 || (N + 63) / 64 <= cu_count();
+}
+// The same for the gate/up pair; [K][N] weights in panels of 64 columns, up to 32 rows (16 x 14336 x 4096: 46.8 us against 48.0).
+static bool rows_pay_dual(int M, int K, bool b_col) { return M > 0 && M <= (b_col ? kRowsMax : 32) && K >= 3 * kRowsClasses * 64; }
+
+// Rounds of workgroups times what one of them reads (16-row panels of weights and of A).
+static int rows_cost(int N, int nt, int m_tiles, int a_panels) { return ((N + nt * 16 - 1) / (nt * 16) * m_tiles + cu_count() - 1) / cu_count() * (nt + a_panels); }
+
+template <class E, bool kSums>
+static int dispatch_rows(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
+                         int ldc, hipStream_t s) {
+  if (M <= 8)  // a tie goes to fewer, wider workgroups (1 x 6144 x 4096: 9.9 us against 11.2)
+    return rows_cost(N, 1, 1, 0) < rows_cost(N, 2, 1, 0) ? launch_rows<E, 8, 1, 8, 1, 3, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s)
+                                                         : launch_rows<E, 8, 2, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  if (M <= 16)
+    return rows_cost(N, 1, 1, 1) < rows_cost(N, 2, 1, 1) ? launch_rows<E, 16, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s)
+                                                         : launch_rows<E, 16, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  const int half = (M + 31) / 32;  // m tiles of 32 rows
+  const int c1 = rows_cost(N, 1, half, 2), c2 = rows_cost(N, 2, half, 2);
+  const int w2 = M <= 32 ? 1 << 30 : rows_cost(N, 2, 1, 4), w4 = rows_cost(N, 4, 1, M <= 32 ? 2 : 4);
+  const int best = std::min(std::min(c1, c2), std::min(w2, w4));
+  if (best == c1) return launch_rows<E, 32, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  if (best == c2) return launch_rows<E, 32, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  if (best == w2) return launch_rows<E, 64, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  return M <= 32 ? launch_rows<E, 32, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s)
+                 : launch_rows<E, 64, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+}
+
+template <class E, bool kBCol>
+static int dispatch_rows_dual(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* out, int M, int N, int K, hipStream_t s) {
+  if constexpr (kBCol) {
+    if (M <= 8) return launch_rows<E, 8, 1, 8, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    if (M <= 16) return launch_rows<E, 16, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    if (M <= 32) return launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    return launch_rows<E, 64, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+  } else {
+    if (M <= 8) return launch_rows<E, 8, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    if (M <= 16) return launch_rows<E, 16, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    return launch_rows<E, 32, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+  }
+}
+
+// 17 to 64 rows against k-contiguous weights where rows_pay says no: 64 x 64 tiles, two workgroups a CU, and only as many shares
+// of K as give every CU a workgroup (64 x 4096 x 14336: 26.4 us in 4 shares against 30.1 on 64 x 256 tiles in 16).
+static int splitk_plan_narrow(int N, int K, int* k_per) {
+  if (K <= 4096) return 1;
+  const int shares = std::min(std::min(cu_count() / ((N + 63) / 64), K / 512), kMaxShares);
+  if (shares < 2) return 1;
+  *k_per = ((K + shares - 1) / shares + BK - 1) / BK * BK;
+  return (K + *k_per - 1) / *k_per;
+}
+
+}  // namespace nf

@@ -1,0 +1,72 @@
+"""Products of at most 64 rows on whole-K workgroups (csrc/kernels/gemm_rows.h): every tile of the dispatch at its edges, against
+float64.  An element may be off by its one rounding to 16 bits and by what fp32 sums of K terms can lose:
+2^-p |r| + K 2^-24 sum |a||b| (p = 11 significant bits for fp16, 8 for bf16)."""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+BITS = {torch.float16: 11, torch.bfloat16: 8}
+
+
+def operands(M, N, K, dtype, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed + M + N + K)
+    return (torch.empty(s, device="cuda").normal_(0, d, generator=g).to(dtype) for s, d in (((M, K), 1.0), ((N, K), K ** -0.5)))
+
+
+def check(got, want, a, b, K, bits, scale=1.0):
+    sums = a.double().abs() @ b.double().abs().t()
+    bound = 2.0 ** -bits * want.abs() + scale * K * 2.0 ** -24 * sums + 1e-7
+    assert bool(((got.double() - want).abs() <= bound).all()), float(((got.double() - want).abs() / bound).max())
+
+
+# rows at the edges of the row tiles, columns at those of the panels (and a lone one), K of whole and of cut units
+SHAPES = [(m, n, k) for m in (1, 8, 9, 16, 17, 32, 33, 64) for n, k in ((8, 1536), (72, 1544), (4104, 2048), (264, 4096))] + \
+    [(3, 8200, 1600), (13, 16392, 1536), (30, 16392, 1536), (64, 8200, 1544), (61, 16384, 1536), (40, 24, 6000), (17, 520, 8192), (5, 24, 8200)]
+
+
+@pytest.mark.parametrize("M,N,K_", SHAPES)
+def test_products_of_few_rows(M, N, K_):
+    from nanoflow_amd import kernels as K
+    a, b = operands(M, N, K_, torch.float16)
+    want = a.double() @ b.double().t()
+    got, _ = K.gemm_ws(a, b, b_col_major=True)
+    check(got, want, a, b, K_, 11)
+    c = torch.randn(M, N, device="cuda").half()
+    d = c.clone()
+    K.gemm_ws(a, b, d, alpha=0.5, beta=1.0, b_col_major=True, out=d)                 # in place, as the residual stream is
+    check(d, 0.5 * want + c.double(), a, b, K_, 11)
+    bias = torch.randn(N, device="cuda").half()
+    check(K.gemm_ws(a, b, bias=bias, beta=1.0, b_col_major=True)[0], want + bias.double(), a, b, K_, 11)
+    if M <= 16 or K_ <= 4096:   # a row is the same whatever comes with it
+        assert torch.equal(got[M - 1:], K.gemm_ws(a[M - 1:].clone(), b, b_col_major=True)[0])
+
+
+@pytest.mark.parametrize("M,N,K_", [(1, 2048, 2048), (16, 40, 1544), (33, 72, 2048), (64, 2056, 4096), (40, 264, 8192)])
+def test_bfloat16_products_and_sums(M, N, K_):
+    from nanoflow_amd import kernels as K
+    a, b = operands(M, N, K_, torch.bfloat16)
+    ws = torch.empty(max(K.lib().nf_gemm_nk_workspace_bytes_upto(M, N, K_), 16), dtype=torch.uint8, device="cuda")
+    want = a.double() @ b.double().t()
+    check(K.gemm_nk(a, b, workspace=ws), want, a, b, K_, 8)
+    check(K.gemm_nk(a, b, workspace=ws, squared_relu=True), want.clamp(min=0).square(), a, b, K_, 7, scale=2 * float(want.abs().max()) + 1)
+    bias = torch.randn(N, device="cuda").bfloat16()
+    check(K.gemm_nk(a, b, workspace=ws, bias=bias), want + bias.double(), a, b, K_, 8)
+    check(K.gemm_nk_sums(a, b, 16).sum(0), want, a, b, K_, 20)
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K_", [(72, 1544), (520, 2048), (1160, 4096)])
+def test_gate_up_pair_of_few_rows(M, N, K_):
+    from nanoflow_amd import kernels as K
+    a, g = operands(M, N, K_, torch.float16)
+    _, u = operands(M, N, K_, torch.float16, seed=1)
+    gv, uv = (a.double() @ w.double().t() for w in (g, u))
+    want = torch.nn.functional.silu(gv) * uv
+    got, _ = K.dual_swiglu_ws(a, g, u, b_col_major=True)
+    # both products are rounded to fp16 ahead of silu(g) * u, whose slopes are at most 1.1 |u| and |g|
+    lost = lambda v, w: 2.0 ** -11 * v.abs() + K_ * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
+    bound = 1.1 * uv.abs() * lost(gv, g) + gv.abs() * lost(uv, u) + 2.0 ** -10 * want.abs() + 1e-6
+    assert bool(((got.double() - want).abs() <= bound).all())
+    if M <= 32:                 # [K][N] weights: the same bits
+        assert torch.equal(got, K.dual_swiglu_ws(a, g.t().contiguous(), u.t().contiguous())[0])
