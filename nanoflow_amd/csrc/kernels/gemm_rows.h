@@ -27,6 +27,17 @@
 namespace nf {
 
 constexpr int kRowsMax = 64;       // rows of A
+// e4m3 operands: a unit is 128 k, a lane's two chunks of it go through one MFMA, and the sums are multiplied by a scale per row of A
+// and one per output column.
+struct RowsF8 {
+  static __device__ __forceinline__ float widen(uint32_t bits) { return h2f_bits(bits); }  // C and D are fp16
+  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return pack_f16x2(lo, hi); }
+  static __device__ __forceinline__ float rounded(float x) { return __half2float(__float2half_rn(x)); }
+  static __device__ __forceinline__ float4_t finish(float4_t v) { return v; }
+};
+struct RowsScales {
+  const float *a = nullptr, *b = nullptr, *b1 = nullptr;
+};
 constexpr int kRowsClasses = 8;    // K is summed in this many interleaved classes of units
 
 template <int AR, int NT, int NW, int NB, int S>
@@ -39,11 +50,16 @@ struct RowsSmem {
 };
 
 // AR: rows of A a workgroup takes (8, 16, 32 or 64).  NB: 2 = the gate/up pair.  kSums: D is float, sums as they are.
+// A, B, B1: elements of E's operand type.
 template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, bool kSums>
-__global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                                                            const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D, int M,
-                                                            int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n) {
+__global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restrict__ A, const void* __restrict__ B,
+                                                            const void* __restrict__ B1, const uint16_t* C, uint16_t* D, int M,
+                                                            int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n,
+                                                            RowsScales scales) {
   using SM = RowsSmem<AR, NT, NW, NB, S>;
+  constexpr bool kF8 = std::is_same_v<E, RowsF8>;
+  static_assert(!kF8 || (kBCol && !kSums), "e4m3 weights are k-contiguous");
+  const uint32_t row_bytes = (uint32_t)K * (kF8 ? 1u : 2u);  // of A and of [N][K] weights
   constexpr int MT = (AR + 15) / 16, PAR = kRowsClasses / NW;  // classes per wavefront
   static_assert(NW * PAR == kRowsClasses && S % PAR == 0, "a ring slot belongs to one class");
   const int total = tiles_m * tiles_n, logical = xcd_order(blockIdx.x, total);
@@ -55,11 +71,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __re
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   const uint32_t mine_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * (S * SM::slot));
   const uint8_t* mine = smem + wave * (S * SM::slot);
-  const rsrc_t a_rsrc = make_rsrc(A, (size_t)M * K * 2);
+  const rsrc_t a_rsrc = make_rsrc(A, (size_t)M * row_bytes);
   rsrc_t b_rsrc[NB];
 #pragma unroll
-  for (int b = 0; b < NB; ++b) b_rsrc[b] = make_rsrc(b ? B1 : B, (size_t)N * K * 2);
-  const int units = (K + 63) / 64;
+  for (int b = 0; b < NB; ++b) b_rsrc[b] = make_rsrc(b ? B1 : B, (size_t)N * row_bytes);
+  const int units = (int)((row_bytes + 127) / 128);
 
   // Rows of 128 bytes (A, [N][K] weights): lane -> row lane / 8 of the instruction's 8, position lane % 8, which holds chunk
   // position ^ ((row >> 1) & 7) of the 16-row tile (an odd instruction has its rows 8..15): fragment reads without conflicts.
@@ -67,12 +83,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __re
   const uint32_t kc[2] = {(uint32_t)((lane & 7) ^ (r8 >> 1)) * 16u, (uint32_t)((lane & 7) ^ ((r8 >> 1) | 4)) * 16u};
   uint32_t a_off[AR / 8], b_off[NT * 2];
 #pragma unroll
-  for (int i = 0; i < AR / 8; ++i) a_off[i] = (uint32_t)(m0 + i * 8 + r8) * (uint32_t)K * 2u + kc[i & 1];
+  for (int i = 0; i < AR / 8; ++i) a_off[i] = (uint32_t)(m0 + i * 8 + r8) * row_bytes + kc[i & 1];
   // [K][N] weights: 64 k rows of NT * 32 bytes, as they lie; columns from N on belong to the next row and are not stored
   constexpr int CPR = NT * 2;  // 16-byte chunks of such a row
 #pragma unroll
   for (int j = 0; j < NT * 2; ++j) {
-    if constexpr (kBCol) b_off[j] = (uint32_t)(n0 + j * 8 + r8) * (uint32_t)K * 2u + kc[j & 1];
+    if constexpr (kBCol) b_off[j] = (uint32_t)(n0 + j * 8 + r8) * row_bytes + kc[j & 1];
     else b_off[j] = ((uint32_t)((j * 64 + lane) / CPR) * (uint32_t)N + n0 + (j * 64 + lane) % CPR * 8) * 2u;
   }
   // Rows past the operands' last ones lie past the end of the buffers and read as zero.
@@ -80,7 +96,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __re
     constexpr int s = decltype(s_c)::value;
     const uint32_t kb = (uint32_t)u * 128u;
     const bool in = u < units;
-    const bool ok[2] = {in && kb + kc[0] < (uint32_t)K * 2u, in && kb + kc[1] < (uint32_t)K * 2u};
+    const bool ok[2] = {in && kb + kc[0] < row_bytes, in && kb + kc[1] < row_bytes};
     static_for<NB>([&](auto b_c) {
       static_for<NT * 2>([&](auto j_c) {
         constexpr int b = decltype(b_c)::value, j = decltype(j_c)::value, dst = s * SM::slot + (b * NT * 2 + j) * 1024;
@@ -131,14 +147,30 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __re
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments are in registers, the slot may be refilled
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
+    if constexpr (kF8) {
+      typedef int v4i32 __attribute__((ext_vector_type(4)));
+      typedef int v8i32 __attribute__((ext_vector_type(8)));
+      auto both = [](half8_t lo, half8_t hi) {
+        return (v8i32)__builtin_shufflevector(__builtin_bit_cast(v4i32, lo), __builtin_bit_cast(v4i32, hi), 0, 1, 2, 3, 4, 5, 6, 7);
+      };
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-          for (int i = 0; i < MT; ++i) acc[s % PAR][b][i][j] = E::mfma16(w[h][b][j], a[h][i], acc[s % PAR][b][i][j]);
+          for (int i = 0; i < MT; ++i)
+            acc[s % PAR][b][i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(both(w[0][b][j], w[1][b][j]), both(a[0][i], a[1][i]),
+                                                                                    acc[s % PAR][b][i][j], 0, 0, 0, 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[s % PAR][b][i][j] = E::mfma16(w[h][b][j], a[h][i], acc[s % PAR][b][i][j]);
+    }
   };
   constexpr int kLoads = SM::slot / 1024, kYounger = kLoads * (S - 1);
   static_assert(kYounger < 64, "vmcnt range");
@@ -186,11 +218,16 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __re
         *reinterpret_cast<float4_t*>(reinterpret_cast<float*>(D) + (size_t)m * N + n) = v[0];
       } else {
         float4_t o;
+        if constexpr (kF8) {
+          const float row_scale = scales.a[m];
+          v[0] = v[0] * (*reinterpret_cast<const float4_t*>(scales.b + n) * alpha) * row_scale;
+          if constexpr (NB == 2) v[1] = v[1] * *reinterpret_cast<const float4_t*>(scales.b1 + n) * row_scale;
+        }
         if constexpr (NB == 2) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[e] = swiglu_rounded<E>(v[0][e], v[NB - 1][e]);
         } else {
-          o = v[0] * alpha;
+          o = kF8 ? v[0] : v[0] * alpha;
           if (beta != 0.f) {
             const u32x2 c = *reinterpret_cast<const u32x2*>(C + (size_t)m * ldc + n);
             o[0] += beta * E::widen(c.x & 0xffffu);
@@ -207,8 +244,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const uint16_t* __re
 }
 
 template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, bool kSums>
-static int launch_rows(const uint16_t* A, const uint16_t* B, const uint16_t* B1, const uint16_t* C, uint16_t* D, int M, int N, int K,
-                       float alpha, float beta, int ldc, hipStream_t stream) {
+static int launch_rows(const void* A, const void* B, const void* B1, const uint16_t* C, uint16_t* D, int M, int N, int K,
+                       float alpha, float beta, int ldc, hipStream_t stream, const RowsScales& scales = {}) {
   using SM = RowsSmem<AR, NT, NW, NB, S>;
   auto kern = gemm_rows_kernel<E, AR, NT, NW, NB, S, kBCol, kSums>;
   static bool attr_set = false;  // benign race: the call is idempotent
@@ -221,7 +258,7 @@ static int launch_rows(const uint16_t* A, const uint16_t* B, const uint16_t* B1,
     attr_set = true;
   }
   const int tiles_m = (M + AR - 1) / AR, tiles_n = (N + NT * 16 - 1) / (NT * 16);
-  kern<<<(tiles_m * tiles_n + 7) / 8 * 8, NW * 64, SM::bytes, stream>>>(A, B, B1, C, D, M, N, K, alpha, beta, ldc, tiles_m, tiles_n);
+  kern<<<(tiles_m * tiles_n + 7) / 8 * 8, NW * 64, SM::bytes, stream>>>(A, B, B1, C, D, M, N, K, alpha, beta, ldc, tiles_m, tiles_n, scales);
   return check_launch("gemm (few rows) launch");
 }
 
@@ -230,49 +267,51 @@ static int launch_rows(const uint16_t* A, const uint16_t* B, const uint16_t* B1,
 // contraction against a narrow N is better off split over K between workgroups (64 x 4096 x 14336: 26.4 us against 37.5;
 // 64 x 8192 x 8192: even at 31), and from 33 rows on more workgroups than CUs re-read A once too often (64 x 128256 x 4096: 215
 // us against 181 on 64 x 256 tiles).
-static bool rows_pay(int M, int N, int K) {
-  if (M <= 0 || M > kRowsMax || K < 3 * kRowsClasses * 64) return false;
+static bool rows_pay(int M, int N, int K, int row_bytes = 0) {
+  if (row_bytes == 0) row_bytes = K * 2;  // of 16-bit operands
+  if (M <= 0 || M > kRowsMax || row_bytes < 3 * kRowsClasses * 128) return false;
   if (M <= 16) return true;
-  if (K > 4096 && N < 8192) return false;
+  if (row_bytes > 8192 && N < 8192) return false;
   return M <= 32 || (N + 63) / 64 <= cu_count();
 }
 // The same for the gate/up pair; [K][N] weights in panels of 64 columns, up to 32 rows (16 x 14336 x 4096: 46.8 us against 48.0).
-static bool rows_pay_dual(int M, int K, bool b_col) { return M > 0 && M <= (b_col ? kRowsMax : 32) && K >= 3 * kRowsClasses * 64; }
+static bool rows_pay_dual(int M, int row_bytes, bool b_col) { return M > 0 && M <= (b_col ? kRowsMax : 32) && row_bytes >= 3 * kRowsClasses * 128; }
 
 // Rounds of workgroups times what one of them reads (16-row panels of weights and of A).
 static int rows_cost(int N, int nt, int m_tiles, int a_panels) { return ((N + nt * 16 - 1) / (nt * 16) * m_tiles + cu_count() - 1) / cu_count() * (nt + a_panels); }
 
 template <class E, bool kSums>
-static int dispatch_rows(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
-                         int ldc, hipStream_t s) {
+static int dispatch_rows(const void* A, const void* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
+                         int ldc, hipStream_t s, const RowsScales& sc = {}) {
   if (M <= 8)  // a tie goes to fewer, wider workgroups (1 x 6144 x 4096: 9.9 us against 11.2)
-    return rows_cost(N, 1, 1, 0) < rows_cost(N, 2, 1, 0) ? launch_rows<E, 8, 1, 8, 1, 3, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s)
-                                                         : launch_rows<E, 8, 2, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+    return rows_cost(N, 1, 1, 0) < rows_cost(N, 2, 1, 0) ? launch_rows<E, 8, 1, 8, 1, 3, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc)
+                                                         : launch_rows<E, 8, 2, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
   if (M <= 16)
-    return rows_cost(N, 1, 1, 1) < rows_cost(N, 2, 1, 1) ? launch_rows<E, 16, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s)
-                                                         : launch_rows<E, 16, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+    return rows_cost(N, 1, 1, 1) < rows_cost(N, 2, 1, 1) ? launch_rows<E, 16, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc)
+                                                         : launch_rows<E, 16, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
   const int half = (M + 31) / 32;  // m tiles of 32 rows
   const int c1 = rows_cost(N, 1, half, 2), c2 = rows_cost(N, 2, half, 2);
   const int w2 = M <= 32 ? 1 << 30 : rows_cost(N, 2, 1, 4), w4 = rows_cost(N, 4, 1, M <= 32 ? 2 : 4);
   const int best = std::min(std::min(c1, c2), std::min(w2, w4));
-  if (best == c1) return launch_rows<E, 32, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
-  if (best == c2) return launch_rows<E, 32, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
-  if (best == w2) return launch_rows<E, 64, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
-  return M <= 32 ? launch_rows<E, 32, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s)
-                 : launch_rows<E, 64, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  if (best == c1) return launch_rows<E, 32, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
+  if (best == c2) return launch_rows<E, 32, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
+  if (best == w2) return launch_rows<E, 64, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
+  return M <= 32 ? launch_rows<E, 32, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc)
+                 : launch_rows<E, 64, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
 }
 
 template <class E, bool kBCol>
-static int dispatch_rows_dual(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* out, int M, int N, int K, hipStream_t s) {
+static int dispatch_rows_dual(const void* A, const void* Bg, const void* Bu, uint16_t* out, int M, int N, int K, hipStream_t s,
+                              const RowsScales& sc = {}) {
   if constexpr (kBCol) {
-    if (M <= 8) return launch_rows<E, 8, 1, 8, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
-    if (M <= 16) return launch_rows<E, 16, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
-    if (M <= 32) return launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
-    return launch_rows<E, 64, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    if (M <= 8) return launch_rows<E, 8, 1, 8, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+    if (M <= 16) return launch_rows<E, 16, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+    if (M <= 32) return launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+    return launch_rows<E, 64, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
   } else {
-    if (M <= 8) return launch_rows<E, 8, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
-    if (M <= 16) return launch_rows<E, 16, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
-    return launch_rows<E, 32, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    if (M <= 8) return launch_rows<E, 8, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+    if (M <= 16) return launch_rows<E, 16, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+    return launch_rows<E, 32, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
   }
 }
 

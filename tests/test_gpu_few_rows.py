@@ -70,3 +70,25 @@ def test_gate_up_pair_of_few_rows(M, N, K_):
     assert bool(((got.double() - want).abs() <= bound).all())
     if M <= 32:                 # [K][N] weights: the same bits
         assert torch.equal(got, K.dual_swiglu_ws(a, g.t().contiguous(), u.t().contiguous())[0])
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K_", [(72, 3088), (4104, 4096), (264, 8192)])
+def test_e4m3_products_of_few_rows(M, N, K_):
+    from nanoflow_amd import kernels as K
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K_)
+    codes = lambda r: (torch.randn((r, K_), generator=gen, device="cuda")).to(torch.float8_e4m3fn)
+    a, b, u = codes(M), codes(N), codes(N)
+    sa, sb, su = (torch.rand(n, generator=gen, device="cuda") * K_ ** -0.25 + 0.01 for n in (M, N, N))
+    value = lambda q, s: q.float().double() * s.double()[:, None]
+    av, bv, uv = value(a, sa), value(b, sb), value(u, su)
+    c = torch.randn(M, N, generator=gen, device="cuda").half()
+    raw = lambda q: q.view(torch.uint8)
+    want = av @ bv.t()
+    check(K.gemm_f8(raw(a), sa, raw(b), sb), want, av, bv, K_, 11)
+    check(K.gemm_f8q(raw(a), sa, raw(b), sb, c, alpha=0.5, beta=1.0), 0.5 * want + c.double(), av, bv, K_, 11)
+    g, up = want, av @ uv.t()
+    lost = lambda v, w: 2.0 ** -11 * v.abs() + K_ * 2.0 ** -24 * (av.abs() @ w.abs().t())
+    pair = torch.nn.functional.silu(g) * up
+    got = K.dual_swiglu_f8q(raw(a), sa, raw(b), sb, raw(u), su)
+    assert bool(((got.double() - pair).abs() <= 1.1 * up.abs() * lost(g, bv) + g.abs() * lost(up, uv) + 2.0 ** -10 * pair.abs() + 1e-6).all())
