@@ -110,19 +110,31 @@ __device__ __forceinline__ uint32_t f32_to_e4m3(float x) {
   }
   return sign | code;
 }
-// Eight halves (a 16-byte chunk) divided by s and rounded to e4m3: 8 bytes.
-__device__ __forceinline__ u32x2 quantize_chunk_e4m3(const u32x4& v, float s) {
+// Eight halves (a 16-byte chunk) divided by s and rounded to e4m3: 8 bytes.  r = 1 / s, correctly rounded.  The quotient is
+// x r corrected by one residual, which is the correctly rounded x / s (Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000", 1990): 4 instructions instead of a division's 10, and the hardware's conversion instead of
+// f32_to_e4m3's 12.  The sign is put back for -0.  What the conversion does not take as f32_to_e4m3 does (464 and up, NaN) and an
+// infinite s go the long way.  The same bytes for every half and every maximum.
+__device__ __forceinline__ u32x2 quantize_chunk_e4m3(const u32x4& v, float s, float r) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  uint32_t q[8];
+  float q[8];
+  uint32_t largest = 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    q[2 * i] = f32_to_e4m3(h2f_bits(w[i] & 0xffffu) / s);
-    q[2 * i + 1] = f32_to_e4m3(h2f_bits(w[i] >> 16) / s);
+  for (int i = 0; i < 8; ++i) {
+    const float x = h2f_bits(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu), q0 = x * r;
+    q[i] = copysignf(__builtin_fmaf(__builtin_fmaf(-q0, s, x), r, q0), x);
+    largest = max(largest, __float_as_uint(q[i]) & 0x7fffffffu);
   }
-  u32x2 o;
-  o.x = q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24);
-  o.y = q[4] | (q[5] << 8) | (q[6] << 16) | (q[7] << 24);
-  return o;
+  if (largest >= 0x43E80000u || !(s < INFINITY)) {  // 464
+    uint32_t c[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) c[i] = f32_to_e4m3(h2f_bits(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu) / s);
+    return u32x2{c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24), c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24)};
+  }
+  int lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false), hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false);
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], hi, true);
+  return u32x2{(uint32_t)lo, (uint32_t)hi};
 }
 // Two floats rounded to nearest-even fp16, lo in bits 15:0 (one v_cvt_pk_f16_f32 on gfx950).
 __device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {

@@ -34,52 +34,53 @@ struct F8Smem {
   static constexpr size_t bytes = (size_t)stages * stage_bytes;
 };
 
-// One workgroup per row.  kChunks > 0: the row (at most kChunks x 256 chunks of 8 halves) stays in
-// registers between the maximum and the rounding, so it is read once; kChunks == 0: any length, the
-// second pass reads the row again.
-template <int kChunks>
-__global__ __launch_bounds__(256) void quantize_rows_e4m3_kernel(const uint16_t* __restrict__ X,
-                                                                 uint8_t* __restrict__ Xq,
-                                                                 float* __restrict__ scale, int K) {
-  __shared__ float red[4];
+// One workgroup of kThreads per row.  kChunks > 0: the row (at most kChunks x kThreads chunks of 8 halves) stays in registers
+// between the maximum and the rounding, so it is read once; kChunks == 0: any length, the second pass reads the row
+// again.
+template <int kChunks, int kThreads>
+__global__ __launch_bounds__(kThreads) void quantize_rows_e4m3_kernel(const uint16_t* __restrict__ X,
+                                                                      uint8_t* __restrict__ Xq,
+                                                                      float* __restrict__ scale, int K) {
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  __shared__ float red[kThreads / 64];
   const int row = blockIdx.x, tid = threadIdx.x;
   const u32x4* src = reinterpret_cast<const u32x4*>(X + (size_t)row * K);
   const int chunks = K / 8;
   constexpr int kHeld = kChunks > 0 ? kChunks : 1;
   u32x4 held[kHeld];
-  float amax = 0.f;
+  f16x2 top = {(_Float16)0.f, (_Float16)0.f};  // NaN never wins
   auto chunk_max = [&](const u32x4& v) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      amax = fmaxf(amax, fabsf(h2f_bits(w[i] & 0xffffu)));
-      amax = fmaxf(amax, fabsf(h2f_bits(w[i] >> 16)));
-    }
+    for (int i = 0; i < 4; ++i) top = __builtin_elementwise_max(top, __builtin_bit_cast(f16x2, w[i] & 0x7fff7fffu));
   };
   if constexpr (kChunks > 0) {
 #pragma unroll
     for (int u = 0; u < kChunks; ++u)
-      if (tid + u * 256 < chunks) held[u] = src[tid + u * 256];
+      if (tid + u * kThreads < chunks) held[u] = src[tid + u * kThreads];
 #pragma unroll
     for (int u = 0; u < kChunks; ++u)
-      if (tid + u * 256 < chunks) chunk_max(held[u]);
+      if (tid + u * kThreads < chunks) chunk_max(held[u]);
   } else {
-    for (int c = tid; c < chunks; c += 256) chunk_max(src[c]);
+    for (int c = tid; c < chunks; c += kThreads) chunk_max(src[c]);
   }
+  float amax = fmaxf((float)top[0], (float)top[1]);
 #pragma unroll
   for (int m = 32; m > 0; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const float s = amax > 0.f ? amax / 448.f : 1.f;
+  amax = red[0];
+#pragma unroll
+  for (int i = 1; i < kThreads / 64; ++i) amax = fmaxf(amax, red[i]);
+  const float s = amax > 0.f ? amax / 448.f : 1.f, r = 1.f / s;
   if (tid == 0) scale[row] = s;
   u32x2* dst = reinterpret_cast<u32x2*>(Xq + (size_t)row * K);
   if constexpr (kChunks > 0) {
 #pragma unroll
     for (int u = 0; u < kChunks; ++u)
-      if (tid + u * 256 < chunks) dst[tid + u * 256] = quantize_chunk_e4m3(held[u], s);
+      if (tid + u * kThreads < chunks) dst[tid + u * kThreads] = quantize_chunk_e4m3(held[u], s, r);
   } else {
-    for (int c = tid; c < chunks; c += 256) dst[c] = quantize_chunk_e4m3(src[c], s);
+    for (int c = tid; c < chunks; c += kThreads) dst[c] = quantize_chunk_e4m3(src[c], s, r);
   }
 }
 
@@ -591,9 +592,9 @@ int nf_quantize_rows_e4m3(const uint16_t* X, uint8_t* Xq, float* row_scale, int 
   NF_REQUIRE(((uintptr_t)X | (uintptr_t)Xq) % 16 == 0, "nf_quantize_rows_e4m3: operands must be 16-byte aligned");
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (K <= 4 * 2048) quantize_rows_e4m3_kernel<4><<<M, 256, 0, s>>>(X, Xq, row_scale, K);
-  else if (K <= 16 * 2048) quantize_rows_e4m3_kernel<16><<<M, 256, 0, s>>>(X, Xq, row_scale, K);
-  else quantize_rows_e4m3_kernel<0><<<M, 256, 0, s>>>(X, Xq, row_scale, K);
+  if (K <= 2 * 2048) quantize_rows_e4m3_kernel<2, 256><<<M, 256, 0, s>>>(X, Xq, row_scale, K);
+  else if (K <= 4 * 8192) quantize_rows_e4m3_kernel<4, 1024><<<M, 1024, 0, s>>>(X, Xq, row_scale, K);
+  else quantize_rows_e4m3_kernel<0, 1024><<<M, 1024, 0, s>>>(X, Xq, row_scale, K);
   return check_launch("quantize_rows_e4m3 launch");
 }
 

@@ -181,11 +181,12 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(u32x4* __restrict__ out,
     __syncthreads();
     amax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
     const float s = amax > 0.f ? amax / 448.f : 1.f;
+    const float inv_s = 1.f / s;
     if (threadIdx.x == 0) q_scale[r] = s;
     u32x2* dst = reinterpret_cast<u32x2*>(q_out + (size_t)r * vec_per_row * 8);
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-      if ((int)threadIdx.x + k * 256 < vec_per_row) dst[threadIdx.x + k * 256] = quantize_chunk_e4m3(held[k], s);
+      if ((int)threadIdx.x + k * 256 < vec_per_row) dst[threadIdx.x + k * 256] = quantize_chunk_e4m3(held[k], s, inv_s);
   }
 }
 

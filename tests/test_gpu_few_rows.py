@@ -92,3 +92,25 @@ def test_e4m3_products_of_few_rows(M, N, K_):
     pair = torch.nn.functional.silu(g) * up
     got = K.dual_swiglu_f8q(raw(a), sa, raw(b), sb, raw(u), su)
     assert bool(((got.double() - pair).abs() <= 1.1 * up.abs() * lost(g, bv) + g.abs() * lost(up, uv) + 2.0 ** -10 * pair.abs() + 1e-6).all())
+
+
+@pytest.mark.parametrize("K_", [4096, 8192, 14336, 32784])
+def test_row_quantiser_over_every_half(oracle, K_):
+    """Rows that hold all halves up to a maximum (the largest, ordinary ones, the smallest, subnormal ones, infinity) and NaN, on every
+    row length's kernel: the oracle's bytes and scales."""
+    import numpy as np
+    from nanoflow_amd import kernels as K
+    every = np.arange(65536, dtype=np.uint16)
+    every = every[~((every & 0x7fff) > 0x7c00)]
+    maxima = [0x7bff, 0x7c00, 0x5640, 0x3c00, 0x3555, 0x0401, 0x0400, 0x0003, 0x0001]
+    rows = []
+    for m in maxima:
+        some = every[(every & 0x7fff) <= m]
+        for at in range(0, len(some), K_):
+            rows.append(np.concatenate(([np.uint16(m)], np.resize(some[at:at + K_], K_ - 1))))
+    x = np.stack(rows).view(np.float16)
+    q, s = K.quantize_rows_e4m3(torch.from_numpy(x.copy()).cuda())
+    q_ref, s_ref = oracle.quantize_rows_e4m3(x)
+    finite = np.isfinite(x.astype(np.float32)).all(1)
+    assert np.array_equal(s.cpu().numpy(), s_ref)
+    assert np.array_equal(q.cpu().numpy()[finite], q_ref[finite])
