@@ -15,25 +15,33 @@ struct TilePlace {
 
 // Tile `logical` of the launch; group -1: past the end.  Inside a routed group the m tiles are fastest: they run side by
 // side and share a panel of the expert's weights, which is read once.
-template <int BM>
+// kSpread: every XCD takes an eighth of every group's panels instead of its own run of the launch's tiles, for launches whose tiles
+// cost very unlike: the last XCD would have all of an expert that every token goes to (256 rows, 32 experts of 2048 x 2048 and
+// such a one: 92 -> 75 us).  An eighth is a run of neighbours: every eighth panel is 25 % slower (64 rows of 3584 x 4096: 182 us,
+// 139).
+template <int BM, bool kSpread = false>
 __device__ __forceinline__ TilePlace find_tile(const nf_grouped_gemm_args& a, int bid, int tiles_n) {
   const int tiles_m = (a.M + BM - 1) / BM;
+  const int per = (tiles_n + 7) / 8, start = kSpread ? bid % 8 * per : 0;
+  if constexpr (kSpread) {
+    tiles_n = min(per, tiles_n - start);
+    if (tiles_n <= 0) return {-1, 0, 0, 0, 0};
+  }
   const int m_tiles = a.routing.n_tiles ? *a.routing.n_tiles : tiles_m * a.groups;
-  const int total = m_tiles * tiles_n, logical = xcd_order(bid, total);
-  if (bid / 8 >= (total + 7) / 8 || logical >= total) return {-1, 0, 0, 0, 0};
+  const int total = m_tiles * tiles_n, logical = kSpread ? bid / 8 : xcd_order(bid, total);
+  if ((!kSpread && bid / 8 >= (total + 7) / 8) || logical >= total) return {-1, 0, 0, 0, 0};
   const int mt = logical / tiles_n, n_tile = logical % tiles_n;
   if (a.routing.n_tiles) {
-    const int g = a.routing.tile_group[mt], first = a.routing.offsets[g], rows = a.routing.offsets[g + 1] - first;
+    const int g = a.routing.tile_group[mt], row0 = a.routing.offsets[g], rows = a.routing.offsets[g + 1] - row0;
     const int i = logical - (mt - a.routing.tile_row[mt] / BM) * tiles_n, tiles = (rows + BM - 1) / BM;
-    return {g, i % tiles * BM, rows, i / tiles, (size_t)first};
+    return {g, i % tiles * BM, rows, i / tiles + start, (size_t)row0};
   }
-  return {mt / tiles_m, mt % tiles_m * BM, a.M, n_tile, 0};
+  return {mt / tiles_m, mt % tiles_m * BM, a.M, n_tile + start, 0};
 }
 
-template <class E, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_grouped_kernel(nf_grouped_gemm_args a, int tiles_n) {
-  const TilePlace t = find_tile<BM>(a, blockIdx.x, tiles_n);
-  if (t.group < 0) return;
+// The BM x BN tile of a group from row t.m_base and column n_base.
+template <class E, int BM, int BN, int WM, int WN, int kCap>
+__device__ __forceinline__ void grouped_tile(const nf_grouped_gemm_args& a, const TilePlace& t, int n_base) {
   const bool routed = a.routing.n_tiles != nullptr;
   const int32_t* rows = routed && a.gather ? a.routing.row_of + t.row0 : nullptr;
   const uint16_t* A = (const uint16_t*)a.a + (routed ? (rows ? 0 : t.row0 * a.lda) : (size_t)t.group * a.a_group);
@@ -45,9 +53,85 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_grouped_kernel(nf_grouped_g
     ep.shift = a.gated.shift;
     if (a.gated.limits) ep.limit = a.gated.limits[t.group];
   }
-  gemm_tile<E, BM, BN, WM, WN, false, true, false, true>(A, (const uint16_t*)a.b + (size_t)t.group * a.N * a.K, nullptr, nullptr, D,
-                                                         t.rows, a.N, a.K, 1.f, 0.f, a.N, t.m_base, t.n_tile * BN, a.lda, a.K, a.ldd,
-                                                         rows, a.M, ep);
+  gemm_tile<E, BM, BN, WM, WN, false, true, false, true, kCap>(A, (const uint16_t*)a.b + (size_t)t.group * a.N * a.K, nullptr, nullptr, D,
+                                                               t.rows, a.N, a.K, 1.f, 0.f, a.N, t.m_base, n_base, a.lda, a.K,
+                                                               a.ldd, rows, a.M, ep);
+}
+
+template <class E, int BM, int BN, int WM, int WN, int kCap>
+__global__ __launch_bounds__(WM * WN * 64, kCap == kHalfCu ? 2 : 1) void gemm_grouped_kernel(nf_grouped_gemm_args a, int tiles_n) {
+  const TilePlace t = find_tile<BM>(a, blockIdx.x, tiles_n);
+  if (t.group >= 0) grouped_tile<E, BM, BN, WM, WN, kCap>(a, t, t.n_tile * BN);
+}
+
+unsigned grid_of(const nf_grouped_gemm_args& a, int bm, int tiles_n) {
+  const long long m_tiles = a.routing.n_tiles ? (long long)a.max_rows / bm + std::min(a.groups, a.max_rows) : (long long)((a.M + bm - 1) / bm) * a.groups;
+  return (unsigned)((m_tiles * tiles_n + 7) / 8 * 8);
+}
+
+// Experts with few rows (tile lists of 64): the weight stream of gemm_rows.h, 32 output columns of an expert a workgroup, on a tile
+// that fits the rows that are there.  An expert with more of them than that (one that every token goes to) has 128 x 32 tiles,
+// which leave the other half of its entries in the list out.
+constexpr int kFewRows = 48;  // three 16-row tiles beside 32 columns: 80 KB of ring, two workgroups a CU
+template <class E, bool kSpread>
+__global__ __launch_bounds__(256) void gemm_grouped_rows_kernel(nf_grouped_gemm_args a, int tiles_n) {
+  const TilePlace t = find_tile<64, kSpread>(a, blockIdx.x, tiles_n);
+  if (t.group < 0) return;
+  const int32_t* from = a.gather ? a.routing.row_of + t.row0 : nullptr;
+  const uint16_t* A = (const uint16_t*)a.a + (from ? 0 : t.row0 * a.lda);
+  uint16_t* D = (uint16_t*)a.d + t.row0 * a.ldd;
+  const float* row_scale = a.weigh ? a.routing.row_weight + t.row0 : nullptr;
+  GroupEpilogue ep;
+  if constexpr (std::is_same_v<E, BF16Gated>) {
+    ep.slope = a.gated.slope;
+    ep.shift = a.gated.shift;
+    if (a.gated.limits) ep.limit = a.gated.limits[t.group];
+  }
+  const rsrc_t a_rsrc = make_rsrc(A, ((size_t)((from ? a.M : t.rows) - 1) * a.lda + a.K) * 2);
+  const rsrc_t b_rsrc[1] = {make_rsrc((const uint16_t*)a.b + (size_t)t.group * a.N * a.K, (size_t)a.N * a.K * 2)};
+  const int end = t.rows;
+  auto pass = [&](auto rows_c, int m0) {
+    rows_tile<E, decltype(rows_c)::value, 2, 4, 1, 2, true>(
+        a_rsrc, b_rsrc, (uint32_t)a.K * 2u, a.N, m0, t.n_tile * 32,
+        [&](int m) { return m < end ? (uint32_t)(from ? from[m] : m) * (uint32_t)a.lda * 2u : kOob; },
+        [&](int m, int n, float4_t(&v)[1]) {
+          if (m >= end) return;
+          if (row_scale) v[0] *= row_scale[m];
+          if constexpr (std::is_same_v<E, BF16Gated>) {
+            *reinterpret_cast<uint32_t*>(D + (size_t)m * a.ldd + n / 2) = E::pack2(ep.gated(v[0][0], v[0][1]), ep.gated(v[0][2], v[0][3]));
+          } else {
+            const float4_t o = E::finish(v[0]);
+            *reinterpret_cast<u32x2*>(D + (size_t)m * a.ldd + n) = u32x2{E::pack2(o[0], o[1]), E::pack2(o[2], o[3])};
+          }
+        });
+  };
+  if (t.rows > kFewRows) {
+    if (t.m_base % 128 == 0) grouped_tile<E, 128, 32, 4, 1, kHalfCu>(a, t, t.n_tile * 32);
+  } else if (t.rows <= 16) {
+    pass(ic<16>{}, t.m_base);
+  } else if (t.rows <= 32) {
+    pass(ic<32>{}, t.m_base);
+  } else {
+    pass(ic<kFewRows>{}, t.m_base);
+  }
+}
+
+template <class E, bool kSpread>
+int launch_grouped_rows(const nf_grouped_gemm_args& a, hipStream_t s) {
+  constexpr int lds = RowsSmem<kFewRows, 2, 4, 1, 2>::bytes;
+  auto kern = gemm_grouped_rows_kernel<E, kSpread>;
+  static bool attr_set = false;  // benign race: the call is idempotent
+  if (!attr_set) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) {
+      set_error("nf_gemm_grouped: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
+      return NF_ERR_RUNTIME;
+    }
+    attr_set = true;
+  }
+  const int tiles_n = (a.N + 31) / 32;
+  kern<<<grid_of(a, 64, kSpread ? (tiles_n + 7) / 8 * 8 : tiles_n), 256, lds, s>>>(a, tiles_n);
+  return check_launch("nf_gemm_grouped");
 }
 
 template <int kAct>
@@ -69,15 +153,10 @@ __global__ __launch_bounds__(256) void gemm_grouped_f32_kernel(nf_grouped_gemm_a
                       t.n_tile * kF32Tile, ep);
 }
 
-unsigned grid_of(const nf_grouped_gemm_args& a, int bm, int tiles_n) {
-  const long long m_tiles = a.routing.n_tiles ? (long long)a.max_rows / bm + std::min(a.groups, a.max_rows) : (long long)((a.M + bm - 1) / bm) * a.groups;
-  return (unsigned)((m_tiles * tiles_n + 7) / 8 * 8);
-}
-
-template <class E, int BM, int BN, int WM, int WN>
+template <class E, int BM, int BN, int WM, int WN, int kCap = kWholeCu>
 int launch_grouped(const nf_grouped_gemm_args& a, hipStream_t s) {
-  using SM = GemmSmem<BM, BN, 1>;
-  auto kern = gemm_grouped_kernel<E, BM, BN, WM, WN>;
+  using SM = GemmSmem<BM, BN, 1, kCap>;
+  auto kern = gemm_grouped_kernel<E, BM, BN, WM, WN, kCap>;
   static bool attr_set = false;  // benign race: the call is idempotent
   if (!attr_set) {
     const hipError_t e =
@@ -95,6 +174,23 @@ int launch_grouped(const nf_grouped_gemm_args& a, hipStream_t s) {
 
 template <class E>
 int dispatch_grouped(const nf_grouped_gemm_args& a, int tile_rows, hipStream_t s) {
+  if (a.routing.n_tiles) {
+    // Few rows an expert: as gemm_rows.h.  Its workgroups re-read an expert's rows for every 32 columns, which the larger tiles do
+    // not, so from 17 rows on it pays for short contractions only.  32 experts, 4 of them a token, us against 64 x 256 tiles:
+    //   N x K         1 token   16 tokens   64 tokens   256 tokens (32 rows an expert)
+    //   2048 x 2048   19 -> 13   59 -> 46    65 -> 47    66 -> 56
+    //   4096 x 3584   44 -> 21  136 -> 116  159 -> 139  165 -> 185: not taken
+    // 64 tokens, 2 of 8 of 4096 x 14336 (16 rows an expert): 202 -> 156.
+    const long long rows = a.max_rows, groups = a.groups;
+    if (tile_rows == 64 && a.K >= 1536 && (rows <= 16 * groups || (rows <= 48 * groups && a.K <= 2048)))
+      return a.N >= 512 ? launch_grouped_rows<E, true>(a, s) : launch_grouped_rows<E, false>(a, s);
+    // Short contractions: a third of a tile's time is its start and its end, so two workgroups share a CU and one runs under the
+    // other's (2000 rows, 8 of 64 experts of 1024 x 1024: 80 -> 62 us; 1946 rows, 5 of 33 gated experts of 4096 x 2048: 242 ->
+    // 225).  Longer ones want the larger tile's lower LDS traffic (512 rows, 4 of 32 of 4096 x 3584: 187 us against 205; 2048 rows:
+    // 311 against 325).
+    if (a.K <= 2048)
+      return tile_rows == 64 ? launch_grouped<E, 64, 128, 2, 2, kHalfCu>(a, s) : launch_grouped<E, 128, 128, 2, 2, kHalfCu>(a, s);
+  }
   if (tile_rows == 64) return a.N <= 128 ? launch_grouped<E, 64, 128, 2, 2>(a, s) : launch_grouped<E, 64, 256, 1, 4>(a, s);
   return a.N > 128 && a.N % 256 == 0 ? launch_grouped<E, 128, 256, 2, 2>(a, s) : launch_grouped<E, 128, 128, 2, 2>(a, s);
 }
@@ -103,10 +199,11 @@ int dispatch_grouped(const nf_grouped_gemm_args& a, int tile_rows, hipStream_t s
 
 extern "C" {
 
-// Rows of an m tile: what the routing's tile list has to be made for.
+// Rows of an m tile: what the routing's tile list has to be made for.  (748 rows, 5 of 32 experts and 8 identities of 2048 x 2048,
+// 117 slots an expert: 77 us on 64 rows, 92 on 128.)
 int nf_grouped_tile_rows(int dtype, int rows, int groups) {
   if (dtype == NF_F32) return kF32Tile;
-  return (long long)rows <= 96ll * std::max(groups, 1) ? 64 : 128;
+  return (long long)rows <= 120ll * std::max(groups, 1) ? 64 : 128;
 }
 
 int nf_gemm_grouped(const nf_grouped_gemm_args* args, nf_stream_t stream) {
@@ -128,7 +225,7 @@ int nf_gemm_grouped(const nf_grouped_gemm_args* args, nf_stream_t stream) {
   const int a_rows = routed && !a.gather ? a.max_rows : a.M;
   NF_REQUIRE(((size_t)a_rows + 256) * ((size_t)a.lda + 512) * 2 < 0xFFFFFF00ull && ((size_t)a.N + 256) * ((size_t)a.K + 512) * 2 < 0xFFFFFF00ull,
              "%s: an operand exceeds the 4 GiB buffer-addressing limit", who);
-  const int tile_rows = nf_grouped_tile_rows(a.dtype, routed ? a.max_rows : a.M * a.groups, a.groups);
+  const int tile_rows = a.dtype == NF_F32 || routed ? nf_grouped_tile_rows(a.dtype, a.max_rows, a.groups) : a.M <= 96 ? 64 : 128;
   NF_REQUIRE(!routed || a.routing.tile_rows == tile_rows, "%s: the tile list is for tiles of %d rows, not %d", who, a.routing.tile_rows, tile_rows);
   hipStream_t s = (hipStream_t)stream;
   if (a.dtype == NF_F32) {

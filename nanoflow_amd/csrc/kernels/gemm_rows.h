@@ -49,32 +49,22 @@ struct RowsSmem {
   static_assert(bytes <= 160 * 1024 && NB * ((AR + 15) / 16) * NT % (pass * NB) == 0, "rows tile");
 };
 
-// AR: rows of A a workgroup takes (8, 16, 32 or 64).  NB: 2 = the gate/up pair.  kSums: D is float, sums as they are.
-// A, B, B1: elements of E's operand type.
-template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, bool kSums>
-__global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restrict__ A, const void* __restrict__ B,
-                                                            const void* __restrict__ B1, const uint16_t* C, uint16_t* D, int M,
-                                                            int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n,
-                                                            RowsScales scales) {
+// The tile of AR rows (8, 16, 32, 48 or 64) from row m0 and NT * 16 output columns from n0.  NB: 2 = two weight matrices.  a_row(m): byte
+// offset of row m in A, kOob past the last one (nothing is fetched then).  store(m, n, v): what becomes of the sums v[NB] of row
+// m, columns n .. n + 3.
+template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, class ARow, class Store>
+__device__ __forceinline__ void rows_tile(const rsrc_t a_rsrc, const rsrc_t (&b_rsrc)[NB], const uint32_t row_bytes, const int N,
+                                          const int m0, const int n0, ARow&& a_row, Store&& store) {
   using SM = RowsSmem<AR, NT, NW, NB, S>;
-  constexpr bool kF8 = std::is_same_v<E, RowsF8>;
-  static_assert(!kF8 || (kBCol && !kSums), "e4m3 weights are k-contiguous");
-  const uint32_t row_bytes = (uint32_t)K * (kF8 ? 1u : 2u);  // of A and of [N][K] weights
   constexpr int MT = (AR + 15) / 16, PAR = kRowsClasses / NW;  // classes per wavefront
+  constexpr bool kF8 = std::is_same_v<E, RowsF8>;
   static_assert(NW * PAR == kRowsClasses && S % PAR == 0, "a ring slot belongs to one class");
-  const int total = tiles_m * tiles_n, logical = xcd_order(blockIdx.x, total);
-  if (logical >= total) return;
-  // the m tiles of a weight panel side by side: the panel is fetched once
-  const int tm = logical % tiles_m, tn = logical / tiles_m, m0 = tm * AR, n0 = tn * NT * 16;
+  static_assert(!kF8 || kBCol, "e4m3 weights are k-contiguous");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, lq = lane >> 4;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
   const uint32_t mine_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * (S * SM::slot));
   const uint8_t* mine = smem + wave * (S * SM::slot);
-  const rsrc_t a_rsrc = make_rsrc(A, (size_t)M * row_bytes);
-  rsrc_t b_rsrc[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) b_rsrc[b] = make_rsrc(b ? B1 : B, (size_t)N * row_bytes);
   const int units = (int)((row_bytes + 127) / 128);
 
   // Rows of 128 bytes (A, [N][K] weights): lane -> row lane / 8 of the instruction's 8, position lane % 8, which holds chunk
@@ -82,8 +72,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restri
   const int r8 = lane >> 3;
   const uint32_t kc[2] = {(uint32_t)((lane & 7) ^ (r8 >> 1)) * 16u, (uint32_t)((lane & 7) ^ ((r8 >> 1) | 4)) * 16u};
   uint32_t a_off[AR / 8], b_off[NT * 2];
-#pragma unroll
-  for (int i = 0; i < AR / 8; ++i) a_off[i] = (uint32_t)(m0 + i * 8 + r8) * row_bytes + kc[i & 1];
   // [K][N] weights: 64 k rows of NT * 32 bytes, as they lie; columns from N on belong to the next row and are not stored
   constexpr int CPR = NT * 2;  // 16-byte chunks of such a row
 #pragma unroll
@@ -91,8 +79,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restri
     if constexpr (kBCol) b_off[j] = (uint32_t)(n0 + j * 8 + r8) * row_bytes + kc[j & 1];
     else b_off[j] = ((uint32_t)((j * 64 + lane) / CPR) * (uint32_t)N + n0 + (j * 64 + lane) % CPR * 8) * 2u;
   }
-  // Rows past the operands' last ones lie past the end of the buffers and read as zero.
-  auto issue = [&](auto s_c, int u) {
+  // Weight rows past the last one lie past the end of the buffer and read as zero.
+  auto issue_b = [&](auto s_c, int u) {
     constexpr int s = decltype(s_c)::value;
     const uint32_t kb = (uint32_t)u * 128u;
     const bool in = u < units;
@@ -104,9 +92,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restri
         else load16_to_lds<dst, (NT >= 4)>(b_rsrc[b], in ? b_off[j] + (uint32_t)u * 64u * (uint32_t)N * 2u : kOob, mine_lds);
       });
     });
+  };
+  auto issue_a = [&](auto s_c, int u) {
+    constexpr int s = decltype(s_c)::value;
+    const uint32_t kb = (uint32_t)u * 128u;
+    const bool in = u < units;
+    const bool ok[2] = {in && kb + kc[0] < row_bytes, in && kb + kc[1] < row_bytes};
     static_for<AR / 8>([&](auto i_c) {
       constexpr int i = decltype(i_c)::value;
-      load16_to_lds<s * SM::slot + SM::w_bytes + i * 1024>(a_rsrc, ok[i & 1] ? a_off[i] + kb : kOob, mine_lds);
+      load16_to_lds<s * SM::slot + SM::w_bytes + i * 1024>(a_rsrc, ok[i & 1] && a_off[i] != kOob ? a_off[i] + kc[i & 1] + kb : kOob, mine_lds);
     });
   };
 
@@ -121,7 +115,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restri
         for (int j = 0; j < NT; ++j) acc[p][b][i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
   const uint32_t f_row = (uint32_t)l16 * 128u, f_swz = (l16 >> 1) & 7;
   // eight rows of A stand for sixteen: the upper half of the products is not stored
-  const uint32_t a_row = AR == 8 ? (uint32_t)(l16 & 7) * 128u : f_row, a_swz = AR == 8 ? (l16 & 7) >> 1 : f_swz;
+  const uint32_t af_row = AR == 8 ? (uint32_t)(l16 & 7) * 128u : f_row, a_swz = AR == 8 ? (l16 & 7) >> 1 : f_swz;
   auto consume = [&](auto s_c) {
     constexpr int s = decltype(s_c)::value;
     const uint8_t* slot = mine + s * SM::slot;
@@ -143,7 +137,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restri
         }
 #pragma unroll
       for (int i = 0; i < MT; ++i)
-        a[h][i] = *reinterpret_cast<const half8_t*>(slot + SM::w_bytes + i * 2048 + a_row + (((h * 4 + lq) ^ a_swz) << 4));
+        a[h][i] = *reinterpret_cast<const half8_t*>(slot + SM::w_bytes + i * 2048 + af_row + (((h * 4 + lq) ^ a_swz) << 4));
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments are in registers, the slot may be refilled
     __builtin_amdgcn_sched_barrier(0);
@@ -172,22 +166,32 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restri
             for (int i = 0; i < MT; ++i) acc[s % PAR][b][i][j] = E::mfma16(w[h][b][j], a[h][i], acc[s % PAR][b][i][j]);
     }
   };
-  constexpr int kLoads = SM::slot / 1024, kYounger = kLoads * (S - 1);
-  static_assert(kYounger < 64, "vmcnt range");
-  int u = wave;
-  static_for<S>([&](auto s_c) {
-    issue(s_c, u);
-    u += NW;
-  });
-  for (int done = wave; done < units; done += NW * S) {  // units past the last one read as zero
+  // vmcnt(n): all but the n youngest loads of this wavefront have landed
+  auto wait_but = [](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    static_assert(n < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int kA = AR / 8, kLoads = SM::slot / 1024;
+  // The weights of the first S units are under way before the rows of A are looked up, which may take a load of its own.
+  static_for<S>([&](auto s_c) { issue_b(s_c, wave + decltype(s_c)::value * NW); });
+#pragma unroll
+  for (int i = 0; i < kA; ++i) a_off[i] = a_row(m0 + i * 8 + r8);
+  static_for<S>([&](auto s_c) { issue_a(s_c, wave + decltype(s_c)::value * NW); });
+  int u = wave + S * NW;
+  auto round = [&](auto first_c) {  // units past the last one read as zero
     static_for<S>([&](auto s_c) {
-      __builtin_amdgcn_s_waitcnt(0x0F70 | (kYounger & 15) | ((kYounger >> 4) << 14));  // vmcnt(kYounger): the slot has landed
-      __builtin_amdgcn_sched_barrier(0);
+      constexpr int s = decltype(s_c)::value;
+      wait_but(ic<decltype(first_c)::value ? (S - 1 - s) * kA + s * kLoads : (S - 1) * kLoads>{});  // the slot has landed
       consume(s_c);
-      issue(s_c, u);
+      issue_b(s_c, u);
+      issue_a(s_c, u);
       u += NW;
     });
-  }
+  };
+  if (wave < units) round(ic<1>{});
+  for (int done = wave + NW * S; done < units; done += NW * S) round(ic<0>{});
   __builtin_amdgcn_s_waitcnt(0x0070);
   __syncthreads();
 
@@ -212,35 +216,57 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restri
 #pragma unroll
         for (int c = 1; c < kRowsClasses; ++c) v[b] += red[((c * TP + t) * NB + b) * 64 + ln];
       }
-      const int row = tt / NT * 16 + (ln & 15), m = m0 + row, n = n0 + tt % NT * 16 + (ln >> 4) * 4;
-      if (row >= AR || m >= M || n >= N) continue;
-      if constexpr (kSums) {
-        *reinterpret_cast<float4_t*>(reinterpret_cast<float*>(D) + (size_t)m * N + n) = v[0];
-      } else {
-        float4_t o;
-        if constexpr (kF8) {
-          const float row_scale = scales.a[m];
-          v[0] = v[0] * (*reinterpret_cast<const float4_t*>(scales.b + n) * alpha) * row_scale;
-          if constexpr (NB == 2) v[1] = v[1] * *reinterpret_cast<const float4_t*>(scales.b1 + n) * row_scale;
-        }
-        if constexpr (NB == 2) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = swiglu_rounded<E>(v[0][e], v[NB - 1][e]);
-        } else {
-          o = kF8 ? v[0] : v[0] * alpha;
-          if (beta != 0.f) {
-            const u32x2 c = *reinterpret_cast<const u32x2*>(C + (size_t)m * ldc + n);
-            o[0] += beta * E::widen(c.x & 0xffffu);
-            o[1] += beta * E::widen(c.x >> 16);
-            o[2] += beta * E::widen(c.y & 0xffffu);
-            o[3] += beta * E::widen(c.y >> 16);
-          }
-          o = E::finish(o);
-        }
-        *reinterpret_cast<u32x2*>(D + (size_t)m * N + n) = u32x2{E::pack2(o[0], o[1]), E::pack2(o[2], o[3])};
-      }
+      const int row = tt / NT * 16 + (ln & 15), n = n0 + tt % NT * 16 + (ln >> 4) * 4;
+      if (row < AR && n < N) store(m0 + row, n, v);
     }
   });
+}
+
+// kSums: D is float, sums as they are.  A, B, B1: elements of E's operand type.
+template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, bool kSums>
+__global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(const void* __restrict__ A, const void* __restrict__ B,
+                                                            const void* __restrict__ B1, const uint16_t* C, uint16_t* D, int M,
+                                                            int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n,
+                                                            RowsScales scales) {
+  constexpr bool kF8 = std::is_same_v<E, RowsF8>;
+  const int total = tiles_m * tiles_n, logical = xcd_order(blockIdx.x, total);
+  if (logical >= total) return;
+  const uint32_t row_bytes = (uint32_t)K * (kF8 ? 1u : 2u);  // of A and of [N][K] weights
+  rsrc_t b_rsrc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) b_rsrc[b] = make_rsrc(b ? B1 : B, (size_t)N * row_bytes);
+  // the m tiles of a weight panel side by side: the panel is fetched once
+  rows_tile<E, AR, NT, NW, NB, S, kBCol>(
+      make_rsrc(A, (size_t)M * row_bytes), b_rsrc, row_bytes, N, logical % tiles_m * AR, logical / tiles_m * (NT * 16),
+      [&](int m) { return m < M ? (uint32_t)m * row_bytes : kOob; },
+      [&](int m, int n, float4_t(&v)[NB]) {
+        if (m >= M) return;
+        if constexpr (kSums) {
+          *reinterpret_cast<float4_t*>(reinterpret_cast<float*>(D) + (size_t)m * N + n) = v[0];
+        } else {
+          if constexpr (kF8) {
+            const float row_scale = scales.a[m];
+            v[0] = v[0] * (*reinterpret_cast<const float4_t*>(scales.b + n) * alpha) * row_scale;
+            if constexpr (NB == 2) v[1] = v[1] * *reinterpret_cast<const float4_t*>(scales.b1 + n) * row_scale;
+          }
+          float4_t o;
+          if constexpr (NB == 2) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = swiglu_rounded<E>(v[0][e], v[NB - 1][e]);
+          } else {
+            o = kF8 ? v[0] : v[0] * alpha;
+            if (beta != 0.f) {
+              const u32x2 c = *reinterpret_cast<const u32x2*>(C + (size_t)m * ldc + n);
+              o[0] += beta * E::widen(c.x & 0xffffu);
+              o[1] += beta * E::widen(c.x >> 16);
+              o[2] += beta * E::widen(c.y & 0xffffu);
+              o[3] += beta * E::widen(c.y >> 16);
+            }
+            o = E::finish(o);
+          }
+          *reinterpret_cast<u32x2*>(D + (size_t)m * N + n) = u32x2{E::pack2(o[0], o[1]), E::pack2(o[2], o[3])};
+        }
+      });
 }
 
 template <class E, int AR, int NT, int NW, int NB, int S, bool kBCol, bool kSums>

@@ -114,3 +114,50 @@ def test_row_quantiser_over_every_half(oracle, K_):
     finite = np.isfinite(x.astype(np.float32)).all(1)
     assert np.array_equal(s.cpu().numpy(), s_ref)
     assert np.array_equal(q.cpu().numpy()[finite], q_ref[finite])
+
+
+# rows of each expert, and whether every token also goes to one more
+COUNTS = [([1], False), ([0, 1, 15, 16, 0, 3, 9, 0], False), ([17, 0, 32, 31, 1, 2, 0, 0, 0, 16], False), ([33, 48, 47, 0, 16, 1], False),
+          ([49, 0, 0, 64, 5, 8], False), ([65, 128, 1, 0, 0, 7, 0, 0, 0, 0, 0, 0, 2], False), ([33, 48, 7, 0, 16, 2, 25, 0], True),
+          ([100, 64, 65, 63], False), ([300, 129, 128, 1], False), ([1, 260, 2], True)]
+
+
+@pytest.mark.parametrize("N,K_", [(48, 1536), (272, 1544), (528, 2048), (784, 72), (1040, 2056)])
+@pytest.mark.parametrize("counts,shared", COUNTS)
+def test_experts_at_the_edges_of_their_tiles(counts, shared, N, K_):
+    """Every kernel for the experts' products, each activation with its inputs gathered and weighed or as they lie."""
+    from nanoflow_amd import kernels as K
+    T, e, bf16 = sum(counts), len(counts), torch.bfloat16
+    gen = torch.Generator(device="cuda").manual_seed(T + N + K_)
+    randn = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    of = torch.repeat_interleave(torch.arange(e, device="cuda"), torch.tensor(counts, device="cuda"))[torch.randperm(T, generator=gen, device="cuda")]
+    z = torch.full((1, T, (e + 7) // 8 * 8), -1.0, device="cuda")
+    z[0, torch.arange(T), of] = 2.0
+    n, groups = T * (1 + shared), e + shared
+    r, t = K.route(z, e, e, 1, None, 1.5, K.lib().nf_grouped_tile_rows(K.BF16, n, groups), always=int(shared), scores=K.SCORES_SIGMOID, always_plain=True)
+    offsets = t["offsets"].tolist()
+    assert [b - a for a, b in zip(offsets, offsets[1:])] == counts + [T] * shared
+    h, w = randn(T, K_).to(bf16), (randn(groups, N, K_) * K_ ** -0.5).to(bf16)
+    tokens = t["row_of"].long()
+    for act, gather, weigh in ((K.ACT_NONE, False, False), (K.ACT_GELU, True, False), (K.ACT_SQUARED_RELU, True, True), (K.ACT_GATED, True, True)):
+        a = h if gather else h[tokens].contiguous()
+        d = torch.full((n, N // 2 if act == K.ACT_GATED else N), 9.0, dtype=bf16, device="cuda")
+        K.gemm_grouped_experts(a, w, d, r, n, gather, act, weigh=weigh, gated=(1.7, 1.0, None))
+        for g in range(groups):
+            rows = slice(offsets[g], offsets[g + 1])
+            x = h[tokens[rows]].double()
+            scale = t["row_weight"][rows].double()[:, None] if weigh else 1.0
+            p = x @ w[g].double().t() * scale
+            lost = K_ * 2.0 ** -24 * (x.abs() @ w[g].double().abs().t()) * scale + 2.0 ** -23 * p.abs()
+            if act == K.ACT_GELU:
+                want, lost = torch.nn.functional.gelu(p), 1.13 * lost
+            elif act == K.ACT_SQUARED_RELU:
+                want, lost = p.clamp(min=0) ** 2, 2 * p.abs() * lost + lost ** 2
+            elif act == K.ACT_GATED:
+                gate, up = p[:, ::2], p[:, 1::2] + 1.0
+                want = gate * torch.sigmoid(1.7 * gate) * up
+                lost = 1.2 * lost[:, ::2] * up.abs() + gate.abs() * lost[:, 1::2]  # 1.2: the gate's largest slope
+            else:
+                want = p
+            bound = 2.0 ** -8 * want.abs() + lost + 2.0 ** -18
+            assert bool(((d[rows].double() - want).abs() <= bound).all()), (g, act, float(((d[rows].double() - want).abs() / bound).max()))
