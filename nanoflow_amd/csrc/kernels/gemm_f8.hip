@@ -16,6 +16,7 @@
 // A dot product does not depend on which k a lane slot holds as long as both operands use the
 // same assignment; lane (l32, lg) slot s of k-step kk holds k = kk*64 + lg*32 + s for both.
 #include <algorithm>
+#include <numeric>
 #include <type_traits>
 
 #include "gemm_impl.h"  // the few-row kernel (gemm_rows.h)
@@ -28,10 +29,14 @@ typedef int v8i32 __attribute__((ext_vector_type(8)));
 
 template <int BM, int BN, int NB>
 struct F8Smem {
-  static constexpr int stage_bytes = (BM + NB * BN) * 128;
+  static constexpr int a_bytes = BM * 128, b_bytes = NB * BN * 128;
+  static constexpr int stage_bytes = a_bytes + b_bytes;
   static constexpr int stages = (144 * 1024) / stage_bytes > 4 ? 4 : (144 * 1024) / stage_bytes;
   static_assert(stages >= 2, "tile too large for two LDS stages");
-  static constexpr size_t bytes = (size_t)stages * stage_bytes;
+  // Tiles with room for two stages only keep the activations in two stages and the weights in three (see GemmSmem): a weight load
+  // has two slabs to land, not one.
+  static constexpr bool split = stages == 2 && 2 * a_bytes + 3 * b_bytes <= 160 * 1024;
+  static constexpr size_t bytes = split ? (size_t)2 * a_bytes + (size_t)3 * b_bytes : (size_t)stages * stage_bytes;
 };
 
 // One workgroup of kThreads per row.  kChunks > 0: the row (at most kChunks x kThreads chunks of 8 halves) stays in registers
@@ -228,27 +233,28 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t)
       b_off[b][t] = (uint32_t)(n_base + (t * 4 + wave) * 8 + (lane >> 3)) * (uint32_t)lda + kc;
-  auto load_one = [&](auto t_c, uint32_t st, bool k_ok) {
+  // la / lb: LDS address of the stage the activations / the weights of the slab go to, + wave * 1024
+  auto load_one = [&](auto t_c, uint32_t la, uint32_t lb, bool k_ok) {
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
-      load16_to_lds<t * 4096>(a_rsrc, k_ok ? a_off[t] : kOob, st);
+      load16_to_lds<t * 4096>(a_rsrc, k_ok ? a_off[t] : kOob, la);
       a_off[t] += F8_BK;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
-      load16_to_lds<(BM + b * BN) * 128 + tt * 4096>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, st);
+      load16_to_lds<b * BN * 128 + tt * 4096>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
       b_off[b][tt] += F8_BK;
     }
   };
   auto load_slab = [&](int stage, int k0) {
     const uint32_t st = __builtin_amdgcn_readfirstlane(smem_lds + stage * SM::stage_bytes + wave * 1024);
     const bool k_ok = k0 + kc < K;
-    static_for<LOADS>([&](auto t_c) { load_one(t_c, st, k_ok); });
+    static_for<LOADS>([&](auto t_c) { load_one(t_c, st, st + SM::a_bytes, k_ok); });
   };
 
   // MFMA operand of k-step kk: 32 bytes of row r = the logical chunks 4kk + 2lg and + 1, which
   // sit at positions p and p ^ 1 with p = (4kk + 2lg) ^ ((r >> 1) & 7).
   const uint32_t a_rd = (uint32_t)(wm * (BM / WM) + l32) * 128u;
-  const uint32_t b_rd = (uint32_t)(BM * 128 + (wn * (BN / WN) + l32) * 128);
+  const uint32_t b_rd = (uint32_t)(wn * (BN / WN) + l32) * 128u;
   uint32_t swz[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) swz[kk] = (uint32_t)(((kk * 4 + lg * 2) ^ ((l32 >> 1) & 7)) << 4);
@@ -259,23 +265,24 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
     return v8i32{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
   };
   constexpr int READS = TM + NB * TN;
-  auto read_one = [&](auto q_c, auto kk_c, auto buf_c, const uint8_t* st) {
+  auto read_one = [&](auto q_c, auto kk_c, auto buf_c, const uint8_t* sta, const uint8_t* stb) {
     constexpr int q = decltype(q_c)::value, kk = decltype(kk_c)::value, buf = decltype(buf_c)::value;
     if constexpr (q < TM) {
-      af[buf][q] = read32(st + a_rd + q * 32 * 128, swz[kk]);
+      af[buf][q] = read32(sta + a_rd + q * 32 * 128, swz[kk]);
     } else {
       constexpr int b = (q - TM) / TN, j = (q - TM) % TN;
-      bf[buf][b][j] = read32(st + b_rd + (b * BN + j * 32) * 128, swz[kk]);
+      bf[buf][b][j] = read32(stb + b_rd + (b * BN + j * 32) * 128, swz[kk]);
     }
   };
 
-  // One k-step: its MFMAs (64 cycles of the matrix pipe each) with the loads LP, LP + PARTS, ...
-  // of the slab being fetched (LP < 0: none) and the fragment reads of k-step RK (RK < 0: none)
+  // One k-step: its MFMAs (64 cycles of the matrix pipe each) with the loads L0, L0 + LSTR, ... (NL of them)
+  // of the slab being fetched and the fragment reads of k-step RK (RK < 0: none)
   // dealt out between them, order pinned -- the scheme of gemm.hip.
   constexpr int NM = NB * TN * TM;
-  auto step = [&](auto kk_c, auto lp_c, auto rk_c, uint32_t ld_st, bool ld_ok, const uint8_t* rd_st) {
-    constexpr int kk = decltype(kk_c)::value, LP = decltype(lp_c)::value, RK = decltype(rk_c)::value;
-    constexpr int NL = LP < 0 ? 0 : (LOADS - LP + PARTS - 1) / PARTS;
+  auto step = [&](auto kk_c, auto l0_c, auto lstr_c, auto nl_c, auto rk_c, uint32_t la, uint32_t lb, bool ld_ok, const uint8_t* sta,
+                  const uint8_t* stb) {
+    constexpr int kk = decltype(kk_c)::value, L0 = decltype(l0_c)::value, LSTR = decltype(lstr_c)::value;
+    constexpr int NL = decltype(nl_c)::value, RK = decltype(rk_c)::value;
     constexpr int NR = RK < 0 ? 0 : READS;
     constexpr int S = NL + NR;
     static_for<NM>([&](auto n_c) {
@@ -285,12 +292,65 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
       constexpr int lo = n * S / NM, hi = (n + 1) * S / NM;
       static_for<hi - lo>([&](auto d_c) {
         constexpr int q = lo + decltype(d_c)::value;
-        if constexpr (q < NL) load_one(ic<(LP < 0 ? 0 : LP) + PARTS * q>{}, ld_st, ld_ok);
-        else read_one(ic<q - NL>{}, ic<(RK < 0 ? 0 : RK)>{}, ic<1 - kk>{}, rd_st);
+        if constexpr (q < NL) load_one(ic<L0 + LSTR * q>{}, la, lb, ld_ok);
+        else read_one(ic<q - NL>{}, ic<(RK < 0 ? 0 : RK)>{}, ic<1 - kk>{}, sta, stb);
       });
       __builtin_amdgcn_sched_barrier(0);
     });
   };
+  using T_ = std::true_type;
+  using F_ = std::false_type;
+  const int nslab = (K + F8_BK - 1) / F8_BK;
+
+  if constexpr (SM::split) {
+  // Slab s has its activations in stage s % 2 and its weights in stage s % 3.  Step 0 of slab s issues all weight loads of slab
+  // s+2; then the wavefront waits until everything but those has landed -- its loads of slab s+1 -- and meets the others; step 1
+  // issues the activation loads of slab s+2 into the stage that the barrier has just freed.  (2048 rows, against two whole stages
+  // with a slab for every load: 8192 x 28672 332 -> 306 us, pairs of 14336 x 4096 201 -> 189 and of 28672 x 8192 673 -> 638.
+  // With every operand in the L2 these are 5 % faster: what is left is the matrix pipe and a tile's start and end, 11 us a round.)
+  constexpr int BL = NB * B_LOADS;
+  constexpr int wait_but_b = 0x0070 | (BL & 15) | ((BL >> 4) << 14);  // vmcnt(BL), lgkmcnt(0)
+  auto a_ptr = [&](int s) { return smem8 + (s & 1) * SM::a_bytes; };
+  auto b_ptr = [&](int stage) { return smem8 + 2 * SM::a_bytes + stage * SM::b_bytes; };
+  auto a_lds = [&](int s) { return __builtin_amdgcn_readfirstlane(smem_lds + (s & 1) * SM::a_bytes + wave * 1024); };
+  auto b_lds = [&](int stage) { return __builtin_amdgcn_readfirstlane(smem_lds + 2 * SM::a_bytes + stage * SM::b_bytes + wave * 1024); };
+  auto k_ok_of = [&](int slab_idx) { return slab_idx * F8_BK + kc < K; };
+  // prologue: activations and weights of slab 0, weights of slab 1
+  static_for<LOADS>([&](auto t_c) { load_one(t_c, a_lds(0), b_lds(0), k_ok_of(0)); });
+  if (nslab > 1) {
+    static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, 0, b_lds(1), k_ok_of(1)); });
+    __builtin_amdgcn_s_waitcnt(wait_but_b);
+  } else {
+    __builtin_amdgcn_s_waitcnt(0x0070);
+  }
+  __syncthreads();
+  static_for<READS>([&](auto q_c) { read_one(q_c, ic<0>{}, ic<0>{}, a_ptr(0), b_ptr(0)); });
+  if (nslab > 1) static_for<A_LOADS>([&](auto t_c) { load_one(t_c, a_lds(1), 0, k_ok_of(1)); });
+  // H1: slab s+1 exists, H2: slab s+2 exists; bs = s % 3
+  auto slab = [&](auto h1_c, auto h2_c, int s, int bs) {
+    constexpr bool H1 = decltype(h1_c)::value, H2 = decltype(h2_c)::value;
+    const int bs1 = bs == 2 ? 0 : bs + 1, bs2 = bs1 == 2 ? 0 : bs1 + 1;
+    const uint32_t lb2 = b_lds(bs2), la2 = a_lds(s);
+    step(ic<0>{}, ic<A_LOADS>{}, ic<1>{}, ic<H2 ? BL : 0>{}, ic<1>{}, la2, lb2, k_ok_of(s + 2), a_ptr(s), b_ptr(bs));
+    if constexpr (H1) {
+      __builtin_amdgcn_s_waitcnt(H2 ? wait_but_b : 0x0070);
+      __syncthreads();
+    }
+    step(ic<1>{}, ic<0>{}, ic<1>{}, ic<H2 ? A_LOADS : 0>{}, ic<H1 ? 0 : -1>{}, la2, lb2, k_ok_of(s + 2), a_ptr(s + 1), b_ptr(bs1));
+  };
+  int s = 0, bs = 0;
+  for (; s + 2 < nslab; ++s) {
+    slab(T_{}, T_{}, s, bs);
+    bs = bs == 2 ? 0 : bs + 1;
+  }
+  if (s + 1 < nslab) {
+    slab(T_{}, F_{}, s, bs);
+    bs = bs == 2 ? 0 : bs + 1;
+    ++s;
+  }
+  slab(F_{}, F_{}, s, bs);
+  } else {
+
   // vmcnt(n) with lgkmcnt(0): n in bits [3:0] and [15:14]
   auto wait_loads = [&](int younger) {
     if (younger == 0) __builtin_amdgcn_s_waitcnt(0x0070);
@@ -298,6 +358,7 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
   };
   static_assert(LOADS * (NS - 2) < 64, "vmcnt range");
   auto next = [](int st) { return st + 1 == NS ? 0 : st + 1; };
+  constexpr auto nl = [](int lp) { return (LOADS - lp + PARTS - 1) / PARTS; };  // loads lp, lp + PARTS, ...
 
   // Slab s lives in LDS stage s % NS and is two k-steps.  Step 0 prefetches the fragments of step
   // 1; then the wavefront waits for its own loads of slab s+1 and its reads of this stage, and
@@ -309,31 +370,30 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
     constexpr bool IA = decltype(ia_c)::value, IB = decltype(ib_c)::value, LAST = decltype(last_c)::value;
     const uint8_t* st = smem8 + cs * SM::stage_bytes;
     const uint32_t ld_a = __builtin_amdgcn_readfirstlane(smem_lds + ls * SM::stage_bytes + wave * 1024);
-    step(ic<0>{}, ic<(IA && PARTS > 1) ? 1 : -1>{}, ic<1>{}, ld_a, (s + NS - 1) * F8_BK + kc < K, st);
+    step(ic<0>{}, ic<1>{}, ic<PARTS>{}, ic<(IA && PARTS > 1) ? nl(1) : 0>{}, ic<1>{}, ld_a, ld_a + SM::a_bytes,
+         (s + NS - 1) * F8_BK + kc < K, st, st + SM::a_bytes);
     if constexpr (!LAST) {
       wait_loads(IA ? 1 : 0);
       __syncthreads();
     }
     const uint32_t ld_b = __builtin_amdgcn_readfirstlane(smem_lds + cs * SM::stage_bytes + wave * 1024);
-    step(ic<1>{}, ic<IB ? 0 : -1>{}, ic<LAST ? -1 : 0>{}, ld_b, (s + NS) * F8_BK + kc < K,
-         smem8 + next(cs) * SM::stage_bytes);
+    const uint8_t* nst = smem8 + next(cs) * SM::stage_bytes;
+    step(ic<1>{}, ic<0>{}, ic<PARTS>{}, ic<IB ? nl(0) : 0>{}, ic<LAST ? -1 : 0>{}, ld_b, ld_b + SM::a_bytes,
+         (s + NS) * F8_BK + kc < K, nst, nst + SM::a_bytes);
   };
 
-  const int nslab = (K + F8_BK - 1) / F8_BK;
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
     if (p < nslab) load_slab(p, p * F8_BK);
   wait_loads(nslab >= NS - 1 ? 1 : 0);
   __syncthreads();
-  static_for<READS>([&](auto q_c) { read_one(q_c, ic<0>{}, ic<0>{}, smem8); });
+  static_for<READS>([&](auto q_c) { read_one(q_c, ic<0>{}, ic<0>{}, smem8, smem8 + SM::a_bytes); });
   if (NS - 1 < nslab) {  // the share of slab NS-1 that a slab's step 1 would have issued
     const uint32_t st = __builtin_amdgcn_readfirstlane(smem_lds + (NS - 1) * SM::stage_bytes + wave * 1024);
     const bool k_ok = (NS - 1) * F8_BK + kc < K;
-    static_for<(LOADS + PARTS - 1) / PARTS>([&](auto q_c) { load_one(ic<PARTS * decltype(q_c)::value>{}, st, k_ok); });
+    static_for<(LOADS + PARTS - 1) / PARTS>([&](auto q_c) { load_one(ic<PARTS * decltype(q_c)::value>{}, st, st + SM::a_bytes, k_ok); });
   }
   int cs = 0, ls = NS - 1, s = 0;
-  using T_ = std::true_type;
-  using F_ = std::false_type;
   for (; s + NS < nslab; ++s) {  // steady state
     slab(T_{}, T_{}, F_{}, s, cs, ls);
     cs = next(cs);
@@ -346,26 +406,33 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
     ls = next(ls);
   }
   slab(F_{}, F_{}, T_{}, s, cs, ls);
+  }  // one ring for both operands
 
   // Epilogue, as in gemm.hip: acc[i][j][r] is D[m][n] with m = tile row l32 and
   // n = (r/4)*8 + lg*4 + r%4; each wavefront turns its block around through LDS, 32 rows at a
   // time in fp32, and stores (and reads C and the row scales) in whole runs through buffer
   // descriptors that end with the matrix, so a pass has no branches.
   constexpr int CW = BN / WN, ROWP = CW * 4 + 16, CPR = CW / 4, ITER = 32 * CPR / 64;
-  static_assert(NB * 4 * 32 * ROWP <= (int)SM::bytes && (32 * CPR) % 64 == 0 && 64 % CPR == 0, "epilogue staging");
+  static_assert(NB * 4 * 32 * ROWP <= (int)SM::bytes && (32 * CPR) % 64 == 0, "epilogue staging");
+  constexpr int PER = 64 % CPR == 0 ? 1 : CPR / std::gcd(CPR, 64);  // a lane's columns repeat after PER iterations
   typedef unsigned int u32v2_t __attribute__((ext_vector_type(2)));
   __syncthreads();  // every wavefront has read its last fragments
   uint8_t* ep = smem8 + wave * (32 * ROWP);
   uint8_t* ep1 = smem8 + (4 + wave) * (32 * ROWP);  // kDual: the second product
   const int gn0 = n_base + wn * CW;
-  const int gn = gn0 + (lane % CPR) * 4;  // the same 4 columns in every pass: 64 % CPR == 0
-  float4_t cs4 = float4_t{0.f, 0.f, 0.f, 0.f}, cu4 = float4_t{0.f, 0.f, 0.f, 0.f};
-  if constexpr (!kPartial) {
-    if (gn < N) cs4 = *reinterpret_cast<const float4_t*>(sb + gn);
-    if constexpr (kDual) {
-      if (gn < N) cu4 = *reinterpret_cast<const float4_t*>(sb1 + gn);
-    } else {
-      cs4 *= alpha;
+  int gns[PER];
+  float4_t cs4[PER], cu4[PER];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int gn = gns[p] = gn0 + ((p * 64 + lane) % CPR) * 4;
+    cs4[p] = cu4[p] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if constexpr (!kPartial) {
+      if (gn < N) cs4[p] = *reinterpret_cast<const float4_t*>(sb + gn);
+      if constexpr (kDual) {
+        if (gn < N) cu4[p] = *reinterpret_cast<const float4_t*>(sb1 + gn);
+      } else {
+        cs4[p] *= alpha;
+      }
     }
   }
 #pragma unroll
@@ -397,7 +464,7 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
           const int c = it * 64 + lane;
           const float4_t p4 = *reinterpret_cast<const float4_t*>(ep + (c / CPR) * ROWP + (c % CPR) * 16);
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32v4_t, p4), p_rsrc,
-                                                 gn < N ? (uint32_t)((c / CPR) * N + gn) * 4u : kOob, 0, 0);
+                                                 gns[it % PER] < N ? (uint32_t)((c / CPR) * N + gns[it % PER]) * 4u : kOob, 0, 0);
         }
       }
       continue;
@@ -410,7 +477,7 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
 #pragma unroll
     for (int it = 0; it < ITER; ++it) {
       const int r = (it * 64 + lane) / CPR;
-      off[it] = gn < N ? (uint32_t)(r * N + gn) * 2u : kOob;
+      off[it] = gns[it % PER] < N ? (uint32_t)(r * N + gns[it % PER]) * 2u : kOob;
       rs[it] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, r * 4, 0, 0));
     }
     u32v2_t cv[ITER];
@@ -447,7 +514,7 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
       for (int it = 0; it < ITER; ++it) {
         const int c = it * 64 + lane;
         const float4_t u4 = *reinterpret_cast<const float4_t*>(ep1 + (c / CPR) * ROWP + (c % CPR) * 16);
-        const float4_t g = a4[it] * cs4 * rs[it], u = u4 * cu4 * rs[it];
+        const float4_t g = a4[it] * cs4[it % PER] * rs[it], u = u4 * cu4[it % PER] * rs[it];
         float4_t v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = swiglu_rounded_f16(g[e], u[e]);
@@ -455,11 +522,11 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
       }
     } else if (beta == 0.f) {
 #pragma unroll
-      for (int it = 0; it < ITER; ++it) store_group(it, a4[it] * cs4 * rs[it]);
+      for (int it = 0; it < ITER; ++it) store_group(it, a4[it] * cs4[it % PER] * rs[it]);
     } else {
 #pragma unroll
       for (int it = 0; it < ITER; ++it) {
-        float4_t v = a4[it] * cs4 * rs[it];
+        float4_t v = a4[it] * cs4[it % PER] * rs[it];
         v[0] += beta * h2f_bits(cv[it].x & 0xffffu);
         v[1] += beta * h2f_bits(cv[it].x >> 16);
         v[2] += beta * h2f_bits(cv[it].y & 0xffffu);
@@ -616,9 +683,10 @@ int nf_gemm_f8_f16(const uint8_t* Aq, const float* a_scale, const uint8_t* Bq, c
   if (M <= 64) return launch_gemm_f8<64, 256, 1, 4>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
   // Tile choice by cost, as for the fp16 kernels: rounds of one tile per CU, a partly filled last
   // round charged 0.47 + 0.53 x its fill, a round costing the tile's area over its efficiency
-  // (1 / 0.80 / 0.60 for 256x256 / 128x256 / 128x128, from full rounds with the weights streamed
-  // from HBM).  Picks the fastest tile on the Llama-3-8B and -70B layer shapes at 1024 and 2048
-  // rows (2048 x 6144 x 4096: 49 us on 192 tiles of 256x256, 64 us on 384 of 128x256).
+  // (1 / 0.95 / 0.80 / 0.60 for 256x256 / 256x192 / 128x256 / 128x128, from full rounds with the weights
+  // streamed from HBM).  Picks the fastest tile on the Llama-3-8B and -70B layer shapes at 1024 and 2048
+  // rows (2000 x 6144 x 4096: 48 us on 192 tiles of 256x256, 45 on 256 of 256x192, 56 on 384 of 128x256;
+  // 2000 x 10240 x 4096: 91, 78 and 95).
   static int cus = 0;  // benign race: every thread computes the same value
   if (cus == 0) {
     int dev = 0, v = 0;
@@ -632,8 +700,10 @@ int nf_gemm_f8_f16(const uint8_t* Aq, const float* a_scale, const uint8_t* Bq, c
     return ((double)full + (rest ? 0.47 + 0.53 * (double)rest / cus : 0.0)) * bm * bn / eff;
   };
   const double c256 = cost(256, 256, 1.0), c128x256 = cost(128, 256, 0.80), c128 = cost(128, 128, 0.60);
-  const double best = std::min(c256, std::min(c128x256, c128));
+  const double c192 = cost(256, 192, 0.95);
+  const double best = std::min(std::min(c256, c192), std::min(c128x256, c128));
   if (best == c256) return launch_gemm_f8<256, 256, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
+  if (best == c192) return launch_gemm_f8<256, 192, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
   if (best == c128x256) return launch_gemm_f8<128, 256, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
   return launch_gemm_f8<128, 128, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
 }
