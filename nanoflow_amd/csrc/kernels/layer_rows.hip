@@ -343,8 +343,9 @@ int nf_residual_rows(const nf_residual_args* args, nf_stream_t stream) {
     if (a.y && a.y_dtype == NF_BF16) return b16 ? go(residual_rows_kernel<bf16_t, bf16_t, V, false, N>) : go(residual_rows_kernel<bf16_t, float, V, false, N>);
     return b16 ? go(residual_rows_kernel<float, bf16_t, V, false, N>) : go(residual_rows_kernel<float, float, V, false, N>);
   };
-  // a row on more wavefronts where rows alone leave the CUs mostly empty, and where it is put together from many
-  if ((a.rows <= kFewRows || a.routing) && a.ld > 1024) return a.ld <= 4096 ? sized(ic<1>{}, ic<1024>{}) : a.ld <= 8192 ? sized(ic<2>{}, ic<1024>{}) : sized(ic<4>{}, ic<1024>{});
+  // a row on more wavefronts where rows alone leave the CUs mostly empty.  (Not where rows are many and each is put together from
+  // several: a CU holds two such workgroups, eight of four wavefronts; 2047 rows of 2048, 5 experts a row: 29 us, 16.)
+  if (a.rows <= kFewRows && a.ld > 1024) return a.ld <= 4096 ? sized(ic<1>{}, ic<1024>{}) : a.ld <= 8192 ? sized(ic<2>{}, ic<1024>{}) : sized(ic<4>{}, ic<1024>{});
   return with_vec(a.ld, [&](auto v) { return sized(v, ic<kRowThreads>{}); });
 }
 
