@@ -119,14 +119,20 @@ __global__ __launch_bounds__(256) void attn_plan_kernel(const int32_t* __restric
 //   * A page is addressed through its own buffer descriptor (base = page, 64 KiB range), so
 //     pools larger than 4 GiB need no 64-bit per-lane arithmetic and out-of-page offsets
 //     (used to zero-fill V rows past the end of the sequence) read as zero.
-template <int GROUP, int NW>
+//   * F > 1: F workgroups share a request and kv head.  Each takes all keys, 128 / F features of V and of the output, so its
+//     stream is (1 + 1/F) / 2 as long, the K tiles come out of the L2 for all but the first, and the sums stay what they
+//     are.  (Sharing the keys out instead needs a second launch that adds the parts.  One request, 8 heads: 8.2 us for
+//     1000 keys against 11.7, but 7 for 100 against 4.5, and the length is not known where the launch is chosen.)
+template <int GROUP, int NW, int F>
 __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
     const uint16_t* __restrict__ q, uint16_t* __restrict__ o, const int32_t* __restrict__ qo_indptr,
     const uint16_t* __restrict__ kv_data, const int32_t* __restrict__ kv_indptr,
     const int32_t* __restrict__ kv_indices, const int32_t* __restrict__ kv_last_page_len, int batch,
     int Hq, int Hkv, int causal, float scale_log2) {
   constexpr int TPB = 16 / GROUP;  // tokens per 16-column block = tokens per work item pass
-  constexpr int WAVE_LDS = 32768;  // per wavefront: K0 K1 V0 V1, 8 KB each
+  constexpr int V_BYTES = 8192 / F, WAVE_LDS = 16384 + 2 * V_BYTES;  // per wavefront: K0 K1 of 8 KB, V0 V1
+  constexpr int NF = 8 / F, VROW = 256 / F;  // 16-feature blocks, bytes of a V row
+  constexpr int KL = 8, VL = 8 / F;          // load instructions of a K and of a V tile
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
@@ -144,12 +150,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
   for (int j = 0; j < 4; ++j) kx[j] = (uint32_t)(c16 * 256 + (((j * 4 + g) ^ c16) << 4));
   // V: lanes 16g..16g+15 read the 4(key) x 16(feature) block of keys 4g.. and features 16i..;
   // lane i16 addresses key 4g + i16/4, features 16i + 4(i16&3)..+3; 32-byte unit i of a row
-  // sits at i ^ (key & 7) (the 8 keys x 32 bytes of a read cycle then cover all 64 banks).
-  const int i16 = lane & 15, vx_x = ((g & 1) << 2) | ((i16 >> 2) & 3);
-  uint32_t vx[8];
+  // sits at i ^ (key & 7) / F (the 8 keys x 32 bytes of a read cycle then cover all 64 banks).
+  const int i16 = lane & 15, vx_x = (((g & 1) << 2) | ((i16 >> 2) & 3)) / F;
+  uint32_t vx[NF];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-    vx[i] = (uint32_t)((g * 4 + (i16 >> 2)) * 256 + ((i ^ vx_x) * 32) + (i16 & 3) * 8);
+  for (int i = 0; i < NF; ++i)
+    vx[i] = (uint32_t)((g * 4 + (i16 >> 2)) * VROW + ((i ^ vx_x) * 32) + (i16 & 3) * 8);
 
   // Work item w -> (request, kv head).  Workgroup ids go round the 8 XCDs, so in groups of 8
   // requests the item order is (head, request): the workgroups an XCD starts one after the other
@@ -157,14 +163,18 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
   // each key's 256-byte rows of all heads -- one contiguous Hkv x 256 bytes in the pool -- together
   // (the bare load pattern: 6.55 -> 6.76 TB/s).  The requests past the last whole group of 8 keep
   // (request, head) order.
-  const long long grouped = (long long)(batch / 8) * 8 * Hkv;
-  for (long long w = blockIdx.x; w < (long long)batch * Hkv; w += gridDim.x) {
-    int req = (int)(w / Hkv), kvh = (int)(w % Hkv);
+  // The F workgroups of a head come after all heads' firsts: with 8 kv heads, on one XCD again.
+  const int sharers = Hkv * F;
+  const long long grouped = (long long)(batch / 8) * 8 * sharers;
+  for (long long w = blockIdx.x; w < (long long)batch * sharers; w += gridDim.x) {
+    int req = (int)(w / sharers), kvh = (int)(w % sharers);
     if (w < grouped) {
-      const int j = (int)(w % (8 * Hkv));
-      req = (int)(w / (8 * Hkv)) * 8 + j % 8;
+      const int j = (int)(w % (8 * sharers));
+      req = (int)(w / (8 * sharers)) * 8 + j % 8;
       kvh = j / 8;
     }
+    const int f = F > 1 ? kvh / Hkv : 0;
+    kvh -= f * Hkv;
     const int qo0 = qo_indptr[req];
     const int qo_len = qo_indptr[req + 1] - qo0;
     const int pg0 = kv_indptr[req];
@@ -172,21 +182,27 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
     const int kv_len = npages > 0 ? (npages - 1) * PAGE + kv_last_page_len[req] : 0;
     // DMA source offsets inside a page: instruction t4 moves keys 4*t4 .. 4*t4+3 of a page
     // (64 lanes x 16 bytes = 4 rows), lane -> key 4*t4 + lane/16, position lane%16.
-    uint32_t k_src[4], v_src[4];
+    // V: 4 F rows of 256 / F bytes.
+    uint32_t k_src[4], v_src[4 / F];
 #pragma unroll
     for (int t4 = 0; t4 < 4; ++t4) {
       const int key = 4 * t4 + (lane >> 4), pos = lane & 15;
       const uint32_t row = (uint32_t)((key * Hkv + kvh) * D * 2);
       k_src[t4] = row + (uint32_t)(((pos ^ key) & 15) << 4);
-      v_src[t4] = v_half + row + (uint32_t)((pos ^ ((key & 7) << 1)) << 4);
+    }
+    const int v_key = lane / (16 / F);  // of this lane inside a V instruction
+#pragma unroll
+    for (int t4 = 0; t4 < 4 / F; ++t4) {
+      const int key = 4 * F * t4 + v_key, pos = lane % (16 / F);
+      v_src[t4] = v_half + (uint32_t)((key * Hkv + kvh) * D * 2 + f * VROW) + (uint32_t)((pos ^ ((key & 7) / F << 1)) << 4);
     }
     const int n_sub = (qo_len + TPB - 1) / TPB;
     for (int sub = 0; sub < n_sub; ++sub) {
       const int tok0 = sub * TPB;
-      float4_t oacc[8];
+      float4_t oacc[NF];
       float m_run = -1e30f, l_run = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) oacc[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < NF; ++i) oacc[i] = float4_t{0.f, 0.f, 0.f, 0.f};
 
       // Q operand: column c16 = (token tok0 + c16/GROUP, head c16%GROUP)
       H8 qf[4];
@@ -211,29 +227,31 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
       auto dma_k = [&](int pp, int buf) {
         const rsrc_t ra = page_rsrc(2 * pp), rb = page_rsrc(2 * pp + 1);
         const uint32_t dst = wlds + buf * 8192;
+        auto load = [&](const rsrc_t& r, uint32_t off, uint32_t to) {  // shared K tiles stay in the L2
+          if constexpr (F == 1) load16_to_lds_nt(r, off, to);
+          else load16_to_lds(r, off, to);
+        };
 #pragma unroll
-        for (int t4 = 0; t4 < 4; ++t4) load16_to_lds_nt(ra, k_src[t4], dst + t4 * 1024);
+        for (int t4 = 0; t4 < 4; ++t4) load(ra, k_src[t4], dst + t4 * 1024);
 #pragma unroll
-        for (int t4 = 0; t4 < 4; ++t4) load16_to_lds_nt(rb, k_src[t4], dst + 4096 + t4 * 1024);
+        for (int t4 = 0; t4 < 4; ++t4) load(rb, k_src[t4], dst + 4096 + t4 * 1024);
       };
       auto dma_v = [&](int pp, int buf) {
         const rsrc_t ra = page_rsrc(2 * pp), rb = page_rsrc(2 * pp + 1);
-        const uint32_t dst = wlds + 16384 + buf * 8192;
+        const uint32_t dst = wlds + 16384 + buf * V_BYTES;
         // rows past the end of the sequence may hold anything (NaN x 0 = NaN): zero-fill them
-        const int first_key = pp * 32 + (lane >> 4);
+        const int first_key = pp * 32 + v_key;
 #pragma unroll
-        for (int t4 = 0; t4 < 4; ++t4)
-          load16_to_lds_nt(ra, first_key + 4 * t4 < kv_len ? v_src[t4] : kOob, dst + t4 * 1024);
+        for (int t4 = 0; t4 < 4 / F; ++t4)
+          load16_to_lds_nt(ra, first_key + 4 * F * t4 < kv_len ? v_src[t4] : kOob, dst + t4 * 1024);
 #pragma unroll
-        for (int t4 = 0; t4 < 4; ++t4)
-          load16_to_lds_nt(rb, first_key + 16 + 4 * t4 < kv_len ? v_src[t4] : kOob, dst + 4096 + t4 * 1024);
+        for (int t4 = 0; t4 < 4 / F; ++t4)
+          load16_to_lds_nt(rb, first_key + 16 + 4 * F * t4 < kv_len ? v_src[t4] : kOob, dst + V_BYTES / 2 + t4 * 1024);
       };
       // vmcnt(n): everything but the n youngest load instructions of this wavefront has landed
-      auto wait_but = [&](int younger) {
-        if (younger >= 24) __builtin_amdgcn_s_waitcnt(0x0F70 | (24 & 15) | ((24 >> 4) << 14));
-        else if (younger >= 16) __builtin_amdgcn_s_waitcnt(0x0F70 | (16 & 15) | ((16 >> 4) << 14));
-        else if (younger >= 8) __builtin_amdgcn_s_waitcnt(0x0F70 | 8);
-        else __builtin_amdgcn_s_waitcnt(0x0F70);
+      auto wait_but = [&](auto younger_c) {
+        constexpr int younger = decltype(younger_c)::value;
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (younger & 15) | ((younger >> 4) << 14));
       };
 
       // two steps in flight before the loop
@@ -256,10 +274,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
         const int t_base = pp * 32;
         const bool n1 = pp + NW < npairs, n2 = pp + 2 * NW < npairs;
         const uint8_t* kt = wptr + buf * 8192;
-        const uint8_t* vt = wptr + 16384 + buf * 8192;
+        const uint8_t* vt = wptr + 16384 + buf * V_BYTES;
 
         // ---- scores: K(pp) has landed once only V(pp), K(pp+4), V(pp+4) may still be in flight
-        wait_but(n1 ? 24 : 8);
+        if (n1) wait_but(ic<2 * VL + KL>{});
+        else wait_but(ic<VL>{});
         float4_t s[2];
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
@@ -309,12 +328,14 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
         l_run = l_run * alpha + psum;
 
         // ---- P.V: V(pp) has landed once only K(pp+4), V(pp+4), K(pp+8) may still be in flight
-        wait_but((n1 ? 16 : 0) + (n2 ? 8 : 0));
+        if (n2) wait_but(ic<2 * KL + VL>{});
+        else if (n1) wait_but(ic<KL + VL>{});
+        else wait_but(ic<0>{});
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < NF; ++i) {
           const uint8_t* vp = vt + vx[i];
-          const short4_t lo = lds_read_tr16(vp);         // keys 4g..4g+3 of the first page
-          const short4_t hi = lds_read_tr16(vp + 4096);  // ... of the second page
+          const short4_t lo = lds_read_tr16(vp);                // keys 4g..4g+3 of the first page
+          const short4_t hi = lds_read_tr16(vp + V_BYTES / 2);  // ... of the second page
           typedef short short8_t __attribute__((ext_vector_type(8)));
           const short8_t v8 = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
           oacc[i] *= alpha;
@@ -330,11 +351,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
 
       // ---- merge the wavefronts.  oacc[i][r] = O[column c16][feature 16i + 4g + r].  Each
       // wavefront parks its partial result in its own LDS region (its streaming is over).
-      float* s_o = reinterpret_cast<float*>(wptr);             // [8][4][64]
+      float* s_o = reinterpret_cast<float*>(wptr);             // [NF][4][64]
       float* s_m = reinterpret_cast<float*>(wptr + 8192);      // [64]
       float* s_l = reinterpret_cast<float*>(wptr + 8192 + 256);
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < NF; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s_o[(i * 4 + r) * 64 + lane] = oacc[i][r];
       s_m[lane] = m_run;
@@ -354,11 +375,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
       }
       const float inv = L > 0.f ? 1.0f / L : 0.f;
       if (live) {
-        // wavefront w finishes 8/NW of the 16-feature blocks: 4 consecutive features per lane and i
-        uint16_t* op = o + ((size_t)(qo0 + tq) * Hq + kvh * GROUP + c16 % GROUP) * D;
+        // wavefront w finishes every NW-th of the 16-feature blocks: 4 consecutive features per lane and i
+        uint16_t* op = o + ((size_t)(qo0 + tq) * Hq + kvh * GROUP + c16 % GROUP) * D + f * (D / F);
 #pragma unroll
-        for (int e = 0; e < 8 / NW; ++e) {
-          const int i = (8 / NW) * wave + e;
+        for (int e = 0; e < (NF + NW - 1) / NW; ++e) {
+          const int i = NW * e + wave;
+          if (NF % NW && i >= NF) break;
           float v[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -737,10 +759,10 @@ static int launch_attn(const uint16_t* q, uint16_t* o, const int32_t* qo_indptr,
     // CU, and one streams while the other starts or merges -- a few percent faster than 4 or 1.
     // A batch so small that its workgroups leave CUs empty (at most one per CU) runs with 4
     // wavefronts per workgroup instead: twice the loads in flight per request.
-    auto launch = [&](auto waves_c) -> int {
-      constexpr int kWaves = decltype(waves_c)::value;
-      constexpr int kDecodeLds = kWaves * 32768;
-      auto kern = attn_decode_kernel<GROUP, kWaves>;
+    auto launch = [&](auto waves_c, auto share_c) -> int {
+      constexpr int kWaves = decltype(waves_c)::value, kShare = decltype(share_c)::value;
+      constexpr int kDecodeLds = kWaves * (16384 + 16384 / kShare);
+      auto kern = attn_decode_kernel<GROUP, kWaves, kShare>;
       static bool attr_set = false;  // benign race: the call is idempotent
       if (!attr_set) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -751,11 +773,17 @@ static int launch_attn(const uint16_t* q, uint16_t* o, const int32_t* qo_indptr,
         }
         attr_set = true;
       }
-      kern<<<(int)bound, kWaves * 64, kDecodeLds, stream>>>(q, o, qo_indptr, kv_data, kv_indptr, kv_indices,
+      kern<<<(int)bound * kShare, kWaves * 64, kDecodeLds, stream>>>(q, o, qo_indptr, kv_data, kv_indptr, kv_indices,
                                                             kv_last_page_len, batch, Hq, Hkv, causal, scale_log2);
       return NF_OK;
     };
-    int rc = (long long)batch * Hkv <= 256 ? launch(ic<4>{}) : launch(ic<2>{});
+    // Up to half of the CUs' worth: four or two workgroups share a request and kv head, as many as leave one a CU (beyond that the
+    // K tiles are read for nothing: 24 requests of 8 kv heads 22 us, 30 on two).  1000 keys a request, 8 kv heads: 1 request
+    // 15.7 -> 11.7 us, 8 requests 17.5 -> 13.1, 16 requests 18.9 -> 17.0; 100 keys: 5.2 -> 4.5, 6.0 -> 4.7, 6.3 -> 5.4.
+    // A capped launch keeps its workgroups.
+    const long long items = (long long)batch * Hkv;
+    const int share = num_blocks > 0 ? 1 : items <= 64 ? 4 : items <= 128 ? 2 : 1;
+    int rc = share == 4 ? launch(ic<4>{}, ic<4>{}) : share == 2 ? launch(ic<4>{}, ic<2>{}) : items <= 256 ? launch(ic<4>{}, ic<1>{}) : launch(ic<2>{}, ic<1>{});
     if (rc) return rc;
   } else {
     auto kern = attn_prefill_kernel<GROUP, NQB_PREFILL, kPrefillStages, kPrefillMinWg>;
