@@ -655,7 +655,7 @@ __global__ __launch_bounds__(256, 2) void recur_chunk_out_kernel(nf_recurrence_a
         vr[vt][r] = s.v[(4 * g + r) * C::vPitch + (wave * NVT + vt) * 16 + l16];
         o[vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(at[r], vr[vt][r], o[vt], 0, 0, 0);
       }
-    update_state<KIND, NKT, NVT, true>(S, s, n, ld2, vr);
+    if (t0 + n < ch.n) update_state<KIND, NKT, NVT, true>(S, s, n, ld2, vr);  // what the last step leaves, the scan has
 
     // per-head norm over all columns, gate; through LDS, so that rows are written in whole runs
 #pragma unroll
