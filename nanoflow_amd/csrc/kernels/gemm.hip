@@ -42,14 +42,15 @@ size_t nf_gemm_workspace_bytes(int M, int N, int K) {
   int k_per = 0;
   int shares = splitk_plan(M, N, K, &k_per);
   if (shares < 2) shares = dense_split_plan(M, N, K, &k_per);
+  if (shares < 2 && M <= kMidRows && K >= kDenseSplitMinK) shares = mid_split_plan(M, N, K, kMidBytes).shares;
   return shares < 2 ? 0 : (size_t)shares * M * N * sizeof(float);
 }
 
 size_t nf_gemm_workspace_bytes_upto(int max_M, int N, int K) {
   size_t need = 0;
-  for (int m = 1; m <= max_M && m <= kSplitMaxRows; ++m) need = std::max(need, nf_gemm_workspace_bytes(m, N, K));
+  for (int m = 1; m <= max_M && m <= kMidRows; ++m) need = std::max(need, nf_gemm_workspace_bytes(m, N, K));
   // above that only the two-share split of launches with few 256 x 256 tiles: every count of tile rows
-  for (int m = kSplitMaxRows + 1; m <= max_M; m = (m + 255) / 256 * 256 + 1)
+  for (int m = kMidRows + 1; m <= max_M; m = (m + 255) / 256 * 256 + 1)
     need = std::max(need, nf_gemm_workspace_bytes(std::min((m + 255) / 256 * 256, max_M), N, K));
   return need;
 }

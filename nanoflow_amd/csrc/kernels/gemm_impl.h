@@ -947,10 +947,8 @@ static int cu_count() {
 // as fill them, each at least 512 deep.  Above 256 rows the unsplit launch already fills the chip
 // with 128 x 128 tiles, but those pass the weight bytes through LDS once per 128 rows.  From 257
 // to 320 rows one 320-row tile per column panel passes them once (267 x 10240 x 8192: 72 -> 63 us,
-// 267 x 8192 x 28672: 209 -> 188 us, 267 x 4096 x 4096: 32 -> 28 us).  From 321 to 512 rows two
-// 256-row tiles per panel pass them twice instead of four times, but half of the second tile's
-// MFMAs are padding: measured, that pays for a long contraction only (the down projection), so
-// there the split needs K >= 12288.
+// 267 x 8192 x 28672: 209 -> 188 us, 267 x 4096 x 4096: 32 -> 28 us).  From 321 to 512 rows this is only what a
+// launch of K >= 12288 asks for: it runs as mid_split_plan says, on no more shares.
 // Returns the number of shares (1 = no split) and their depth.
 constexpr int kSplitMaxRows = 512;
 constexpr int kTallRows = 320;  // 257 .. 320 rows: one 320 x 128 tile per column panel
@@ -970,7 +968,8 @@ static int splitk_plan(int M, int N, int K, int* k_per) {
 // (the 8B down projection: 2048 x 4096 x 14336, 128 tiles): two shares of K on 256 x 256 tiles fill
 // the chip, and with K that long the 67 MB of fp32 sums written, read back and added by a second
 // launch cost less than the smaller 128 x 256 tile does (measured with streamed [N][K] weights:
-// 199 us against 211; at K = 4096, the O projection, the split loses: 78 us against 64).
+// 199 us against 211; at K = 4096, the O projection, the split loses: 78 us against 64).  What fp32 sums are stored by,
+// and what other launches ask for above 768 rows.
 constexpr int kDenseSplitMinK = 8192;
 static int dense_split_plan(int M, int N, int K, int* k_per) {
   if (M <= kSplitMaxRows || K < kDenseSplitMinK) return 1;
@@ -978,6 +977,56 @@ static int dense_split_plan(int M, int N, int K, int* k_per) {
   if (t256 * 2 > cu_count() || t256 * 2 <= cu_count() / 2) return 1;
   *k_per = ((K + 1) / 2 + BK - 1) / BK * BK;
   return 2;
+}
+
+// More than 320 rows whose tiles leave CUs idle, which two shares of 256 x 256 answer for few shapes only (640 x 4096 x 14336 ran on
+// 160 tiles of 128 x 128): tile and shares by the time they take, in us -- a tile's start and end, each k of it (slower where the
+// chip is full: the part is at its power cap), and with shares the second launch and the sums written and read.  Fitted to 128 x 128
+// (4 to 256 workgroups), 128 x 256 and 256 x 256 tiles on 336 .. 1536 rows of 2048 .. 8192 columns, 2048 .. 14336 deep; the choice is
+// within 8 % of the fastest there.  Against the unsplit launch: 512 x 2048 x 8192 55 -> 32 us, 640 x 4096 x 14336 124 -> 85, 1024 rows
+// of it 135 -> 114, 448 x 4096 x 8192 60 -> 46, 512 x 2048 x 4096 28 -> 21; 2048 deep and less is never split.
+struct MidPlan {
+  int tile;  // 0: 128 x 128, 1: 128 x 256, 2: 256 x 256
+  int shares, k_per;
+};
+constexpr int kMidRows = 768;                   // up to here, and from kDenseSplitMinK on, a launch asks for the sums' workspace;
+constexpr size_t kMidBytes = (size_t)64 << 20;  // others take what there is for other row counts, up to this
+static MidPlan mid_split_plan(int M, int N, int K, size_t bytes) {
+  constexpr struct {
+    int bm, bn;
+    double ends, per_k, full;
+  } tiles[3] = {{128, 128, 4.5, 0.0065, 0.6}, {128, 256, 3.5, 0.0128, 0.25}, {256, 256, 10.0, 0.0162, 0.6}};
+  MidPlan best{0, 1, K};
+  if (M <= kTallRows || K < 2048) return best;
+  const int cus = cu_count();
+  const size_t sums = (size_t)M * N * sizeof(float);
+  double whole = 1e30, split = 1e30;
+  for (int i = 0; i < 3; ++i) {
+    const auto& t = tiles[i];
+    const long long n = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    auto time = [&](double used, int k) { return t.ends + k * t.per_k * (1.0 + std::max(0.0, used - 0.5) * t.full); };
+    const long long rest = n % cus;
+    whole = std::min(whole, n <= cus ? time((double)n / cus, K) : ((double)(n / cus) + (rest ? 0.47 + 0.53 * (double)rest / cus : 0.0)) * time(1.0, K));
+    for (int s = 2; s <= kMaxShares && n * s <= cus && K / s >= 1024 && s * sums <= std::min(bytes, kMidBytes); ++s) {
+      const int k_per = ((K + s - 1) / s + BK - 1) / BK * BK;
+      const double used = (double)(n * s) / cus;
+      const double us = time(used, k_per) + 3.0 + 0.35e-6 * (double)(s * sums) + (i == 0 && used > 0.9 ? 4.0 : 0.0);
+      if (us < split) {
+        split = us;
+        best = MidPlan{i, (K + k_per - 1) / k_per, k_per};
+      }
+    }
+  }
+  if (split >= 0.95 * whole) best.shares = 1;
+  return best;
+}
+
+template <class E, bool kBCol>
+static int launch_mid(const MidPlan& p, const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha,
+                      float beta, int ldc, float* P, hipStream_t s) {
+  if (p.tile == 0) return launch_splitk<E, 128, 128, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
+  if (p.tile == 1) return launch_splitk<E, 128, 256, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
+  return launch_splitk<E, 256, 256, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
 }
 
 // The same for the fused gate/up pair (tiles of 64 x 128 up to 64 rows, 128 x 128 up to 256,
@@ -1154,9 +1203,9 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
                          size_t workspace_bytes, nf_stream_t stream, bool c_is_row = false) {
   int k_per = 0;
   const bool shape_ok = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && !(b_col_major && rows_pay(M, N, K));
-  int shares = shape_ok ? splitk_plan(M, N, K, &k_per) : 1;
-  const bool dense = shares < 2 && shape_ok && (shares = dense_split_plan(M, N, K, &k_per)) > 1;
-  if (shares < 2 || !workspace || workspace_bytes < (size_t)shares * M * N * sizeof(float))
+  const int shares = shape_ok && M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
+  const MidPlan mid = shape_ok && M > kTallRows && workspace ? mid_split_plan(M, N, K, workspace_bytes) : MidPlan{0, 1, K};
+  if (mid.shares < 2 && (shares < 2 || !workspace || workspace_bytes < (size_t)shares * M * N * sizeof(float)))
     return gemm_entry<E>(who, A, B, C, D, M, N, K, alpha, beta, b_col_major, stream, c_is_row);
   int rc = check_gemm_args(who, A, B, D, M, N, K);
   if (rc) return rc;
@@ -1164,16 +1213,13 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   NF_REQUIRE(((uintptr_t)C) % 8 == 0 && (uintptr_t)workspace % 16 == 0, "%s: C must be 8-byte and the workspace 16-byte aligned", who);
   hipStream_t s = (hipStream_t)stream;
   float* P = static_cast<float*>(workspace);
-  if (dense)
-    return b_col_major ? launch_splitk<E, 256, 256, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
-                       : launch_splitk<E, 256, 256, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
+  if (mid.shares > 1)
+    return b_col_major ? launch_mid<E, true>(mid, A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, P, s)
+                       : launch_mid<E, false>(mid, A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, P, s);
   if (M <= 64) return launch_splitk_64<E>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, b_col_major, s);
-  if (M > 256 && M <= kTallRows)
+  if (M > 256)
     return b_col_major ? launch_splitk<E, 320, 128, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
                        : launch_splitk<E, 320, 128, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
-  if (M > 256)
-    return b_col_major ? launch_splitk<E, 256, 256, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
-                       : launch_splitk<E, 256, 256, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
   return b_col_major ? launch_splitk<E, 128, 128, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
                      : launch_splitk<E, 128, 128, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
 }

@@ -71,6 +71,10 @@ size_t nf_gemm_nk_workspace_bytes_upto(int max_M, int N, int K) {
     const int shares = splitk_plan(m, N, K, &k_per);
     if (shares > 1) need = std::max(need, (size_t)shares * m * N * sizeof(float));
   }
+  for (int m = kTallRows + 1; m <= max_M; ++m) {
+    const int shares = mid_split_plan(m, N, K, kMidBytes).shares;
+    if (shares > 1) need = std::max(need, (size_t)shares * m * N * sizeof(float));
+  }
   return need;
 }
 

@@ -1,0 +1,39 @@
+"""Products of more than 320 rows that are split over K (mid_split_plan in csrc/kernels/gemm_impl.h) against float64, with the bound
+of test_gpu_few_rows.py: one rounding to 16 bits, and K 2^-24 sum |a||b| of fp32 sums."""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+from test_gpu_few_rows import check, operands
+
+SHAPES = [(321, 2048, 4096), (383, 520, 2048), (385, 264, 8200), (512, 2048, 4104), (513, 4096, 14336), (640, 2056, 8192), (767, 1032, 6152),
+          (769, 520, 4096), (1000, 4096, 8192), (1025, 2048, 8200), (1281, 1024, 4096), (1500, 4096, 14336)]
+
+
+@pytest.mark.parametrize("M,N,K_", SHAPES)
+def test_split_products(M, N, K_):
+    from nanoflow_amd import kernels as K
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+    a, b = operands(M, N, K_, torch.float16)
+    want = a.double() @ b.double().t()
+    kn = b.t().contiguous()
+    c, bias = torch.randn(M, N, device="cuda").half(), torch.randn(N, device="cuda").half()
+    for w, col in ((b, True), (kn, False)):
+        got, _ = K.gemm_ws(a, w, b_col_major=col, workspace=ws)
+        check(got, want, a, b, K_, 11)
+        d = c.clone()
+        K.gemm_ws(a, w, d, alpha=0.5, beta=1.0, b_col_major=col, out=d, workspace=ws)
+        check(d, 0.5 * want + c.double(), a, b, K_, 11)
+        check(K.gemm_ws(a, w, bias=bias, beta=1.0, b_col_major=col, workspace=ws)[0], want + bias.double(), a, b, K_, 11)
+        small, _ = K.gemm_ws(a, w, b_col_major=col, workspace=ws[:16])              # no room: unsplit
+        assert torch.equal(small, K.gemm(a, w, b_col_major=col))
+    need = K.lib().nf_gemm_nk_workspace_bytes_upto(M, N, K_)
+    assert K.lib().nf_gemm_workspace_bytes_upto(M, N, K_) <= max(64 << 20, 2 * M * N * 4)
+    a, b = operands(M, N, K_, torch.bfloat16)
+    want = a.double() @ b.double().t()
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    check(K.gemm_nk(a, b, workspace=ws), want, a, b, K_, 8)
+    relu2 = K.gemm_nk(a, b, workspace=ws, act=K.ACT_SQUARED_RELU)
+    lost = 2 * want.abs() * K_ * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t())
+    r = want.clamp(min=0) ** 2
+    assert bool(((relu2.double() - r).abs() <= 2.0 ** -8 * r + 1.1 * lost + 1e-7).all())
