@@ -197,7 +197,7 @@ __device__ __forceinline__ void load16_to_lds(rsrc_t r, uint32_t byte_off, uint3
 // The same with the non-temporal hint: data that is read once (the K and V pages of decode
 // attention) should not displace what the caches hold.  Measured on MI355X for 64 KiB pages read
 // as 256-byte rows: 6.0 -> 6.65 TB/s; for a contiguous stream 6.3 -> 7.07 TB/s.  (Operands that ARE re-read through the caches lose
-// by it: the GEMM kernels run 5-15 % slower with the hint on either operand.)
+// by it: the GEMM kernels run 5-15 % slower with the hint on an operand that several tiles share.)
 __device__ __forceinline__ void load16_to_lds_nt(rsrc_t r, uint32_t byte_off, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
                :: "s"(lds_addr), "v"(byte_off), "s"(r) : "memory", "m0");

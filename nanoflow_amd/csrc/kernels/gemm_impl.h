@@ -165,9 +165,11 @@ __device__ __forceinline__ float swiglu_rounded(float g_acc, float u_acc) {
 // operands (A, and [N][K] weights): equal for a whole GEMM, K < lda for one share of a GEMM split
 // over K, whose operand pointers already point at the share's first k.
 // kPartial: the fp32 sums are stored as they are to D taken as float [M][N] (no alpha, beta, C).
+// kOnce (kBCol only): the weights carry the non-temporal hint.
 // kGroup (kBCol only): operands of one group of a grouped product -- the weights' row stride is ldb, D's is
 // ldd, and where a_rows is not null row m of A is row a_rows[m] of a matrix of a_total rows.
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kPartial = false, bool kGroup = false, int kCap = kWholeCu>
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kPartial = false, bool kGroup = false, int kCap = kWholeCu,
+          bool kOnce = false>
 __device__ __forceinline__ void gemm_tile(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
@@ -287,7 +289,7 @@ __device__ __forceinline__ void gemm_tile(
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       constexpr int dst = b * SM::b_bytes + tt * NW * 1024;
       if constexpr (kBCol) {
-        load16_to_lds<dst>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
+        load16_to_lds<dst, kOnce>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
         b_off[b][tt] += BK * 2;
       } else {
         load16_to_lds<dst>(b_rsrc[b], b_off[b][tt], lb);
@@ -321,7 +323,7 @@ __device__ __forceinline__ void gemm_tile(
       load16_to_lds<t * NW * 1024>(a_rsrc, pend, la);
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
-      load16_to_lds<b * SM::b_bytes + tt * NW * 1024>(b_rsrc[b], pend, lb);
+      load16_to_lds<b * SM::b_bytes + tt * NW * 1024, kOnce>(b_rsrc[b], pend, lb);
     }
   };
   auto load_slab = [&](int stage, int k0) {  // every load of one slab, back to back (one ring for both operands)
@@ -756,14 +758,14 @@ __device__ __forceinline__ bool xcd_tile(int bid, int tiles_m, int tiles_n, int*
   return true;
 }
 
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol>
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kOnce = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_f16_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
     int M, int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n) {
   int tm, tn;
   if (!xcd_tile(blockIdx.x, tiles_m, tiles_n, &tm, &tn)) return;
-  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tm * BM, tn * BN, K);
+  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, false, false, kWholeCu, kOnce>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tm * BM, tn * BN, K);
 }
 
 // Two tile heights in one launch, for shapes whose 256-row tiles fill the 256 CUs a whole number
@@ -887,22 +889,30 @@ static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1
                        uint16_t* D, int M, int N, int K, float alpha, float beta, int ldc,
                        hipStream_t stream) {
   using SM = GemmSmem<BM, BN, kDual ? 2 : 1>;
-  auto kern = gemm_f16_kernel<E, BM, BN, WM, WN, kDual, kBCol>;
-  static bool attr_set = false;  // benign race: the call is idempotent
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)SM::bytes);
-    if (e != hipSuccess) {
-      set_error("gemm: cannot reserve %zu bytes of LDS: %s", SM::bytes, hipGetErrorString(e));
-      return NF_ERR_RUNTIME;
-    }
-    attr_set = true;
-  }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int ntiles = tiles_m * tiles_n;
   const int grid = ((ntiles + 7) / 8) * 8;
-  kern<<<grid, WM * WN * 64, SM::bytes, stream>>>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tiles_m, tiles_n);
-  return check_launch("gemm launch");
+  auto go = [&](auto once_c) {
+    auto kern = gemm_f16_kernel<E, BM, BN, WM, WN, kDual, kBCol, decltype(once_c)::value>;
+    static bool attr_set = false;  // benign race: the call is idempotent
+    if (!attr_set) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)SM::bytes);
+      if (e != hipSuccess) {
+        set_error("gemm: cannot reserve %zu bytes of LDS: %s", SM::bytes, hipGetErrorString(e));
+        return NF_ERR_RUNTIME;
+      }
+      attr_set = true;
+    }
+    kern<<<grid, WM * WN * 64, SM::bytes, stream>>>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tiles_m, tiles_n);
+    return check_launch("gemm launch");
+  };
+  // One row of tiles reads the weights once: with the non-temporal hint (200 x 128256 x 4096: 258 -> 238 us, 66 x 28672 x 8192: 109
+  // -> 96, pairs of it 181 -> 167).  Several rows of tiles share them through the caches, which the hint defeats, and shares of a
+  // split read runs of a row too short for it (128 x 4096 x 4096 in 8: 19 us, 24 with it).
+  if constexpr (kBCol)
+    if (tiles_m == 1) return go(std::true_type{});
+  return go(std::false_type{});
 }
 
 template <class E, int BN, bool kDual, bool kBCol>

@@ -37,3 +37,18 @@ def test_split_products(M, N, K_):
     lost = 2 * want.abs() * K_ * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t())
     r = want.clamp(min=0) ** 2
     assert bool(((relu2.double() - r).abs() <= 2.0 ** -8 * r + 1.1 * lost + 1e-7).all())
+
+
+@pytest.mark.parametrize("M,N,K_", [(65, 520, 512), (128, 4104, 968), (127, 33000, 136), (129, 66008, 72), (200, 65544, 328), (256, 49160, 64), (64, 264, 1000)])
+def test_one_row_of_tiles(M, N, K_):
+    """Unsplit launches whose tiles share no weights: those are read with a hint of their own."""
+    from nanoflow_amd import kernels as K
+    a, b = operands(M, N, K_, torch.float16)
+    check(K.gemm(a, b, b_col_major=True), a.double() @ b.double().t(), a, b, K_, 11)
+    half = N // 16 * 8
+    g, u = b[:half].contiguous(), b[half:2 * half].contiguous()
+    p, q = a.double() @ g.double().t(), a.double() @ u.double().t()
+    pair = torch.nn.functional.silu(p.half().double()) * q.half().double()
+    lost = lambda r, w: 2.0 ** -11 * r.abs() + K_ * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
+    got = K.dual_swiglu(a, g, u, b_col_major=True)
+    assert bool(((got.double() - pair).abs() <= 1.1 * q.abs() * lost(p, g) + p.abs() * lost(q, u) + 2.0 ** -10 * pair.abs() + 1e-6).all())
