@@ -119,6 +119,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_rows_kernel(nf_grouped_gemm_
 template <class E, bool kSpread>
 int launch_grouped_rows(const nf_grouped_gemm_args& a, hipStream_t s) {
   constexpr int lds = RowsSmem<kFewRows, 2, 4, 1, 2>::bytes;
+  static_assert(GemmSmem<128, 32, 1, kHalfCu>::bytes <= lds, "the other tile runs in the same LDS");
   auto kern = gemm_grouped_rows_kernel<E, kSpread>;
   static bool attr_set = false;  // benign race: the call is idempotent
   if (!attr_set) {

@@ -334,7 +334,7 @@ def gemm(A, B, Cmat=None, alpha=1.0, beta=0.0, b_col_major=False, out=None, bias
 def gemm_ws(A, B, Cmat=None, alpha=1.0, beta=0.0, b_col_major=False, out=None, workspace=None, bias=None):
     """nf_gemm_f16_ws: fp16 GEMM that is split over K through a workspace when few rows against a narrow
     N would leave most of the chip idle.  Returns (out, shares_bytes) where shares_bytes is the
-    workspace the shape asked for (0: not split)."""
+    workspace the shape asked for (0: none)."""
     _f16(A); _f16(B)
     M, K = A.shape
     N = B.shape[0] if b_col_major else B.shape[1]
