@@ -77,11 +77,11 @@ NF_API int nf_gemm_f16(const uint16_t* A, const uint16_t* B, const uint16_t* C, 
 
 /* nf_gemm_f16 with scratch: a GEMM whose output tiles would leave most of the chip idle (few rows
  * against a narrow N: the QKV, O and down projections of a small decode batch; up to 320 rows any
- * contraction of 1024 or more, above that those of 2048 or more that profit) is split over K into
- * shares that fill it, summed in fp32 through `workspace`, 16-byte aligned.
- * nf_gemm_workspace_bytes(M, N, K) is what a shape asks for: 0 = none, where it is not split (up to 320
- * rows) or only gains with a workspace of up to 64 MiB that is there for other row counts.  With a
- * null or short workspace, or a shape that does not profit, it is nf_gemm_f16.  The sum over k is
+ * contraction of 1024 or more, up to 512 rows those of 12288 or more, above that those of 8192 or
+ * more) is split over K into shares that fill it, summed in fp32 through `workspace`
+ * (nf_gemm_workspace_bytes(M, N, K) bytes, 16-byte aligned; 0 = this shape is not split and the
+ * workspace is not touched).  Tile and shares depend on the shape alone: a larger workspace changes
+ * nothing.  With a null or short workspace, or a shape that does not profit, it is nf_gemm_f16.  The sum over k is
  * then taken share by share, so results differ from nf_gemm_f16 in fp32 rounding only.
  * nf_gemm_workspace_bytes_upto(max_M, N, K): the largest requirement over 1..max_M rows.
  * No counterpart in the reference (its serial split-K is a tag field of the CUTLASS kernel,
@@ -101,8 +101,8 @@ NF_API int nf_gemm_f16_ws(const uint16_t* A, const uint16_t* B, const uint16_t* 
  * split run as nf_gemm_f16 and never touch the array.  Nothing in the array has to start at zero
  * (every share overwrites its sums before the reduction reads them), but all calls on one device
  * share it: calls that overlap in time on one device (two streams) race.
- * Results are bit-identical to nf_gemm_f16_ws with a workspace of nf_gemm_workspace_bytes(), except where that splits
- * contractions below 12288 of more than 320 rows, or more than 512 rows: those run unsplit here.
+ * Results are bit-identical to nf_gemm_f16_ws with a workspace of nf_gemm_workspace_bytes() up to 512 rows;
+ * more rows run unsplit here.
  * No counterpart in the reference. */
 NF_API int nf_gemm_f16_noalloc(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N,
                                int K, float alpha, float beta, int b_col_major, nf_stream_t stream);

@@ -38,12 +38,7 @@ int nf_gemm_f16(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_
 }
 
 size_t nf_gemm_workspace_bytes(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  int k_per = 0;
-  int shares = splitk_plan(M, N, K, &k_per);
-  if (shares < 2) shares = dense_split_plan(M, N, K, &k_per);
-  if (shares < 2 && M <= kMidRows && K >= kDenseSplitMinK) shares = mid_split_plan(M, N, K, kMidBytes).shares;
-  return shares < 2 ? 0 : (size_t)shares * M * N * sizeof(float);
+  return M <= 0 || N <= 0 || K <= 0 ? 0 : split_bytes(M, N, K, nullptr);
 }
 
 size_t nf_gemm_workspace_bytes_upto(int max_M, int N, int K) {
@@ -85,11 +80,8 @@ int nf_gemm_f16_ws(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint
 
 int nf_gemm_f16_noalloc(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K,
                         float alpha, float beta, int b_col_major, nf_stream_t stream) {
-  // the few-row split only: the two-share split of dense launches is an optimisation that needs more
-  // than the array holds at any shape it applies to, and such a launch runs unsplit here
-  int k_per = 0;
-  const int few = M > 0 && N > 0 && K > 0 ? splitk_plan(M, N, K, &k_per) : 1;
-  const size_t need = few < 2 ? 0 : (size_t)few * M * N * sizeof(float);
+  // up to 512 rows only: more rows run unsplit here, though the array would hold the sums of some of them
+  const size_t need = M > 0 && N > 0 && K > 0 && M <= kSplitMaxRows ? split_bytes(M, N, K, nullptr) : 0;
   NF_REQUIRE(need <= kStaticScratchBytes,
              "nf_gemm_f16_noalloc: %d x %d x %d is split over K through %zu bytes of partial sums; the static "
              "scratch array holds %zu (use nf_gemm_f16_ws with a workspace of your own, or nf_gemm_f16)",

@@ -957,8 +957,8 @@ static int cu_count() {
 // as fill them, each at least 512 deep.  Above 256 rows the unsplit launch already fills the chip
 // with 128 x 128 tiles, but those pass the weight bytes through LDS once per 128 rows.  From 257
 // to 320 rows one 320-row tile per column panel passes them once (267 x 10240 x 8192: 72 -> 63 us,
-// 267 x 8192 x 28672: 209 -> 188 us, 267 x 4096 x 4096: 32 -> 28 us).  From 321 to 512 rows this is only what a
-// launch of K >= 12288 asks for: it runs as mid_split_plan says, on no more shares.
+// 267 x 8192 x 28672: 209 -> 188 us, 267 x 4096 x 4096: 32 -> 28 us).  From 321 to 512 rows, and only for
+// K >= 12288, this is how much workspace a launch asks for: it runs as mid_split_plan says, on no more shares.
 // Returns the number of shares (1 = no split) and their depth.
 constexpr int kSplitMaxRows = 512;
 constexpr int kTallRows = 320;  // 257 .. 320 rows: one 320 x 128 tile per column panel
@@ -978,8 +978,8 @@ static int splitk_plan(int M, int N, int K, int* k_per) {
 // (the 8B down projection: 2048 x 4096 x 14336, 128 tiles): two shares of K on 256 x 256 tiles fill
 // the chip, and with K that long the 67 MB of fp32 sums written, read back and added by a second
 // launch cost less than the smaller 128 x 256 tile does (measured with streamed [N][K] weights:
-// 199 us against 211; at K = 4096, the O projection, the split loses: 78 us against 64).  What fp32 sums are stored by,
-// and what other launches ask for above 768 rows.
+// 199 us against 211; at K = 4096, the O projection, the split loses: 78 us against 64).  What fp32 sums are stored by, and
+// how much workspace other launches ask for: those run as mid_split_plan says.
 constexpr int kDenseSplitMinK = 8192;
 static int dense_split_plan(int M, int N, int K, int* k_per) {
   if (M <= kSplitMaxRows || K < kDenseSplitMinK) return 1;
@@ -994,13 +994,12 @@ static int dense_split_plan(int M, int N, int K, int* k_per) {
 // chip is full: the part is at its power cap), and with shares the second launch and the sums written and read.  Fitted to 128 x 128
 // (4 to 256 workgroups), 128 x 256 and 256 x 256 tiles on 336 .. 1536 rows of 2048 .. 8192 columns, 2048 .. 14336 deep; the choice is
 // within 8 % of the fastest there.  Against the unsplit launch: 512 x 2048 x 8192 55 -> 32 us, 640 x 4096 x 14336 124 -> 85, 1024 rows
-// of it 135 -> 114, 448 x 4096 x 8192 60 -> 46, 512 x 2048 x 4096 28 -> 21; 2048 deep and less is never split.
+// of it 135 -> 114, 448 x 4096 x 8192 60 -> 46, 512 x 2048 x 4096 28 -> 21; 2048 deep and less is never split.  `bytes`: what the sums may take, a function of the shape and never of the workspace at hand.
 struct MidPlan {
   int tile;  // 0: 128 x 128, 1: 128 x 256, 2: 256 x 256
   int shares, k_per;
 };
-constexpr int kMidRows = 768;                   // up to here, and from kDenseSplitMinK on, a launch asks for the sums' workspace;
-constexpr size_t kMidBytes = (size_t)64 << 20;  // others take what there is for other row counts, up to this
+constexpr size_t kMidBytes = (size_t)64 << 20;
 static MidPlan mid_split_plan(int M, int N, int K, size_t bytes) {
   constexpr struct {
     int bm, bn;
@@ -1029,6 +1028,27 @@ static MidPlan mid_split_plan(int M, int N, int K, size_t bytes) {
   }
   if (split >= 0.95 * whole) best.shares = 1;
   return best;
+}
+
+// What the fp16 entries split, and the bytes of sums that it takes: 0 = never split, the workspace is not touched.  Up to 512 rows
+// what splitk_plan says, above that what dense_split_plan says and, up to kMidRows rows, long contractions of other launches.
+// From 321 rows on `mid` (may be null) has the tile and shares: mid_split_plan within those bytes.
+constexpr int kMidRows = 768;
+static size_t split_bytes(int M, int N, int K, MidPlan* mid) {
+  const size_t sums = (size_t)M * N * sizeof(float);
+  int k_per = 0;
+  MidPlan plan{0, 1, K};
+  size_t bytes = 0;
+  const int shares = M <= kSplitMaxRows ? splitk_plan(M, N, K, &k_per) : dense_split_plan(M, N, K, &k_per);
+  if (shares > 1) {
+    bytes = shares * sums;
+    if (M > kTallRows) plan = mid_split_plan(M, N, K, bytes);
+  } else if (M > kSplitMaxRows && M <= kMidRows && K >= kDenseSplitMinK) {
+    plan = mid_split_plan(M, N, K, kMidBytes);
+    if (plan.shares > 1) bytes = plan.shares * sums;
+  }
+  if (mid) *mid = plan;
+  return bytes;
 }
 
 template <class E, bool kBCol>
@@ -1211,12 +1231,13 @@ template <class E>
 static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D,
                          int M, int N, int K, float alpha, float beta, int b_col_major, void* workspace,
                          size_t workspace_bytes, nf_stream_t stream, bool c_is_row = false) {
-  int k_per = 0;
   const bool shape_ok = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && !(b_col_major && rows_pay(M, N, K));
-  const int shares = shape_ok && M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
-  const MidPlan mid = shape_ok && M > kTallRows && workspace ? mid_split_plan(M, N, K, workspace_bytes) : MidPlan{0, 1, K};
-  if (mid.shares < 2 && (shares < 2 || !workspace || workspace_bytes < (size_t)shares * M * N * sizeof(float)))
+  MidPlan mid{0, 1, K};
+  const size_t need = shape_ok ? split_bytes(M, N, K, &mid) : 0;
+  if (need == 0 || !workspace || workspace_bytes < need || (M > kTallRows && mid.shares < 2))
     return gemm_entry<E>(who, A, B, C, D, M, N, K, alpha, beta, b_col_major, stream, c_is_row);
+  int k_per = 0;
+  const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
   int rc = check_gemm_args(who, A, B, D, M, N, K);
   if (rc) return rc;
   NF_REQUIRE(beta == 0.f || C, "%s: beta=%g needs C", who, (double)beta);

@@ -17,9 +17,10 @@ static int gemm_nk_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   hipStream_t s = (hipStream_t)stream;
   if (rows_pay(M, N, K)) return dispatch_rows<E, false>(A, B, bias, D, M, N, K, 1.f, beta, ldc, s);
   if (workspace && M > kTallRows) {
-    const MidPlan mid = mid_split_plan(M, N, K, workspace_bytes);
+    const MidPlan mid = mid_split_plan(M, N, K, kMidBytes);
     NF_REQUIRE(mid.shares < 2 || (uintptr_t)workspace % 16 == 0, "%s: the workspace must be 16-byte aligned", who);
-    if (mid.shares > 1) return launch_mid<E, true>(mid, A, B, bias, D, M, N, K, 1.f, beta, ldc, static_cast<float*>(workspace), s);
+    if (mid.shares > 1 && workspace_bytes >= (size_t)mid.shares * M * N * sizeof(float))
+      return launch_mid<E, true>(mid, A, B, bias, D, M, N, K, 1.f, beta, ldc, static_cast<float*>(workspace), s);
   }
   int k_per = 0;
   const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;

@@ -39,6 +39,40 @@ def test_split_products(M, N, K_):
     assert bool(((relu2.double() - r).abs() <= 2.0 ** -8 * r + 1.1 * lost + 1e-7).all())
 
 
+@pytest.mark.parametrize("col", [True, False])
+@pytest.mark.parametrize("M,N,K_", [(321, 2048, 4096), (400, 4096, 8192), (400, 4096, 14336), (512, 2048, 4104), (600, 1024, 4096), (640, 2056, 8192),
+                                    (640, 4096, 14336), (769, 520, 4096), (1024, 4096, 14336), (1500, 4096, 14336)])
+def test_workspace_beyond_what_a_shape_asks_for_changes_nothing(M, N, K_, col):
+    """nf_gemm_workspace_bytes is the whole contract: 0 = the workspace is not touched, and bytes past the ones asked for neither."""
+    from nanoflow_amd import kernels as K
+    a, b = operands(M, N, K_, torch.float16)
+    w = b if col else b.t().contiguous()
+    need = K.lib().nf_gemm_workspace_bytes(M, N, K_)
+    ws = torch.full(((96 << 20) + 16,), 0x5a, dtype=torch.uint8, device="cuda")
+    big, _ = K.gemm_ws(a, w, b_col_major=col, workspace=ws)
+    untouched = bool((ws[need:] == 0x5a).all())
+    assert untouched
+    exact = K.gemm_ws(a, w, b_col_major=col, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))[0] if need else K.gemm(a, w, b_col_major=col)
+    assert torch.equal(big, exact)
+    ab, bb = a.bfloat16(), b.bfloat16()                          # the bf16 entry: two sizes that both suffice
+    upto = K.lib().nf_gemm_nk_workspace_bytes_upto(M, N, K_)
+    assert torch.equal(K.gemm_nk(ab, bb, workspace=ws), K.gemm_nk(ab, bb, workspace=torch.empty(max(upto, 16), dtype=torch.uint8, device="cuda")))
+
+
+@pytest.mark.parametrize("col", [True, False])
+@pytest.mark.parametrize("M,N,K_", [(321, 2048, 4096), (330, 256, 12288), (383, 520, 16384), (400, 2048, 8192), (400, 1024, 14336), (512, 2048, 4104), (512, 512, 14336)])
+def test_products_without_a_workspace_of_the_callers(M, N, K_, col):
+    """nf_gemm_f16_noalloc has the bits of nf_gemm_f16_ws up to 512 rows."""
+    from nanoflow_amd import kernels as K
+    l = K.lib()
+    assert l.nf_gemm_workspace_bytes(M, N, K_) <= l.nf_gemm_noalloc_scratch_bytes()
+    a, b = operands(M, N, K_, torch.float16)
+    w = b if col else b.t().contiguous()
+    out = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    assert l.nf_gemm_f16_noalloc(a.data_ptr(), w.data_ptr(), None, out.data_ptr(), M, N, K_, 1.0, 0.0, int(col), torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out, K.gemm_ws(a, w, b_col_major=col)[0])
+
+
 @pytest.mark.parametrize("M,N,K_", [(65, 520, 512), (128, 4104, 968), (127, 33000, 136), (129, 66008, 72), (200, 65544, 328), (256, 49160, 64), (64, 264, 1000)])
 def test_one_row_of_tiles(M, N, K_):
     """Unsplit launches whose tiles share no weights: those are read with a hint of their own."""
