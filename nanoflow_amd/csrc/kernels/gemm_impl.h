@@ -994,7 +994,8 @@ static int dense_split_plan(int M, int N, int K, int* k_per) {
 // chip is full: the part is at its power cap), and with shares the second launch and the sums written and read.  Fitted to 128 x 128
 // (4 to 256 workgroups), 128 x 256 and 256 x 256 tiles on 336 .. 1536 rows of 2048 .. 8192 columns, 2048 .. 14336 deep; the choice is
 // within 8 % of the fastest there.  Against the unsplit launch: 512 x 2048 x 8192 55 -> 32 us, 640 x 4096 x 14336 124 -> 85, 1024 rows
-// of it 135 -> 114, 448 x 4096 x 8192 60 -> 46, 512 x 2048 x 4096 28 -> 21; 2048 deep and less is never split.  `bytes`: what the sums may take, a function of the shape and never of the workspace at hand.
+// of it 135 -> 114, 448 x 4096 x 8192 60 -> 46, 512 x 2048 x 4096 28 -> 21; 2048 deep and less is never split (448 x 2048 x 2048: 17.4 us
+// in two shares, 15.9 whole).  `bytes`: what the sums may take, a function of the shape and never of the workspace at hand.
 struct MidPlan {
   int tile;  // 0: 128 x 128, 1: 128 x 256, 2: 256 x 256
   int shares, k_per;
@@ -1006,7 +1007,7 @@ static MidPlan mid_split_plan(int M, int N, int K, size_t bytes) {
     double ends, per_k, full;
   } tiles[3] = {{128, 128, 4.5, 0.0065, 0.6}, {128, 256, 3.5, 0.0128, 0.25}, {256, 256, 10.0, 0.0162, 0.6}};
   MidPlan best{0, 1, K};
-  if (M <= kTallRows || K < 2048) return best;
+  if (M <= kTallRows || K <= 2048) return best;
   const int cus = cu_count();
   const size_t sums = (size_t)M * N * sizeof(float);
   double whole = 1e30, split = 1e30;

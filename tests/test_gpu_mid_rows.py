@@ -59,6 +59,13 @@ def test_workspace_beyond_what_a_shape_asks_for_changes_nothing(M, N, K_, col):
     assert torch.equal(K.gemm_nk(ab, bb, workspace=ws), K.gemm_nk(ab, bb, workspace=torch.empty(max(upto, 16), dtype=torch.uint8, device="cuda")))
 
 
+@pytest.mark.parametrize("M,N", [(321, 2048), (448, 2048), (512, 1024)])
+def test_contractions_of_2048_are_not_split(M, N):
+    from nanoflow_amd import kernels as K
+    a, b = operands(M, N, 2048, torch.bfloat16)
+    assert torch.equal(K.gemm_nk(a, b, workspace=torch.empty(64 << 20, dtype=torch.uint8, device="cuda")), K.gemm_nk(a, b))
+
+
 @pytest.mark.parametrize("col", [True, False])
 @pytest.mark.parametrize("M,N,K_", [(321, 2048, 4096), (330, 256, 12288), (383, 520, 16384), (400, 2048, 8192), (400, 1024, 14336), (512, 2048, 4104), (512, 512, 14336)])
 def test_products_without_a_workspace_of_the_callers(M, N, K_, col):
