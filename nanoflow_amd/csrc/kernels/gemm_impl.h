@@ -1232,17 +1232,19 @@ template <class E>
 static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D,
                          int M, int N, int K, float alpha, float beta, int b_col_major, void* workspace,
                          size_t workspace_bytes, nf_stream_t stream, bool c_is_row = false) {
-  const bool shape_ok = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && !(b_col_major && rows_pay(M, N, K));
   MidPlan mid{0, 1, K};
-  const size_t need = shape_ok ? split_bytes(M, N, K, &mid) : 0;
-  if (need == 0 || !workspace || workspace_bytes < need || (M > kTallRows && mid.shares < 2))
-    return gemm_entry<E>(who, A, B, C, D, M, N, K, alpha, beta, b_col_major, stream, c_is_row);
+  const size_t need = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 ? split_bytes(M, N, K, &mid) : 0;
+  const bool given = need > 0 && workspace && workspace_bytes >= need, aligned = (uintptr_t)workspace % 16 == 0;
   int k_per = 0;
+  // a workspace for the sums of at most 512 rows, or of a dense launch, has to be aligned, whatever runs; others run unsplit without
+  NF_REQUIRE(!given || aligned || (M > kSplitMaxRows && dense_split_plan(M, N, K, &k_per) < 2), "%s: the workspace must be 16-byte aligned", who);
+  const bool whole = M > kTallRows ? mid.shares < 2 : b_col_major && rows_pay(M, N, K);
+  if (!given || !aligned || whole) return gemm_entry<E>(who, A, B, C, D, M, N, K, alpha, beta, b_col_major, stream, c_is_row);
   const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
   int rc = check_gemm_args(who, A, B, D, M, N, K);
   if (rc) return rc;
   NF_REQUIRE(beta == 0.f || C, "%s: beta=%g needs C", who, (double)beta);
-  NF_REQUIRE(((uintptr_t)C) % 8 == 0 && (uintptr_t)workspace % 16 == 0, "%s: C must be 8-byte and the workspace 16-byte aligned", who);
+  NF_REQUIRE(((uintptr_t)C) % 8 == 0, "%s: C must be 8-byte aligned", who);
   hipStream_t s = (hipStream_t)stream;
   float* P = static_cast<float*>(workspace);
   if (mid.shares > 1)
@@ -1290,12 +1292,14 @@ static int dual_ws_entry(const char* who, const uint16_t* A, const uint16_t* Bga
                          uint16_t* out, int M, int N, int K, void* workspace, size_t workspace_bytes,
                          nf_stream_t stream) {
   int k_per = 0;
-  const int shares = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && !rows_pay_dual(M, 2 * K, kBCol) ? splitk_plan_dual(M, N, K, &k_per) : 1;
-  if (shares < 2 || !workspace || workspace_bytes < (size_t)2 * shares * M * N * sizeof(float))
+  const int shares = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 ? splitk_plan_dual(M, N, K, &k_per) : 1;
+  const bool given = shares > 1 && workspace && workspace_bytes >= (size_t)2 * shares * M * N * sizeof(float);
+  NF_REQUIRE(!given || (uintptr_t)workspace % 16 == 0, "%s: the workspace must be 16-byte aligned", who);
+  if (!given || rows_pay_dual(M, 2 * K, kBCol))
     return dual_entry<E, kBCol>(who, A, Bgate, Bup, out, M, N, K, stream);
   int rc = check_gemm_args(who, A, Bgate, out, M, N, K);
   if (rc) return rc;
-  NF_REQUIRE(Bup && ((uintptr_t)Bup | (uintptr_t)workspace) % 16 == 0, "%s: Bup and the workspace must be 16-byte aligned", who);
+  NF_REQUIRE(Bup && ((uintptr_t)Bup) % 16 == 0, "%s: Bup must be 16-byte aligned", who);
   hipStream_t s = (hipStream_t)stream;
   float* P = static_cast<float*>(workspace);
   if (M <= 64)

@@ -15,18 +15,17 @@ static int gemm_nk_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   const int ldc = bias ? 0 : N;
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
+  int k_per = 0;
+  const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
+  const bool aligned = (uintptr_t)workspace % 16 == 0, given = shares > 1 && workspace && workspace_bytes >= (size_t)shares * M * N * sizeof(float);
+  NF_REQUIRE(!given || aligned, "%s: the workspace must be 16-byte aligned", who);  // whatever runs
   if (rows_pay(M, N, K)) return dispatch_rows<E, false>(A, B, bias, D, M, N, K, 1.f, beta, ldc, s);
-  if (workspace && M > kTallRows) {
+  if (workspace && aligned && M > kTallRows) {
     const MidPlan mid = mid_split_plan(M, N, K, kMidBytes);
-    NF_REQUIRE(mid.shares < 2 || (uintptr_t)workspace % 16 == 0, "%s: the workspace must be 16-byte aligned", who);
     if (mid.shares > 1 && workspace_bytes >= (size_t)mid.shares * M * N * sizeof(float))
       return launch_mid<E, true>(mid, A, B, bias, D, M, N, K, 1.f, beta, ldc, static_cast<float*>(workspace), s);
   }
-  int k_per = 0;
-  const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
-  if (shares < 2 || !workspace || workspace_bytes < (size_t)shares * M * N * sizeof(float))
-    return dispatch_plain<E, true>(A, B, bias, D, M, N, K, 1.f, beta, ldc, s);
-  NF_REQUIRE((uintptr_t)workspace % 16 == 0, "%s: the workspace must be 16-byte aligned", who);
+  if (!given) return dispatch_plain<E, true>(A, B, bias, D, M, N, K, 1.f, beta, ldc, s);
   float* P = static_cast<float*>(workspace);
   if (M <= 64) return launch_splitk_64<E>(A, B, bias, D, M, N, K, 1.f, beta, ldc, shares, k_per, P, true, s);
   if (M > 256) return launch_splitk<E, 320, 128, 2, 2, true>(A, B, bias, D, M, N, K, 1.f, beta, ldc, shares, k_per, P, s);

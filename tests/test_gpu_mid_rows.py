@@ -66,6 +66,31 @@ def test_contractions_of_2048_are_not_split(M, N):
     assert torch.equal(K.gemm_nk(a, b, workspace=torch.empty(64 << 20, dtype=torch.uint8, device="cuda")), K.gemm_nk(a, b))
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 4096, 4096), (16, 2048, 2048), (33, 4096, 14336), (64, 4096, 4096), (200, 2048, 4096), (300, 4096, 4096), (400, 1024, 14336),
+                                    (400, 2048, 4096), (640, 4096, 14336), (1024, 4096, 14336), (1500, 4096, 14336)])
+def test_a_workspace_that_is_not_aligned(M, N, K_):
+    """Refused where it would hold sums (up to 512 rows whatever the launch runs on, and of dense launches); else not looked at."""
+    from nanoflow_amd import kernels as K
+    a, b = operands(M, N, K_, torch.float16)
+    ws = torch.empty((96 << 20) + 8, dtype=torch.uint8, device="cuda")[8:]
+    asked = K.lib().nf_gemm_workspace_bytes(M, N, K_) > 0
+    for w, col in ((b, True), (b.t().contiguous(), False)):
+        if asked and not 512 < M <= 768:
+            with pytest.raises(K.NanoflowKernelError, match="aligned"):
+                K.gemm_ws(a, w, b_col_major=col, workspace=ws)
+        else:
+            assert torch.equal(K.gemm_ws(a, w, b_col_major=col, workspace=ws)[0], K.gemm(a, w, b_col_major=col))
+        if K.lib().nf_dual_swiglu_workspace_bytes(M, N, K_):
+            with pytest.raises(K.NanoflowKernelError, match="aligned"):
+                K.dual_swiglu_ws(a, w, w, b_col_major=col, workspace=ws)
+    ab, bb = a.bfloat16(), b.bfloat16()
+    if asked and M <= 320:
+        with pytest.raises(K.NanoflowKernelError, match="aligned"):
+            K.gemm_nk(ab, bb, workspace=ws)
+    else:
+        assert torch.equal(K.gemm_nk(ab, bb, workspace=ws), K.gemm_nk(ab, bb))
+
+
 @pytest.mark.parametrize("col", [True, False])
 @pytest.mark.parametrize("M,N,K_", [(321, 2048, 4096), (330, 256, 12288), (383, 520, 16384), (400, 2048, 8192), (400, 1024, 14336), (512, 2048, 4104), (512, 512, 14336)])
 def test_products_without_a_workspace_of_the_callers(M, N, K_, col):
