@@ -200,11 +200,13 @@ int dispatch_grouped(const nf_grouped_gemm_args& a, int tile_rows, hipStream_t s
 
 extern "C" {
 
-// Rows of an m tile: what the routing's tile list has to be made for.  (748 rows, 5 of 32 experts and 8 identities of 2048 x 2048,
-// 117 slots an expert: 77 us on 64 rows, 92 on 128.)
+// Rows of an m tile: what the routing's tile list has to be made for.  From 96 slots an expert on most experts have more than 64 rows, and two
+// tiles of 64 pass their weights twice.  us on 128 / 64 rows: 32 experts of 4096 x 3584 at 100 slots 186 / 219 and at 117 223 / 253, 8 of
+// 4096 x 4096 at 117 76 / 106, 32 of 2048 x 2560 at 110 109 / 118; 2048 deep and less 64 rows win up to 120 (2048 x 2048 at 117 95 / 84),
+// but the list is made before the contraction is known.
 int nf_grouped_tile_rows(int dtype, int rows, int groups) {
   if (dtype == NF_F32) return kF32Tile;
-  return (long long)rows <= 120ll * std::max(groups, 1) ? 64 : 128;
+  return (long long)rows <= 96ll * std::max(groups, 1) ? 64 : 128;
 }
 
 int nf_gemm_grouped(const nf_grouped_gemm_args* args, nf_stream_t stream) {

@@ -141,3 +141,11 @@ def test_nanobatch_split_and_attention_groups_are_checked_on_the_host():
     assert grp(LOCAL, 640, 256, 768, 1000, g(300, 340, 360, 0)) == 0     # two-way: only the 0+1 rule
     assert grp(SEQ, 0, 0, 0, 1000, g(1000, 0, 0, 0)) == 0
     assert grp(PLLM, 640, 256, 768, 1000, None) == -1
+
+
+def test_rows_of_an_experts_tile_without_a_gpu():
+    """The tile list of a routing: 64 rows up to 96 sorted rows an expert on average, then 128; fp32 has one tile."""
+    from nanoflow_amd import kernels as K
+    rows = K.lib().nf_grouped_tile_rows
+    assert [rows(K.BF16, n, 32) for n in (1, 96 * 32, 96 * 32 + 1, 117 * 32, 120 * 32, 5000)] == [64, 64, 128, 128, 128, 128]
+    assert len({rows(K.F32, n, 32) for n in (1, 4000)}) == 1
