@@ -182,8 +182,11 @@ int dispatch_grouped(const nf_grouped_gemm_args& a, int tile_rows, hipStream_t s
     //   2048 x 2048   19 -> 13   59 -> 46    65 -> 47    66 -> 56
     //   4096 x 3584   44 -> 21  136 -> 116  159 -> 139  165 -> 185: not taken
     // 64 tokens, 2 of 8 of 4096 x 14336 (16 rows an expert): 202 -> 156.
+    // Where it ends: 2048 deep 40 rows an expert 67 -> 61.5, 48 rows 68 -> 71 (4096 x 2048: 126 -> 114, 126 -> 131); 1536 deep 17 rows
+    // 41 -> 41, 24 rows 41 -> 42.5, 40 rows 41 -> 50.  The line between: 16 rows at 1536, 40 at 2048.
     const long long rows = a.max_rows, groups = a.groups;
-    if (tile_rows == 64 && a.K >= 1536 && (rows <= 16 * groups || (rows <= 48 * groups && a.K <= 2048)))
+    const int most = a.K < 1536 ? 0 : a.K <= 2048 ? 16 + (a.K - 1536) * 24 / 512 : 16;
+    if (tile_rows == 64 && rows <= most * groups)
       return a.N >= 512 ? launch_grouped_rows<E, true>(a, s) : launch_grouped_rows<E, false>(a, s);
     // Short contractions: a third of a tile's time is its start and its end, so two workgroups share a CU and one runs under the
     // other's (2000 rows, 8 of 64 experts of 1024 x 1024: 80 -> 62 us; 1946 rows, 5 of 33 gated experts of 4096 x 2048: 242 ->
