@@ -1267,7 +1267,7 @@ static int dual_entry(const char* who, const uint16_t* A, const uint16_t* Bgate,
   NF_REQUIRE(((uintptr_t)Bup) % 16 == 0, "%s: operands must be 16-byte aligned", who);
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (rows_pay_dual(M, 2 * K, kBCol)) return dispatch_rows_dual<E, kBCol>(A, Bgate, Bup, out, M, N, K, s);
+  if (rows_pay_dual(M, N, 2 * K, kBCol, false)) return dispatch_rows_dual<E, kBCol>(A, Bgate, Bup, out, M, N, K, s);
   if (M <= 64)
     return launch_gemm<E, 64, 128, 2, 2, true, kBCol>(A, Bgate, Bup, nullptr, out, M, N, K, 1.f, 0.f, N, s);
   // 257 .. 320 rows against enough column panels to fill the chip: one 320-row tile per panel, so
@@ -1295,7 +1295,7 @@ static int dual_ws_entry(const char* who, const uint16_t* A, const uint16_t* Bga
   const int shares = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 ? splitk_plan_dual(M, N, K, &k_per) : 1;
   const bool given = shares > 1 && workspace && workspace_bytes >= (size_t)2 * shares * M * N * sizeof(float);
   NF_REQUIRE(!given || (uintptr_t)workspace % 16 == 0, "%s: the workspace must be 16-byte aligned", who);
-  if (!given || rows_pay_dual(M, 2 * K, kBCol))
+  if (!given || rows_pay_dual(M, N, 2 * K, kBCol, false))
     return dual_entry<E, kBCol>(who, A, Bgate, Bup, out, M, N, K, stream);
   int rc = check_gemm_args(who, A, Bgate, out, M, N, K);
   if (rc) return rc;

@@ -300,8 +300,23 @@ static bool rows_pay(int M, int N, int K, int row_bytes = 0) {
   if (row_bytes > 8192 && N < 8192) return false;
   return M <= 32 || (N + 63) / 64 <= cu_count();
 }
-// The same for the gate/up pair; [K][N] weights in panels of 64 columns, up to 32 rows (16 x 14336 x 4096: 46.8 us against 48.0).
-static bool rows_pay_dual(int M, int row_bytes, bool b_col) { return M > 0 && M <= (b_col ? kRowsMax : 32) && row_bytes >= 3 * kRowsClasses * 128; }
+// The same for the gate/up pair of 16-bit or e4m3 (f8) operands; [K][N] weights in panels of 64 columns, up to 32 rows (16 x 14336 x 4096:
+// 46.8 us against 48.0).  Few columns against a long contraction, or workgroups that spill over into another round, lose to the tiles
+// and their split over K: 64 x 512 x 14336 63 us against 20, 16 x 4096 x 14336 56 against 46, 64 x 10240 x 8192 86 against 73, e4m3 64 x 512 x
+// 14336 29 against 15.  Both sides by what they take in: here a workgroup's rows of both weights and of A over the whole of K at
+// 50 GB/s, round after round, or all weights at 6.4 TB/s; there 10 us (e4m3: 9) and the weights at 6.  Fitted to 132 and 531 launches
+// of 1 to 64 rows, 64 to 28672 columns, K of 2048 to 14336, and within 5 % of the faster one except e4m3 against 16384 x 4096 (35 us, 31).
+// More than 32 rows against more than 64 columns a CU, and e4m3 rows below 4 KB there from 17 rows on, are the tiles' (64 x 28672 x 8192 181 us
+// against 168, e4m3 64 x 28672 x 3072 49 against 37).
+static bool rows_pay_dual(int M, int N, int row_bytes, bool b_col, bool f8) {
+  if (M <= 0 || M > (b_col ? kRowsMax : 32) || row_bytes < 3 * kRowsClasses * 128) return false;
+  const int cus = cu_count(), cols = M <= 8 ? 16 : 32, ar = M <= 8 ? 8 : M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  const bool wide = N > 64 * cus;
+  if (wide && (M > 32 || (f8 && M > 16 && row_bytes < 4096))) return false;
+  const int rounds = ((N + cols - 1) / cols + cus - 1) / cus;
+  const double weights = 2.0 * N * row_bytes, intake = (double)rounds * (2 * cols + ar) * row_bytes;
+  return std::max(weights / 6.4e6, intake / 50e3) * 1.1 + 1.0 + (f8 ? rounds : 0) < (f8 ? 9.0 : 10.0) + weights / 6e6;
+}
 
 // Rounds of workgroups times what one of them reads (16-row panels of weights and of A).
 static int rows_cost(int N, int nt, int m_tiles, int a_panels) { return ((N + nt * 16 - 1) / (nt * 16) * m_tiles + cu_count() - 1) / cu_count() * (nt + a_panels); }
