@@ -71,14 +71,24 @@ __device__ __forceinline__ float sum_over_lane_groups(float v) {
 }
 
 // Sum over the shares of a GEMM split over K, for 4 neighbouring outputs: P[s * mn + at .. +3],
-// s = 0 .. shares-1 (at most kMaxShares), added in that order.  Every load is issued before the
+// s = 0 .. shares-1 (at most kMaxShares), added in that order (kPairs: 2, 4 or 8 of them, neighbours
+// first, then the pairs, then those).  Every load is issued before the
 // first addition, so the lane waits for one memory round trip instead of one per share.
 constexpr int kMaxShares = 16;
+template <bool kPairs = false>
 __device__ __forceinline__ float4_t sum_shares(const float* __restrict__ P, size_t mn, size_t at, int shares) {
   float4_t p[kMaxShares];
 #pragma unroll
   for (int s = 0; s < kMaxShares; ++s)
     if (s < shares) p[s] = *reinterpret_cast<const float4_t*>(P + s * mn + at);
+  if constexpr (kPairs) {
+#pragma unroll
+    for (int d = 1; d < 8; d *= 2)
+#pragma unroll
+      for (int s = 0; s < 8; s += 2 * d)
+        if (s + d < shares) p[s] += p[s + d];
+    return p[0];
+  }
   float4_t v = p[0];
 #pragma unroll
   for (int s = 1; s < kMaxShares; ++s)

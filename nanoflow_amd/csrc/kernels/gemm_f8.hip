@@ -735,7 +735,7 @@ int nf_dual_swiglu_f8_f16(const uint8_t* Aq, const float* a_scale, const uint8_t
              "nf_dual_swiglu_f8_f16: an operand of %d x %d x %d exceeds the 4 GiB buffer-addressing limit", M, N, K);
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (rows_pay_dual(M, N, K, true, true)) return dispatch_rows_dual<RowsF8, true>(Aq, Gq, Uq, out, M, N, K, s, RowsScales{a_scale, g_scale, u_scale});
+  if (rows_pay_dual(M, N, K, true)) return dispatch_rows_dual<RowsF8>(Aq, Gq, Uq, out, M, N, K, s, RowsScales{a_scale, g_scale, u_scale});
   if (M <= 64)
     return launch_gemm_f8<64, 128, 2, 2, true>(Aq, Gq, a_scale, g_scale, nullptr, out, M, N, K, 1.f, 0.f, s, Uq, u_scale);
   const long long t256 = (long long)((M + 255) / 256) * ((N + 127) / 128);
@@ -829,7 +829,7 @@ static int dual_swiglu_f8q(const uint8_t* Aq, const float* sa, const uint8_t* Gq
                            const uint8_t* Uq, const float* u_scale, uint16_t* out, int M, int N, int K, void* workspace,
                            size_t workspace_bytes, nf_stream_t stream) {
   int k_per = 0;
-  const int shares = N > 0 && N % 8 == 0 && K % 16 == 0 && !rows_pay_dual(M, N, K, true, true) ? splitk_plan_f8(M, N, K, true, &k_per) : 1;
+  const int shares = N > 0 && N % 8 == 0 && K % 16 == 0 && !rows_pay_dual(M, N, K, true) ? splitk_plan_f8(M, N, K, true, &k_per) : 1;
   const size_t p_at = (nf_gemm_f8w_workspace_bytes(M, K) + 255) / 256 * 256;
   if (shares >= 2 && workspace && (uintptr_t)workspace % 16 == 0 &&
       workspace_bytes >= p_at + (size_t)2 * shares * M * N * sizeof(float) && Gq && g_scale && Uq &&

@@ -166,16 +166,20 @@ __device__ __forceinline__ float swiglu_rounded(float g_acc, float u_acc) {
 // over K, whose operand pointers already point at the share's first k.
 // kPartial: the fp32 sums are stored as they are to D taken as float [M][N] (no alpha, beta, C).
 // kOnce (kBCol only): the weights carry the non-temporal hint.
+// kClasses > 0 ([K][N] weights): K is summed as the weight stream of gemm_rows.h sums it -- eight classes of slabs (slab mod 8), each
+// in the order of k, added up in pairs, the pairs in pairs and those two -- here the classes first_class .. first_class + n_classes - 1 (1, 2,
+// 4 or 8 of them, at most 2^kClasses), which the loads walk one after the other without a break.
 // kGroup (kBCol only): operands of one group of a grouped product -- the weights' row stride is ldb, D's is
 // ldd, and where a_rows is not null row m of A is row a_rows[m] of a matrix of a_total rows.
 template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kPartial = false, bool kGroup = false, int kCap = kWholeCu,
-          bool kOnce = false>
+          bool kOnce = false, int kClasses = 0>
 __device__ __forceinline__ void gemm_tile(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
     int M, int N, int K, float alpha, float beta, const int ldc, const int m_base, const int n_base,
     const int lda, const int group_ldb = 0, const int group_ldd = 0, const int32_t* a_rows = nullptr, const int a_total = 0,
-    const GroupEpilogue& group = {}) {
+    const GroupEpilogue& group = {}, const int first_class = 0, const int n_classes = 1) {
+  static_assert(kClasses == 0 || (!kBCol && WM * WN == 4 && !GemmSmem<BM, BN, kDual ? 2 : 1, kCap>::split), "classes: [K][N] weights, one ring, 16 x 16 MFMAs");
   static_assert(!kGroup || (kBCol && !kDual && !kPartial), "grouped products: plain, k-contiguous weights");
   const int ldb = kGroup ? group_ldb : lda, ldd = kGroup ? group_ldd : N;
   constexpr int NB = kDual ? 2 : 1;
@@ -273,6 +277,25 @@ __device__ __forceinline__ void gemm_tile(
     for (int b = 0; b < NB; ++b) b_off[b][t] = off;
   }
 
+  // kClasses: slab `u` of K is followed by the next of its class, the class's last by the next class's first.  Every class has as
+  // many slabs; those past the end of K read as zero.
+  const int class_slabs = (K + 8 * BK - 1) / (8 * BK);
+  auto after = [&](int u) { return u >= 8 * (class_slabs - 1) ? (u & 7) + 1 : u + 8; };
+  int slab_step = 8;    // from the slab being fetched to the next one
+  bool slab_in = true;  // it starts below K
+  auto fetch = [&](int u) {
+    slab_step = after(u) - u;
+    slab_in = u * BK < K;
+  };
+  if constexpr (kClasses > 0) {
+#pragma unroll
+    for (int t = 0; t < A_LOADS; ++t) a_off[t] += (uint32_t)first_class * BK * 2;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int t = 0; t < B_LOADS; ++t) b_off[b][t] += (uint32_t)first_class * b_slab;
+  }
+
   // ---- global -> LDS, one 1 KB load instruction at a time.  Load t of a slab: t < A_LOADS
   // fetches activation rows, the rest weight rows.  st = LDS address of the stage + wave * 1024.
   constexpr int NS = SM::stages;
@@ -284,7 +307,7 @@ __device__ __forceinline__ void gemm_tile(
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
       load16_to_lds<t * NW * 1024>(a_rsrc, k_ok ? a_off[t] : kOob, la);
-      a_off[t] += BK * 2;
+      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : BK * 2;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       constexpr int dst = b * SM::b_bytes + tt * NW * 1024;
@@ -292,8 +315,8 @@ __device__ __forceinline__ void gemm_tile(
         load16_to_lds<dst, kOnce>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
         b_off[b][tt] += BK * 2;
       } else {
-        load16_to_lds<dst>(b_rsrc[b], b_off[b][tt], lb);
-        b_off[b][tt] += b_slab;
+        load16_to_lds<dst>(b_rsrc[b], kClasses == 0 || slab_in ? b_off[b][tt] : kOob, lb);
+        b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;
       }
     }
   };
@@ -305,15 +328,15 @@ __device__ __forceinline__ void gemm_tile(
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
       pend = k_ok ? a_off[t] : kOob;
-      a_off[t] += BK * 2;
+      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : BK * 2;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       if constexpr (kBCol) {
         pend = k_ok ? b_off[b][tt] : kOob;
         b_off[b][tt] += BK * 2;
       } else {
-        pend = b_off[b][tt];
-        b_off[b][tt] += b_slab;
+        pend = kClasses == 0 || slab_in ? b_off[b][tt] : kOob;
+        b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;
       }
     }
   };
@@ -453,7 +476,9 @@ __device__ __forceinline__ void gemm_tile(
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
-  const int nslab = (K + BK - 1) / BK;
+  const int nslab = kClasses > 0 ? n_classes * class_slabs : (K + BK - 1) / BK;
+  // k of slab s, or of slab number u of K
+  auto slab_k = [&](int s, int u) { return (kClasses > 0 ? u : s) * BK; };
 
   if constexpr (SM::split) {
     // ---- two activation stages, three weight stages.  Slab s has its activations in stage s % 2
@@ -541,12 +566,39 @@ __device__ __forceinline__ void gemm_tile(
   // loads must land within the same slab and are issued in the first two of those steps only.)
   //   IA: slab s+NS-1 exists (loads in steps 0..2), IB: slab s+NS exists (loads in step 3),
   //   LAST: no slab s+1.
+  // kClasses: sums of whole classes that wait for their other half
+  acc_t waiting[kClasses > 0 ? kClasses : 1][NB][TM][TNG];
+  auto each_sum = [&](auto f) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TNG; ++j) f(b, i, j);
+  };
+  auto end_class = [&](int c) {  // c: of this workgroup's classes
+    auto level = [&](auto self, auto l_c) -> void {
+      constexpr int l = decltype(l_c)::value;
+      if constexpr (l < kClasses) {
+        if ((c >> l) & 1) {
+          each_sum([&](int b, int i, int j) { acc[b][i][j] = waiting[l][b][i][j] + acc[b][i][j]; });
+          self(self, ic<l + 1>{});
+        } else {
+          each_sum([&](int b, int i, int j) { waiting[l][b][i][j] = acc[b][i][j]; });
+        }
+      }
+    };
+    level(level, ic<0>{});
+    if (c + 1 < n_classes) each_sum([&](int b, int i, int j) { acc[b][i][j] = acc_t{}; });
+  };
+  int u_now = first_class, u_ahead = first_class;  // slab of K that is multiplied, and slab s + NS - 1, which is fetched
   auto slab = [&](auto ia_c, auto ib_c, auto last_c, int s, int cs, int ls) {
     constexpr bool IA = decltype(ia_c)::value, IB = decltype(ib_c)::value, LAST = decltype(last_c)::value;
     const uint8_t* st = smem + cs * SM::stage_bytes;
     const uint8_t* sb = st + SM::a_bytes;
     const uint32_t ld_a = __builtin_amdgcn_readfirstlane(smem_lds + ls * SM::stage_bytes + wave * 1024);
-    const bool ok_a = (s + NS - 1) * BK + a_kc < K;
+    if constexpr (kClasses > 0) fetch(u_ahead);
+    const bool ok_a = slab_k(s + NS - 1, u_ahead) + a_kc < K;
     step(ic<0>{}, ic<1>{}, ic<PARTS>{}, ic<(IA && PARTS > 1) ? nl(1) : 0>{}, ic<1>{}, ld_a, ld_a + SM::a_bytes, ok_a, st, sb);
     step(ic<1>{}, ic<2>{}, ic<PARTS>{}, ic<(IA && PARTS > 2) ? nl(2) : 0>{}, ic<2>{}, ld_a, ld_a + SM::a_bytes, ok_a, st, sb);
     step(ic<2>{}, ic<3>{}, ic<PARTS>{}, ic<(IA && PARTS > 3) ? nl(3) : 0>{}, ic<3>{}, ld_a, ld_a + SM::a_bytes, ok_a, st, sb);
@@ -556,13 +608,24 @@ __device__ __forceinline__ void gemm_tile(
     }
     const uint32_t ld_b = __builtin_amdgcn_readfirstlane(smem_lds + cs * SM::stage_bytes + wave * 1024);
     const uint8_t* nst = smem + next(cs) * SM::stage_bytes;
+    if constexpr (kClasses > 0) {
+      u_ahead = after(u_ahead);
+      fetch(u_ahead);
+    }
     step(ic<3>{}, ic<0>{}, ic<PARTS>{}, ic<IB ? nl(0) : 0>{}, ic<LAST ? -1 : 0>{}, ld_b, ld_b + SM::a_bytes,
-         (s + NS) * BK + a_kc < K, nst, nst + SM::a_bytes);
+         slab_k(s + NS, u_ahead) + a_kc < K, nst, nst + SM::a_bytes);
+    if constexpr (kClasses > 0) {
+      if (u_now >= 8 * (class_slabs - 1)) end_class((u_now & 7) - first_class);
+      u_now = after(u_now);
+    }
   };
 
 #pragma unroll
-  for (int p = 0; p < NS - 1; ++p)
-    if (p < nslab) load_slab(p, p * BK);
+  for (int p = 0; p < NS - 1; ++p) {
+    if constexpr (kClasses > 0) fetch(u_ahead);
+    if (p < nslab) load_slab(p, slab_k(p, u_ahead));
+    if constexpr (kClasses > 0) u_ahead = after(u_ahead);
+  }
   // slab 0 must have landed; later prologue loads may still be in flight (exact count only
   // matters for speed: waiting for everything is always correct)
   wait_loads(nslab >= NS - 1 ? 1 : 0);
@@ -570,7 +633,8 @@ __device__ __forceinline__ void gemm_tile(
   static_for<(kM16 ? TM + CH : READS)>([&](auto q_c) { read_one(q_c, ic<0>{}, ic<0>{}, smem, smem + SM::a_bytes); });
   if (NS - 1 < nslab) {  // the share of slab NS-1 that a slab's k-step 3 would have issued
     const uint32_t st = __builtin_amdgcn_readfirstlane(smem_lds + (NS - 1) * SM::stage_bytes + wave * 1024);
-    const bool k_ok = (NS - 1) * BK + a_kc < K;
+    if constexpr (kClasses > 0) fetch(u_ahead);
+    const bool k_ok = slab_k(NS - 1, u_ahead) + a_kc < K;
     static_for<(LOADS + PARTS - 1) / PARTS>([&](auto q_c) { load_one(ic<PARTS * decltype(q_c)::value>{}, st, st + SM::a_bytes, k_ok); });
   }
   int cs = 0, ls = NS - 1, s = 0;
@@ -758,14 +822,15 @@ __device__ __forceinline__ bool xcd_tile(int bid, int tiles_m, int tiles_n, int*
   return true;
 }
 
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kOnce = false>
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kOnce = false, int kClasses = 0>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_f16_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
     int M, int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n) {
   int tm, tn;
   if (!xcd_tile(blockIdx.x, tiles_m, tiles_n, &tm, &tn)) return;
-  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, false, false, kWholeCu, kOnce>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tm * BM, tn * BN, K);
+  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, false, false, kWholeCu, kOnce, kClasses>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tm * BM, tn * BN, K, 0,
+                                                                                      0, nullptr, 0, {}, 0, 1 << kClasses);
 }
 
 // Two tile heights in one launch, for shapes whose 256-row tiles fill the 256 CUs a whole number
@@ -798,8 +863,8 @@ __global__ __launch_bounds__(256) void gemm_f16_hybrid_kernel(
 // A GEMM with too few output tiles to fill the chip (few rows against a narrow N), split over K:
 // workgroup (tile, share) computes the tile's sums over k in [share * k_per, ...) and stores them
 // as fp32 to P[share][M][N]; splitk_reduce_kernel adds the shares and applies alpha, beta and C.
-// kDual: two weight matrices; the sums of the second go to P1[share][M][N].
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, int kCap = kWholeCu>
+// kDual: two weight matrices; the sums of the second go to P1[share][M][N].  kClasses: a share is a run of the eight classes.
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, int kCap = kWholeCu, int kClasses = 0>
 __global__ __launch_bounds__(WM * WN * 64, kCap == kHalfCu ? 2 : 1) void gemm_f16_splitk_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, const uint16_t* __restrict__ B1,
     float* __restrict__ P, float* __restrict__ P1, int M, int N, int K, int shares, int k_per, int tiles_m,
@@ -808,24 +873,25 @@ __global__ __launch_bounds__(WM * WN * 64, kCap == kHalfCu ? 2 : 1) void gemm_f1
   const int logical = xcd_order(blockIdx.x, total);
   if (logical >= total) return;
   const int share = logical % shares, tile = logical / shares;
-  const int k0 = share * k_per;
+  const int k0 = kClasses > 0 ? 0 : share * k_per, classes = 8 / shares;
+  if constexpr (kClasses > 0) k_per = K;
   const int k_len = K - k0 < k_per ? K - k0 : k_per;
   const size_t b_off = kBCol ? (size_t)k0 : (size_t)k0 * N, p_off = (size_t)share * M * N;
-  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, true, false, kCap>(
+  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, true, false, kCap, false, kClasses>(
       A + k0, B + b_off, kDual ? B1 + b_off : nullptr,
       kDual ? reinterpret_cast<const uint16_t*>(P1 + p_off) : nullptr, reinterpret_cast<uint16_t*>(P + p_off), M, N,
-      k_len, 1.f, 0.f, N, (tile % tiles_m) * BM, (tile / tiles_m) * BN, K);
+      k_len, 1.f, 0.f, N, (tile % tiles_m) * BM, (tile / tiles_m) * BN, K, 0, 0, nullptr, 0, {}, share * classes, classes);
 }
 
 // out[m][n..n+3] = round(silu(g) * u) with g = round(sum_s P0[s][m][n..]), u likewise from P1: the
 // epilogue of the fused gate/up pair on the summed shares.
-template <class E>
+template <class E, bool kPairs = false>
 __global__ __launch_bounds__(256) void splitk_reduce_dual_kernel(const float* __restrict__ P0,
                                                                  const float* __restrict__ P1, int shares,
                                                                  uint16_t* out, int M, int N) {
   const size_t groups = (size_t)M * N / 4, mn = (size_t)M * N;
   for (size_t g = (size_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += (size_t)gridDim.x * 256) {
-    const float4_t a = sum_shares(P0, mn, g * 4, shares), b = sum_shares(P1, mn, g * 4, shares);
+    const float4_t a = sum_shares<kPairs>(P0, mn, g * 4, shares), b = sum_shares<kPairs>(P1, mn, g * 4, shares);
     float4_t v;
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = swiglu_rounded<E>(a[e], b[e]);
@@ -834,13 +900,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_dual_kernel(const float* __
 }
 
 // D[m][n..n+3] = round(alpha * sum_s P[s][m][n..] + beta * C[m][n..]); C has row stride ldc.
-template <class E>
+template <class E, bool kPairs = false>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ P, int shares,
                                                             const uint16_t* C, int ldc, uint16_t* D,
                                                             int M, int N, float alpha, float beta) {
   const size_t groups = (size_t)M * N / 4, mn = (size_t)M * N;
   for (size_t g = (size_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += (size_t)gridDim.x * 256) {
-    float4_t v = sum_shares(P, mn, g * 4, shares) * alpha;
+    float4_t v = sum_shares<kPairs>(P, mn, g * 4, shares) * alpha;
     if (beta != 0.f) {
       const size_t m = g * 4 / N, n = g * 4 % N;
       const u32x2 c = *reinterpret_cast<const u32x2*>(C + m * ldc + n);
@@ -855,12 +921,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 }
 
 // kDual: B1 is the second weight matrix, C is not used, D = the SwiGLU output.
-template <class E, int BM, int BN, int WM, int WN, bool kBCol, bool kDual = false, int kCap = kWholeCu>
+template <class E, int BM, int BN, int WM, int WN, bool kBCol, bool kDual = false, int kCap = kWholeCu, int kClasses = 0>
 static int launch_splitk(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N,
                          int K, float alpha, float beta, int ldc, int shares, int k_per, float* P,
                          hipStream_t stream, const uint16_t* B1 = nullptr) {
   using SM = GemmSmem<BM, BN, kDual ? 2 : 1, kCap>;
-  auto kern = gemm_f16_splitk_kernel<typename E::Mul, BM, BN, WM, WN, kDual, kBCol, kCap>;
+  auto kern = gemm_f16_splitk_kernel<typename E::Mul, BM, BN, WM, WN, kDual, kBCol, kCap, kClasses>;
   float* P1 = kDual ? P + (size_t)shares * M * N : nullptr;
   static bool attr_set = false;  // benign race: the call is idempotent
   if (!attr_set) {
@@ -879,12 +945,12 @@ static int launch_splitk(const uint16_t* A, const uint16_t* B, const uint16_t* C
   if (rc) return rc;
   const size_t groups = (size_t)M * N / 4;
   const int rgrid = (int)std::min<size_t>((groups + 255) / 256, 2048);
-  if constexpr (kDual) splitk_reduce_dual_kernel<E><<<rgrid, 256, 0, stream>>>(P, P1, shares, D, M, N);
-  else splitk_reduce_kernel<E><<<rgrid, 256, 0, stream>>>(P, shares, C, ldc, D, M, N, alpha, beta);
+  if constexpr (kDual) splitk_reduce_dual_kernel<E, (kClasses > 0)><<<rgrid, 256, 0, stream>>>(P, P1, shares, D, M, N);
+  else splitk_reduce_kernel<E, (kClasses > 0)><<<rgrid, 256, 0, stream>>>(P, shares, C, ldc, D, M, N, alpha, beta);
   return check_launch("gemm split-K reduction launch");
 }
 
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol>
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, int kClasses = 0>
 static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1, const uint16_t* C,
                        uint16_t* D, int M, int N, int K, float alpha, float beta, int ldc,
                        hipStream_t stream) {
@@ -893,7 +959,7 @@ static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1
   const int ntiles = tiles_m * tiles_n;
   const int grid = ((ntiles + 7) / 8) * 8;
   auto go = [&](auto once_c) {
-    auto kern = gemm_f16_kernel<E, BM, BN, WM, WN, kDual, kBCol, decltype(once_c)::value>;
+    auto kern = gemm_f16_kernel<E, BM, BN, WM, WN, kDual, kBCol, decltype(once_c)::value, kClasses>;
     static bool attr_set = false;  // benign race: the call is idempotent
     if (!attr_set) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -951,6 +1017,9 @@ static int cu_count() {
   }
   return n;
 }
+
+static bool in_a_gap(int N, int K);  // gemm_rows.h
+static bool rows_pay_dual(int M, int N, int row_bytes, bool f8);
 
 // Split over K: for at most 512 rows whose tiles (64 x 256 up to 64 rows, 128 x 128 up to 256,
 // 320 x 128 up to 320, else 256 x 256) would leave more than half of the CUs idle, as many shares
@@ -1042,7 +1111,7 @@ static size_t split_bytes(int M, int N, int K, MidPlan* mid) {
   size_t bytes = 0;
   const int shares = M <= kSplitMaxRows ? splitk_plan(M, N, K, &k_per) : dense_split_plan(M, N, K, &k_per);
   if (shares > 1) {
-    bytes = shares * sums;
+    bytes = (M <= 8 && in_a_gap(N, K) ? 8 : shares) * sums;
     if (M > kTallRows) plan = mid_split_plan(M, N, K, bytes);
   } else if (M > kSplitMaxRows && M <= kMidRows && K >= kDenseSplitMinK) {
     plan = mid_split_plan(M, N, K, kMidBytes);
@@ -1066,8 +1135,9 @@ static int splitk_plan_dual(int M, int N, int K, int* k_per) {
   if (M > kTallRows || K < 1024) return 1;
   const int bm = M <= 64 ? 64 : M <= 256 ? 128 : 320;
   const int tiles = ((M + bm - 1) / bm) * ((N + 127) / 128);
-  const int shares = std::min(std::min(cu_count() / tiles, K / 512), kMaxShares);
+  int shares = std::min(std::min(cu_count() / tiles, K / 512), kMaxShares);
   if (shares < 2) return 1;
+  if (shares > 4 && shares < 8 && tiles * 8 <= cu_count() && rows_pay_dual(M, N, 2 * K, false)) shares = 8;  // launch_classes_dual takes 2, 4 or 8
   *k_per = ((K + shares - 1) / shares + BK - 1) / BK * BK;
   return (K + *k_per - 1) / *k_per;
 }
@@ -1210,21 +1280,25 @@ static int gemm_entry(const char* who, const uint16_t* A, const uint16_t* B, con
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
   const int ldc = c_is_row ? 0 : N;  // row stride of C: 0 reads the same row for every m
-  if (b_col_major && rows_pay(M, N, K)) return dispatch_rows<E, false>(A, B, C, D, M, N, K, alpha, beta, ldc, s);
+  if (few_pay(M, N, K))
+    return b_col_major ? dispatch_rows<E, false>(A, B, C, D, M, N, K, alpha, beta, ldc, s)
+                       : launch_classes<E>(A, B, C, D, M, N, K, alpha, beta, ldc, 1, nullptr, s);
   return b_col_major ? dispatch_plain<E, true>(A, B, C, D, M, N, K, alpha, beta, ldc, s)
                      : dispatch_plain<E, false>(A, B, C, D, M, N, K, alpha, beta, ldc, s);
 }
 
-// At most 64 rows, split over K into `shares` (what the workspace holds the sums of); k-contiguous weights in no more of them
-// than their narrower tiles need.
+// At most 64 rows, split over K into `shares` (what the workspace holds the sums of), or in no more of them than narrower tiles
+// need.
 template <class E>
 static int launch_splitk_64(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
                             int ldc, int shares, int k_per, float* P, int b_col_major, hipStream_t s) {
-  if (!b_col_major) return launch_splitk<E, 64, 256, 1, 4, false>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
   int k_narrow = 0;
-  const int narrow = M > 16 ? splitk_plan_narrow(N, K, &k_narrow) : 1;
-  if (narrow > 1 && narrow <= shares) return launch_splitk<E, 64, 64, 2, 2, true, false, kHalfCu>(A, B, C, D, M, N, K, alpha, beta, ldc, narrow, k_narrow, P, s);
-  return launch_splitk<E, 64, 256, 1, 4, true>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
+  const int narrow = splitk_plan_narrow(N, K, 2, &k_narrow);
+  if (narrow > 1 && narrow <= shares)
+    return b_col_major ? launch_splitk<E, 64, 64, 2, 2, true, false, kHalfCu>(A, B, C, D, M, N, K, alpha, beta, ldc, narrow, k_narrow, P, s)
+                       : launch_splitk<E, 64, 128, 2, 2, false, false, kHalfCu>(A, B, C, D, M, N, K, alpha, beta, ldc, narrow, k_narrow, P, s);
+  return b_col_major ? launch_splitk<E, 64, 256, 1, 4, true>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s)
+                     : launch_splitk<E, 64, 256, 1, 4, false>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
 }
 
 // gemm_entry with a workspace: shapes that profit are split over K through it.
@@ -1238,7 +1312,7 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   int k_per = 0;
   // a workspace for the sums of at most 512 rows, or of a dense launch, has to be aligned, whatever runs; others run unsplit without
   NF_REQUIRE(!given || aligned || (M > kSplitMaxRows && dense_split_plan(M, N, K, &k_per) < 2), "%s: the workspace must be 16-byte aligned", who);
-  const bool whole = M > kTallRows ? mid.shares < 2 : b_col_major && rows_pay(M, N, K);
+  const bool few = few_pay(M, N, K), whole = M > kTallRows ? mid.shares < 2 : few && b_col_major;
   if (!given || !aligned || whole) return gemm_entry<E>(who, A, B, C, D, M, N, K, alpha, beta, b_col_major, stream, c_is_row);
   const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
   int rc = check_gemm_args(who, A, B, D, M, N, K);
@@ -1250,6 +1324,7 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   if (mid.shares > 1)
     return b_col_major ? launch_mid<E, true>(mid, A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, P, s)
                        : launch_mid<E, false>(mid, A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, P, s);
+  if (few) return launch_classes<E>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, (int)(need / ((size_t)M * N * sizeof(float))), P, s);
   if (M <= 64) return launch_splitk_64<E>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, b_col_major, s);
   if (M > 256)
     return b_col_major ? launch_splitk<E, 320, 128, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
@@ -1267,7 +1342,10 @@ static int dual_entry(const char* who, const uint16_t* A, const uint16_t* Bgate,
   NF_REQUIRE(((uintptr_t)Bup) % 16 == 0, "%s: operands must be 16-byte aligned", who);
   if (M == 0) return NF_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (rows_pay_dual(M, N, 2 * K, kBCol, false)) return dispatch_rows_dual<E, kBCol>(A, Bgate, Bup, out, M, N, K, s);
+  if (rows_pay_dual(M, N, 2 * K, false)) {
+    if constexpr (kBCol) return dispatch_rows_dual<E>(A, Bgate, Bup, out, M, N, K, s);
+    else return launch_classes_dual<E>(A, Bgate, Bup, out, M, N, K, 1, nullptr, s);
+  }
   if (M <= 64)
     return launch_gemm<E, 64, 128, 2, 2, true, kBCol>(A, Bgate, Bup, nullptr, out, M, N, K, 1.f, 0.f, N, s);
   // 257 .. 320 rows against enough column panels to fill the chip: one 320-row tile per panel, so
@@ -1295,13 +1373,16 @@ static int dual_ws_entry(const char* who, const uint16_t* A, const uint16_t* Bga
   const int shares = M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 ? splitk_plan_dual(M, N, K, &k_per) : 1;
   const bool given = shares > 1 && workspace && workspace_bytes >= (size_t)2 * shares * M * N * sizeof(float);
   NF_REQUIRE(!given || (uintptr_t)workspace % 16 == 0, "%s: the workspace must be 16-byte aligned", who);
-  if (!given || rows_pay_dual(M, N, 2 * K, kBCol, false))
+  const bool few = rows_pay_dual(M, N, 2 * K, false);
+  if (!given || (kBCol && few))
     return dual_entry<E, kBCol>(who, A, Bgate, Bup, out, M, N, K, stream);
   int rc = check_gemm_args(who, A, Bgate, out, M, N, K);
   if (rc) return rc;
   NF_REQUIRE(Bup && ((uintptr_t)Bup) % 16 == 0, "%s: Bup must be 16-byte aligned", who);
   hipStream_t s = (hipStream_t)stream;
   float* P = static_cast<float*>(workspace);
+  if constexpr (!kBCol)
+    if (few) return launch_classes_dual<E>(A, Bgate, Bup, out, M, N, K, shares, P, s);
   if (M <= 64)
     return launch_splitk<E, 64, 128, 2, 2, kBCol, true>(A, Bgate, nullptr, out, M, N, K, 1.f, 0.f, N, shares, k_per, P, s, Bup);
   if (M > 256)

@@ -21,7 +21,7 @@ SumPlan sum_plan(int M, int N, int K, int max_shares) {
   }
   if (M > 16 && M <= 64) {
     int k_narrow = 0;
-    const int narrow = splitk_plan_narrow(N, K, &k_narrow);
+    const int narrow = splitk_plan_narrow(N, K, 1, &k_narrow);
     if (narrow > 1 && narrow <= max_shares) return SumPlan{4, narrow, k_narrow};
   }
   const long long t256 = (long long)((M + 255) / 256) * ((N + 255) / 256);

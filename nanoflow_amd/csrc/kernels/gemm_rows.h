@@ -8,11 +8,12 @@
 // nobody until the end and refills a slot as soon as its fragments are in registers.  An instruction fetches 8 rows of 128
 // bytes: whole lines, with the non-temporal hint, reach 6.3 - 7.0 TB/s where fragments loaded straight into registers
 // (16 rows of 64 bytes) stop at 5.0 (the gate/up pair of 1 x 14336 x 4096: 37 us against 47).  Weights may be [K][N] as well
-// (kBCol false): rows of NT * 32 bytes per k, read back through the transposing LDS read.
+// (kBCol false): rows of NT * 32 bytes per k, read back through the transposing LDS read.  That stream is slower than tiles
+// which are split over K where those can be (16 x 4096 x 14336: 50 us against 26) and runs where they cannot.
 //
 // The sum of an output element is taken in the same order whatever the tile: eight classes of units (unit mod 8), each in the
-// order of k, then the classes one after the other.  A row's result does not depend on how many rows come with it, nor on
-// the weights' layout.
+// order of k, neighbouring classes added first, then the pairs, then those.  A row's result does not depend on how many rows come
+// with it, nor on the weights' layout: the tiles for [K][N] weights take their slabs in this order (kClasses in gemm_impl.h).
 //
 // Measured against the tiles and the split over K that it replaces (us, one launch after the other on streamed weights):
 //   rows x N x K              before   here         rows x N x K              before   here
@@ -58,7 +59,8 @@ __device__ __forceinline__ void rows_tile(const rsrc_t a_rsrc, const rsrc_t (&b_
   using SM = RowsSmem<AR, NT, NW, NB, S>;
   constexpr int MT = (AR + 15) / 16, PAR = kRowsClasses / NW;  // classes per wavefront
   constexpr bool kF8 = std::is_same_v<E, RowsF8>;
-  static_assert(NW * PAR == kRowsClasses && S % PAR == 0, "a ring slot belongs to one class");
+  static_assert(NW * PAR == kRowsClasses && (S % PAR == 0 || S == 1), "classes take turns in the ring's slots");
+  constexpr int R = S > PAR ? S : PAR;  // units of a round
   static_assert(!kF8 || kBCol, "e4m3 weights are k-contiguous");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, lq = lane >> 4;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -116,8 +118,8 @@ __device__ __forceinline__ void rows_tile(const rsrc_t a_rsrc, const rsrc_t (&b_
   const uint32_t f_row = (uint32_t)l16 * 128u, f_swz = (l16 >> 1) & 7;
   // eight rows of A stand for sixteen: the upper half of the products is not stored
   const uint32_t af_row = AR == 8 ? (uint32_t)(l16 & 7) * 128u : f_row, a_swz = AR == 8 ? (l16 & 7) >> 1 : f_swz;
-  auto consume = [&](auto s_c) {
-    constexpr int s = decltype(s_c)::value;
+  auto consume = [&](auto s_c, auto p_c) {
+    constexpr int s = decltype(s_c)::value, P = decltype(p_c)::value;
     const uint8_t* slot = mine + s * SM::slot;
     half8_t w[2][NB][NT], a[2][MT];
 #pragma unroll
@@ -153,8 +155,8 @@ __device__ __forceinline__ void rows_tile(const rsrc_t a_rsrc, const rsrc_t (&b_
         for (int j = 0; j < NT; ++j)
 #pragma unroll
           for (int i = 0; i < MT; ++i)
-            acc[s % PAR][b][i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(both(w[0][b][j], w[1][b][j]), both(a[0][i], a[1][i]),
-                                                                                    acc[s % PAR][b][i][j], 0, 0, 0, 0, 0, 0);
+            acc[P][b][i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(both(w[0][b][j], w[1][b][j]), both(a[0][i], a[1][i]),
+                                                                                    acc[P][b][i][j], 0, 0, 0, 0, 0, 0);
     } else {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -163,7 +165,7 @@ __device__ __forceinline__ void rows_tile(const rsrc_t a_rsrc, const rsrc_t (&b_
 #pragma unroll
           for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[s % PAR][b][i][j] = E::mfma16(w[h][b][j], a[h][i], acc[s % PAR][b][i][j]);
+            for (int i = 0; i < MT; ++i) acc[P][b][i][j] = E::mfma16(w[h][b][j], a[h][i], acc[P][b][i][j]);
     }
   };
   // vmcnt(n): all but the n youngest loads of this wavefront have landed
@@ -181,17 +183,17 @@ __device__ __forceinline__ void rows_tile(const rsrc_t a_rsrc, const rsrc_t (&b_
   static_for<S>([&](auto s_c) { issue_a(s_c, wave + decltype(s_c)::value * NW); });
   int u = wave + S * NW;
   auto round = [&](auto first_c) {  // units past the last one read as zero
-    static_for<S>([&](auto s_c) {
-      constexpr int s = decltype(s_c)::value;
-      wait_but(ic<decltype(first_c)::value ? (S - 1 - s) * kA + s * kLoads : (S - 1) * kLoads>{});  // the slot has landed
-      consume(s_c);
-      issue_b(s_c, u);
-      issue_a(s_c, u);
+    static_for<R>([&](auto r_c) {
+      constexpr int r = decltype(r_c)::value, s = r % S;
+      wait_but(ic<decltype(first_c)::value && r < S ? (S - 1 - r) * kA + r * kLoads : (S - 1) * kLoads>{});  // the slot has landed
+      consume(ic<s>{}, ic<r % PAR>{});
+      issue_b(ic<s>{}, u);
+      issue_a(ic<s>{}, u);
       u += NW;
     });
   };
   if (wave < units) round(ic<1>{});
-  for (int done = wave + NW * S; done < units; done += NW * S) round(ic<0>{});
+  for (int done = wave + NW * R; done < units; done += NW * R) round(ic<0>{});
   __builtin_amdgcn_s_waitcnt(0x0070);
   __syncthreads();
 
@@ -212,9 +214,14 @@ __device__ __forceinline__ void rows_tile(const rsrc_t a_rsrc, const rsrc_t (&b_
       float4_t v[NB];
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        v[b] = red[(t * NB + b) * 64 + ln];
+        float4_t sum[kRowsClasses];
 #pragma unroll
-        for (int c = 1; c < kRowsClasses; ++c) v[b] += red[((c * TP + t) * NB + b) * 64 + ln];
+        for (int c = 0; c < kRowsClasses; ++c) sum[c] = red[((c * TP + t) * NB + b) * 64 + ln];
+#pragma unroll
+        for (int d = 1; d < kRowsClasses; d *= 2)
+#pragma unroll
+          for (int c = 0; c < kRowsClasses; c += 2 * d) sum[c] += sum[c + d];
+        v[b] = sum[0];
       }
       const int row = tt / NT * 16 + (ln & 15), n = n0 + tt % NT * 16 + (ln >> 4) * 4;
       if (row < AR && n < N) store(m0 + row, n, v);
@@ -300,19 +307,25 @@ static bool rows_pay(int M, int N, int K, int row_bytes = 0) {
   if (row_bytes > 8192 && N < 8192) return false;
   return M <= 32 || (N + 63) / 64 <= cu_count();
 }
-// The same for the gate/up pair of 16-bit or e4m3 (f8) operands; [K][N] weights in panels of 64 columns, up to 32 rows (16 x 14336 x 4096:
-// 46.8 us against 48.0).  Few columns against a long contraction, or workgroups that spill over into another round, lose to the tiles
-// and their split over K: 64 x 512 x 14336 63 us against 20, 16 x 4096 x 14336 56 against 46, 64 x 10240 x 8192 86 against 73, e4m3 64 x 512 x
-// 14336 29 against 15.  Both sides by what they take in: here a workgroup's rows of both weights and of A over the whole of K at
+// fp16 and bf16 launches that may come with either layout: from 9 rows on not against 33 to 44 columns a CU and K >= 4096, where [K][N]
+// weights have no tiles in this order that are as fast (16 x 10240 x 8192: 42 us in 4 shares, 31.6 as splitk_plan_narrow says, 34.6 on
+// 64 x 256; k-contiguous ones 36.2 here, 35.2 and 37.6).
+static bool in_a_gap(int N, int K) { return N > 32 * cu_count() && N <= 44 * cu_count() && K >= 4096; }
+static bool few_pay(int M, int N, int K) { return rows_pay(M, N, K) && (M <= 8 || !in_a_gap(N, K)); }
+
+// The same for the gate/up pair of 16-bit or e4m3 (f8) operands.  Few columns against a long contraction, or workgroups that spill over
+// into another round, lose to the tiles and their split over K: 64 x 512 x 14336 63 us against 20, 16 x 4096 x 14336 56 against 46, 64 x
+// 10240 x 8192 86 against 73, e4m3 64 x 512 x 14336 29 against 15.  Both sides by what they take in: here a workgroup's rows of both weights and of A over the whole of K at
 // 50 GB/s, round after round, or all weights at 6.4 TB/s; there 10 us (e4m3: 9) and the weights at 6.  Fitted to 132 and 531 launches
 // of 1 to 64 rows, 64 to 28672 columns, K of 2048 to 14336, and within 5 % of the faster one except e4m3 against 16384 x 4096 (35 us, 31).
 // More than 32 rows against more than 64 columns a CU, and e4m3 rows below 4 KB there from 17 rows on, are the tiles' (64 x 28672 x 8192 181 us
 // against 168, e4m3 64 x 28672 x 3072 49 against 37).
-static bool rows_pay_dual(int M, int N, int row_bytes, bool b_col, bool f8) {
-  if (M <= 0 || M > (b_col ? kRowsMax : 32) || row_bytes < 3 * kRowsClasses * 128) return false;
+static bool rows_pay_dual(int M, int N, int row_bytes, bool f8) {
+  if (M <= 0 || M > kRowsMax || row_bytes < 3 * kRowsClasses * 128) return false;
   const int cus = cu_count(), cols = M <= 8 ? 16 : 32, ar = M <= 8 ? 8 : M <= 16 ? 16 : M <= 32 ? 32 : 64;
   const bool wide = N > 64 * cus;
-  if (wide && (M > 32 || (f8 && M > 16 && row_bytes < 4096))) return false;
+  if ((wide && (M > 32 || (f8 && M > 16 && row_bytes < 4096))) || (row_bytes > 16384 && N < 16 * cus)) return false;
+  if (!f8 && M > 8 && in_a_gap(N, row_bytes / 2)) return false;
   const int rounds = ((N + cols - 1) / cols + cus - 1) / cus;
   const double weights = 2.0 * N * row_bytes, intake = (double)rounds * (2 * cols + ar) * row_bytes;
   return std::max(weights / 6.4e6, intake / 50e3) * 1.1 + 1.0 + (f8 ? rounds : 0) < (f8 ? 9.0 : 10.0) + weights / 6e6;
@@ -341,29 +354,69 @@ static int dispatch_rows(const void* A, const void* B, const uint16_t* C, uint16
                  : launch_rows<E, 64, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
 }
 
-template <class E, bool kBCol>
+template <class E>
 static int dispatch_rows_dual(const void* A, const void* Bg, const void* Bu, uint16_t* out, int M, int N, int K, hipStream_t s,
                               const RowsScales& sc = {}) {
-  if constexpr (kBCol) {
-    if (M <= 8) return launch_rows<E, 8, 1, 8, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-    if (M <= 16) return launch_rows<E, 16, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-    if (M <= 32) return launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-    return launch_rows<E, 64, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-  } else {
-    if (M <= 8) return launch_rows<E, 8, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-    if (M <= 16) return launch_rows<E, 16, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-    return launch_rows<E, 32, 4, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-  }
+  if (M <= 8) return launch_rows<E, 8, 1, 8, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+  if (M <= 16) return launch_rows<E, 16, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+  if (M <= 32) return launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+  return launch_rows<E, 64, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
 }
 
-// 17 to 64 rows against k-contiguous weights where rows_pay says no: 64 x 64 tiles, two workgroups a CU, and only as many shares
-// of K as give every CU a workgroup (64 x 4096 x 14336: 26.4 us in 4 shares against 30.1 on 64 x 256 tiles in 16).
-static int splitk_plan_narrow(int N, int K, int* k_per) {
+// Up to 64 rows where few_pay says no: narrow tiles (64 x 64, of [K][N] weights 64 x 128), two workgroups a CU, and as many shares of K
+// as give every CU `per_cu` of 64 x 64 (64 x 4096 x 14336: 4 shares 27.6 us, 8 29.2, 64 x 256 tiles in 16 29.9; on [K][N] weights 8 shares
+// 27.9, 4 37, 64 x 256 in 16 29.8: both layouts take 8, for the same bits).
+static int splitk_plan_narrow(int N, int K, int per_cu, int* k_per) {
   if (K <= 4096) return 1;
-  const int shares = std::min(std::min(cu_count() / ((N + 63) / 64), K / 512), kMaxShares);
+  const int shares = std::min(std::min(per_cu * cu_count() / ((N + 63) / 64), K / 512), kMaxShares);
   if (shares < 2) return 1;
   *k_per = ((K + shares - 1) / shares + BK - 1) / BK * BK;
   return (K + *k_per - 1) / *k_per;
+}
+
+// [K][N] weights where k-contiguous ones run on the weight stream, in its order of sums: 64 x 128 tiles, two workgroups a CU, in 2, 4 or 8
+// shares of the classes, no more than `most` (what the workspace holds) and fewer against more columns, whose sums are to be written.
+// Against 64 x 256 tiles in runs of K, 1 to 64 rows: 4096 x 4096 13.2 .. 15.8 -> 10.7 .. 13.7 us, 6144 x 4096 14.7 .. 18.1 -> 14.6 ..
+// 17.4, 4096 x 14336 24.9 .. 29.7 -> 22.6 .. 27.8, 12288 x 4096 22.4 .. 26.0 -> 23.1 .. 26.6.  The stream, in the longest pieces of a k row
+// that still give the CUs work, where nothing is to be split, against more than 64 columns a CU and in the gap below 6144: 28672 x 4096
+// 43 -> 40 us, 128256 x 4096 171 -> 160; without a workspace 4096 x 4096 40 -> 16.
+template <class E>
+static int launch_classes(const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
+                          int ldc, int most, float* P, hipStream_t s) {
+  const int tiles = (N + 127) / 128, cus = cu_count();
+  int shares = tiles <= cus / 8 || in_a_gap(N, K) ? 8 : tiles <= cus / 4 ? 4 : tiles <= cus / 2 ? 2 : 1;
+  if (most >= 8 && N > 16 * cus && N <= 22 * cus)  // 5120 x 5120: 15.3 us, 16.2 in 4 shares of the others
+    return launch_splitk<E, 64, 256, 1, 4, false, false, kWholeCu, 1>(A, B, C, D, M, N, K, alpha, beta, ldc, 8, 0, P, s);
+  if (in_a_gap(N, K) && K < 6144) shares = 1;
+  while (shares > most) shares /= 2;
+  if (shares > 1) return launch_splitk<E, 64, 128, 2, 2, false, false, kHalfCu, 2>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, 0, P, s);
+  auto rows = [&](auto ar_c) {
+    constexpr int AR = decltype(ar_c)::value;
+    if (N <= 16 * cus) return launch_rows<E, AR, 1, 8, 1, 1, false, false>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+    if (N <= 32 * cus) return launch_rows<E, AR, 2, 8, 1, 1, false, false>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+    if constexpr (AR <= 32)
+      if (N > 64 * cus) return launch_rows<E, AR, 8, 8, 1, 1, false, false>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+    return launch_rows<E, AR, 4, 8, 1, 1, false, false>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  };
+  return M <= 8 ? rows(ic<8>{}) : M <= 16 ? rows(ic<16>{}) : M <= 32 ? rows(ic<32>{}) : rows(ic<64>{});
+}
+
+// The same for the pair: 64 x 128 tiles (1 to 64 rows of 8192 x 8192 57 .. 63 -> 53 .. 61 us), or the stream, also against few columns and a
+// short contraction (32 x 2048 x 2048 14.4 -> 12.5; 28672 x 8192 167 -> 157).
+template <class E>
+static int launch_classes_dual(const uint16_t* A, const uint16_t* Bg, const uint16_t* Bu, uint16_t* out, int M, int N, int K, int most, float* P,
+                               hipStream_t s) {
+  const int cus = cu_count(), shares = most >= 8 ? 8 : most >= 4 ? 4 : 2;
+  const bool narrow = N <= 4 * cus && K < 4096;
+  if (most > 1 && !narrow) return launch_splitk<E, 64, 128, 2, 2, false, true, kWholeCu, 2>(A, Bg, nullptr, out, M, N, K, 1.f, 0.f, N, shares, 0, P, s, Bu);
+  auto rows = [&](auto ar_c) {
+    constexpr int AR = decltype(ar_c)::value;
+    if (narrow) return launch_rows<E, AR, 2, 8, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    if constexpr (AR <= 32)
+      if (N > 64 * cus) return launch_rows<E, AR, 8, 4, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+    return launch_rows<E, AR, 4, 4, 2, 1, false, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+  };
+  return M <= 8 ? rows(ic<8>{}) : M <= 16 ? rows(ic<16>{}) : M <= 32 || narrow ? rows(ic<32>{}) : rows(ic<64>{});
 }
 
 }  // namespace nf

@@ -42,6 +42,39 @@ def test_products_of_few_rows(M, N, K_):
         assert torch.equal(got[M - 1:], K.gemm_ws(a[M - 1:].clone(), b, b_col_major=True)[0])
 
 
+# every count of shares that the [K][N] tiles take (1, 2, 4, 8 of the classes), units that do not fill the classes evenly, cut slabs; and
+# launches that are split over K into runs
+LAYOUTS = SHAPES + [(1, 4096, 4096), (16, 1000, 5000), (33, 8192, 4104), (64, 2056, 4160), (9, 10240, 8192), (48, 12296, 4096), (64, 28680, 2048),
+                    (5, 33000, 1536), (17, 4096, 14336), (64, 40, 8200), (50, 5120, 5128)]
+
+
+@pytest.mark.parametrize("M,N,K_", LAYOUTS)
+def test_both_layouts_of_the_weights_have_the_same_bits(M, N, K_):
+    from nanoflow_amd import kernels as K
+    a, b = operands(M, N, K_, torch.float16)
+    kn = b.t().contiguous()
+    c, bias = torch.randn(M, N, device="cuda").half(), torch.randn(N, device="cuda").half()
+    need = K.lib().nf_gemm_workspace_bytes(M, N, K_)
+    for size in {max(need, 16), 64 << 20}:
+        ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+        both = lambda **kw: [K.gemm_ws(a, w, b_col_major=col, workspace=ws, **kw)[0] for w, col in ((b, True), (kn, False))]
+        assert torch.equal(*both())
+        assert torch.equal(*both(Cmat=c, alpha=0.7, beta=-1.3))
+        assert torch.equal(*both(bias=bias, alpha=0.7, beta=1.9))
+    assert torch.equal(K.gemm(a, b, c, 0.7, -1.3, b_col_major=True), K.gemm(a, kn, c, 0.7, -1.3))
+    ab, bb = a.bfloat16(), b.bfloat16()
+    assert torch.equal(K.gemm(ab, bb, b_col_major=True), K.gemm(ab, bb.t().contiguous()))
+    check(K.gemm_ws(a, kn)[0], a.double() @ b.double().t(), a, b, K_, 11)
+    half = max(N // 16 * 8, 8)                                   # the pair, with its workspace, with a short one and without
+    g, u = b[:half].contiguous(), b[-half:].contiguous()
+    kg, ku = g.t().contiguous(), u.t().contiguous()
+    need = K.lib().nf_dual_swiglu_workspace_bytes(M, half, K_)
+    for size in {max(need, 16), 16}:
+        ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+        assert torch.equal(K.dual_swiglu_ws(a, g, u, b_col_major=True, workspace=ws)[0], K.dual_swiglu_ws(a, kg, ku, workspace=ws)[0])
+    assert torch.equal(K.dual_swiglu(a, g, u, b_col_major=True), K.dual_swiglu(a, kg, ku))
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 2048, 2048), (16, 40, 1544), (33, 72, 2048), (64, 2056, 4096), (40, 264, 8192)])
 def test_bfloat16_products_and_sums(M, N, K_):
     from nanoflow_amd import kernels as K
