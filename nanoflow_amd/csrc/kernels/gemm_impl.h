@@ -1312,7 +1312,7 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   int k_per = 0;
   // a workspace for the sums of at most 512 rows, or of a dense launch, has to be aligned, whatever runs; others run unsplit without
   NF_REQUIRE(!given || aligned || (M > kSplitMaxRows && dense_split_plan(M, N, K, &k_per) < 2), "%s: the workspace must be 16-byte aligned", who);
-  const bool few = few_pay(M, N, K), whole = M > kTallRows ? mid.shares < 2 : few && b_col_major;
+  const bool few = few_pay(M, N, K) && !(given && aligned && narrow_and_deep(M, N, K)), whole = M > kTallRows ? mid.shares < 2 : few && b_col_major;
   if (!given || !aligned || whole) return gemm_entry<E>(who, A, B, C, D, M, N, K, alpha, beta, b_col_major, stream, c_is_row);
   const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
   int rc = check_gemm_args(who, A, B, D, M, N, K);

@@ -5,7 +5,9 @@
 namespace {
 
 // Tile of a launch that stores fp32 sums, and its split over K.  Few rows: whole sums where the kernel of gemm_rows.h pays, else
-// 64 x 64 tiles in as many shares as give every CU a workgroup.  Other launches: enough shares of at least 128 to give
+// 64 x 64 tiles in as many shares as give every CU a workgroup.  Up to 4 columns a CU (8 from K = 8192 on) that kernel has too few workgroups for more than
+// 16 rows or a contraction of 4096 or more, and sums need no second launch: 64 x 64 tiles in shares of 256 or more (64 x 64 x 2048 5.3
+// -> 3.3 us, 64 x 1024 x 4096 7.9 -> 4.9, 16 x 1024 x 14336 18.1 -> 7.9).  Other launches: enough shares of at least 128 to give
 // every CU a tile while the sums stay within 64 MiB; two shares of 256 x 256 tiles where dense_split_plan
 // says so; else, from 257 rows on, the largest tile that still gives every CU work.
 struct SumPlan {
@@ -15,6 +17,12 @@ struct SumPlan {
 
 SumPlan sum_plan(int M, int N, int K, int max_shares) {
   SumPlan p{M <= 64 ? 0 : 1, 1, (K + BK - 1) / BK * BK};
+  if (max_shares > 1 && rows_pay(M, N, K) && N <= (K >= 8192 ? 8 : 4) * cu_count() && (M > 16 || K >= 4096)) {
+    const int shares = std::min(std::min(2 * cu_count() / ((N + 63) / 64), K / 256), std::min(max_shares, kMaxShares));
+    p = SumPlan{4, 1, ((K + shares - 1) / shares + BK - 1) / BK * BK};
+    p.shares = (K + p.k_per - 1) / p.k_per;
+    return p;
+  }
   if (rows_pay(M, N, K)) {
     p.tile = 3;
     return p;

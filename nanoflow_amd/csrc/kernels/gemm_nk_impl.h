@@ -19,7 +19,7 @@ static int gemm_nk_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   const int shares = M <= kTallRows ? splitk_plan(M, N, K, &k_per) : 1;
   const bool aligned = (uintptr_t)workspace % 16 == 0, given = shares > 1 && workspace && workspace_bytes >= (size_t)shares * M * N * sizeof(float);
   NF_REQUIRE(!given || aligned, "%s: the workspace must be 16-byte aligned", who);  // whatever runs
-  if (rows_pay(M, N, K)) return dispatch_rows<E, false>(A, B, bias, D, M, N, K, 1.f, beta, ldc, s);
+  if (rows_pay(M, N, K) && !(given && narrow_and_deep(M, N, K))) return dispatch_rows<E, false>(A, B, bias, D, M, N, K, 1.f, beta, ldc, s);
   if (workspace && aligned && M > kTallRows) {
     const MidPlan mid = mid_split_plan(M, N, K, kMidBytes);
     if (mid.shares > 1 && workspace_bytes >= (size_t)mid.shares * M * N * sizeof(float))

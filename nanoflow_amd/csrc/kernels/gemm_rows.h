@@ -313,6 +313,12 @@ static bool rows_pay(int M, int N, int K, int row_bytes = 0) {
 static bool in_a_gap(int N, int K) { return N > 32 * cu_count() && N <= 44 * cu_count() && K >= 4096; }
 static bool few_pay(int M, int N, int K) { return rows_pay(M, N, K) && (M <= 8 || !in_a_gap(N, K)); }
 
+// With a workspace there is another choice: few columns against a long contraction are few workgroups, each with all of K to take in, and
+// better off split (splitk_plan_narrow; 16 x 1024 x 14336 17.6 us here, 11.2 so, 16 x 2048 x 14336 19.6 and 15.6, one row of it 13.9 and
+// 15.2, 8 x 512 x 14336 12.7 and 8.9, 16 x 1024 x 8192 9.5 and 8.7, 16 x 2048 x 8192 10.9 and 11.8; [K][N] weights 1 x 2048 x 14336 18.7
+// and 15.7).
+static bool narrow_and_deep(int M, int N, int K) { return M <= 16 && K >= 8192 && N <= (K > 8192 ? 8 : 4) * cu_count(); }
+
 // The same for the gate/up pair of 16-bit or e4m3 (f8) operands.  Few columns against a long contraction, or workgroups that spill over
 // into another round, lose to the tiles and their split over K: 64 x 512 x 14336 63 us against 20, 16 x 4096 x 14336 56 against 46, 64 x
 // 10240 x 8192 86 against 73, e4m3 64 x 512 x 14336 29 against 15.  Both sides by what they take in: here a workgroup's rows of both weights and of A over the whole of K at

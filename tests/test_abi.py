@@ -149,3 +149,12 @@ def test_rows_of_an_experts_tile_without_a_gpu():
     rows = K.lib().nf_grouped_tile_rows
     assert [rows(K.BF16, n, 32) for n in (1, 96 * 32, 96 * 32 + 1, 117 * 32, 120 * 32, 5000)] == [64, 64, 128, 128, 128, 128]
     assert len({rows(K.F32, n, 32) for n in (1, 4000)}) == 1
+
+
+def test_sums_of_few_columns_are_split_without_a_gpu():
+    """Whole sums of few rows leave most of the chip idle against few columns: shares of 256 or more of K where the caller takes them."""
+    from nanoflow_amd import kernels as K
+    shares = K.lib().nf_gemm_nk_sums_shares
+    assert shares(64, 64, 2048, 16) == 8 and shares(17, 1024, 4096, 16) == 16 and shares(16, 1024, 14336, 16) == 16
+    assert shares(64, 64, 2048, 4) == 4 and shares(64, 64, 2048, 1) == 1
+    assert shares(16, 64, 2048, 16) == 1 and shares(64, 4096, 4096, 16) == 1 and shares(64, 2048, 2048, 16) == 1

@@ -45,7 +45,7 @@ def test_products_of_few_rows(M, N, K_):
 # every count of shares that the [K][N] tiles take (1, 2, 4, 8 of the classes), units that do not fill the classes evenly, cut slabs; and
 # launches that are split over K into runs
 LAYOUTS = SHAPES + [(1, 4096, 4096), (16, 1000, 5000), (33, 8192, 4104), (64, 2056, 4160), (9, 10240, 8192), (48, 12296, 4096), (64, 28680, 2048),
-                    (5, 33000, 1536), (17, 4096, 14336), (64, 40, 8200), (50, 5120, 5128)]
+                    (5, 33000, 1536), (3, 1024, 8200), (16, 2048, 14336), (9, 1032, 9000), (17, 4096, 14336), (64, 40, 8200), (50, 5120, 5128)]
 
 
 @pytest.mark.parametrize("M,N,K_", LAYOUTS)
@@ -75,7 +75,8 @@ def test_both_layouts_of_the_weights_have_the_same_bits(M, N, K_):
     assert torch.equal(K.dual_swiglu(a, g, u, b_col_major=True), K.dual_swiglu(a, kg, ku))
 
 
-@pytest.mark.parametrize("M,N,K_", [(1, 2048, 2048), (16, 40, 1544), (33, 72, 2048), (64, 2056, 4096), (40, 264, 8192)])
+@pytest.mark.parametrize("M,N,K_", [(1, 2048, 2048), (16, 40, 1544), (33, 72, 2048), (64, 2056, 4096), (40, 264, 8192), (64, 64, 2048), (17, 1024, 4104),
+                                    (16, 1024, 14336), (9, 520, 9000), (2, 40, 4096)])
 def test_bfloat16_products_and_sums(M, N, K_):
     from nanoflow_amd import kernels as K
     a, b = operands(M, N, K_, torch.bfloat16)
