@@ -194,29 +194,47 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(u32x4* __restrict__ out,
 
 // Candidate order of the reference sampler: larger value wins; equal values: smaller key,
 // key = bitreverse10(col mod 1024) << 20 | col.  Values <= -10000 (and NaN) never win.
-__device__ __forceinline__ uint32_t arg_key(uint32_t col) {
-  return ((__brev(col & 1023u) >> 22) << 20) | col;
+// Columns c .. c + 7 (c = 8 i) of a thread's vector i: their bits of col mod 1024 reversed are those of the place e in the vector, then
+// those of i mod 128, the same for all vectors of a thread.  What is left of the key here: kPlace[e] on top, e below.
+__device__ __forceinline__ uint32_t arg_key_of_equals(const u32x4& v, _Float16 best) {
+  constexpr uint32_t kPlace[8] = {0, 4, 2, 6, 1, 5, 3, 7};
+  const uint32_t p[4] = {v.x, v.y, v.z, v.w};
+  uint32_t key = 0xffffffffu;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const _Float16 h = __builtin_bit_cast(_Float16, (uint16_t)(p[e / 2] >> (e % 2 * 16)));
+    key = min(key, h == best ? kPlace[e] << 27 | (uint32_t)e : 0xffffffffu);
+  }
+  return key;
 }
 
-// Bound by reading a row once.  First the row's maximum, two halves an instruction and eight 16-byte loads in flight a thread, then
-// the threads that hold it read their columns again and look which of them it is.  (200 rows of 128256: 26 -> 16 us; comparing
-// value and key at every element took three times the loads' time.)
+// Bound by reading a row once.  First the row's maximum, two halves an instruction, then the threads that hold it look which of
+// their columns it is.  kHeld > 0: a row of at most kHeld x 8192 columns stays in registers between the two; one vector a thread
+// (kHeld 1) finds both at once and meets the others with the pair.  Longer rows are read in eight loads a thread, and again by the
+// threads that hold the maximum.  us, comparing value and key at every element before: 200 rows of 128256 19.9 -> 12.8, 200 x 32000 8.0 ->
+// 5.6, 2048 x 8192 16.9 -> 12.6, 2048 x 1024 12.6 -> 9.4.  (Slower: rows of more than 65536 columns that are all equal, 2048 x 128256
+// 108 -> 148.)
+template <int kHeld>
 __global__ __launch_bounds__(1024) void argmax_kernel(const uint16_t* __restrict__ logits,
                                                       uint16_t* __restrict__ max_vals,
                                                       int32_t* __restrict__ arg, int cols) {
   typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
   __shared__ float s_v[16];
   __shared__ uint32_t s_k[16];
-  constexpr int kAhead = 8;
+  constexpr int kAhead = kHeld > 0 ? kHeld : 8;
   const int r = blockIdx.x, tid = threadIdx.x;
   const uint16_t* x = logits + (long long)r * cols;
   const int nvec = cols >> 3;
   const u32x4* xv = reinterpret_cast<const u32x4*>(x);
-  f16x2 top = {(_Float16)-10000.f, (_Float16)-10000.f};  // NaN never wins
-  for (int i0 = tid; i0 < nvec; i0 += kAhead * 1024) {
-    u32x4 v[kAhead];
+  const uint32_t none = 0xf0e2f0e2u;  // -10000 twice
+  f16x2 top = __builtin_bit_cast(f16x2, none);  // NaN never wins
+  u32x4 v[kAhead];
+  auto load = [&](int i0) {
 #pragma unroll
-    for (int u = 0; u < kAhead; ++u) v[u] = xv[min(i0 + u * 1024, nvec - 1)];  // past the row: its last columns once more
+    for (int u = 0; u < kAhead; ++u) v[u] = i0 + u * 1024 < nvec ? xv[i0 + u * 1024] : u32x4{none, none, none, none};
+  };
+  for (int i0 = tid; i0 < nvec; i0 += kAhead * 1024) {
+    load(i0);
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const uint32_t p[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
@@ -226,39 +244,57 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const uint16_t* __restrict
   }
   const float mine = fmaxf((float)top[0], (float)top[1]);
   float best = mine;
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) best = fmaxf(best, __shfl_xor(best, m, 64));
-  if ((tid & 63) == 0) s_v[tid >> 6] = best;
-  __syncthreads();
-  best = s_v[tid & 15];
-#pragma unroll
-  for (int m = 8; m > 0; m >>= 1) best = fmaxf(best, __shfl_xor(best, m, 64));
   uint32_t key = 0xffffffffu;
-  if (mine == best && best > -10000.f)
+  auto find = [&]() {  // smallest key of this thread's columns that equal `mine`
+    const uint32_t of_thread = (__brev((uint32_t)tid & 127u) >> 25) << 20;
     for (int i0 = tid; i0 < nvec; i0 += kAhead * 1024) {
-      u32x4 v[kAhead];
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u) v[u] = xv[min(i0 + u * 1024, nvec - 1)];
+      if constexpr (kHeld == 0) load(i0);
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
-        const uint32_t p[4] = {v[u].x, v[u].y, v[u].z, v[u].w}, c = (uint32_t)min(i0 + u * 1024, nvec - 1) * 8u;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (h2f_bits(p[j] & 0xffffu) == best) key = min(key, arg_key(c + 2 * j));
-          if (h2f_bits(p[j] >> 16) == best) key = min(key, arg_key(c + 2 * j + 1));
-        }
+        const uint32_t k = arg_key_of_equals(v[u], (_Float16)mine);
+        if (k != 0xffffffffu && i0 + u * 1024 < nvec) key = min(key, k + of_thread + (uint32_t)(i0 + u * 1024) * 8u);
       }
     }
+  };
+  auto take = [&](float ov, uint32_t ok) {
+    if (ov > best || (ov == best && ok < key)) {
+      best = ov;
+      key = ok;
+    }
+  };
+  if constexpr (kHeld == 1) {
+    if (mine > -10000.f) find();
 #pragma unroll
-  for (int m = 32; m > 0; m >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, m, 64));
-  if ((tid & 63) == 0) s_k[tid >> 6] = key;
+    for (int m = 32; m > 0; m >>= 1) take(__shfl_xor(best, m, 64), (uint32_t)__shfl_xor((int)key, m, 64));
+  } else {
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) best = fmaxf(best, __shfl_xor(best, m, 64));
+    if ((tid & 63) == 0) s_v[tid >> 6] = best;
+    __syncthreads();
+    best = s_v[tid & 15];
+#pragma unroll
+    for (int m = 8; m > 0; m >>= 1) best = fmaxf(best, __shfl_xor(best, m, 64));
+    if (mine == best && best > -10000.f) find();
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, m, 64));
+    __syncthreads();  // s_v has been read
+  }
+  if ((tid & 63) == 0) {
+    s_v[tid >> 6] = best;
+    s_k[tid >> 6] = key;
+  }
   __syncthreads();
-  if (tid == 0) {
-    for (int i = 1; i < 16; ++i) key = min(key, s_k[i]);
-    const bool any = key != 0xffffffffu;  // else nothing above -10000
-    const int32_t col = any ? (int32_t)(key & 0xfffffu) : 0;
-    arg[r] = col;
-    if (max_vals) max_vals[r] = any ? x[col] : (uint16_t)f2h_bits(-10000.f);
+  if (tid < 64) {
+    best = s_v[tid & 15];
+    key = s_k[tid & 15];
+#pragma unroll
+    for (int m = 8; m > 0; m >>= 1) take(__shfl_xor(best, m, 64), (uint32_t)__shfl_xor((int)key, m, 64));
+    if (tid == 0) {
+      const bool any = key != 0xffffffffu;  // else nothing above -10000
+      const int32_t col = any ? (int32_t)(key & 0xfffffu) : 0;
+      arg[r] = col;
+      if (max_vals) max_vals[r] = any && best == 0.f ? x[col] : (uint16_t)f2h_bits(any ? best : -10000.f);  // 0 or -0, as it lies
+    }
   }
 }
 
@@ -519,7 +555,8 @@ int nf_argmax_f16(const uint16_t* logits, uint16_t* max_vals, int32_t* argmax, i
              "nf_argmax_f16: cols=%d must be a multiple of 8 below 2^20 (rows=%d)", cols, rows);
   if (rows == 0) return NF_OK;
   NF_REQUIRE(logits && argmax, "nf_argmax_f16: null pointer");
-  argmax_kernel<<<rows, 1024, 0, (hipStream_t)stream>>>(logits, max_vals, argmax, cols);
+  auto kern = cols <= 8192 ? argmax_kernel<1> : cols <= 65536 ? argmax_kernel<8> : argmax_kernel<0>;
+  kern<<<rows, 1024, 0, (hipStream_t)stream>>>(logits, max_vals, argmax, cols);
   return check_launch("nf_argmax_f16");
 }
 

@@ -17,7 +17,7 @@ def literal(x):
     return best, x[best]
 
 
-@pytest.mark.parametrize("cols", [8, 1016, 8184, 8192, 8200, 65528, 65544, 128256, (1 << 20) - 8])
+@pytest.mark.parametrize("cols", [8, 1016, 8184, 8192, 8200, 65528, 65536, 65544, 128256, (1 << 20) - 8])
 def test_argmax_of_halves(cols):
     from nanoflow_amd import kernels as K
     rng = np.random.default_rng(cols)
