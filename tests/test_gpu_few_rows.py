@@ -1,4 +1,5 @@
-"""Products of at most 64 rows on whole-K workgroups (csrc/kernels/gemm_rows.h): every tile of the dispatch at its edges, against
+"""Products of at most 64 rows on whole-K workgroups (csrc/kernels/gemm_rows.h), and on the tiles that take [K][N] weights in the same
+order: every tile of the dispatches (for 256 CUs) on ragged columns and at the edges of its rows, against
 float64.  An element may be off by its one rounding to 16 bits and by what fp32 sums of K terms can lose:
 2^-p |r| + K 2^-24 sum |a||b| (p = 11 significant bits for fp16, 8 for bf16)."""
 import pytest
@@ -44,7 +45,7 @@ def test_products_of_few_rows(M, N, K_):
 
 # every count of shares that the [K][N] tiles take (1, 2, 4, 8 of the classes), units that do not fill the classes evenly, cut slabs; and
 # launches that are split over K into runs
-LAYOUTS = SHAPES + [(1, 4096, 4096), (16, 1000, 5000), (33, 8192, 4104), (64, 2056, 4160), (9, 10240, 8192), (48, 12296, 4096), (64, 28680, 2048),
+LAYOUTS = SHAPES + [(17, 8200, 1600), (32, 14344, 1544), (16, 8264, 1544), (16, 5128, 4160), (33, 4104, 4104), (16, 33000, 1536), (24, 33008, 1544), (1, 4096, 4096), (16, 1000, 5000), (33, 8192, 4104), (64, 2056, 4160), (9, 10240, 8192), (48, 12296, 4096), (64, 28680, 2048),
                     (5, 33000, 1536), (3, 1024, 8200), (16, 2048, 14336), (9, 1032, 9000), (17, 4096, 14336), (64, 40, 8200), (50, 5120, 5128)]
 
 
@@ -76,7 +77,8 @@ def test_both_layouts_of_the_weights_have_the_same_bits(M, N, K_):
 
 
 @pytest.mark.parametrize("M,N,K_", [(1, 2048, 2048), (16, 40, 1544), (33, 72, 2048), (64, 2056, 4096), (40, 264, 8192), (64, 64, 2048), (17, 1024, 4104),
-                                    (16, 1024, 14336), (9, 520, 9000), (2, 40, 4096)])
+                                    (16, 1024, 14336), (9, 520, 9000), (2, 40, 4096), (1, 4104, 1536), (16, 4104, 1544), (32, 2056, 1536), (64, 4104, 1544),
+                                    (32, 8200, 1544), (64, 8200, 1536)])
 def test_bfloat16_products_and_sums(M, N, K_):
     from nanoflow_amd import kernels as K
     a, b = operands(M, N, K_, torch.bfloat16)
@@ -128,10 +130,39 @@ def test_e4m3_products_of_few_rows(M, N, K_):
     assert bool(((got.double() - pair).abs() <= 1.1 * up.abs() * lost(g, bv) + g.abs() * lost(up, uv) + 2.0 ** -10 * pair.abs() + 1e-6).all())
 
 
+@pytest.mark.parametrize("M,N,K_", [(17, 14344, 3088), (32, 8200, 3104), (33, 8264, 3072), (64, 8200, 3088)])
+def test_e4m3_products_of_few_rows_against_many_columns(M, N, K_):
+    test_e4m3_products_of_few_rows(M, N, K_)
+
+
+@pytest.mark.parametrize("K_", [4096, 8192, 14336, 32784])
+def test_row_quantiser_of_nan_and_infinity(oracle, K_):
+    """NaN takes no part in a row's maximum and becomes 448 like everything above it, of either sign; beside an infinity finite values become
+    zeros of their sign.  Quiet and signalling NaN of both signs in every lane position of a chunk, on every row length's kernel."""
+    import numpy as np
+    from nanoflow_amd import kernels as K
+    rng = np.random.default_rng(K_)
+    x = (rng.standard_normal((24, K_)) * 10.0 ** rng.integers(-6, 4, (24, 1))).astype(np.float16).view(np.uint16)
+    for row in range(24):
+        at = rng.choice(K_, 64, replace=False)
+        at[:8] = np.arange(8) + 8 * rng.integers(0, K_ // 8)                      # a whole chunk of them
+        x[row, at] = np.resize(np.array([0x7e00, 0xfe00, 0x7c01, 0xfc01, 0x7d55, 0xffff], dtype=np.uint16), 64)
+    x[16:20, rng.integers(0, K_, 3)] = 0x7c00
+    x[18:22, rng.integers(0, K_, 3)] = 0xfc00
+    x[22] = np.resize(np.array([0x7e00, 0xfc01], dtype=np.uint16), K_)           # nothing else: the scale of a row of zeros
+    v = x.view(np.float16).astype(np.float32)
+    q, s = K.quantize_rows_e4m3(torch.from_numpy(x.view(np.float16).copy()).cuda())
+    q_ref, s_ref = oracle.quantize_rows_e4m3(x.view(np.float16))
+    assert np.array_equal(s.cpu().numpy(), s_ref) and s_ref[22] == 1 and np.isinf(s_ref[16:22]).all()
+    q, special = q.cpu().numpy(), np.isnan(v) | (np.isinf(v) & np.isinf(s_ref)[:, None])   # NaN, or infinity over infinity: no sign to speak of
+    assert np.array_equal(q[~special], q_ref[~special])
+    assert (q[special] & 0x7f == 0x7e).all() and (q_ref[special] & 0x7f == 0x7e).all()
+
+
 @pytest.mark.parametrize("K_", [4096, 8192, 14336, 32784])
 def test_row_quantiser_over_every_half(oracle, K_):
-    """Rows that hold all halves up to a maximum (the largest, ordinary ones, the smallest, subnormal ones, infinity) and NaN, on every
-    row length's kernel: the oracle's bytes and scales."""
+    """Rows that hold all halves up to a maximum (the largest, ordinary ones, the smallest, subnormal ones), on every row length's
+    kernel: the oracle's bytes and scales; of rows with an infinity the scales."""
     import numpy as np
     from nanoflow_amd import kernels as K
     every = np.arange(65536, dtype=np.uint16)

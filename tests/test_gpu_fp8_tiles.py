@@ -17,7 +17,8 @@ def operands(M, N, K_, n):
 
 
 @pytest.mark.parametrize("K_", DEPTHS)
-@pytest.mark.parametrize("M,N", [(2048, 8192), (1800, 8008), (2000, 6152), (1793, 5960)])  # 256 x 256 tiles, 256 x 192
+@pytest.mark.parametrize("M,N", [(2048, 8192), (1800, 8008), (2000, 6152), (1793, 5960), (2000, 6144), (2000, 10240), (1990, 10216)])
+# 256 x 256 tiles of the first three, 256 x 192 of the others (whole and ragged columns; 32 to 54 tiles of columns)
 def test_products(M, N, K_):
     from nanoflow_amd import kernels as K
     (a, b), (sa, sb), (av, bv), gen = operands(M, N, K_, 1)
