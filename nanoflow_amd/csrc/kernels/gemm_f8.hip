@@ -750,13 +750,23 @@ size_t nf_gemm_f8w_workspace_bytes(int M, int K) {
   return ((size_t)M * K + 255) / 256 * 256 + (size_t)M * sizeof(float);
 }
 
+// Where the weight stream takes the launch and a split over K is still faster: 33 to 44 columns a CU, whose workgroups leave half a round
+// empty, against a long contraction (16 x 9728 x 12288 28.9 us there, 24.1 in shares, 32 rows 30.7 and 25.2, 64 rows 37.4 and 27.8; 64 x
+// 10240 x 14336 39.8 and 34.2).  From 33 rows on it begins earlier and ends later (64 x 10240 x 9216 30.6 and 26.7, x 8192 24.3 and 25.1;
+// 48 x 12288 x 10240 30.8 and 28.2, x 13312 33.8 and 31.6).  At 16 x 10240 x 9216 and 16384 the stream is ahead again (22.3 and 22.6, 36.4
+// and 39), and 64 x 13312 x 16384 has 46 and 53.
+static bool split_pays_f8(int M, int N, int K) {
+  const int cus = cu_count();
+  return M > 8 && K > (M > 32 ? 8192 : 9216) && K <= 14336 && N > 32 * cus && N <= (M > 32 ? 48 : 44) * cus;
+}
+
 // The GEMM on rows that are quantised already: split over K when the launch has few rows against a
 // narrow N and the workspace holds the partial sums behind the place of the quantised rows.
 static int gemm_f8q(const uint8_t* Aq, const float* sa, const uint8_t* Bq, const float* b_scale, const uint16_t* C,
                     uint16_t* D, int M, int N, int K, float alpha, float beta, void* workspace, size_t workspace_bytes,
                     nf_stream_t stream) {
   int k_per = 0;
-  const int shares = N > 0 && N % 8 == 0 && K % 16 == 0 && !rows_pay(M, N, K, K) ? splitk_plan_f8(M, N, K, false, &k_per) : 1;
+  const int shares = N > 0 && N % 8 == 0 && K % 16 == 0 && (!rows_pay(M, N, K, K) || split_pays_f8(M, N, K)) ? splitk_plan_f8(M, N, K, false, &k_per) : 1;
   const size_t p_at = (nf_gemm_f8w_workspace_bytes(M, K) + 255) / 256 * 256;
   if (shares >= 2 && workspace && (uintptr_t)workspace % 16 == 0 &&
       workspace_bytes >= p_at + (size_t)shares * M * N * sizeof(float) && Bq && b_scale && D &&

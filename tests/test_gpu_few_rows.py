@@ -135,6 +135,25 @@ def test_e4m3_products_of_few_rows_against_many_columns(M, N, K_):
     test_e4m3_products_of_few_rows(M, N, K_)
 
 
+# 33 to 44 columns a CU against a long contraction: shares of K from 9 rows on, where the workspace holds their sums
+@pytest.mark.parametrize("M,N,K_,shared", [(9, 8200, 9232, True), (32, 11264, 9232, True), (33, 12288, 8208, True), (64, 8200, 14336, True),
+                                           (8, 8200, 9232, False), (32, 8200, 9216, False), (64, 8200, 8192, False), (16, 8200, 14352, False)])
+def test_e4m3_products_in_shares(M, N, K_, shared):
+    from nanoflow_amd import kernels as K
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K_)
+    codes = lambda r: torch.randn((r, K_), generator=gen, device="cuda").to(torch.float8_e4m3fn)
+    scales = lambda r: torch.rand(r, generator=gen, device="cuda") + 0.5
+    a, b, sa, sb = codes(M), codes(N), scales(M), scales(N) * K_ ** -0.5
+    av, bv = a.float().double() * sa.double()[:, None], b.float().double() * sb.double()[:, None]
+    need = K.lib().nf_gemm_f8w_split_workspace_bytes(M, N, K_)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device="cuda")
+    check(K.gemm_f8q(a.view(torch.uint8), sa, b.view(torch.uint8), sb, workspace=ws), av @ bv.t(), av, bv, K_, 11)
+    assert bool((ws != 255).any()) == shared
+    short = torch.full((need - 256,), 255, dtype=torch.uint8, device="cuda")
+    check(K.gemm_f8q(a.view(torch.uint8), sa, b.view(torch.uint8), sb, workspace=short), av @ bv.t(), av, bv, K_, 11)
+    assert bool((short == 255).all())
+
+
 @pytest.mark.parametrize("K_", [4096, 8192, 14336, 32784])
 def test_row_quantiser_of_nan_and_infinity(oracle, K_):
     """NaN takes no part in a row's maximum and becomes 448 like everything above it, of either sign; beside an infinity finite values become
