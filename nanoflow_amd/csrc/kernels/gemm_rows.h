@@ -343,18 +343,23 @@ static int rows_cost(int N, int nt, int m_tiles, int a_panels) { return ((N + nt
 template <class E, bool kSums>
 static int dispatch_rows(const void* A, const void* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
                          int ldc, hipStream_t s, const RowsScales& sc = {}) {
+  // Short e4m3 rows against many columns want workgroups of 32, whatever the rounds say: 16 are over too soon (1 x 28672 x 4096 25.0 us, 21.9
+  // so, 4 x 20480 x 6144 22.8 and 21.3; from 8 KB on the same in both), and 64 have few wavefronts a CU (17 x 28672 x 4096 25.7 and
+  // 23.9, 17 x 57344 x 4096 47.5 and 40.7; but 32 x 28672 x 6144 34.1 and 36.5).
+  const bool f8 = std::is_same_v<E, RowsF8>, brief = f8 && K < 8192 && N > 64 * cu_count();
   if (M <= 8)  // a tie goes to fewer, wider workgroups (1 x 6144 x 4096: 9.9 us against 11.2)
-    return rows_cost(N, 1, 1, 0) < rows_cost(N, 2, 1, 0) ? launch_rows<E, 8, 1, 8, 1, 3, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc)
+    return !brief && rows_cost(N, 1, 1, 0) < rows_cost(N, 2, 1, 0) ? launch_rows<E, 8, 1, 8, 1, 3, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc)
                                                          : launch_rows<E, 8, 2, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
   if (M <= 16)
     return rows_cost(N, 1, 1, 1) < rows_cost(N, 2, 1, 1) ? launch_rows<E, 16, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc)
                                                          : launch_rows<E, 16, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
+  const bool pairs = f8 && M <= 32 && K <= 4096 && N > 96 * cu_count();
   const int half = (M + 31) / 32;  // m tiles of 32 rows
   const int c1 = rows_cost(N, 1, half, 2), c2 = rows_cost(N, 2, half, 2);
   const int w2 = M <= 32 ? 1 << 30 : rows_cost(N, 2, 1, 4), w4 = rows_cost(N, 4, 1, M <= 32 ? 2 : 4);
   const int best = std::min(std::min(c1, c2), std::min(w2, w4));
-  if (best == c1) return launch_rows<E, 32, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
-  if (best == c2) return launch_rows<E, 32, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
+  if (best == c1 && !pairs) return launch_rows<E, 32, 1, 8, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
+  if (best == c2 || pairs) return launch_rows<E, 32, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
   if (best == w2) return launch_rows<E, 64, 2, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);
   return M <= 32 ? launch_rows<E, 32, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc)
                  : launch_rows<E, 64, 4, 4, 1, 2, true, kSums>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s, sc);

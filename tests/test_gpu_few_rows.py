@@ -130,7 +130,8 @@ def test_e4m3_products_of_few_rows(M, N, K_):
     assert bool(((got.double() - pair).abs() <= 1.1 * up.abs() * lost(g, bv) + g.abs() * lost(up, uv) + 2.0 ** -10 * pair.abs() + 1e-6).all())
 
 
-@pytest.mark.parametrize("M,N,K_", [(17, 14344, 3088), (32, 8200, 3104), (33, 8264, 3072), (64, 8200, 3088)])
+@pytest.mark.parametrize("M,N,K_", [(17, 14344, 3088), (32, 8200, 3104), (33, 8264, 3072), (64, 8200, 3088), (1, 16392, 3088), (8, 20488, 8176),
+                                    (8, 20488, 8192), (17, 24584, 4096), (32, 24584, 3088), (32, 24584, 4112)])
 def test_e4m3_products_of_few_rows_against_many_columns(M, N, K_):
     test_e4m3_products_of_few_rows(M, N, K_)
 
