@@ -204,7 +204,7 @@ def test_row_quantiser_over_every_half(oracle, K_):
 # rows of each expert, and whether every token also goes to one more
 COUNTS = [([1], False), ([0, 1, 15, 16, 0, 3, 9, 0], False), ([17, 0, 32, 31, 1, 2, 0, 0, 0, 16], False), ([33, 48, 47, 0, 16, 1], False),
           ([49, 0, 0, 64, 5, 8], False), ([65, 128, 1, 0, 0, 7, 0, 0, 0, 0, 0, 0, 2], False), ([33, 48, 7, 0, 16, 2, 25, 0], True),
-          ([100, 64, 65, 63], False), ([300, 129, 128, 1], False), ([1, 260, 2], True)]
+          ([100, 64, 65, 63], False), ([300, 129, 128, 1], False), ([1, 260, 2], True), ([192, 193, 64, 65], False)]
 
 
 @pytest.mark.parametrize("N,K_", [(48, 1536), (272, 1544), (528, 2048), (784, 72), (1040, 2056)])
