@@ -306,7 +306,8 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
   // Slab s has its activations in stage s % 2 and its weights in stage s % 3.  Step 0 of slab s issues all weight loads of slab
   // s+2; then the wavefront waits until everything but those has landed -- its loads of slab s+1 -- and meets the others; step 1
   // issues the activation loads of slab s+2 into the stage that the barrier has just freed.  (2048 rows, against two whole stages
-  // with a slab for every load: 8192 x 28672 332 -> 306 us, pairs of 14336 x 4096 201 -> 189 and of 28672 x 8192 673 -> 638.
+  // with a slab for every load, on one card in turn: 8192 x 28672 343 -> 314 us, pairs of 14336 x 4096 207 -> 197 and of 28672 x 8192
+  // 691 -> 653; 4096 columns, on the smaller tiles, as before.
   // With every operand in the L2 these are 5 % faster: what is left is the matrix pipe and a tile's start and end, 11 us a round.)
   constexpr int BL = NB * B_LOADS;
   constexpr int wait_but_b = 0x0070 | (BL & 15) | ((BL >> 4) << 14);  // vmcnt(BL), lgkmcnt(0)

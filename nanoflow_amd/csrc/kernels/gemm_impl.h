@@ -973,8 +973,8 @@ static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1
     kern<<<grid, WM * WN * 64, SM::bytes, stream>>>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tiles_m, tiles_n);
     return check_launch("gemm launch");
   };
-  // One row of tiles reads the weights once: with the non-temporal hint (200 x 128256 x 4096: 258 -> 238 us, 66 x 28672 x 8192: 109
-  // -> 96, pairs of it 181 -> 167).  Several rows of tiles share them through the caches, which the hint defeats, and shares of a
+  // One row of tiles reads the weights once: with the non-temporal hint (three turns on one card: 256 x 128256 x 4096 258 -> 238 us, 66 x
+  // 28672 x 8192 103 -> 91, pairs of it 176 -> 158; 200 x 128256 x 4096 between 224 and 263 either way).  Several rows of tiles share them through the caches, which the hint defeats, and shares of a
   // split read runs of a row too short for it (128 x 4096 x 4096 in 8: 19 us, 24 with it).
   if constexpr (kBCol)
     if (tiles_m == 1) return go(std::true_type{});
