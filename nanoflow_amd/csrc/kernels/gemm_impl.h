@@ -170,7 +170,8 @@ __device__ __forceinline__ float swiglu_rounded(float g_acc, float u_acc) {
 // in the order of k, added up in pairs, the pairs in pairs and those two -- here the classes first_class .. first_class + n_classes - 1 (1, 2,
 // 4 or 8 of them, at most 2^kClasses), which the loads walk one after the other without a break.
 // kGroup (kBCol only): operands of one group of a grouped product -- the weights' row stride is ldb, D's is
-// ldd, and where a_rows is not null row m of A is row a_rows[m] of a matrix of a_total rows.
+// ldd, and where a_rows is not null row m of A is row a_rows[m] of a matrix of a_total rows; the contraction starts at slab `turn` of K and goes
+// round.
 template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kPartial = false, bool kGroup = false, int kCap = kWholeCu,
           bool kOnce = false, int kClasses = 0>
 __device__ __forceinline__ void gemm_tile(
@@ -178,7 +179,7 @@ __device__ __forceinline__ void gemm_tile(
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
     int M, int N, int K, float alpha, float beta, const int ldc, const int m_base, const int n_base,
     const int lda, const int group_ldb = 0, const int group_ldd = 0, const int32_t* a_rows = nullptr, const int a_total = 0,
-    const GroupEpilogue& group = {}, const int first_class = 0, const int n_classes = 1) {
+    const GroupEpilogue& group = {}, const int first_class = 0, const int n_classes = 1, const int turn = 0) {
   static_assert(kClasses == 0 || (!kBCol && WM * WN == 4 && !GemmSmem<BM, BN, kDual ? 2 : 1, kCap>::split), "classes: [K][N] weights, one ring, 16 x 16 MFMAs");
   static_assert(!kGroup || (kBCol && !kDual && !kPartial), "grouped products: plain, k-contiguous weights");
   const int ldb = kGroup ? group_ldb : lda, ldd = kGroup ? group_ldd : N;
@@ -254,7 +255,7 @@ __device__ __forceinline__ void gemm_tile(
     if constexpr (kGroup) {
       // rows past the group's last one start at the end of the buffer and read as zero
       const size_t row = a_rows ? (size_t)a_rows[gm < M ? gm : 0] : (size_t)gm;
-      a_off[t] = gm < M ? ((uint32_t)row * (uint32_t)lda + a_kc) * 2u : (uint32_t)((a_extent + 15) & ~(size_t)15);
+      a_off[t] = (gm < M ? ((uint32_t)row * (uint32_t)lda + a_kc) * 2u : (uint32_t)((a_extent + 15) & ~(size_t)15)) + (uint32_t)turn * (BK * 2u);
     } else {
       a_off[t] = ((uint32_t)gm * (uint32_t)lda + a_kc) * 2u;
     }
@@ -266,7 +267,7 @@ __device__ __forceinline__ void gemm_tile(
     uint32_t off;
     if constexpr (kBCol) {
       const int gn = n_base + (t * NW + wave) * 8 + (lane >> 3);
-      off = ((uint32_t)gn * (uint32_t)ldb + a_kc) * 2u;
+      off = ((uint32_t)gn * (uint32_t)ldb + a_kc) * 2u + (kGroup ? (uint32_t)turn * (BK * 2u) : 0u);
     } else {
       const int g = (t * NW + wave) * 64 + lane;  // 16-byte slot of the slab's LDS image
       const int row = g / B_CPR;
@@ -277,6 +278,10 @@ __device__ __forceinline__ void gemm_tile(
     for (int b = 0; b < NB; ++b) b_off[b][t] = off;
   }
 
+  // kGroup: slab s is slab k_slab(s) of K; from the last one the loads go back to the first.
+  const int k_slabs = (K + BK - 1) / BK;
+  auto k_slab = [&](int s) { return kGroup && s + turn >= k_slabs ? s + turn - k_slabs : s + turn; };
+  auto on_from = [&](int s) { return kGroup && k_slab(s) == k_slabs - 1 ? -(k_slabs - 1) * (BK * 2) : BK * 2; };
   // kClasses: slab `u` of K is followed by the next of its class, the class's last by the next class's first.  Every class has as
   // many slabs; those past the end of K read as zero.
   const int class_slabs = (K + 8 * BK - 1) / (8 * BK);
@@ -303,17 +308,17 @@ __device__ __forceinline__ void gemm_tile(
   constexpr int PARTS = NS == 2 ? 3 : 4;         // k-steps the loads of one slab are spread over
   // k_ok: this lane's 16 bytes of the slab's 128-byte rows lie below K.  la / lb: LDS address of
   // the stage the activations / the weights of the slab go to, + wave * 1024.
-  auto load_one = [&](auto t_c, uint32_t la, uint32_t lb, bool k_ok) {
+  auto load_one = [&](auto t_c, uint32_t la, uint32_t lb, bool k_ok, int by = BK * 2) {
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
       load16_to_lds<t * NW * 1024>(a_rsrc, k_ok ? a_off[t] : kOob, la);
-      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : BK * 2;
+      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kGroup ? by : BK * 2;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       constexpr int dst = b * SM::b_bytes + tt * NW * 1024;
       if constexpr (kBCol) {
         load16_to_lds<dst, kOnce>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
-        b_off[b][tt] += BK * 2;
+        b_off[b][tt] += kGroup ? by : BK * 2;
       } else {
         load16_to_lds<dst>(b_rsrc[b], kClasses == 0 || slab_in ? b_off[b][tt] : kOob, lb);
         b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;
@@ -324,16 +329,16 @@ __device__ __forceinline__ void gemm_tile(
   // instructions each: the offset (masked, and advanced for the next slab) first, the M0 write and
   // the load instruction one MFMA later.
   uint32_t pend = 0;
-  auto load_prepare = [&](auto t_c, bool k_ok) {
+  auto load_prepare = [&](auto t_c, bool k_ok, int by) {
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
       pend = k_ok ? a_off[t] : kOob;
-      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : BK * 2;
+      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kGroup ? by : BK * 2;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       if constexpr (kBCol) {
         pend = k_ok ? b_off[b][tt] : kOob;
-        b_off[b][tt] += BK * 2;
+        b_off[b][tt] += kGroup ? by : BK * 2;
       } else {
         pend = kClasses == 0 || slab_in ? b_off[b][tt] : kOob;
         b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;
@@ -349,10 +354,10 @@ __device__ __forceinline__ void gemm_tile(
       load16_to_lds<b * SM::b_bytes + tt * NW * 1024, kOnce>(b_rsrc[b], pend, lb);
     }
   };
-  auto load_slab = [&](int stage, int k0) {  // every load of one slab, back to back (one ring for both operands)
+  auto load_slab = [&](int stage, int k0, int by) {  // every load of one slab, back to back (one ring for both operands)
     const uint32_t st = __builtin_amdgcn_readfirstlane(smem_lds + stage * SM::stage_bytes + wave * 1024);
     const bool k_ok = k0 + a_kc < K;
-    static_for<LOADS>([&](auto t_c) { load_one(t_c, st, st + SM::a_bytes, k_ok); });
+    static_for<LOADS>([&](auto t_c) { load_one(t_c, st, st + SM::a_bytes, k_ok, by); });
   };
 
   // ---- LDS -> MFMA operand fragments, double-buffered across k-steps
@@ -415,7 +420,7 @@ __device__ __forceinline__ void gemm_tile(
   //   loads L0, L0 + LSTR, ... (NL of them) of a slab being fetched, into the stages at la / lb;
   //   then the fragment reads of k-step RK from the stages sa / sb into the other buffer (RK < 0: none).
   constexpr int NM = NB * TN * TM;
-  auto step = [&](auto kk_c, auto l0_c, auto lstr_c, auto nl_c, auto rk_c, uint32_t la, uint32_t lb, bool ld_ok,
+  auto step = [&](auto kk_c, auto l0_c, auto lstr_c, auto nl_c, auto rk_c, uint32_t la, uint32_t lb, bool ld_ok, int by,
                   const uint8_t* sa, const uint8_t* sb) {
     constexpr int kk = decltype(kk_c)::value, L0 = decltype(l0_c)::value, LSTR = decltype(lstr_c)::value;
     constexpr int NL = decltype(nl_c)::value, RK = decltype(rk_c)::value;
@@ -444,7 +449,7 @@ __device__ __forceinline__ void gemm_tile(
           constexpr int NRD = NRB + NRA;
           constexpr int qq = q < NRA ? 2 * NL + NRB + q : q < NRD ? 2 * NL + (q - NRA) : q - NRD;
           if constexpr (qq < 2 * NL) {
-            if constexpr (qq % 2 == 0) load_prepare(ic<L0 + LSTR * (qq / 2)>{}, ld_ok);
+            if constexpr (qq % 2 == 0) load_prepare(ic<L0 + LSTR * (qq / 2)>{}, ld_ok, by);
             else load_issue(ic<L0 + LSTR * (qq / 2)>{}, la, lb);
           } else if constexpr (qq < 2 * NL + NRB) {
             read_one(ic<TM + HN * CH + (qq - 2 * NL)>{}, ic<K2N>{}, ic<HN>{}, sa, sb);
@@ -467,7 +472,7 @@ __device__ __forceinline__ void gemm_tile(
       constexpr int lo = n * S / NM, hi = (n + 1) * S / NM;
       static_for<hi - lo>([&](auto d_c) {
         constexpr int q = lo + decltype(d_c)::value;
-        if constexpr (q < NL) load_one(ic<L0 + LSTR * q>{}, la, lb, ld_ok);
+        if constexpr (q < NL) load_one(ic<L0 + LSTR * q>{}, la, lb, ld_ok, by);
         else read_one(ic<q - NL>{}, ic<(RK < 0 ? 0 : RK)>{}, ic<(kk + 1) & 1>{}, sa, sb);
       });
       __builtin_amdgcn_sched_barrier(0);
@@ -478,7 +483,7 @@ __device__ __forceinline__ void gemm_tile(
   using F_ = std::false_type;
   const int nslab = kClasses > 0 ? n_classes * class_slabs : (K + BK - 1) / BK;
   // k of slab s, or of slab number u of K
-  auto slab_k = [&](int s, int u) { return (kClasses > 0 ? u : s) * BK; };
+  auto slab_k = [&](int s, int u) { return (kClasses > 0 ? u : k_slab(s)) * BK; };
 
   if constexpr (SM::split) {
     // ---- two activation stages, three weight stages.  Slab s has its activations in stage s % 2
@@ -499,14 +504,14 @@ __device__ __forceinline__ void gemm_tile(
     };
     auto a_ptr = [&](int stage) { return smem + stage * SM::a_bytes; };
     auto b_ptr = [&](int stage) { return smem + SM::b_ring + stage * NB * SM::b_bytes; };
-    auto k_ok_of = [&](int slab_idx) { return slab_idx * BK + a_kc < K; };
+    auto k_ok_of = [&](int slab_idx) { return k_slab(slab_idx) * BK + a_kc < K; };
     // prologue: activations and weights of slab 0, weights of slab 1
     {
       const uint32_t la = a_lds(0), lb0 = b_lds(0), lb1 = b_lds(1);
-      static_for<A_LOADS>([&](auto t_c) { load_one(t_c, la, lb0, k_ok_of(0)); });
-      static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb0, k_ok_of(0)); });
+      static_for<A_LOADS>([&](auto t_c) { load_one(t_c, la, lb0, k_ok_of(0), on_from(0)); });
+      static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb0, k_ok_of(0), on_from(0)); });
       if (nslab > 1) {
-        static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb1, k_ok_of(1)); });
+        static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb1, k_ok_of(1), on_from(1)); });
         __builtin_amdgcn_s_waitcnt(wait_but_b);
       } else {
         __builtin_amdgcn_s_waitcnt(0x0070);
@@ -516,7 +521,7 @@ __device__ __forceinline__ void gemm_tile(
     static_for<(kM16 ? TM + CH : READS)>([&](auto q_c) { read_one(q_c, ic<0>{}, ic<0>{}, a_ptr(0), b_ptr(0)); });
     if (nslab > 1) {  // what k-step 3 of a slab before slab 0 would have issued
       const uint32_t la = a_lds(1);
-      static_for<HA>([&](auto t_c) { load_one(t_c, la, la, k_ok_of(1)); });
+      static_for<HA>([&](auto t_c) { load_one(t_c, la, la, k_ok_of(1), on_from(1)); });
     }
     // H1: slab s+1 exists, H2: slab s+2 exists
     auto slab2 = [&](auto h1_c, auto h2_c, int s, int bs) {
@@ -524,15 +529,15 @@ __device__ __forceinline__ void gemm_tile(
       const uint8_t *sa = a_ptr(s & 1), *sb = b_ptr(bs);
       const int bs1 = bs == 2 ? 0 : bs + 1, bs2 = bs1 == 2 ? 0 : bs1 + 1;
       const uint32_t la1 = a_lds((s + 1) & 1), lb2 = b_lds(bs2);
-      step(ic<0>{}, ic<HA>{}, ic<1>{}, ic<H1 ? A_LOADS - HA : 0>{}, ic<1>{}, la1, la1, k_ok_of(s + 1), sa, sb);
-      step(ic<1>{}, ic<A_LOADS>{}, ic<1>{}, ic<H2 ? HB : 0>{}, ic<2>{}, lb2, lb2, k_ok_of(s + 2), sa, sb);
-      step(ic<2>{}, ic<A_LOADS + HB>{}, ic<1>{}, ic<H2 ? BL - HB : 0>{}, ic<3>{}, lb2, lb2, k_ok_of(s + 2), sa, sb);
+      step(ic<0>{}, ic<HA>{}, ic<1>{}, ic<H1 ? A_LOADS - HA : 0>{}, ic<1>{}, la1, la1, k_ok_of(s + 1), on_from(s + 1), sa, sb);
+      step(ic<1>{}, ic<A_LOADS>{}, ic<1>{}, ic<H2 ? HB : 0>{}, ic<2>{}, lb2, lb2, k_ok_of(s + 2), on_from(s + 2), sa, sb);
+      step(ic<2>{}, ic<A_LOADS + HB>{}, ic<1>{}, ic<H2 ? BL - HB : 0>{}, ic<3>{}, lb2, lb2, k_ok_of(s + 2), on_from(s + 2), sa, sb);
       if constexpr (H1) {
         __builtin_amdgcn_s_waitcnt(H2 ? wait_but_b : 0x0070);
         __syncthreads();
       }
       const uint32_t la2 = a_lds(s & 1);  // slab s+2's activations reuse this slab's stage
-      step(ic<3>{}, ic<0>{}, ic<1>{}, ic<H2 ? HA : 0>{}, ic<H1 ? 0 : -1>{}, la2, la2, k_ok_of(s + 2), a_ptr((s + 1) & 1),
+      step(ic<3>{}, ic<0>{}, ic<1>{}, ic<H2 ? HA : 0>{}, ic<H1 ? 0 : -1>{}, la2, la2, k_ok_of(s + 2), on_from(s + 2), a_ptr((s + 1) & 1),
            b_ptr(bs1));
     };
     int s = 0, bs = 0;
@@ -599,9 +604,9 @@ __device__ __forceinline__ void gemm_tile(
     const uint32_t ld_a = __builtin_amdgcn_readfirstlane(smem_lds + ls * SM::stage_bytes + wave * 1024);
     if constexpr (kClasses > 0) fetch(u_ahead);
     const bool ok_a = slab_k(s + NS - 1, u_ahead) + a_kc < K;
-    step(ic<0>{}, ic<1>{}, ic<PARTS>{}, ic<(IA && PARTS > 1) ? nl(1) : 0>{}, ic<1>{}, ld_a, ld_a + SM::a_bytes, ok_a, st, sb);
-    step(ic<1>{}, ic<2>{}, ic<PARTS>{}, ic<(IA && PARTS > 2) ? nl(2) : 0>{}, ic<2>{}, ld_a, ld_a + SM::a_bytes, ok_a, st, sb);
-    step(ic<2>{}, ic<3>{}, ic<PARTS>{}, ic<(IA && PARTS > 3) ? nl(3) : 0>{}, ic<3>{}, ld_a, ld_a + SM::a_bytes, ok_a, st, sb);
+    step(ic<0>{}, ic<1>{}, ic<PARTS>{}, ic<(IA && PARTS > 1) ? nl(1) : 0>{}, ic<1>{}, ld_a, ld_a + SM::a_bytes, ok_a, on_from(s + NS - 1), st, sb);
+    step(ic<1>{}, ic<2>{}, ic<PARTS>{}, ic<(IA && PARTS > 2) ? nl(2) : 0>{}, ic<2>{}, ld_a, ld_a + SM::a_bytes, ok_a, on_from(s + NS - 1), st, sb);
+    step(ic<2>{}, ic<3>{}, ic<PARTS>{}, ic<(IA && PARTS > 3) ? nl(3) : 0>{}, ic<3>{}, ld_a, ld_a + SM::a_bytes, ok_a, on_from(s + NS - 1), st, sb);
     if constexpr (!LAST) {
       wait_loads(IA ? 1 : 0);
       __syncthreads();
@@ -613,7 +618,7 @@ __device__ __forceinline__ void gemm_tile(
       fetch(u_ahead);
     }
     step(ic<3>{}, ic<0>{}, ic<PARTS>{}, ic<IB ? nl(0) : 0>{}, ic<LAST ? -1 : 0>{}, ld_b, ld_b + SM::a_bytes,
-         slab_k(s + NS, u_ahead) + a_kc < K, nst, nst + SM::a_bytes);
+         slab_k(s + NS, u_ahead) + a_kc < K, on_from(s + NS), nst, nst + SM::a_bytes);
     if constexpr (kClasses > 0) {
       if (u_now >= 8 * (class_slabs - 1)) end_class((u_now & 7) - first_class);
       u_now = after(u_now);
@@ -623,7 +628,7 @@ __device__ __forceinline__ void gemm_tile(
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p) {
     if constexpr (kClasses > 0) fetch(u_ahead);
-    if (p < nslab) load_slab(p, slab_k(p, u_ahead));
+    if (p < nslab) load_slab(p, slab_k(p, u_ahead), on_from(p));
     if constexpr (kClasses > 0) u_ahead = after(u_ahead);
   }
   // slab 0 must have landed; later prologue loads may still be in flight (exact count only
@@ -635,7 +640,7 @@ __device__ __forceinline__ void gemm_tile(
     const uint32_t st = __builtin_amdgcn_readfirstlane(smem_lds + (NS - 1) * SM::stage_bytes + wave * 1024);
     if constexpr (kClasses > 0) fetch(u_ahead);
     const bool k_ok = slab_k(NS - 1, u_ahead) + a_kc < K;
-    static_for<(LOADS + PARTS - 1) / PARTS>([&](auto q_c) { load_one(ic<PARTS * decltype(q_c)::value>{}, st, st + SM::a_bytes, k_ok); });
+    static_for<(LOADS + PARTS - 1) / PARTS>([&](auto q_c) { load_one(ic<PARTS * decltype(q_c)::value>{}, st, st + SM::a_bytes, k_ok, on_from(NS - 1)); });
   }
   int cs = 0, ls = NS - 1, s = 0;
   for (; s + NS < nslab; ++s) {  // steady state

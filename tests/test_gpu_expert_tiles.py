@@ -1,0 +1,65 @@
+"""Products of routed experts over small whole numbers: every sum is exact in fp32 whatever its order, so the results are those of
+integer arithmetic, rounded once.  Experts with no row, one, a few more than a tile's and several tiles; contractions of one slab of
+64 and a few, of whole slabs and not; columns that end inside a tile."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+FEW = (0, 1, 16, 33, 49, 64, 65)                       # tile lists of 64 rows
+MANY = (0, 129, 1, 300, 128, 96, 257, 511, 32)         # of 128
+
+
+def routing(K, counts, tile, rows, rng):
+    """Rows of the tokens in the order of their experts, and the tile list."""
+    e, slots = len(counts), int(sum(counts))
+    i32 = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).cuda()
+    tiles = [(g, r) for g in range(e) for r in range(0, counts[g], tile)]
+    room = K.lib().nf_routing_max_tiles(slots, e, tile)
+    assert len(tiles) <= room
+    pad = [(0, 0)] * (room - len(tiles))
+    row_of = rng.integers(0, rows, slots)
+    weight = rng.integers(1, 4, slots).astype(np.float32)
+    t = dict(row_of=i32(row_of), offsets=i32(np.concatenate([[0], np.cumsum(counts)])), tile_group=i32([g for g, _ in tiles + pad]),
+             tile_row=i32([r for _, r in tiles + pad]), n_tiles=i32([len(tiles)]), row_weight=torch.from_numpy(weight).cuda())
+    return K.Routing(tile_rows=tile, **{k: v.data_ptr() for k, v in t.items()}), t, row_of, weight
+
+
+@pytest.mark.parametrize("counts", [FEW, MANY], ids=["lists of 64", "lists of 128"])
+@pytest.mark.parametrize("N,Kd", [(8, 64), (136, 72), (256, 128), (264, 200), (520, 1000), (1032, 2048), (2048, 2056), (1024, 2112), (1048, 2184), (512, 3000)])
+def test_whole_numbers(counts, N, Kd):
+    from nanoflow_amd import kernels as K
+    rng = np.random.default_rng(N + Kd)
+    counts = np.array(counts)
+    e, slots, rows = len(counts), int(counts.sum()), 300
+    tile = K.lib().nf_grouped_tile_rows(K.BF16, slots, e)
+    assert tile == (128 if max(counts) > 65 else 64)
+    r, hold, row_of, weight = routing(K, counts, tile, rows, rng)
+    a, b = rng.integers(-2, 3, (rows, Kd)), rng.integers(-2, 3, (e, N, Kd))
+    gather, given = torch.from_numpy(a).cuda(), torch.from_numpy(a[row_of]).cuda().bfloat16()
+    w = torch.from_numpy(b).cuda()
+    group = np.repeat(np.arange(e), counts)
+    product = torch.cat([gather[row_of[group == g]].double() @ w[g].double().T for g in range(e)])      # whole numbers below 2^24
+    bf16 = lambda x: x.float().bfloat16()
+    gather, w = gather.bfloat16(), w.bfloat16()
+
+    def run(act, source, out, **kw):
+        d = torch.full((slots, out), 9.0, dtype=torch.bfloat16, device="cuda")
+        K.gemm_grouped_experts(source, w, d, r, slots, source is gather, act, **kw)
+        return d
+
+    assert torch.equal(run(K.ACT_NONE, gather, N), bf16(product))
+    assert torch.equal(run(K.ACT_NONE, given, N), bf16(product))
+    assert torch.equal(run(K.ACT_SQUARED_RELU, gather, N), bf16(product.clamp(min=0).float().square()))
+    assert torch.equal(run(K.ACT_NONE, given, N, weigh=True), bf16(product * torch.from_numpy(weight).cuda()[:, None].double()))
+    # gate and up, weighed first: the sigmoid's rounding and one to bf16
+    x = product * torch.from_numpy(weight).cuda()[:, None].double() / 64
+    limits = torch.full((e,), 7.0, device="cuda")
+    scaled = (w.float() / 64).bfloat16()
+    d = torch.full((slots, N // 2), 9.0, dtype=torch.bfloat16, device="cuda")
+    if N // 2 % 8 == 0:
+        K.gemm_grouped_experts(gather, scaled, d, r, slots, True, K.ACT_GATED, weigh=True, gated=(1.702, 1.0, limits))
+        g, u = x[:, 0::2].clamp(max=7.0), x[:, 1::2].clamp(-7.0, 7.0)
+        ref = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        assert (d.double() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
