@@ -4,7 +4,7 @@
 //
 // bf16: the tiles of the plain GEMM family; an m tile never spans two groups.  fp32: gemm_f32's tile.
 #include "gemm_f32_tile.h"
-#include "gemm_impl.h"
+#include "gemm_chain.h"
 
 namespace {
 
@@ -186,6 +186,55 @@ int launch_grouped(const nf_grouped_gemm_args& a, hipStream_t s) {
   return check_launch("nf_gemm_grouped");
 }
 
+// Each XCD takes a run of the launch's tiles (m tiles of an expert fastest), its workgroups every n-th of them.
+template <class E, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(WM * WN * 64, 1) void gemm_chain_kernel(nf_grouped_gemm_args a, int tiles_n) {
+  typedef const __attribute__((address_space(4))) int32_t* list_t;  // read-only: by scalar loads, which the operands' waits do not count
+  const list_t n_tiles = (list_t)a.routing.n_tiles, groups = (list_t)a.routing.tile_group, tile_row = (list_t)a.routing.tile_row, offsets = (list_t)a.routing.offsets;
+  const int total = n_tiles[0] * tiles_n, per = (total + 7) / 8, x = blockIdx.x % 8, end = min((x + 1) * per, total);
+  const int first = x * per + blockIdx.x / 8, nslab = (a.K + BK - 1) / BK;
+  if (first >= end) return;
+  gemm_chain<E, BM, BN, WM, WN>(a, first, end, gridDim.x / 8, [&](int logical) {
+    if (logical >= end) return ChainTile{0, 0, 0, 0, 0, 0};
+    const int mt = logical / tiles_n, g = groups[mt], row0 = offsets[g], rows = offsets[g + 1] - row0;
+    const int i = logical - (mt - tile_row[mt] / BM) * tiles_n, tiles = (rows + BM - 1) / BM, n_tile = i / tiles;
+    const int h = ((rows + tiles - 1) / tiles + 16 * WM - 1) / (16 * WM) * (16 * WM), m_base = i % tiles * h;
+    return ChainTile{g, m_base, min(rows, m_base + h), n_tile * BN, row0, (n_tile + g * 4) % nslab};
+  });
+}
+
+template <class E>
+int launch_chain(const nf_grouped_gemm_args& a, hipStream_t s) {
+  constexpr int BM = 128, BN = 256;
+  using SM = ChainSmem<BM, BN>;
+  auto kern = gemm_chain_kernel<E, BM, BN, 2, 4>;
+  static bool attr_set = false;  // benign race: the call is idempotent
+  if (!attr_set) {
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)SM::bytes);
+    if (e != hipSuccess) {
+      set_error("nf_gemm_grouped: cannot reserve %zu bytes of LDS: %s", SM::bytes, hipGetErrorString(e));
+      return NF_ERR_RUNTIME;
+    }
+    attr_set = true;
+  }
+  const int tiles_n = (a.N + BN - 1) / BN;
+  kern<<<std::min(grid_of(a, BM, tiles_n), (unsigned)std::max(cu_count() / 8 * 8, 8)), 512, SM::bytes, s>>>(a, tiles_n);
+  return check_launch("nf_gemm_grouped");
+}
+
+// Tile lists of 128 rows that run on gemm_chain.h.  Contractions beyond 2048 against whole column tiles do, where a 128 x 256 tile on four
+// wavefronts ran before: 0.90 to 1.00 of its time over 300 to 2048 rows, 8 to 65 experts of 512 to 4096 columns 2304 to 3584 deep.
+// At 2048 two workgroups of 128 x 128 a CU stand against it, which leave less of a round idle: it pays where its own rounds are at least four
+// fifths full, or one is at least half full (2.9 and 5.8 rounds: 0.91 of their time, 0.6 of one 0.88; 1.1 to 2.2: 1.02 to 1.14).  The rows of
+// an expert are not known here: half a tile each over the sorted rows.  Below 2048 neither wins.
+bool chain_pays(const nf_grouped_gemm_args& a) {
+  if (a.K < 2048 || a.N < 256 || a.ldd > 1 << 22 || (a.act == NF_ACT_GATED ? a.N % 16 != 0 : a.weigh)) return false;
+  if (a.K > 2048) return a.N % 256 == 0;
+  const double rounds = (a.max_rows / 128.0 + a.groups * 0.5) * ((a.N + 255) / 256) / cu_count();
+  return rounds < 1 ? rounds >= 0.5 : std::ceil(rounds) <= 1.25 * rounds;
+}
+
 template <class E>
 int dispatch_grouped(const nf_grouped_gemm_args& a, int tile_rows, hipStream_t s) {
   if (a.routing.n_tiles) {
@@ -203,8 +252,8 @@ int dispatch_grouped(const nf_grouped_gemm_args& a, int tile_rows, hipStream_t s
       return a.N >= 512 ? launch_grouped_rows<E, true>(a, s) : launch_grouped_rows<E, false>(a, s);
     // Short contractions: a third of a tile's time is its start and its end, so two workgroups share a CU and one runs under the
     // other's (2000 rows, 8 of 64 experts of 1024 x 1024: 80 -> 62 us; 1946 rows, 5 of 33 gated experts of 4096 x 2048: 242 ->
-    // 225).  Longer ones want the larger tile's lower LDS traffic (512 rows, 4 of 32 of 4096 x 3584: 187 us against 205; 2048 rows:
-    // 311 against 325).
+    // 225).  Longer ones want the larger tile's lower LDS traffic (512 rows, 4 of 32 of 4096 x 3584: 187 us against 205).
+    if (tile_rows == 128 && chain_pays(a)) return launch_chain<E>(a, s);
     if (a.K <= 2048)
       return tile_rows == 64 ? launch_grouped<E, 64, 128, 2, 2, kHalfCu>(a, s) : launch_grouped<E, 128, 128, 2, 2, kHalfCu, true>(a, s);
   }

@@ -27,7 +27,7 @@ def routing(K, counts, tile, rows, rng):
 
 
 @pytest.mark.parametrize("counts", [FEW, MANY], ids=["lists of 64", "lists of 128"])
-@pytest.mark.parametrize("N,Kd", [(8, 64), (136, 72), (256, 128), (264, 200), (520, 1000), (1032, 2048), (2048, 2056), (1024, 2112), (1048, 2184), (512, 3000)])
+@pytest.mark.parametrize("N,Kd", [(8, 64), (136, 72), (256, 128), (264, 200), (520, 1000), (1032, 2048), (2048, 2056), (1024, 2112), (1048, 2184), (512, 3000), (2192, 2048)])
 def test_whole_numbers(counts, N, Kd):
     from nanoflow_amd import kernels as K
     rng = np.random.default_rng(N + Kd)
@@ -36,7 +36,7 @@ def test_whole_numbers(counts, N, Kd):
     tile = K.lib().nf_grouped_tile_rows(K.BF16, slots, e)
     assert tile == (128 if max(counts) > 65 else 64)
     r, hold, row_of, weight = routing(K, counts, tile, rows, rng)
-    a, b = rng.integers(-2, 3, (rows, Kd)), rng.integers(-2, 3, (e, N, Kd))
+    a, b = rng.integers(-2, 3, (rows, Kd), dtype=np.int8), rng.integers(-2, 3, (e, N, Kd), dtype=np.int8)
     gather, given = torch.from_numpy(a).cuda(), torch.from_numpy(a[row_of]).cuda().bfloat16()
     w = torch.from_numpy(b).cuda()
     group = np.repeat(np.arange(e), counts)
