@@ -1144,7 +1144,14 @@ static int launch_window(const nf_window_attention_args& a, hipStream_t s) {
   const unsigned gy = (unsigned)(a.kv.kv_heads * chunks);
   if (a.decode) {
     auto lds_of = [&](int w) { return (size_t)w * kMaps * (32 + (size_t)gs * a.kv.v_pad) * sizeof(float); };
-    int waves = (long long)a.req_num * gy >= 512 || window_threads(kMaps, VD) < 512 ? 4 : 8;
+    // As many wavefronts a workgroup as leave every workgroup resident at once (eight wavefronts a CU by their registers): a second round pays the
+    // page lookups, the first keys and the merge again.  us, window 512: 256 requests of 4 kv heads, two maps 61 on four wavefronts, 56 on two; 200
+    // requests of 300 36 and 31; 300 of 500 64 and, on one, 60; 500 of 1000 113 and 101; one map 256 requests 59 and 54.  From 2048 workgroups
+    // on there are several rounds however few the wavefronts (1000 requests: four 176, one 192).
+    const long long groups = (long long)a.req_num * gy;
+    int waves = 4;
+    if (window_threads(kMaps, VD) == 512 && groups <= 2048)
+      for (waves = 8; waves > 1 && groups * waves > 2048;) waves /= 2;
     while (waves > 1 && lds_of(waves) > 64 * 1024) waves /= 2;
     attn_window_kernel<KD, VD, 1, kMaps, true><<<dim3((unsigned)a.req_num, gy), waves * 64, lds_of(waves), s>>>(a, gs, chunks, 0);
     return check_launch("nf_window_attention (decode)");

@@ -175,6 +175,14 @@ def test_difference_of_two_maps(heads, kv_heads, dim, vdim, window):
         close(got, want, dtype, f"{dtype}", factor=1.5)
 
 
+@pytest.mark.parametrize("requests,kv_heads", [(64, 4), (65, 4), (129, 4), (129, 8), (257, 8)])
+def test_decoding_with_fewer_wavefronts(requests, kv_heads):
+    """8, 4, 2, 1 and again 4 wavefronts a workgroup, with the short requests whose keys do not reach all of them."""
+    b = cases.batch(np.random.default_rng(requests).integers(0, 90, requests).tolist(), [], seed=3)
+    got, want = maps_case(BF16, kv_heads, kv_heads, 32, 32, 60, b, requests, seed=5)
+    close(got, want, BF16, factor=1.5)
+
+
 @pytest.mark.parametrize("cap,scale,weight,diff", [(None, 0.3, 0.2, 0.8), (0.5, 0.3, 1.4, 0.0), (50.0, 0.02, -0.3, 0.5), (3.0, 2.0, 0.6, 0.1),
                                                    (4.0, -0.4, 0.3, 0.3), (200.0, 1.5, 0.3, 0.3)])
 def test_caps_and_weights(cap, scale, weight, diff):
