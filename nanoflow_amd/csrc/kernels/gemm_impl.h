@@ -981,9 +981,13 @@ static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1
   // One row of tiles reads the weights once: with the non-temporal hint (three turns on one card: 256 x 128256 x 4096 258 -> 238 us, 66 x
   // 28672 x 8192 103 -> 91, pairs of it 176 -> 158; 200 x 128256 x 4096 between 224 and 263 either way).  Several rows of tiles share them through the caches, which the hint defeats, and shares of a
   // split read runs of a row too short for it (128 x 4096 x 4096 in 8: 19 us, 24 with it).
-  if constexpr (kBCol)
-    if (tiles_m == 1) return go(std::true_type{});
-  return go(std::false_type{});
+  if constexpr (kBCol && BM % 128 != 0 && BM > 128) {
+    return go(std::true_type{});  // heights of one row of tiles
+  } else {
+    if constexpr (kBCol)
+      if (tiles_m == 1) return go(std::true_type{});
+    return go(std::false_type{});
+  }
 }
 
 template <class E, int BN, bool kDual, bool kBCol>
@@ -1191,6 +1195,15 @@ static int dispatch_plain(const uint16_t* A, const uint16_t* B, const uint16_t* 
       return launch_gemm<E, 256, 192, 2, 2, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
   if (best == c256 && two_heights)
     return launch_hybrid<E, 256, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, (int)(t256 - rest256), s);
+  // One row of tiles: no higher than its rows need, for the padding is multiplied at the power cap's price (us against 256 x 256, x 128256 x 4096:
+  // 140 rows 238 -> 199, 180 rows 249 -> 222, 192 rows 250 -> 227, 200 rows 253 -> 240; from 225 rows on it is the same tile).  Wavefronts
+  // beside each other, since 224 and 160 rows are no two blocks of whole passes.
+  if constexpr (kBCol)
+    if (best == c256 && M <= 224) {
+      if (M <= 160) return launch_gemm<E, 160, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+      if (M <= 192) return launch_gemm<E, 192, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+      return launch_gemm<E, 224, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+    }
   if (best == c256) return launch_gemm<E, 256, 256, 2, 2, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
   if (best == c128x256) return launch_gemm<E, 128, 256, 2, 2, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
   return launch_gemm<E, 128, 128, 2, 2, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);

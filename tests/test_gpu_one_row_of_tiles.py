@@ -1,0 +1,23 @@
+"""Products of 129 to 256 rows against many columns, whose tiles are as high as the rows need: whole numbers, so every result is exact."""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M", [129, 160, 161, 192, 193, 224, 225])
+@pytest.mark.parametrize("N,Kd", [(65536, 64), (65400, 136), (65288, 712)])
+def test_heights(dtype, M, N, Kd):
+    from nanoflow_amd import kernels as K
+    gen = torch.Generator(device="cuda").manual_seed(M + Kd)
+    whole = lambda *shape, top: torch.randint(-top, top + 1, shape, generator=gen, device="cuda")
+    a, b, c = whole(M, Kd, top=1), whole(N, Kd, top=1), whole(M, N, top=8)      # results stay below 256 but for a chance of 1e-20
+    want = a.double() @ b.double().t()
+    cast = lambda t: t.to(getattr(torch, dtype))
+    assert want.abs().max() < 240
+    guard = torch.full((M + 1, N), 77.0, dtype=getattr(torch, dtype), device="cuda")
+    K.gemm(cast(a), cast(b), b_col_major=True, out=guard[:M])
+    assert torch.equal(guard[:M].double(), want) and (guard[M] == 77.0).all()
+    K.gemm(cast(a), cast(b), Cmat=cast(c), beta=1.0, b_col_major=True, out=guard[:M])
+    assert torch.equal(guard[:M].double(), want + c) and (guard[M] == 77.0).all()
