@@ -1,14 +1,18 @@
 #pragma once
 // 16-bit x 16-bit -> fp32 -> 16-bit GEMM family for gfx950 on v_mfma_f32_16x16x32_f16 (fp16, the
-// pipeline's type; 32x32x16 for the tiles on eight wavefronts) and the bf16 forms of the same
+// pipeline's type; 32x32x16 for the pair's 320-row tile) and the bf16 forms of the same
 // instructions (bf16: same kernels, other element type).
 //
 //   D = half(alpha * A.B + beta * C)                     (plain; QKV, O, down, LM head)
 //   D = half(silu(half(A.Bg)) * half(A.Bu))              (dual; gate/up SwiGLU)
 //
-// Workgroup = 256 threads = 4 wavefronts in a WM x WN grid; each wavefront owns a
+// Workgroup = 4 or 8 wavefronts in a WM x WN grid; each wavefront owns a
 // (BM/WM) x (BN/WN) block of 16x16 (or 32x32) MFMA tiles.  K is walked in slabs of 64 through a
 // ring of two to four LDS stages (as many as fit 144 KB).
+// Tiles of 128 rows run on eight: their sub-steps are too short for a wavefront alone on its SIMD to wait out an LDS read in, and a tile's start
+// and end halve (us, four -> eight: 2046 x 4096 x 4096 63.3 -> 60.1, 2048 deep 37.8 -> 33.6; 2019 x 2048 x 512 9.8 -> 7.9, 8192 deep 67.6 and 67.7; split
+// 128 x 4096 x 4096 18.0 -> 16.6; fp32 sums of 748 x 2048 x 2048 13.7 -> 12.2; pair 128 x 4096 x 4096 27.8 -> 25.3).  Those of 256 rows on four where
+// the contraction is long (dispatch_plain).
 //
 // Operands go from global memory STRAIGHT INTO LDS (buffer_load_dwordx4 ... lds): a CU moves
 // about 38 GB/s through the load-to-register path but well over 100 GB/s through this one, and
@@ -28,7 +32,7 @@
 //       read cycle touches (two k-groups of 8 rows, 8 rows apart) sit in 8 different 32-byte
 //       bank groups.
 // With these two permutations SQ_LDS_BANK_CONFLICT reads zero for the kernel.
-// No staging registers, no permutes, no LDS stores in the main loop.  A wavefront is alone on
+// No staging registers, no permutes, no LDS stores in the main loop.  A wavefront is alone or one of two on
 // its SIMD, so nothing hides a stall of its instruction stream: the loads of later slabs and
 // the fragment reads of the next k-step are dealt out one at a time between the MFMAs of the
 // current k-step, in a pinned order; one barrier per slab.
@@ -158,7 +162,7 @@ __device__ __forceinline__ float swiglu_rounded(float g_acc, float u_acc) {
 }
 
 // WM x WN wavefronts: four (one per SIMD, up to 512 registers each) or eight (two per SIMD, up to
-// 256 each: for tiles whose accumulators do not fit four wavefronts, the 320 x 128 gate/up pair).
+// 256 each: for tiles of 128 rows, short contractions, and the 320 x 128 gate/up pair, whose accumulators do not fit four).
 // kDual: two weight matrices, SwiGLU epilogue.  kBCol: weights stored [N][K].
 // One BM x BN output tile at (m_base, n_base), computed by the whole workgroup.
 // K is the extent of the contraction and lda the row stride (elements) of the k-contiguous
@@ -196,8 +200,8 @@ __device__ __forceinline__ void gemm_tile(
   // sub-step reads the columns of the next one -- so that everything but the accumulators fits
   // the 256 architectural registers and the compiler has no reason to shuffle accumulators
   // between the two register files.
-  // Eight-wavefront tiles keep 32x32x16 (256 registers per wavefront in all).
-  constexpr bool kM16 = NW == 4;
+  // The pair's 320-row tile on eight wavefronts keeps 32x32x16 (256 registers per wavefront in all).
+  constexpr bool kM16 = NW == 4 || BM != 320;
   constexpr int MT = kM16 ? 16 : 32;  // rows and columns of an MFMA tile
   constexpr int TM = BM / WM / MT;    // MFMA tiles per wave along M
   constexpr int TN = BN / WN / MT;
@@ -1133,8 +1137,8 @@ static size_t split_bytes(int M, int N, int K, MidPlan* mid) {
 template <class E, bool kBCol>
 static int launch_mid(const MidPlan& p, const uint16_t* A, const uint16_t* B, const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha,
                       float beta, int ldc, float* P, hipStream_t s) {
-  if (p.tile == 0) return launch_splitk<E, 128, 128, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
-  if (p.tile == 1) return launch_splitk<E, 128, 256, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
+  if (p.tile == 0) return launch_splitk<E, 128, 128, 2, 4, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
+  if (p.tile == 1) return launch_splitk<E, 128, 256, 2, 4, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
   return launch_splitk<E, 256, 256, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, p.shares, p.k_per, P, s);
 }
 
@@ -1204,9 +1208,14 @@ static int dispatch_plain(const uint16_t* A, const uint16_t* B, const uint16_t* 
       if (M <= 192) return launch_gemm<E, 192, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
       return launch_gemm<E, 224, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
     }
-  if (best == c256) return launch_gemm<E, 256, 256, 2, 2, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
-  if (best == c128x256) return launch_gemm<E, 128, 256, 2, 2, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
-  return launch_gemm<E, 128, 128, 2, 2, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  // Two wavefronts a SIMD start and end a tile sooner and lose at the power cap what the larger block of one saves in LDS reads: 2048 x 8192 of
+  // k-contiguous weights 2048 deep 59.0 us on four, 57.1 on eight, 3584 deep 93.7 and 91.0, 4096 104.4 and 103.8, 8192 199 and 206;
+  // of [K][N] weights 62.6 and 57.9, 109.8 and 103.6, 205.5 and 204.9.
+  if (best == c256 && (!kBCol || K < 4096)) return launch_gemm<E, 256, 256, 2, 4, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  if constexpr (kBCol)
+    if (best == c256) return launch_gemm<E, 256, 256, 2, 2, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  if (best == c128x256) return launch_gemm<E, 128, 256, 2, 4, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  return launch_gemm<E, 128, 128, 2, 4, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
 }
 
 // ---- a caller-chosen tile and split over K (the cta_m / cta_n / split_k fields of a GEMM tag).
@@ -1255,8 +1264,8 @@ static int dispatch_menu(int index, const uint16_t* A, const uint16_t* B, const 
                          int K, float alpha, float beta, int ldc, int shares, int k_per, float* P, hipStream_t s) {
   switch (index) {
     case 0: return launch_menu<E, 64, 256, 1, 4, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
-    case 1: return launch_menu<E, 128, 128, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
-    case 2: return launch_menu<E, 128, 256, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
+    case 1: return launch_menu<E, 128, 128, 2, 4, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
+    case 2: return launch_menu<E, 128, 256, 2, 4, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
     case 3: return launch_menu<E, 256, 256, 2, 2, kBCol>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
     case 4:
       if constexpr (kBCol) return launch_menu<E, 256, 192, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, ldc, shares, k_per, P, s);
@@ -1347,8 +1356,8 @@ static int gemm_ws_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   if (M > 256)
     return b_col_major ? launch_splitk<E, 320, 128, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
                        : launch_splitk<E, 320, 128, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
-  return b_col_major ? launch_splitk<E, 128, 128, 2, 2, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
-                     : launch_splitk<E, 128, 128, 2, 2, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
+  return b_col_major ? launch_splitk<E, 128, 128, 2, 4, true>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s)
+                     : launch_splitk<E, 128, 128, 2, 4, false>(A, B, C, D, M, N, K, alpha, beta, c_is_row ? 0 : N, shares, k_per, P, s);
 }
 
 template <class E, bool kBCol>
@@ -1380,7 +1389,7 @@ static int dual_entry(const char* who, const uint16_t* A, const uint16_t* Bgate,
       return launch_hybrid<E, 128, true, kBCol>(A, Bgate, Bup, nullptr, out, M, N, K, 1.f, 0.f, N, (int)(t256 - rest), s);
     return launch_gemm<E, 256, 128, 2, 2, true, kBCol>(A, Bgate, Bup, nullptr, out, M, N, K, 1.f, 0.f, N, s);
   }
-  return launch_gemm<E, 128, 128, 2, 2, true, kBCol>(A, Bgate, Bup, nullptr, out, M, N, K, 1.f, 0.f, N, s);
+  return launch_gemm<E, 128, 128, 2, 4, true, kBCol>(A, Bgate, Bup, nullptr, out, M, N, K, 1.f, 0.f, N, s);
 }
 
 template <class E, bool kBCol>
@@ -1405,6 +1414,6 @@ static int dual_ws_entry(const char* who, const uint16_t* A, const uint16_t* Bga
     return launch_splitk<E, 64, 128, 2, 2, kBCol, true>(A, Bgate, nullptr, out, M, N, K, 1.f, 0.f, N, shares, k_per, P, s, Bup);
   if (M > 256)
     return launch_splitk<E, 320, 128, 2, 4, kBCol, true>(A, Bgate, nullptr, out, M, N, K, 1.f, 0.f, N, shares, k_per, P, s, Bup);
-  return launch_splitk<E, 128, 128, 2, 2, kBCol, true>(A, Bgate, nullptr, out, M, N, K, 1.f, 0.f, N, shares, k_per, P, s, Bup);
+  return launch_splitk<E, 128, 128, 2, 4, kBCol, true>(A, Bgate, nullptr, out, M, N, K, 1.f, 0.f, N, shares, k_per, P, s, Bup);
 }
 

@@ -122,7 +122,7 @@ int nf_gemm_nk_sums_bf16(const uint16_t* A, const uint16_t* B, float* P, size_t 
   if (p.tile == 3) return dispatch_rows<BF16, true>(A, B, nullptr, reinterpret_cast<uint16_t*>(P), M, N, K, 1.f, 0.f, N, s);
   if (p.tile == 4) return launch_sums<64, 64, 2, 2, kHalfCu>(A, B, P, M, N, K, p, s);
   if (p.tile == 0) return launch_sums<64, 256, 1, 4>(A, B, P, M, N, K, p, s);
-  if (p.tile == 1) return launch_sums<128, 128, 2, 2>(A, B, P, M, N, K, p, s);
+  if (p.tile == 1) return launch_sums<128, 128, 2, 4>(A, B, P, M, N, K, p, s);
   return launch_sums<256, 256, 2, 2>(A, B, P, M, N, K, p, s);
 }
 

@@ -29,5 +29,5 @@ static int gemm_nk_entry(const char* who, const uint16_t* A, const uint16_t* B, 
   float* P = static_cast<float*>(workspace);
   if (M <= 64) return launch_splitk_64<E>(A, B, bias, D, M, N, K, 1.f, beta, ldc, shares, k_per, P, true, s);
   if (M > 256) return launch_splitk<E, 320, 128, 2, 2, true>(A, B, bias, D, M, N, K, 1.f, beta, ldc, shares, k_per, P, s);
-  return launch_splitk<E, 128, 128, 2, 2, true>(A, B, bias, D, M, N, K, 1.f, beta, ldc, shares, k_per, P, s);
+  return launch_splitk<E, 128, 128, 2, 4, true>(A, B, bias, D, M, N, K, 1.f, beta, ldc, shares, k_per, P, s);
 }

@@ -1,4 +1,5 @@
-"""Products of 129 to 256 rows against many columns, whose tiles are as high as the rows need: whole numbers, so every result is exact."""
+"""Products of 129 to 256 rows against many columns, whose tiles are as high as the rows need, and the tiles on eight wavefronts at their edges:
+whole numbers, so every result is exact."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -21,3 +22,20 @@ def test_heights(dtype, M, N, Kd):
     assert torch.equal(guard[:M].double(), want) and (guard[M] == 77.0).all()
     K.gemm(cast(a), cast(b), Cmat=cast(c), beta=1.0, b_col_major=True, out=guard[:M])
     assert torch.equal(guard[:M].double(), want + c) and (guard[M] == 77.0).all()
+
+
+@pytest.mark.parametrize("nk", [True, False])
+@pytest.mark.parametrize("M,N,Kd", [(129, 264, 64), (300, 4104, 200), (513, 6152, 136), (700, 2040, 712), (1000, 4096, 72), (2040, 8184, 136), (1793, 8200, 328)])
+def test_eight_wavefronts(nk, M, N, Kd):
+    from nanoflow_amd import kernels as K
+    gen = torch.Generator(device="cuda").manual_seed(M + Kd)
+    whole = lambda *shape, top: torch.randint(-top, top + 1, shape, generator=gen, device="cuda")
+    a, b, c = whole(M, Kd, top=1), whole(N, Kd, top=1), whole(M, N, top=8)
+    want = a.double() @ b.double().t()
+    guard = torch.full((M + 1, N), 77.0, dtype=torch.float16, device="cuda")
+    w = b.half() if nk else b.half().t().contiguous()
+    K.gemm(a.half(), w, Cmat=c.half(), beta=1.0, b_col_major=nk, out=guard[:M])
+    assert torch.equal(guard[:M].double(), want + c) and (guard[M] == 77.0).all()
+    if nk:
+        sums = K.gemm_nk_sums(a.bfloat16(), b.bfloat16(), 16)
+        assert torch.equal(sums.double().sum(0), want)
