@@ -9,8 +9,9 @@
 // Both operands are stored with k contiguous (Aq [M][K], Bq [N][K]: one row per output
 // channel), so both are staged the same way: a slab is 128 k-bytes per row, moved from global
 // memory straight into LDS (buffer_load ... lds, XOR-swizzled rows, multi-stage ring -- the
-// scheme of gemm.hip with both operands in its row form).  Workgroup = 256 threads = 4
-// wavefronts in a WM x WN grid.  The MFMA is issued as D^T = B.A^T so that a lane owns 4
+// scheme of gemm.hip with both operands in its row form).  Workgroup = 4
+// wavefronts in a WM x WN grid, 8 on tiles of 128 rows (us, 4 -> 8: 1024 x 6144 x 4096 29.0 -> 27.3, 1973 x 4096 x 4096 34.1 -> 33.6, 500 rows
+// 16.8 -> 16.1; 256-row tiles lose: 2048 x 8192 x 8192 96 -> 98).  The MFMA is issued as D^T = B.A^T so that a lane owns 4
 // consecutive output columns.
 //
 // A dot product does not depend on which k a lane slot holds as long as both operands use the
@@ -158,18 +159,19 @@ __device__ __forceinline__ float swiglu_rounded_f16(float g_acc, float u_acc) {
 // k in [share * k_per, ...) and stores the fp32 sums, unscaled, to D taken as float
 // [shares][M][N] (kDual: the sums of the second product to C taken the same way); Kt is then the
 // whole contraction (the row stride of both operands), shares and k_per describe the split.
+// One BM x BN tile at (m_base, n_base).  K: extent of the contraction; lda: row stride of both operands; p_off: this share's slice of the partial sums.
 template <int BM, int BN, int WM, int WN, bool kDual, bool kPartial = false>
-__global__ __launch_bounds__(256) void gemm_f8_kernel(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ B1,
-    const float* __restrict__ sa, const float* __restrict__ sb, const float* __restrict__ sb1,
-    const uint16_t* C, uint16_t* D, int M, int N, int Kt, float alpha, float beta, int tiles_m, int tiles_n,
-    int shares, int k_per) {
+__device__ __forceinline__ void gemm_f8_tile(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ B1,
+                                             const float* __restrict__ sa, const float* __restrict__ sb, const float* __restrict__ sb1, const uint16_t* C,
+                                             uint16_t* D, int M, int N, const int K, const int lda, float alpha, float beta, const int m_base,
+                                             const int n_base, const size_t p_off = 0) {
   constexpr int NB = kDual ? 2 : 1;
   using SM = F8Smem<BM, BN, NB>;
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
-  static_assert(WM * WN == 4, "four wavefronts");
-  constexpr int A_LOADS = BM / 32;  // 1 KB (8 rows) load instructions per wave per slab
-  constexpr int B_LOADS = BN / 32;  // ... per weight matrix
+  constexpr int NW = WM * WN;
+  static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
+  constexpr int A_LOADS = BM / (8 * NW);  // 1 KB (8 rows) load instructions per wave per slab
+  constexpr int B_LOADS = BN / (8 * NW);  // ... per weight matrix
   constexpr int NS = SM::stages;
   constexpr int LOADS = A_LOADS + NB * B_LOADS;
   // k-steps the loads of one slab are spread over; with two stages they must land within one step
@@ -177,28 +179,6 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
 
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem8[];
   const uint32_t smem_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem8;
-
-  // XCD-aware tile order (workgroup ids round-robin over 8 XCDs): each XCD walks one
-  // contiguous range of tiles, M fastest, so a weight panel stays in that XCD's L2.
-  const int ntiles = tiles_m * tiles_n * (kPartial ? shares : 1);
-  const int per_xcd = (ntiles + 7) / 8;
-  int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (logical >= ntiles) return;
-  int K = Kt;                       // extent of this workgroup's contraction
-  const int lda = Kt;               // row stride of both operands (k contiguous)
-  size_t p_off = 0;                 // this share's slice of the partial sums
-  if constexpr (kPartial) {
-    const int share = logical % shares;
-    logical /= shares;
-    const int k0 = share * k_per;
-    K = Kt - k0 < k_per ? Kt - k0 : k_per;
-    A += k0;
-    B += k0;
-    if constexpr (kDual) B1 += k0;
-    p_off = (size_t)share * M * N;
-  }
-  const int tile_m = logical % tiles_m, tile_n = logical / tiles_m;
-  const int m_base = tile_m * BM, n_base = tile_n * BN;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -227,21 +207,21 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
   uint32_t a_off[A_LOADS], b_off[NB][B_LOADS];
 #pragma unroll
   for (int t = 0; t < A_LOADS; ++t)
-    a_off[t] = (uint32_t)(m_base + (t * 4 + wave) * 8 + (lane >> 3)) * (uint32_t)lda + kc;
+    a_off[t] = (uint32_t)(m_base + (t * NW + wave) * 8 + (lane >> 3)) * (uint32_t)lda + kc;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int t = 0; t < B_LOADS; ++t)
-      b_off[b][t] = (uint32_t)(n_base + (t * 4 + wave) * 8 + (lane >> 3)) * (uint32_t)lda + kc;
+      b_off[b][t] = (uint32_t)(n_base + (t * NW + wave) * 8 + (lane >> 3)) * (uint32_t)lda + kc;
   // la / lb: LDS address of the stage the activations / the weights of the slab go to, + wave * 1024
   auto load_one = [&](auto t_c, uint32_t la, uint32_t lb, bool k_ok) {
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
-      load16_to_lds<t * 4096>(a_rsrc, k_ok ? a_off[t] : kOob, la);
+      load16_to_lds<t * NW * 1024>(a_rsrc, k_ok ? a_off[t] : kOob, la);
       a_off[t] += F8_BK;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
-      load16_to_lds<b * BN * 128 + tt * 4096>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
+      load16_to_lds<b * BN * 128 + tt * NW * 1024>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
       b_off[b][tt] += F8_BK;
     }
   };
@@ -414,12 +394,12 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
   // time in fp32, and stores (and reads C and the row scales) in whole runs through buffer
   // descriptors that end with the matrix, so a pass has no branches.
   constexpr int CW = BN / WN, ROWP = CW * 4 + 16, CPR = CW / 4, ITER = 32 * CPR / 64;
-  static_assert(NB * 4 * 32 * ROWP <= (int)SM::bytes && (32 * CPR) % 64 == 0, "epilogue staging");
+  static_assert(NB * NW * 32 * ROWP <= (int)SM::bytes && (32 * CPR) % 64 == 0, "epilogue staging");
   constexpr int PER = 64 % CPR == 0 ? 1 : CPR / std::gcd(CPR, 64);  // a lane's columns repeat after PER iterations
   typedef unsigned int u32v2_t __attribute__((ext_vector_type(2)));
   __syncthreads();  // every wavefront has read its last fragments
   uint8_t* ep = smem8 + wave * (32 * ROWP);
-  uint8_t* ep1 = smem8 + (4 + wave) * (32 * ROWP);  // kDual: the second product
+  uint8_t* ep1 = smem8 + (NW + wave) * (32 * ROWP);  // kDual: the second product
   const int gn0 = n_base + wn * CW;
   int gns[PER];
   float4_t cs4[PER], cu4[PER];
@@ -538,6 +518,72 @@ __global__ __launch_bounds__(256) void gemm_f8_kernel(
   }
 }
 
+template <int BM, int BN, int WM, int WN, bool kDual, bool kPartial = false>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_f8_kernel(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ B1,
+    const float* __restrict__ sa, const float* __restrict__ sb, const float* __restrict__ sb1,
+    const uint16_t* C, uint16_t* D, int M, int N, int Kt, float alpha, float beta, int tiles_m, int tiles_n,
+    int shares, int k_per) {
+  // XCD-aware tile order (workgroup ids round-robin over 8 XCDs): each XCD walks one
+  // contiguous range of tiles, M fastest, so a weight panel stays in that XCD's L2.
+  const int ntiles = tiles_m * tiles_n * (kPartial ? shares : 1);
+  const int per_xcd = (ntiles + 7) / 8;
+  int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (logical >= ntiles) return;
+  int K = Kt;                       // extent of this workgroup's contraction
+  const int lda = Kt;               // row stride of both operands (k contiguous)
+  size_t p_off = 0;                 // this share's slice of the partial sums
+  if constexpr (kPartial) {
+    const int share = logical % shares;
+    logical /= shares;
+    const int k0 = share * k_per;
+    K = Kt - k0 < k_per ? Kt - k0 : k_per;
+    A += k0;
+    B += k0;
+    if constexpr (kDual) B1 += k0;
+    p_off = (size_t)share * M * N;
+  }
+  gemm_f8_tile<BM, BN, WM, WN, kDual, kPartial>(A, B, B1, sa, sb, sb1, C, D, M, N, K, lda, alpha, beta, logical % tiles_m * BM, logical / tiles_m * BN, p_off);
+}
+
+// The pair on tiles of two heights in one launch, as gemm_f16_hybrid_kernel: a last round that 256-row tiles fill at most half takes half its time on 128-row ones (1973 x
+// 14336 x 4096, 896 tiles: 768 + 2 x 128; 197 -> 190 us).
+__global__ __launch_bounds__(256) void gemm_f8_pair_hybrid_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ B1,
+                                                                  const float* __restrict__ sa, const float* __restrict__ sb,
+                                                                  const float* __restrict__ sb1, uint16_t* D, int M, int N, int K, int tiles_m,
+                                                                  int tiles_n, int n_big) {
+  const int big_grid = (n_big + 7) / 8 * 8;
+  if ((int)blockIdx.x < big_grid) {
+    const int t = xcd_order(blockIdx.x, n_big);
+    if (t >= n_big) return;
+    gemm_f8_tile<256, 128, 2, 2, true>(A, B, B1, sa, sb, sb1, nullptr, D, M, N, K, K, 1.f, 0.f, t % tiles_m * 256, t / tiles_m * 128);
+  } else {
+    const int n_small = 2 * (tiles_m * tiles_n - n_big), u = xcd_order(blockIdx.x - big_grid, n_small);
+    if (u >= n_small) return;
+    const int t = n_big + u / 2, m_base = t % tiles_m * 256 + (u & 1) * 128;
+    if (m_base >= M) return;
+    gemm_f8_tile<128, 128, 2, 2, true>(A, B, B1, sa, sb, sb1, nullptr, D, M, N, K, K, 1.f, 0.f, m_base, t / tiles_m * 128);
+  }
+}
+
+static int launch_pair_hybrid_f8(const uint8_t* A, const uint8_t* B, const uint8_t* B1, const float* sa, const float* sb, const float* sb1, uint16_t* D,
+                                 int M, int N, int K, int n_big, hipStream_t stream) {
+  constexpr size_t lds = std::max(F8Smem<256, 128, 2>::bytes, F8Smem<128, 128, 2>::bytes);
+  static bool attr_set = false;  // benign race: the call is idempotent
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f8_pair_hybrid_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) {
+      set_error("gemm_f8: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+      return NF_ERR_RUNTIME;
+    }
+    attr_set = true;
+  }
+  const int tiles_m = (M + 255) / 256, tiles_n = (N + 127) / 128, n_small = 2 * (tiles_m * tiles_n - n_big);
+  const int grid = (n_big + 7) / 8 * 8 + (n_small + 7) / 8 * 8;
+  gemm_f8_pair_hybrid_kernel<<<grid, 256, lds, stream>>>(A, B, B1, sa, sb, sb1, D, M, N, K, tiles_m, tiles_n, n_big);
+  return check_launch("gemm_f8 launch");
+}
+
 template <int BM, int BN, int WM, int WN, bool kDual = false>
 static int launch_gemm_f8(const uint8_t* A, const uint8_t* B, const float* sa, const float* sb,
                           const uint16_t* C, uint16_t* D, int M, int N, int K, float alpha, float beta,
@@ -556,7 +602,7 @@ static int launch_gemm_f8(const uint8_t* A, const uint8_t* B, const float* sa, c
   }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int grid = ((tiles_m * tiles_n + 7) / 8) * 8;
-  kern<<<grid, 256, SM::bytes, stream>>>(A, B, B1, sa, sb, sb1, C, D, M, N, K, alpha, beta, tiles_m, tiles_n, 1, K);
+  kern<<<grid, WM * WN * 64, SM::bytes, stream>>>(A, B, B1, sa, sb, sb1, C, D, M, N, K, alpha, beta, tiles_m, tiles_n, 1, K);
   return check_launch("gemm_f8 launch");
 }
 
@@ -636,7 +682,7 @@ static int launch_splitk_f8(const uint8_t* A, const uint8_t* B, const uint8_t* B
   float* P1 = kDual ? P + (size_t)shares * M * N : nullptr;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int grid = ((tiles_m * tiles_n * shares + 7) / 8) * 8;
-  kern<<<grid, 256, SM::bytes, stream>>>(A, B, B1, nullptr, nullptr, nullptr, reinterpret_cast<const uint16_t*>(P1),
+  kern<<<grid, WM * WN * 64, SM::bytes, stream>>>(A, B, B1, nullptr, nullptr, nullptr, reinterpret_cast<const uint16_t*>(P1),
                                          reinterpret_cast<uint16_t*>(P), M, N, K, 1.f, 0.f, tiles_m, tiles_n,
                                          shares, k_per);
   int rc = check_launch("gemm_f8 split-K launch");
@@ -705,8 +751,8 @@ int nf_gemm_f8_f16(const uint8_t* Aq, const float* a_scale, const uint8_t* Bq, c
   const double best = std::min(std::min(c256, c192), std::min(c128x256, c128));
   if (best == c256) return launch_gemm_f8<256, 256, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
   if (best == c192) return launch_gemm_f8<256, 192, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
-  if (best == c128x256) return launch_gemm_f8<128, 256, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
-  return launch_gemm_f8<128, 128, 2, 2>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
+  if (best == c128x256) return launch_gemm_f8<128, 256, 2, 4>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
+  return launch_gemm_f8<128, 128, 2, 4>(Aq, Bq, a_scale, b_scale, C, D, M, N, K, alpha, beta, s);
 }
 
 int nf_quantize_weight_e4m3(const uint16_t* W, uint8_t* Wq, float* col_scale, int K, int N,
@@ -741,9 +787,12 @@ int nf_dual_swiglu_f8_f16(const uint8_t* Aq, const float* a_scale, const uint8_t
     return launch_gemm_f8<64, 128, 2, 2, true>(Aq, Gq, a_scale, g_scale, nullptr, out, M, N, K, 1.f, 0.f, s, Uq, u_scale);
   const long long t256 = (long long)((M + 255) / 256) * ((N + 127) / 128);
   const int tail = M % 256;  // rows in the last 256-row tile: half-empty tiles go to the 128-row kernel
-  if (t256 >= 192 && (tail == 0 || tail > 128))
+  if (t256 >= 192 && (tail == 0 || tail > 128)) {
+    const int cus = cu_count(), rest = (int)(t256 % cus);  // tiles of the last, partial round
+    if (t256 > cus && rest > 0 && rest <= cus / 2) return launch_pair_hybrid_f8(Aq, Gq, Uq, a_scale, g_scale, u_scale, out, M, N, K, (int)(t256 - rest), s);
     return launch_gemm_f8<256, 128, 2, 2, true>(Aq, Gq, a_scale, g_scale, nullptr, out, M, N, K, 1.f, 0.f, s, Uq, u_scale);
-  return launch_gemm_f8<128, 128, 2, 2, true>(Aq, Gq, a_scale, g_scale, nullptr, out, M, N, K, 1.f, 0.f, s, Uq, u_scale);
+  }
+  return launch_gemm_f8<128, 128, 2, 4, true>(Aq, Gq, a_scale, g_scale, nullptr, out, M, N, K, 1.f, 0.f, s, Uq, u_scale);
 }
 
 size_t nf_gemm_f8w_workspace_bytes(int M, int K) {
@@ -777,7 +826,7 @@ static int gemm_f8q(const uint8_t* Aq, const float* sa, const uint8_t* Bq, const
     hipStream_t s = (hipStream_t)stream;
     if (M <= 64)
       return launch_splitk_f8<64, 256, 1, 4, false>(Aq, Bq, nullptr, sa, b_scale, nullptr, C, D, M, N, K, alpha, beta, shares, k_per, P, s);
-    return launch_splitk_f8<128, 128, 2, 2, false>(Aq, Bq, nullptr, sa, b_scale, nullptr, C, D, M, N, K, alpha, beta, shares, k_per, P, s);
+    return launch_splitk_f8<128, 128, 2, 4, false>(Aq, Bq, nullptr, sa, b_scale, nullptr, C, D, M, N, K, alpha, beta, shares, k_per, P, s);
   }
   return nf_gemm_f8_f16(Aq, sa, Bq, b_scale, C, D, M, N, K, alpha, beta, stream);
 }
@@ -851,7 +900,7 @@ static int dual_swiglu_f8q(const uint8_t* Aq, const float* sa, const uint8_t* Gq
     hipStream_t s = (hipStream_t)stream;
     if (M <= 64)
       return launch_splitk_f8<64, 128, 2, 2, true>(Aq, Gq, Uq, sa, g_scale, u_scale, nullptr, out, M, N, K, 1.f, 0.f, shares, k_per, P, s);
-    return launch_splitk_f8<128, 128, 2, 2, true>(Aq, Gq, Uq, sa, g_scale, u_scale, nullptr, out, M, N, K, 1.f, 0.f, shares, k_per, P, s);
+    return launch_splitk_f8<128, 128, 2, 4, true>(Aq, Gq, Uq, sa, g_scale, u_scale, nullptr, out, M, N, K, 1.f, 0.f, shares, k_per, P, s);
   }
   return nf_dual_swiglu_f8_f16(Aq, sa, Gq, g_scale, Uq, u_scale, out, M, N, K, stream);
 }

@@ -17,8 +17,8 @@ def operands(M, N, K_, n):
 
 
 @pytest.mark.parametrize("K_", DEPTHS)
-@pytest.mark.parametrize("M,N", [(2048, 8192), (1800, 8008), (2000, 6152), (1793, 5960), (2000, 6144), (2000, 10240), (1990, 10216)])
-# 256 x 256 tiles of the first three, 256 x 192 of the others (whole and ragged columns; 32 to 54 tiles of columns)
+@pytest.mark.parametrize("M,N", [(2048, 8192), (1800, 8008), (2000, 6152), (1793, 5960), (2000, 6144), (2000, 10240), (1990, 10216), (1030, 4104), (300, 520)])
+# 256 x 256 tiles of the first three, 256 x 192 of the others (whole and ragged columns; 32 to 54 tiles of columns), at last 128 rows on eight wavefronts
 def test_products(M, N, K_):
     from nanoflow_amd import kernels as K
     (a, b), (sa, sb), (av, bv), gen = operands(M, N, K_, 1)
@@ -29,7 +29,8 @@ def test_products(M, N, K_):
 
 
 @pytest.mark.parametrize("K_", DEPTHS)
-@pytest.mark.parametrize("M,N", [(2048, 3072), (1937, 3080)])
+@pytest.mark.parametrize("M,N", [(2048, 3072), (1937, 3080), (1937, 4232), (2048, 6144), (300, 520)])
+# 256 x 128 tiles; the third and fourth with a last round of half the height; 128 x 128 on eight wavefronts
 def test_pairs(M, N, K_):
     from nanoflow_amd import kernels as K
     (a, b, u), (sa, sb, su), (av, bv, uv), _ = operands(M, N, K_, 2)
