@@ -40,7 +40,7 @@ __device__ __forceinline__ TilePlace find_tile(const nf_grouped_gemm_args& a, in
 }
 
 // The BM x BN tile of a group from row t.m_base and column n_base.
-template <class E, int BM, int BN, int WM, int WN, int kCap>
+template <class E, int BM, int BN, int WM, int WN, int kCap, bool kTurn = true>
 __device__ __forceinline__ void grouped_tile(const nf_grouped_gemm_args& a, const TilePlace& t, int n_base) {
   const bool routed = a.routing.n_tiles != nullptr;
   const int32_t* rows = routed && a.gather ? a.routing.row_of + t.row0 : nullptr;
@@ -57,7 +57,8 @@ __device__ __forceinline__ void grouped_tile(const nf_grouped_gemm_args& a, cons
   // channels at a time (a stream of 8 rows of 128 bytes an instruction: 4.4 TB/s, 6.1 with every workgroup at another k).  So every column tile
   // of an expert starts K at a slab of its own and goes round; the m tiles that share its weights start at the same one.  748 rows, 5 of 32
   // experts of 2048 x 2048: 90 -> 80 us up, 88 -> 79 down; where experts have 200 rows and more and the matrix cores set the pace, the same.
-  const int turn = routed ? (t.n_tile + t.group * 4) % ((a.K + BK - 1) / BK) : 0;
+  // Other strides, and the tiles of the one expert beside a weight stream, lose 2 % by it.
+  const int turn = kTurn && routed && a.K % 2048 == 0 ? (t.n_tile + t.group * 4) % ((a.K + BK - 1) / BK) : 0;
   gemm_tile<E, BM, BN, WM, WN, false, true, false, true, kCap>(A, (const uint16_t*)a.b + (size_t)t.group * a.N * a.K, nullptr, nullptr, D,
                                                                t.rows, a.N, a.K, 1.f, 0.f, a.N, t.m_base, n_base, a.lda, a.K,
                                                                a.ldd, rows, a.M, ep, 0, 1, turn);
@@ -119,7 +120,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_rows_kernel(nf_grouped_gemm_
         });
   };
   if (t.rows > kFewRows) {
-    if (t.m_base % 128 == 0) grouped_tile<E, 128, 32, 4, 1, kHalfCu>(a, t, t.n_tile * 32);
+    if (t.m_base % 128 == 0) grouped_tile<E, 128, 32, 4, 1, kHalfCu, false>(a, t, t.n_tile * 32);
   } else if (t.rows <= 16) {
     pass(ic<16>{}, t.m_base);
   } else if (t.rows <= 32) {
@@ -226,13 +227,14 @@ int launch_chain(const nf_grouped_gemm_args& a, hipStream_t s) {
 // Tile lists of 128 rows that run on gemm_chain.h.  Contractions beyond 2048 against whole column tiles do, where a 128 x 256 tile on four
 // wavefronts ran before: 0.90 to 1.00 of its time over 300 to 2048 rows, 8 to 65 experts of 512 to 4096 columns 2304 to 3584 deep.
 // At 2048 two workgroups of 128 x 128 a CU stand against it, which leave less of a round idle: it pays where its own rounds are at least four
-// fifths full, or one is at least half full (2.9 and 5.8 rounds: 0.91 of their time, 0.6 of one 0.88; 1.1 to 2.2: 1.02 to 1.14).  The rows of
+// fifths full of columns that are there, or one is at least half full (2.9 and 5.8 rounds: 0.91 of their time, 0.6 of one 0.88; 1.1 to 2.2: 1.02 to 1.14;
+// 4.05 with a tenth of it past the columns: 1.05).  The rows of
 // an expert are not known here: half a tile each over the sorted rows.  Below 2048 neither wins.
 bool chain_pays(const nf_grouped_gemm_args& a) {
   if (a.K < 2048 || a.N < 256 || a.ldd > 1 << 22 || (a.act == NF_ACT_GATED ? a.N % 16 != 0 : a.weigh)) return false;
   if (a.K > 2048) return a.N % 256 == 0;
-  const double rounds = (a.max_rows / 128.0 + a.groups * 0.5) * ((a.N + 255) / 256) / cu_count();
-  return rounds < 1 ? rounds >= 0.5 : std::ceil(rounds) <= 1.25 * rounds;
+  const double m_tiles = a.max_rows / 128.0 + a.groups * 0.5, rounds = m_tiles * ((a.N + 255) / 256) / cu_count(), filled = m_tiles * a.N / 256.0 / cu_count();
+  return rounds < 1 ? filled >= 0.5 : std::ceil(rounds) <= 1.25 * filled;
 }
 
 template <class E>
@@ -257,8 +259,10 @@ int dispatch_grouped(const nf_grouped_gemm_args& a, int tile_rows, hipStream_t s
     if (a.K <= 2048)
       return tile_rows == 64 ? launch_grouped<E, 64, 128, 2, 2, kHalfCu>(a, s) : launch_grouped<E, 128, 128, 2, 2, kHalfCu, true>(a, s);
   }
-  if (tile_rows == 64) return a.N <= 128 ? launch_grouped<E, 64, 128, 2, 2>(a, s) : launch_grouped<E, 64, 256, 1, 4>(a, s);
-  return a.N > 128 && a.N % 256 == 0 ? launch_grouped<E, 128, 256, 2, 2>(a, s) : launch_grouped<E, 128, 128, 2, 2>(a, s);
+  // One workgroup a CU: eight wavefronts (us, four -> eight: 16 heads of 128 x 512 for 128 rows 8.1 -> 6.4, of 576 x 128 5.1 -> 4.4; 256 rows, 4 of 33 experts of
+  // 2048 x 4096 156 -> 131, the contraction turned among it).  Two a CU gain nothing by it (1946 rows, 33 experts of 3072 x 1536 144 and 155).
+  if (tile_rows == 64) return a.N <= 128 ? launch_grouped<E, 64, 128, 2, 4>(a, s) : launch_grouped<E, 64, 256, 2, 4>(a, s);
+  return a.N > 128 && a.N % 256 == 0 ? launch_grouped<E, 128, 256, 2, 4>(a, s) : launch_grouped<E, 128, 128, 2, 4>(a, s);
 }
 
 }  // namespace
