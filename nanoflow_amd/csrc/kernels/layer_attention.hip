@@ -1114,9 +1114,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile_kernel(nf_window_attention_a
   }
 }
 
-template <int KD, int VD, int kMaps = 1>
-static int launch_tile(const nf_window_attention_args& a, hipStream_t s) {
-  constexpr int NB = 2 / kMaps;
+template <int KD, int VD, int kMaps, int NB>
+static int launch_tile_of(const nf_window_attention_args& a, hipStream_t s) {
   const int group = a.kv.heads / a.kv.kv_heads;
   const int chunks = (group + 15) / 16, gs = (group + chunks - 1) / chunks;
   const int tile_tokens = 4 * NB * (16 / gs);
@@ -1134,6 +1133,21 @@ static int launch_tile(const nf_window_attention_args& a, hipStream_t s) {
   const unsigned tiles = (unsigned)(a.max_rows / tile_tokens + a.req_num);
   kern<<<dim3((unsigned)(a.kv.kv_heads * chunks), tiles), 256, lds, s>>>(a, gs, chunks, tile_tokens, (long long)tiles * a.kv.kv_heads * chunks <= 2 * 256 + 64);
   return check_launch("nf_window_attention (tiles)");
+}
+
+// One column block a wavefront where that leaves at most three workgroups a CU, else two (of two maps always one).  A tile is bound by its chain
+// of steps -- barrier, scores, softmax, products -- and two workgroups a CU with half the columns run beside each other; beyond, every step's
+// keys pass through a CU twice as often.  us, two blocks -> one: 16 heads over 4, 2 x 1024 tokens in chunks 47 -> 32, window 512 30 -> 24; latents written out,
+// 16 heads, 700 tokens on 300 41 -> 29, 2047 80 -> 59; 64 heads 700 tokens (704 workgroups) 50 -> 45; but 32 heads 4 x 500 on 700 (1032) 65 -> 67 and,
+// latents, 62 -> 74.
+template <int KD, int VD, int kMaps = 1>
+static int launch_tile(const nf_window_attention_args& a, hipStream_t s) {
+  if constexpr (kMaps == 1) {
+    const int group = a.kv.heads / a.kv.kv_heads, chunks = (group + 15) / 16, gs = (group + chunks - 1) / chunks;
+    const long long groups = ((long long)a.max_rows / (4 * (16 / gs)) + a.req_num) * a.kv.kv_heads * chunks;
+    if (groups > 3 * 256) return launch_tile_of<KD, VD, 1, 2>(a, s);
+  }
+  return launch_tile_of<KD, VD, kMaps, 1>(a, s);
 }
 
 template <int KD, int VD, int kMaps = 1>

@@ -252,6 +252,14 @@ def test_scales_that_are_not_positive(scale):
         close(got, want, dtype)
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(40, 40), (45, 45), (46, 46), (64, 64), (96, 24), (192, 48)])
+def test_prompts_on_one_and_two_column_blocks(heads, kv_heads):
+    """Up to 768 workgroups of one block a wavefront (17 tiles of 64 tokens a head, or 64 of 16), and more on two."""
+    b = cases.batch([], [(30, 700), (0, 301)] if heads == kv_heads else [(30, 333), (0, 150)], seed=heads)
+    got, want = attention_case(BF16, heads, kv_heads, 64, 64, 100, 5, b, 0, seed=3, out_scale=1.3)
+    close(got, want, BF16)
+
+
 def test_long_decode_context_and_many_requests():
     b = cases.batch(np.random.default_rng(0).integers(1, 700, 80).tolist(), [], seed=1)
     got, want = attention_case(BF16, 8, 2, 64, 64, 300, 20, b, 80, seed=2)
