@@ -370,7 +370,16 @@ static int dispatch_rows_dual(const void* A, const void* Bg, const void* Bu, uin
                               const RowsScales& sc = {}) {
   if (M <= 8) return launch_rows<E, 8, 1, 8, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
   if (M <= 16) return launch_rows<E, 16, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-  if (M <= 32) return launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+  // A workgroup of 32 columns is one a CU, and its rows of A come with every one, so between 48 and 64 columns a CU two nearly full rounds of
+  // them lose to one round of twice the width, whose LDS holds a ring of one: 64 x 14336 x 4096 52 -> 46 us, 64 x 16384 x 4096 59 -> 52, 40 x
+  // 16384 x 4096 57 -> 51, 32 x 16384 x 4096 58 -> 55, e4m3 64 x 14336 x 4096 32 -> 29, 24 x 14336 x 4096 26 -> 24.  Below, the second round is
+  // short enough to cost less (64 x 8192 x 4096, which has none: 28 and 41; 40 x 11264 x 4096 44 and 46); above, both take as many bytes a
+  // round and the shorter ring shows (64 x 18432 x 4096 66 and 72).  The sums keep their order.
+  const bool wide = N >= 48 * cu_count() && N <= 64 * cu_count();
+  if (M <= 32)
+    return wide ? launch_rows<E, 32, 4, 4, 2, 1, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc)
+                : launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
+  if (wide) return launch_rows<E, 64, 4, 4, 2, 1, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
   return launch_rows<E, 64, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
 }
 

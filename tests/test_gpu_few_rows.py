@@ -108,6 +108,25 @@ def test_gate_up_pair_of_few_rows(M, N, K_):
         assert torch.equal(got, K.dual_swiglu_ws(a, g.t().contiguous(), u.t().contiguous())[0])
 
 
+# between 48 and 64 columns a CU: its edges, a cut tile, a last unit that is cut; a column's sums do not depend on the tile, so the bits are
+# those of the same columns in launches of 32 a CU, whose tile the tests above hold to float64
+@pytest.mark.parametrize("N,K_", [(12280, 1544), (12288, 1544), (14344, 3088), (16376, 1552), (16384, 4096)])
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+def test_gate_up_pair_on_wide_tiles(M, N, K_):
+    from nanoflow_amd import kernels as K
+    a, g = operands(M, N, K_, torch.float16)
+    _, u = operands(M, N, K_, torch.float16, seed=1)
+    halves = lambda pair: torch.cat([pair(slice(0, 8192))[:, :N - 8192], pair(slice(N - 8192, N))], 1)
+    pair = lambda r: K.dual_swiglu_ws(a, g[r], u[r], b_col_major=True)[0]
+    assert torch.equal(pair(slice(0, N)), halves(pair))
+    if K_ < 3072:   # shorter e4m3 rows are not this stream's
+        return
+    qa, qg, qu = ((16 * w).to(torch.float8_e4m3fn).view(torch.uint8) for w in (a, g, u))
+    sa, sg, su = (torch.rand(n, device="cuda") + 0.01 for n in (M, N, N))
+    pair = lambda r: K.dual_swiglu_f8q(qa, sa, qg[r], sg[r], qu[r], su[r])
+    assert torch.equal(pair(slice(0, N)), halves(pair))
+
+
 @pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("N,K_", [(72, 3088), (4104, 4096), (264, 8192)])
 def test_e4m3_products_of_few_rows(M, N, K_):
