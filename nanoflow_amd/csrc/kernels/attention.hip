@@ -17,6 +17,7 @@
 // one XCD starts together are the heads of one request and stream the same 64 KiB pages.  Prefill: a workgroup is a
 // 16-token tile (for GQA 4) whose wavefronts share the streamed K/V tiles; tiles are planned
 // on the device from qo_indptr (prefix of tiles per request) -- no host round trip in either mode.
+#include <climits>
 #include <type_traits>
 
 #include "common.h"
@@ -43,58 +44,106 @@ union H8 {
 //   tiles fit into two such waves every workgroup is resident from the start, nothing fills in
 //   behind anything, and what counts is which two tiles share a CU: the second wave then runs from
 //   the shortest tile up, so that the longest tile shares its CU with the shortest.
-constexpr int kPlanSortMax = 1024;
-__global__ __launch_bounds__(256) void attn_plan_kernel(const int32_t* __restrict__ qo_indptr,
-                                                        const int32_t* __restrict__ kv_indptr,
-                                                        const int32_t* __restrict__ kv_last_page_len,
-                                                        int32_t* __restrict__ tile_start, int32_t* __restrict__ tile_order,
-                                                        int batch, int wg_tok, int causal, int first_wave) {
-  __shared__ int s_sum[256];
-  __shared__ int s_key[kPlanSortMax];
-  const int per = (batch + 255) / 256;
-  const int lo = threadIdx.x * per, hi = min(lo + per, batch);
+//   What bounds it is its chain of dependent reads and barriers on one CU, so up to 1024 requests are read at once, one a thread, every tile finds
+//   its request by bisection in LDS, and the ranks are counted four keys a read by as many threads a tile as there are (us, one thread a tile with a
+//   key a read and 256 requests at once -> this: 2 prompts, 125 tiles 9.9 -> 5.5; 3 prompts of 484, 88 tiles 7.7 -> 5.2; an empty launch takes 4).
+constexpr int kPlanThreads = 1024, kPlanSortMax = 1024;
+__global__ __launch_bounds__(kPlanThreads) void attn_plan_kernel(const int32_t* __restrict__ qo_indptr,
+                                                                 const int32_t* __restrict__ kv_indptr,
+                                                                 const int32_t* __restrict__ kv_last_page_len,
+                                                                 int32_t* __restrict__ tile_start, int32_t* __restrict__ tile_order,
+                                                                 int batch, int wg_tok, int causal, int first_wave) {
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  static_assert(kPlanThreads == kPlanSortMax, "a thread a tile");
+  __shared__ int s_wave[kPlanThreads / 64], s_first[kPlanThreads], s_len[kPlanThreads], s_kv[kPlanThreads], s_rank[kPlanSortMax];
+  __shared__ i32x4 s_key4[kPlanSortMax / 4];
+  int* s_key = reinterpret_cast<int*>(s_key4);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int per = (batch + kPlanThreads - 1) / kPlanThreads;
+  const int lo = min(tid * per, batch), hi = min(lo + per, batch);
+  auto len_of = [&](int i) { return qo_indptr[i + 1] - qo_indptr[i]; };
+  auto kv_of = [&](int i) {
+    const int npages = kv_indptr[i + 1] - kv_indptr[i], last = kv_last_page_len[i];
+    return npages > 0 ? (npages - 1) * PAGE + last : 0;
+  };
+  auto tiles_of = [&](int len) { return len > 0 ? (len + wg_tok - 1) / wg_tok : 0; };
+  auto key_of = [&](int t, int len, int kv_len) {  // keys that tile t of a request sees
+    return causal ? min(kv_len, kv_len - len + min((t + 1) * wg_tok, len)) : kv_len;
+  };
   int sum = 0;
-  for (int i = lo; i < hi; ++i) {
-    int len = qo_indptr[i + 1] - qo_indptr[i];
-    sum += len > 0 ? (len + wg_tok - 1) / wg_tok : 0;
-  }
-  s_sum[threadIdx.x] = sum;
-  __syncthreads();
-  // inclusive scan over the 256 partial sums (Hillis-Steele)
-  for (int off = 1; off < 256; off <<= 1) {
-    int v = threadIdx.x >= off ? s_sum[threadIdx.x - off] : 0;
-    __syncthreads();
-    s_sum[threadIdx.x] += v;
-    __syncthreads();
-  }
-  int run = s_sum[threadIdx.x] - sum;  // exclusive prefix of this thread's range
-  const int total = s_sum[255];
-  if (threadIdx.x == 255) tile_start[batch] = total;
-  for (int i = lo; i < hi; ++i) {
-    tile_start[i] = run;
-    const int len = qo_indptr[i + 1] - qo_indptr[i];
-    const int n = len > 0 ? (len + wg_tok - 1) / wg_tok : 0;
-    if (total <= kPlanSortMax) {  // keys the request's tiles see
-      const int npages = kv_indptr[i + 1] - kv_indptr[i];
-      const int kv_len = npages > 0 ? (npages - 1) * PAGE + kv_last_page_len[i] : 0;
-      for (int t = 0; t < n; ++t) {
-        const int last = min((t + 1) * wg_tok, len) - 1;
-        s_key[run + t] = causal ? min(kv_len, kv_len - len + last + 1) : kv_len;
-      }
+  s_rank[tid] = 0;
+  if (per == 1) {
+    int len = 0, kv_len = 0;
+    if (tid < batch) {
+      len = len_of(tid);
+      kv_len = kv_of(tid);
     }
-    run += n;
+    s_len[tid] = len;
+    s_kv[tid] = kv_len;
+    sum = tiles_of(len);
+  } else {
+    for (int i = lo; i < hi; ++i) sum += tiles_of(len_of(i));
   }
+  int to = sum;  // inclusive sums over the threads
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int x = __shfl_up(to, d, 64);
+    if (lane >= d) to += x;
+  }
+  if (lane == 63) s_wave[wave] = to;
   __syncthreads();
+  int total = 0;
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; ++w) {
+    const int x = s_wave[w];
+    if (w < wave) to += x;
+    total += x;
+  }
+  int run = to - sum;  // exclusive prefix of this thread's range
+  if (tid == 0) tile_start[batch] = total;
+  if (per == 1) {
+    if (tid < batch) tile_start[tid] = run;
+    s_first[tid] = run;
+  } else {
+    for (int i = lo; i < hi; ++i) {
+      tile_start[i] = run;
+      const int len = len_of(i), n = tiles_of(len);
+      if (total <= kPlanSortMax && n > 0) {
+        const int kv_len = kv_of(i);
+        for (int t = 0; t < n; ++t) s_key[run + t] = key_of(t, len, kv_len);
+      }
+      run += n;
+    }
+  }
   if (total > kPlanSortMax) {
-    for (int t = threadIdx.x; t < total; t += 256) tile_order[t] = t;
+    for (int t = tid; t < total; t += kPlanThreads) tile_order[t] = t;
     return;
   }
-  for (int t = threadIdx.x; t < total; t += 256) {
-    const int key = s_key[t];
-    int rank = 0;
-    for (int u = 0; u < total; ++u) rank += (s_key[u] > key) || (s_key[u] == key && u < t);
+  if (per == 1) {
+    __syncthreads();
+    if (tid < total) {  // the last request that starts at this tile or before: those without tiles start where the next one does
+      int r = 0;
+      for (int d = 1 << (31 - __builtin_clz(batch)); d > 0; d >>= 1)
+        if (r + d < batch && s_first[r + d] <= tid) r += d;
+      s_key[tid] = key_of(tid - s_first[r], s_len[r], s_kv[r]);
+    }
+  }
+  if (tid >= total) s_key[tid] = INT_MIN;  // behind every tile
+  __syncthreads();
+  const int width = total <= 64 ? 64 : 1 << (32 - __builtin_clz(total - 1));  // threads that stand for a tile each; `parts` of them share a tile's count
+  const int t = tid & (width - 1), part = tid / width, parts = kPlanThreads / width, key = s_key[t];
+  int ahead = 0;
+  for (int q = part; q < (total + 3) / 4; q += parts) {
+    const i32x4 k = s_key4[q];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ahead += (k[j] > key) || (k[j] == key && 4 * q + j < t);
+  }
+  if (t < total && ahead > 0) atomicAdd(&s_rank[t], ahead);
+  __syncthreads();
+  if (tid < total) {
+    const int rank = s_rank[tid];
     const bool pair_up = first_wave > 0 && total <= 2 * first_wave && rank >= first_wave;
-    tile_order[pair_up ? first_wave + (total - 1 - rank) : rank] = t;
+    tile_order[pair_up ? first_wave + (total - 1 - rank) : rank] = tid;
   }
 }
 
@@ -747,7 +796,7 @@ static int launch_attn(const uint16_t* q, uint16_t* o, const int32_t* qo_indptr,
       cus = v;
     }
     const int first_wave = num_blocks > 0 ? 0 : cus / Hkv;
-    attn_plan_kernel<<<1, 256, 0, stream>>>(qo_indptr, kv_indptr, kv_last_page_len, tile_start, tile_order, batch,
+    attn_plan_kernel<<<1, kPlanThreads, 0, stream>>>(qo_indptr, kv_indptr, kv_last_page_len, tile_start, tile_order, batch,
                                             wg_tok, causal, first_wave);
     bound = ((long long)batch + max_qo_rows / wg_tok) * Hkv;
   }

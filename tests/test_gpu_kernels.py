@@ -792,6 +792,15 @@ def test_attention_long_context_prefill(K, oracle):
     _attn_case(K, oracle, 8, 2, [], [(1900, 147)], seed=14)
 
 
+# a prompt launch's plan: tiles of 8 rows up to and past a wavefront's 64 and a workgroup's 1024, requests likewise, some without rows
+@pytest.mark.parametrize("prefill", [
+    [(0, 512)], [(0, 513)], [(5, 0), (20, 100), (9, 0), (9, 0), (1, 17), (4, 0)], [(7, 8)] * 1024, [(7, 8)] * 1023 + [(0, 16)],
+    [(5, 0), (3, 3)] * 512, [(7, 8)] * 1024 + [(1, 0)], [(5, 0), (3, 3)] * 1024, [(7, 8)] * 1024 + [(0, 2)],
+], ids=["64 tiles", "65 tiles", "empty requests", "1024 tiles", "1025 tiles", "every other empty", "1025 requests", "2048 requests", "1025 of both"])
+def test_attention_prefill_plan(K, oracle, prefill):
+    _attn_case(K, oracle, 8, 1, [], prefill, seed=18)
+
+
 def test_attention_page_permutation_invariance(K):
     rng = np.random.default_rng(15)
     Hq, Hkv, d, P = 32, 8, 128, 16
