@@ -3,7 +3,7 @@
 // route_rows_kernel: one wavefront per token, its scores in registers (fp32 softmax over all outputs, or a sigmoid of each), groups of
 //   outputs closed by the rank of their largest entry, the `top` largest taken one after the other, then the
 //   experts that every token has.
-// route_plan_kernel: one workgroup counts the rows of every expert, places them (an expert's rows consecutive)
+// route_plan_kernel: counts the rows of every expert, places them (an expert's rows consecutive)
 //   and lists the m tiles of the grouped product.  The place of a row inside its expert's run
 //   depends on the order of LDS atomics; nothing computed from it does.
 #include <algorithm>
@@ -120,30 +120,40 @@ __global__ __launch_bounds__(256) void route_rows_kernel(nf_route_args a, int32_
 }
 
 // experts: of the grouped product, the last `always` of which have every token's row, in the tokens' order.
-// kStaged: the sorted rows and weights are put together in LDS and written in whole runs; one CU takes a scattered store's 64 lanes
-// one by one (1946 rows of 5: 15 -> 11 us).  Its bytes for every entry, up to kStagedEntries.
-constexpr int kStagedEntries = 16384;
-template <bool kStaged>
-__global__ __launch_bounds__(1024) void route_plan_kernel(nf_routing r, int rows, int top, int always, int experts) {
-  extern __shared__ int staged[];  // [n] rows, [n] weights
-  __shared__ int count[kMaxOutputs], first[kMaxOutputs], tile0[kMaxOutputs], wave_rows[16], wave_tiles[16];
+// What bounds it is what one CU can read and write, so every workgroup places a share of the entries, kPlanChunk at a time, all of which every workgroup
+// counts: those ahead of its own apart from the rest (us, one workgroup for all -> this: 1946 rows of 5 10.8 -> 7.3, 2047 of 5 9.3 -> 6.8; 748
+// rows of 5 5.4 -> 5.0, 256 of 5 4.7 and 4.7; an empty launch takes 4).
+constexpr int kPlanChunk = 1024, kPlanGroups = 32;
+__global__ __launch_bounds__(kPlanChunk) void route_plan_kernel(nf_routing r, int rows, int top, int always, int experts) {
+  __shared__ int ahead[kMaxOutputs], count[kMaxOutputs], first[kMaxOutputs], wave_rows[16], wave_tiles[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, routed = experts - always, per_token = top + always, n = rows * per_token;
+  const int chunks = (n - 1) / kPlanChunk + 1, per_group = (chunks + gridDim.x - 1) / gridDim.x;
+  const int c0 = min((int)blockIdx.x * per_group, chunks), c1 = min(c0 + per_group, chunks);
+  int own = 0;
+  float weight = 0.f;
+  auto read_own = [&](int c) {
+    const int i = min(c * kPlanChunk + tid, n - 1);
+    own = r.choice[i];
+    weight = r.weight[i];
+  };
+  if (c0 < c1) read_own(c0);
+  ahead[tid] = 0;
   count[tid] = tid >= routed && tid < experts ? rows : 0;
   __syncthreads();
-  constexpr int kAhead = 4;  // choices of a thread requested at once
-  for (int i0 = tid; i0 < n; i0 += kAhead * 1024) {
+  constexpr int kAhead = 8;  // choices of a thread requested at once
+  for (int c = 0; c < chunks; c += kAhead) {
     int e[kAhead];
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) e[k] = r.choice[min(i0 + k * 1024, n - 1)];
+    for (int k = 0; k < kAhead; ++k) e[k] = c + k < chunks ? r.choice[min((c + k) * kPlanChunk + tid, n - 1)] : experts;
 #pragma unroll
     for (int k = 0; k < kAhead; ++k) {
-      const int i = i0 + k * 1024;
-      if (i < n && e[k] < routed) atomicAdd(&count[e[k]], 1);  // those of every token are past the outputs
+      if (c + k == chunks - 1 && tid >= n - (chunks - 1) * kPlanChunk) e[k] = experts;
+      if (e[k] < routed) atomicAdd(c + k < c0 ? &ahead[e[k]] : &count[e[k]], 1);  // those of every token are past the outputs
     }
   }
   __syncthreads();
   // exclusive sums over the experts: rows, tiles
-  const int c = count[tid], tiles = (c + r.tile_rows - 1) / r.tile_rows;
+  const int before = ahead[tid], c = count[tid] + before, tiles = (c + r.tile_rows - 1) / r.tile_rows;
   int rows_to = c, tiles_to = tiles;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -162,57 +172,32 @@ __global__ __launch_bounds__(1024) void route_plan_kernel(nf_routing r, int rows
     rows_to += wave_rows[w];
     tiles_to += wave_tiles[w];
   }
-  first[tid] = rows_to - c;
-  tile0[tid] = tiles_to - tiles;
-  if (tid < experts) {
+  first[tid] = rows_to - c + before;  // nobody's entries are ahead of another's at the experts of every token
+  if (blockIdx.x == 0 && tid < experts) {
+    const int tile0 = tiles_to - tiles;
     r.offsets[tid + 1] = rows_to;
     if (tid == 0) r.offsets[0] = 0;
     if (tid == experts - 1) *r.n_tiles = tiles_to;
     for (int i = 0; i < tiles; ++i) {
-      r.tile_group[tile0[tid] + i] = tid;
-      r.tile_row[tile0[tid] + i] = i * r.tile_rows;
+      r.tile_group[tile0 + i] = tid;
+      r.tile_row[tile0 + i] = i * r.tile_rows;
     }
   }
   __syncthreads();
-  const float inv = 1.f / (float)per_token;
-  for (int i0 = tid; i0 < n; i0 += kAhead * 1024) {
-    int choice[kAhead];
-    float weight[kAhead];
-#pragma unroll
-    for (int x = 0; x < kAhead; ++x) {
-      choice[x] = r.choice[min(i0 + x * 1024, n - 1)];
-      weight[x] = r.weight[min(i0 + x * 1024, n - 1)];
-    }
-#pragma unroll
-    for (int x = 0; x < kAhead; ++x) {
-      const int i = i0 + x * 1024, e = choice[x];
-      if (i >= n) break;
-      // half an entry past a multiple is 2^-7 from the next one at least, fp32 is off by 2^-9 at most below 2^14
-      const int t = kStaged ? (int)(((float)i + 0.5f) * inv) : i / per_token, k = i - t * per_token;
+  for (int c = c0; c < c1; ++c) {
+    const int i = c * kPlanChunk + tid;
+    if (i < n) {
+      const int t = i / per_token, k = i - t * per_token;
       int at = -1;
       if (k >= top) at = first[routed + k - top] + t;
-      else if (e < routed) at = atomicAdd(&first[e], 1);
+      else if (own < routed) at = atomicAdd(&first[own], 1);
       if (at >= 0) {
-        if constexpr (kStaged) {
-          staged[at] = t;
-          staged[n + at] = (int)__float_as_uint(weight[x]);
-        } else {
-          r.row_of[at] = t;
-          if (r.row_weight) r.row_weight[at] = weight[x];
-        }
+        r.row_of[at] = t;
+        if (r.row_weight) r.row_weight[at] = weight;
       }
       r.place[i] = at;
     }
-  }
-  if constexpr (kStaged) {
-    __syncthreads();
-    int sorted = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) sorted += wave_rows[w];
-    for (int i = tid; i < sorted; i += 1024) {
-      r.row_of[i] = staged[i];
-      if (r.row_weight) r.row_weight[i] = __uint_as_float((uint32_t)staged[n + i]);
-    }
+    if (c + 1 < c1) read_own(c + 1);
   }
 }
 
@@ -253,22 +238,8 @@ int nf_route(const nf_route_args* args, const nf_routing* routing, nf_stream_t s
   const int per = (a.outputs + 63) / 64;
   const int rc = per <= 1 ? go(ic<1>{}) : per <= 2 ? go(ic<2>{}) : per <= 4 ? go(ic<4>{}) : per <= 8 ? go(ic<8>{}) : go(ic<16>{});
   if (rc) return rc;
-  const size_t n = (size_t)a.rows * (a.top + a.always);
-  if (n > kStagedEntries) {
-    route_plan_kernel<false><<<1, 1024, 0, s>>>(r, a.rows, a.top, a.always, a.experts + a.always);
-    return check_launch("nf_route (plan)");
-  }
-  static bool attr_set = false;  // benign race: the call is idempotent
-  if (!attr_set) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(route_plan_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             kStagedEntries * 8);
-    if (e != hipSuccess) {
-      set_error("%s: cannot reserve %d bytes of LDS: %s", who, kStagedEntries * 8, hipGetErrorString(e));
-      return NF_ERR_RUNTIME;
-    }
-    attr_set = true;
-  }
-  route_plan_kernel<true><<<1, 1024, n * 8, s>>>(r, a.rows, a.top, a.always, a.experts + a.always);
+  const long long chunks = ((long long)a.rows * per_token + kPlanChunk - 1) / kPlanChunk;
+  route_plan_kernel<<<(unsigned)std::min<long long>(chunks, kPlanGroups), kPlanChunk, 0, s>>>(r, a.rows, a.top, a.always, a.experts + a.always);
   return check_launch("nf_route (plan)");
 }
 

@@ -1,4 +1,4 @@
-"""The order of the routed rows by expert, at the edges of what one workgroup stages: whole numbers and copied weights, so exact."""
+"""The order of the routed rows by expert, at the edges of what one workgroup places: whole numbers and copied weights, so exact."""
 import numpy as np
 import pytest
 
@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,experts,identity,top,always", [(1, 3, 0, 1, 0), (255, 5, 2, 3, 1), (2047, 32, 8, 5, 0), (3276, 33, 0, 4, 1), (4096, 7, 0, 3, 1), (4096, 40, 3, 4, 0),
-                                                           (4097, 40, 3, 4, 0), (273, 100, 20, 58, 2), (16384, 2, 0, 1, 0), (5462, 3, 1, 1, 2)])
+                                                           (4097, 40, 3, 4, 0), (273, 100, 20, 58, 2), (16384, 2, 0, 1, 0), (5462, 3, 1, 1, 2), (1024, 32, 0, 3, 1), (4097, 9, 0, 1, 0), (8200, 5, 0, 4, 1)])
 def test_rows_by_expert(T, experts, identity, top, always):
     from nanoflow_amd import kernels as K
     outputs, per = experts + identity, top + always
