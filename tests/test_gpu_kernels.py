@@ -496,9 +496,9 @@ def _quantize_weights_nk(W):
     return q, sc
 
 
-# row lengths on both sides of what the quantiser keeps in registers (8192 and 32768 halves)
+# row lengths on both sides of what the quantiser keeps in registers (4096, 16384 of more than 512 rows, and 32768 halves)
 @pytest.mark.parametrize("M,K_", [(1, 16), (5, 4096), (33, 144), (64, 28672), (7, 8192), (6, 8208), (9, 14336),
-                                  (4, 32768), (3, 32784), (3, 40960)])
+                                  (4, 32768), (3, 32784), (3, 40960), (513, 4112), (512, 16384), (513, 16384), (513, 16400)])
 def test_quantize_rows_e4m3_bit_exact(K, oracle, M, K_):
     rng = np.random.default_rng(M * 7 + K_)
     X = (rng.normal(0, 1, (M, K_)) * rng.uniform(0.01, 20, (M, 1))).astype(np.float16)
