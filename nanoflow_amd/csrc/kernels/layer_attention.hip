@@ -1158,14 +1158,12 @@ static int launch_window(const nf_window_attention_args& a, hipStream_t s) {
   const unsigned gy = (unsigned)(a.kv.kv_heads * chunks);
   if (a.decode) {
     auto lds_of = [&](int w) { return (size_t)w * kMaps * (32 + (size_t)gs * a.kv.v_pad) * sizeof(float); };
-    // As many wavefronts a workgroup as leave every workgroup resident at once (eight wavefronts a CU by their registers): a second round pays the
-    // page lookups, the first keys and the merge again.  us, window 512: 256 requests of 4 kv heads, two maps 61 on four wavefronts, 56 on two; 200
-    // requests of 300 36 and 31; 300 of 500 64 and, on one, 60; 500 of 1000 113 and 101; one map 256 requests 59 and 54.  From 2048 workgroups
-    // on there are several rounds however few the wavefronts (1000 requests: four 176, one 192).
-    const long long groups = (long long)a.req_num * gy;
-    int waves = 4;
-    if (window_threads(kMaps, VD) == 512 && groups <= 2048)
-      for (waves = 8; waves > 1 && groups * waves > 2048;) waves /= 2;
+    // How far the longest request reaches is not known here, and it is the launch's tail: four wavefronts a workgroup at least.  With as many as leave
+    // every workgroup resident (two from 513 workgroups on, one from 1025) requests of one length gain (us, window 512, 777 keys: 256 of 4 kv heads 64 ->
+    // 59, two maps 64 -> 59, 512 of them 118 -> 107), but any batch with a long one loses more: 300 of 4 kv heads, 8000 keys of one and 40 to 70 of the
+    // others 146 -> 444, two maps 158 -> 507, over a window of 512 31 -> 46; lengths of 1 to 4000 133 -> 248.  Eight up to 511 workgroups (65 of 4 kv heads,
+    // one of 8000 keys 119, on four 140; but all of 777 33 and 31).
+    int waves = (long long)a.req_num * gy >= 512 || window_threads(kMaps, VD) < 512 ? 4 : 8;
     while (waves > 1 && lds_of(waves) > 64 * 1024) waves /= 2;
     attn_window_kernel<KD, VD, 1, kMaps, true><<<dim3((unsigned)a.req_num, gy), waves * 64, lds_of(waves), s>>>(a, gs, chunks, 0);
     return check_launch("nf_window_attention (decode)");

@@ -177,10 +177,30 @@ def test_difference_of_two_maps(heads, kv_heads, dim, vdim, window):
 
 @pytest.mark.parametrize("requests,kv_heads", [(64, 4), (65, 4), (129, 4), (129, 8), (257, 8)])
 def test_decoding_with_fewer_wavefronts(requests, kv_heads):
-    """8, 4, 2, 1 and again 4 wavefronts a workgroup, with the short requests whose keys do not reach all of them."""
+    """8 wavefronts a workgroup and 4, with the short requests whose keys do not reach all of them."""
     b = cases.batch(np.random.default_rng(requests).integers(0, 90, requests).tolist(), [], seed=3)
     got, want = maps_case(BF16, kv_heads, kv_heads, 32, 32, 60, b, requests, seed=5)
     close(got, want, BF16, factor=1.5)
+
+
+@pytest.mark.parametrize("maps", [1, 2])
+@pytest.mark.parametrize("requests,beside", [(65, 40), (127, 40), (128, 700), (129, 700), (260, 700), (512, 700)])
+def test_decoding_order_of_a_request(requests, beside, maps):
+    """Long requests among many short ones are split over as many wavefronts as among few below 512 workgroups, and as among any number from there on:
+    their keys are merged in the same order, bit for bit (another order flips the last bit of one element in some hundreds)."""
+    heads, dim, vdim, long = 4, 32, 128, 40
+    layout = K.kv_layout(BF16, heads, heads, dim, vdim, maps)
+    gen = torch.Generator(device="cuda").manual_seed(maps)
+    b = synth.make_batch([1500] * long + [9] * (700 - long), [], vocab=10, seed=0)
+    pool = K.kv_pool(layout, b.num_pages).normal_(generator=gen)
+    q = torch.randn((700, heads * maps * dim), generator=gen, device="cuda").bfloat16()
+    got = []
+    for n in (requests, beside):
+        d = device_batch(b)
+        for name, size in (("input_indptr", n + 1), ("kv_indptr", n + 1), ("rev_input_indptr", n), ("positions", n)):
+            d[name] = d[name][:size].contiguous()
+        got.append(K.window_attention(layout, q[:n], pool, d, window=0, keep_first=0, scale=0.2, decode=n, map_weight=0.3 if maps == 2 else 0.0)[:long])
+    assert torch.isfinite(got[0].float()).all() and torch.equal(*got)
 
 
 @pytest.mark.parametrize("cap,scale,weight,diff", [(None, 0.3, 0.2, 0.8), (0.5, 0.3, 1.4, 0.0), (50.0, 0.02, -0.3, 0.5), (3.0, 2.0, 0.6, 0.1),
