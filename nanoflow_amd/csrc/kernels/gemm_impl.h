@@ -1208,12 +1208,16 @@ static int dispatch_plain(const uint16_t* A, const uint16_t* B, const uint16_t* 
       if (M <= 192) return launch_gemm<E, 192, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
       return launch_gemm<E, 224, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
     }
-  // Two wavefronts a SIMD start and end a tile sooner and lose at the power cap what the larger block of one saves in LDS reads: 2048 x 8192 of
-  // k-contiguous weights 2048 deep 59.0 us on four, 57.1 on eight, 3584 deep 93.7 and 91.0, 4096 104.4 and 103.8, 8192 199 and 206;
-  // of [K][N] weights 62.6 and 57.9, 109.8 and 103.6, 205.5 and 204.9.
-  if (best == c256 && (!kBCol || K < 4096)) return launch_gemm<E, 256, 256, 2, 4, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
-  if constexpr (kBCol)
-    if (best == c256) return launch_gemm<E, 256, 256, 2, 2, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
+  // Two wavefronts a SIMD start and end a tile sooner, and read more LDS for the same products: a matter of the contraction, and of how full the
+  // rounds are, for fewer busy CUs clock higher and the reads then are the bound.  Time on eight over time on four, by tiles:
+  //   k-contiguous weights  1024 deep 0.92 to 0.99, 1536 0.94 to 1.02, 2048 0.98 to 1.06, 3584 1.00 to 1.12 (1750 x 8192 95.9 us for 87.1)
+  //   [K][N] weights        2048 deep 0.90 to 0.99, 2560 0.94 to 1.00; a round at least 15/16 full and more than one 0.92 to 1.02 up to 8192 (2048 x 8192 x
+  //                         8192 214 us for 224), 0.96 to 1.10 beyond; 7/8 full 0.94 to 1.02 up to 6144; less full 1.00 to 1.09 from 3072
+  //                         on and up to 1.18 from 8192 on (1503 x 6144 x 8192 178 us for 159)
+  const bool eight = kBCol ? K <= 1536 : K <= 2560 || (K <= 8192 && 16 * t256 >= 15 * cus) || (K <= 6144 && 8 * t256 >= 7 * cus);
+  if (best == c256)
+    return eight ? launch_gemm<E, 256, 256, 2, 4, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s)
+                 : launch_gemm<E, 256, 256, 2, 2, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
   if (best == c128x256) return launch_gemm<E, 128, 256, 2, 4, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
   return launch_gemm<E, 128, 128, 2, 4, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
 }
