@@ -40,7 +40,7 @@ __device__ __forceinline__ TilePlace find_tile(const nf_grouped_gemm_args& a, in
 }
 
 // The BM x BN tile of a group from row t.m_base and column n_base.
-template <class E, int BM, int BN, int WM, int WN, int kCap, bool kTurn = true>
+template <class E, int BM, int BN, int WM, int WN, int kCap, bool kTurn>
 __device__ __forceinline__ void grouped_tile(const nf_grouped_gemm_args& a, const TilePlace& t, int n_base) {
   const bool routed = a.routing.n_tiles != nullptr;
   const int32_t* rows = routed && a.gather ? a.routing.row_of + t.row0 : nullptr;
@@ -55,11 +55,9 @@ __device__ __forceinline__ void grouped_tile(const nf_grouped_gemm_args& a, cons
   }
   // Weight rows are whole multiples of 4 KB apart where K is a multiple of 2048, and workgroups that walk K in step then ask a few of the memory's
   // channels at a time (a stream of 8 rows of 128 bytes an instruction: 4.4 TB/s, 6.1 with every workgroup at another k).  So every column tile
-  // of an expert starts K at a slab of its own and goes round; the m tiles that share its weights start at the same one.  748 rows, 5 of 32
-  // experts of 2048 x 2048: 90 -> 80 us up, 88 -> 79 down; where experts have 200 rows and more and the matrix cores set the pace, the same.
-  // Other strides, and the tiles of the one expert beside a weight stream, lose 2 % by it.
-  const int turn = kTurn && routed && a.K % 2048 == 0 ? (t.n_tile + t.group * 4) % ((a.K + BK - 1) / BK) : 0;
-  gemm_tile<E, BM, BN, WM, WN, false, true, false, true, kCap>(A, (const uint16_t*)a.b + (size_t)t.group * a.N * a.K, nullptr, nullptr, D,
+  // of an expert starts K at a slab of its own and goes round; the m tiles that share its weights start at the same one.
+  const int turn = kTurn ? (t.n_tile + t.group * 4) % ((a.K + BK - 1) / BK) : 0;
+  gemm_tile<E, BM, BN, WM, WN, false, true, false, true, kCap, false, 0, kTurn>(A, (const uint16_t*)a.b + (size_t)t.group * a.N * a.K, nullptr, nullptr, D,
                                                                t.rows, a.N, a.K, 1.f, 0.f, a.N, t.m_base, n_base, a.lda, a.K,
                                                                a.ldd, rows, a.M, ep, 0, 1, turn);
 }
@@ -67,15 +65,15 @@ __device__ __forceinline__ void grouped_tile(const nf_grouped_gemm_args& a, cons
 // kFit: a tile with at most half its rows is half as high, with the same sums: of uneven experts many are, and a tile of 2048 deep takes
 // less than its place in a round (748 rows, 5 of 32 experts and 8 identities, 28 to 300 rows each, a layer 401 -> 387 us; 560 rows, 2 of 8
 // experts of 14336 x 2048 140 -> 129; 800 rows, 4 of 32 of 2048 x 2048, nearly all with more than 64, 71 and 71).
-template <class E, int BM, int BN, int WM, int WN, int kCap, bool kFit>
+template <class E, int BM, int BN, int WM, int WN, int kCap, bool kFit, bool kTurn>
 __global__ __launch_bounds__(WM * WN * 64, kCap == kHalfCu ? 2 : 1) void gemm_grouped_kernel(nf_grouped_gemm_args a, int tiles_n) {
   const TilePlace t = find_tile<BM>(a, blockIdx.x, tiles_n);
   if (t.group < 0) return;
   if constexpr (kFit) {
     static_assert(GemmSmem<BM / 2, BN, 1, kCap>::bytes <= GemmSmem<BM, BN, 1, kCap>::bytes, "both heights run in the same LDS");
-    if (t.rows - t.m_base <= BM / 2) return grouped_tile<E, BM / 2, BN, WM, WN, kCap>(a, t, t.n_tile * BN);
+    if (t.rows - t.m_base <= BM / 2) return grouped_tile<E, BM / 2, BN, WM, WN, kCap, kTurn>(a, t, t.n_tile * BN);
   }
-  grouped_tile<E, BM, BN, WM, WN, kCap>(a, t, t.n_tile * BN);
+  grouped_tile<E, BM, BN, WM, WN, kCap, kTurn>(a, t, t.n_tile * BN);
 }
 
 unsigned grid_of(const nf_grouped_gemm_args& a, int bm, int tiles_n) {
@@ -168,10 +166,10 @@ __global__ __launch_bounds__(256) void gemm_grouped_f32_kernel(nf_grouped_gemm_a
                       t.n_tile * kF32Tile, ep);
 }
 
-template <class E, int BM, int BN, int WM, int WN, int kCap = kWholeCu, bool kFit = false>
-int launch_grouped(const nf_grouped_gemm_args& a, hipStream_t s) {
+template <class E, int BM, int BN, int WM, int WN, int kCap, bool kFit, bool kTurn>
+int launch_grouped_of(const nf_grouped_gemm_args& a, hipStream_t s) {
   using SM = GemmSmem<BM, BN, 1, kCap>;
-  auto kern = gemm_grouped_kernel<E, BM, BN, WM, WN, kCap, kFit>;
+  auto kern = gemm_grouped_kernel<E, BM, BN, WM, WN, kCap, kFit, kTurn>;
   static bool attr_set = false;  // benign race: the call is idempotent
   if (!attr_set) {
     const hipError_t e =
@@ -185,6 +183,17 @@ int launch_grouped(const nf_grouped_gemm_args& a, hipStream_t s) {
   const int tiles_n = (a.N + BN - 1) / BN;
   kern<<<grid_of(a, BM, tiles_n), WM * WN * 64, SM::bytes, s>>>(a, tiles_n);
   return check_launch("nf_gemm_grouped");
+}
+
+// Turned contractions: experts whose weights are at least 128 MB, half the last-level cache, which the memory's channels set the pace of (time
+// turned over straight 0.80 to 1.00, 748 rows, 5 of 32 experts of 2048 x 2048 90 -> 80 us; experts of 200 rows and more 1.00).  Of fewer weights, and where K is no
+// multiple of 2048, the offsets that go round only cost (8 of 2048 x 2048 19.0 us and 20.0, 4 of 256 x 4096 28.4 and 30.7; 8 of 768 x 1408, of which none
+// turn, 12.9 and 13.6), nor do the tiles of the one expert beside a weight stream gain.
+template <class E, int BM, int BN, int WM, int WN, int kCap = kWholeCu, bool kFit = false>
+int launch_grouped(const nf_grouped_gemm_args& a, hipStream_t s) {
+  return a.routing.n_tiles && a.K % 2048 == 0 && (size_t)a.groups * a.N * a.K * 2 >= (size_t)128 << 20
+             ? launch_grouped_of<E, BM, BN, WM, WN, kCap, kFit, true>(a, s)
+             : launch_grouped_of<E, BM, BN, WM, WN, kCap, kFit, false>(a, s);
 }
 
 // Each XCD takes a run of the launch's tiles (m tiles of an expert fastest), its workgroups every n-th of them.

@@ -174,10 +174,10 @@ __device__ __forceinline__ float swiglu_rounded(float g_acc, float u_acc) {
 // in the order of k, added up in pairs, the pairs in pairs and those two -- here the classes first_class .. first_class + n_classes - 1 (1, 2,
 // 4 or 8 of them, at most 2^kClasses), which the loads walk one after the other without a break.
 // kGroup (kBCol only): operands of one group of a grouped product -- the weights' row stride is ldb, D's is
-// ldd, and where a_rows is not null row m of A is row a_rows[m] of a matrix of a_total rows; the contraction starts at slab `turn` of K and goes
-// round.
+// ldd, and where a_rows is not null row m of A is row a_rows[m] of a matrix of a_total rows; kTurn: the contraction starts at slab `turn` of K and
+// goes round.
 template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kPartial = false, bool kGroup = false, int kCap = kWholeCu,
-          bool kOnce = false, int kClasses = 0>
+          bool kOnce = false, int kClasses = 0, bool kTurn = false>
 __device__ __forceinline__ void gemm_tile(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
@@ -186,6 +186,7 @@ __device__ __forceinline__ void gemm_tile(
     const GroupEpilogue& group = {}, const int first_class = 0, const int n_classes = 1, const int turn = 0) {
   static_assert(kClasses == 0 || (!kBCol && WM * WN == 4 && !GemmSmem<BM, BN, kDual ? 2 : 1, kCap>::split), "classes: [K][N] weights, one ring, 16 x 16 MFMAs");
   static_assert(!kGroup || (kBCol && !kDual && !kPartial), "grouped products: plain, k-contiguous weights");
+  static_assert(!kTurn || kGroup, "turned contractions: grouped products");
   const int ldb = kGroup ? group_ldb : lda, ldd = kGroup ? group_ldd : N;
   constexpr int NB = kDual ? 2 : 1;
   using SM = GemmSmem<BM, BN, NB, kCap>;
@@ -259,7 +260,7 @@ __device__ __forceinline__ void gemm_tile(
     if constexpr (kGroup) {
       // rows past the group's last one start at the end of the buffer and read as zero
       const size_t row = a_rows ? (size_t)a_rows[gm < M ? gm : 0] : (size_t)gm;
-      a_off[t] = (gm < M ? ((uint32_t)row * (uint32_t)lda + a_kc) * 2u : (uint32_t)((a_extent + 15) & ~(size_t)15)) + (uint32_t)turn * (BK * 2u);
+      a_off[t] = (gm < M ? ((uint32_t)row * (uint32_t)lda + a_kc) * 2u : (uint32_t)((a_extent + 15) & ~(size_t)15)) + (kTurn ? (uint32_t)turn * (BK * 2u) : 0u);
     } else {
       a_off[t] = ((uint32_t)gm * (uint32_t)lda + a_kc) * 2u;
     }
@@ -271,7 +272,7 @@ __device__ __forceinline__ void gemm_tile(
     uint32_t off;
     if constexpr (kBCol) {
       const int gn = n_base + (t * NW + wave) * 8 + (lane >> 3);
-      off = ((uint32_t)gn * (uint32_t)ldb + a_kc) * 2u + (kGroup ? (uint32_t)turn * (BK * 2u) : 0u);
+      off = ((uint32_t)gn * (uint32_t)ldb + a_kc) * 2u + (kTurn ? (uint32_t)turn * (BK * 2u) : 0u);
     } else {
       const int g = (t * NW + wave) * 64 + lane;  // 16-byte slot of the slab's LDS image
       const int row = g / B_CPR;
@@ -282,10 +283,10 @@ __device__ __forceinline__ void gemm_tile(
     for (int b = 0; b < NB; ++b) b_off[b][t] = off;
   }
 
-  // kGroup: slab s is slab k_slab(s) of K; from the last one the loads go back to the first.
+  // kTurn: slab s is slab k_slab(s) of K; from the last one the loads go back to the first.
   const int k_slabs = (K + BK - 1) / BK;
-  auto k_slab = [&](int s) { return kGroup && s + turn >= k_slabs ? s + turn - k_slabs : s + turn; };
-  auto on_from = [&](int s) { return kGroup && k_slab(s) == k_slabs - 1 ? -(k_slabs - 1) * (BK * 2) : BK * 2; };
+  auto k_slab = [&](int s) { return !kTurn ? s : s + turn >= k_slabs ? s + turn - k_slabs : s + turn; };
+  auto on_from = [&](int s) { return kTurn && k_slab(s) == k_slabs - 1 ? -(k_slabs - 1) * (BK * 2) : BK * 2; };
   // kClasses: slab `u` of K is followed by the next of its class, the class's last by the next class's first.  Every class has as
   // many slabs; those past the end of K read as zero.
   const int class_slabs = (K + 8 * BK - 1) / (8 * BK);
@@ -316,13 +317,13 @@ __device__ __forceinline__ void gemm_tile(
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
       load16_to_lds<t * NW * 1024>(a_rsrc, k_ok ? a_off[t] : kOob, la);
-      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kGroup ? by : BK * 2;
+      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kTurn ? by : BK * 2;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       constexpr int dst = b * SM::b_bytes + tt * NW * 1024;
       if constexpr (kBCol) {
         load16_to_lds<dst, kOnce>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
-        b_off[b][tt] += kGroup ? by : BK * 2;
+        b_off[b][tt] += kTurn ? by : BK * 2;
       } else {
         load16_to_lds<dst>(b_rsrc[b], kClasses == 0 || slab_in ? b_off[b][tt] : kOob, lb);
         b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;
@@ -337,12 +338,12 @@ __device__ __forceinline__ void gemm_tile(
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
       pend = k_ok ? a_off[t] : kOob;
-      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kGroup ? by : BK * 2;
+      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kTurn ? by : BK * 2;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       if constexpr (kBCol) {
         pend = k_ok ? b_off[b][tt] : kOob;
-        b_off[b][tt] += kGroup ? by : BK * 2;
+        b_off[b][tt] += kTurn ? by : BK * 2;
       } else {
         pend = kClasses == 0 || slab_in ? b_off[b][tt] : kOob;
         b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;

@@ -63,3 +63,21 @@ def test_whole_numbers(counts, N, Kd):
         g, u = x[:, 0::2].clamp(max=7.0), x[:, 1::2].clamp(-7.0, 7.0)
         ref = g * torch.sigmoid(1.702 * g) * (u + 1.0)
         assert (d.double() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
+
+
+@pytest.mark.parametrize("counts,N,Kd", [((65, 96, 70, 80), 1536, 2048), ((72, 65, 90, 66), 256, 4096), ((300, 129, 65, 140), 520, 6144)],
+                         ids=["lists of 64", "lists of 64, 4096 deep", "lists of 128"])
+def test_few_weights_are_walked_straight(counts, N, Kd):
+    """Experts of less than 128 MB of weights begin at their first k however long a row of weights is: the bits of the plain product of their rows."""
+    from nanoflow_amd import kernels as K
+    rng = np.random.default_rng(N)
+    counts = np.array(counts)
+    slots, e = int(counts.sum()), len(counts)
+    tile = K.lib().nf_grouped_tile_rows(K.BF16, slots, e)
+    r, hold, row_of, _ = routing(K, counts, tile, 300, rng)
+    gen = torch.Generator(device="cuda").manual_seed(Kd)
+    a, w = (torch.randn(shape, generator=gen, device="cuda").bfloat16() for shape in ((300, Kd), (e, N, Kd)))
+    d = torch.zeros((slots, N), dtype=torch.bfloat16, device="cuda")
+    K.gemm_grouped_experts(a, w, d, r, slots, True)
+    group = np.repeat(np.arange(e), counts)
+    assert torch.equal(d, torch.cat([K.gemm_nk(a[row_of[group == g]].contiguous(), w[g]) for g in range(e)]))
