@@ -233,17 +233,19 @@ int launch_chain(const nf_grouped_gemm_args& a, hipStream_t s) {
   return check_launch("nf_gemm_grouped");
 }
 
-// Tile lists of 128 rows that run on gemm_chain.h.  Contractions beyond 2048 against whole column tiles do, where a 128 x 256 tile on four
-// wavefronts ran before: 0.90 to 1.00 of its time over 300 to 2048 rows, 8 to 65 experts of 512 to 4096 columns 2304 to 3584 deep.
-// At 2048 two workgroups of 128 x 128 a CU stand against it, which leave less of a round idle: it pays where its own rounds are at least four
-// fifths full of columns that are there, or one is at least half full (2.9 and 5.8 rounds: 0.91 of their time, 0.6 of one 0.88; 1.1 to 2.2: 1.02 to 1.14;
-// 4.05 with a tenth of it past the columns: 1.05).  The rows of
-// an expert are not known here: half a tile each over the sorted rows.  Below 2048 neither wins.
+// Tile lists of 128 rows that run on gemm_chain.h.  Contractions beyond 2048 against whole column tiles do, where a 128 x 256 tile on eight wavefronts
+// stands against it: 0.93 to 1.04 of its time over 80 launches of more than a round, 2112 to 8192 deep, 0.99 in the mean; below a round it has its even
+// shares of an expert's rows alone, 0.93 where they are 150 and 1.05 to 1.10 where they fill a tile (800 of 8 experts of 512 x 2304).
+// At 2048 two workgroups of 128 x 128 a CU stand against it, which leave less of a round idle: it pays where its own rounds, of which there must be more
+// than one, are at least four fifths full of columns that are there (0.87 to 1.02 of their time; 1.1 to 1.5 rounds 1.00, 2.0 to 2.4 0.99 to 1.01; in
+// one round 0.84 to 0.98, but 1.04 to 1.26 where the 128 x 128 tiles are no more than the CUs).  The rows of
+// an expert are not known here: half a tile each over the sorted rows, among which are those of identity choices, that no expert has: with a fifth
+// of them a launch taken for full rounds can be 1.09 of the other form's time.  Below 2048 neither wins.
 bool chain_pays(const nf_grouped_gemm_args& a) {
   if (a.K < 2048 || a.N < 256 || a.ldd > 1 << 22 || (a.act == NF_ACT_GATED ? a.N % 16 != 0 : a.weigh)) return false;
   if (a.K > 2048) return a.N % 256 == 0;
   const double m_tiles = a.max_rows / 128.0 + a.groups * 0.5, rounds = m_tiles * ((a.N + 255) / 256) / cu_count(), filled = m_tiles * a.N / 256.0 / cu_count();
-  return rounds < 1 ? filled >= 0.5 : std::ceil(rounds) <= 1.25 * filled;
+  return rounds > 1 && std::ceil(rounds) <= 1.25 * filled;
 }
 
 template <class E>

@@ -65,10 +65,12 @@ def test_whole_numbers(counts, N, Kd):
         assert (d.double() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
 
 
-@pytest.mark.parametrize("counts,N,Kd", [((65, 96, 70, 80), 1536, 2048), ((72, 65, 90, 66), 256, 4096), ((300, 129, 65, 140), 520, 6144)],
-                         ids=["lists of 64", "lists of 64, 4096 deep", "lists of 128"])
+@pytest.mark.parametrize("counts,N,Kd", [((65, 96, 70, 80), 1536, 2048), ((72, 65, 90, 66), 256, 4096), ((300, 129, 65, 140), 520, 6144),
+                                             ((70, 120, 128, 100, 129, 110, 75, 90), 2816, 2048)],
+                         ids=["lists of 64", "lists of 64, 4096 deep", "lists of 128", "part of a round"])
 def test_few_weights_are_walked_straight(counts, N, Kd):
-    """Experts of less than 128 MB of weights begin at their first k however long a row of weights is: the bits of the plain product of their rows."""
+    """Experts of less than 128 MB of weights begin at their first k however long a row of weights is, and are not chained where a round holds them: the
+    bits of the plain product of their rows."""
     from nanoflow_amd import kernels as K
     rng = np.random.default_rng(N)
     counts = np.array(counts)
