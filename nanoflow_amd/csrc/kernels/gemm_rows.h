@@ -319,18 +319,33 @@ static bool few_pay(int M, int N, int K) { return rows_pay(M, N, K) && (M <= 8 |
 // and 15.7).
 static bool narrow_and_deep(int M, int N, int K) { return M <= 16 && K >= 8192 && N <= (K > 8192 ? 8 : 4) * cu_count(); }
 
+// The gate/up pair of 17 to 64 rows: a workgroup of 32 columns is one a CU, and its rows of A come with every one, so between 48 and 64 columns a CU two nearly full
+// rounds of them lose to one round of twice the width, whose LDS holds a ring of one: 64 x 14336 x 4096 52 -> 46 us, 64 x 16384 x 4096 59 -> 52, 40 x
+// 16384 x 4096 57 -> 51, 32 x 16384 x 4096 58 -> 55, e4m3 64 x 14336 x 4096 32 -> 29, 24 x 14336 x 4096 26 -> 24.  Below, the second round is
+// short enough to cost less (64 x 8192 x 4096, which has none: 28 and 41; 40 x 11264 x 4096 44 and 46); above, both take as many bytes a
+// round and the shorter ring shows (64 x 18432 x 4096 66 and 72), as it does on rows beyond 10 KB (17 x 15360 x 8192 92 and 104, e4m3 17 x 15360 x 16384
+// 85 and 95).  Up to 32 rows, of 5 sizes against 9 widths and 6 depths: 0.86 to 1.01 of the time, but weight rows whole multiples of 4 KB apart, which
+// few of the memory's channels hold at a time, 0.95 to 1.08 between 50 and 62 columns a CU (17 x 14336 x 4096 45 and 48; 0.80 to 0.90 at 64).  The sums keep their order.
+static bool wide_pair(int M, int N, int row_bytes) {
+  const int cus = cu_count();
+  if (M <= 16 || N < 48 * cus || N > 64 * cus || row_bytes > 10240) return false;
+  return M > 32 || row_bytes % 4096 != 0 || N <= 50 * cus || N > 62 * cus;
+}
+
 // The same for the gate/up pair of 16-bit or e4m3 (f8) operands.  Few columns against a long contraction, or workgroups that spill over
 // into another round, lose to the tiles and their split over K: 64 x 512 x 14336 63 us against 20, 16 x 4096 x 14336 56 against 46, 64 x
 // 10240 x 8192 86 against 73, e4m3 64 x 512 x 14336 29 against 15.  Both sides by what they take in: here a workgroup's rows of both weights and of A over the whole of K at
 // 50 GB/s, round after round, or all weights at 6.4 TB/s; there 10 us (e4m3: 9) and the weights at 6.  Fitted to 132 and 531 launches
-// of 1 to 64 rows, 64 to 28672 columns, K of 2048 to 14336, and within 5 % of the faster one except e4m3 against 16384 x 4096 (35 us, 31).
+// of 1 to 64 rows, 64 to 28672 columns, K of 2048 to 14336, on 32 columns a workgroup, and within 5 % of the faster one except e4m3 against 16384 x 4096
+// (35 us, 31); wide pairs, priced with 64, are the faster ones in 90 launches of 33 to 64 rows (64 x 12288 x 4096 60 -> 50, 48 x 13312 x 4096 65 -> 53, e4m3 64 x
+// 13312 x 8192 64 -> 50; [K][N] weights the same with a workspace, 66 -> 50 without).
 // More than 32 rows against more than 64 columns a CU, and e4m3 rows below 4 KB there from 17 rows on, are the tiles' (64 x 28672 x 8192 181 us
 // against 168, e4m3 64 x 28672 x 3072 49 against 37).
 static bool rows_pay_dual(int M, int N, int row_bytes, bool f8) {
   if (M <= 0 || M > kRowsMax || row_bytes < 3 * kRowsClasses * 128) return false;
-  const int cus = cu_count(), cols = M <= 8 ? 16 : 32, ar = M <= 8 ? 8 : M <= 16 ? 16 : M <= 32 ? 32 : 64;
-  const bool wide = N > 64 * cus;
-  if ((wide && (M > 32 || (f8 && M > 16 && row_bytes < 4096))) || (row_bytes > 16384 && N < 16 * cus)) return false;
+  const int cus = cu_count(), cols = wide_pair(M, N, row_bytes) ? 64 : M <= 8 ? 16 : 32, ar = M <= 8 ? 8 : M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  const bool beyond = N > 64 * cus;
+  if ((beyond && (M > 32 || (f8 && M > 16 && row_bytes < 4096))) || (row_bytes > 16384 && N < 16 * cus)) return false;
   if (!f8 && M > 8 && in_a_gap(N, row_bytes / 2)) return false;
   const int rounds = ((N + cols - 1) / cols + cus - 1) / cus;
   const double weights = 2.0 * N * row_bytes, intake = (double)rounds * (2 * cols + ar) * row_bytes;
@@ -370,12 +385,7 @@ static int dispatch_rows_dual(const void* A, const void* Bg, const void* Bu, uin
                               const RowsScales& sc = {}) {
   if (M <= 8) return launch_rows<E, 8, 1, 8, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
   if (M <= 16) return launch_rows<E, 16, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);
-  // A workgroup of 32 columns is one a CU, and its rows of A come with every one, so between 48 and 64 columns a CU two nearly full rounds of
-  // them lose to one round of twice the width, whose LDS holds a ring of one: 64 x 14336 x 4096 52 -> 46 us, 64 x 16384 x 4096 59 -> 52, 40 x
-  // 16384 x 4096 57 -> 51, 32 x 16384 x 4096 58 -> 55, e4m3 64 x 14336 x 4096 32 -> 29, 24 x 14336 x 4096 26 -> 24.  Below, the second round is
-  // short enough to cost less (64 x 8192 x 4096, which has none: 28 and 41; 40 x 11264 x 4096 44 and 46); above, both take as many bytes a
-  // round and the shorter ring shows (64 x 18432 x 4096 66 and 72).  The sums keep their order.
-  const bool wide = N >= 48 * cu_count() && N <= 64 * cu_count();
+  const bool wide = wide_pair(M, N, K * (std::is_same_v<E, RowsF8> ? 1 : 2));
   if (M <= 32)
     return wide ? launch_rows<E, 32, 4, 4, 2, 1, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc)
                 : launch_rows<E, 32, 2, 4, 2, 2, true, false>(A, Bg, Bu, nullptr, out, M, N, K, 1.f, 0.f, N, s, sc);

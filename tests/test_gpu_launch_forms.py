@@ -1,5 +1,5 @@
-"""Products of 256 x 256 tiles, which run on four or on eight wavefronts by a rule: against the four-wavefront form, which a launch with a chosen tile
-always runs.  On the same operands in turns; the two have the same bits."""
+"""Rules that choose between two forms of a launch, where one of them once was much the slower: against the other form, on the same operands in turns.  The two
+have the same bits."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -30,7 +30,8 @@ def medians(calls, copies, turns=15):
     return [sorted(t)[turns // 2] for t in times]
 
 
-# deep contractions of [K][N] weights on part of the chip take 1.11 to 1.14 of the time on eight wavefronts
+# 256 x 256 tiles on four or eight wavefronts (a launch with a chosen tile has four): deep contractions of [K][N] weights on part of the chip
+# take 1.11 to 1.14 of the time on eight
 @pytest.mark.parametrize("M,N,Kd", [(1503, 6144, 14336), (1024, 10240, 8192)])
 def test_deep_products_on_part_of_the_chip(M, N, Kd):
     from nanoflow_amd import kernels as K
