@@ -329,7 +329,8 @@ NF_API int nf_gemm_nk_sums_bf16(const uint16_t* A, const uint16_t* B, float* P, 
                                 int max_shares, nf_stream_t stream);
 
 /* Where a batch's tokens go in a mixture of experts: device arrays that nf_route fills.  An expert's rows are
- * consecutive ("sorted rows"), experts in order. */
+ * consecutive ("sorted rows"), experts in order.  place may be the array of choice or of weight itself, and, up to 16384
+ * entries, row_of and row_weight may share memory with those two (what nf_route leaves in them is lost); the others are apart. */
 typedef struct nf_routing {
   int32_t* choice;     /* [rows][top] chosen outputs of the router */
   float* weight;       /* [rows][top] */

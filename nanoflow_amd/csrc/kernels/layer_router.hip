@@ -123,8 +123,11 @@ __global__ __launch_bounds__(256) void route_rows_kernel(nf_route_args a, int32_
 // What bounds it is what one CU can read and write, so every workgroup places a share of the entries, kPlanChunk at a time, all of which every workgroup
 // counts: those ahead of its own apart from the rest (us, one workgroup for all -> this: 1946 rows of 5 10.8 -> 7.3, 2047 of 5 9.3 -> 6.8; 748
 // rows of 5 5.4 -> 5.0, 256 of 5 4.7 and 4.7; an empty launch takes 4).
-constexpr int kPlanChunk = 1024, kPlanGroups = 32;
-__global__ __launch_bounds__(kPlanChunk) void route_plan_kernel(nf_routing r, int rows, int top, int always, int experts) {
+// held: for arrays that share memory with the choices or weights.  One workgroup, which has read both when it writes the sorted rows: they stay in LDS till then,
+// up to kHeldEntries; an entry's place is written by the thread that has read the entry.
+constexpr int kPlanChunk = 1024, kPlanGroups = 32, kHeldEntries = 16384;
+__global__ __launch_bounds__(kPlanChunk) void route_plan_kernel(nf_routing r, int rows, int top, int always, int experts, bool held) {
+  extern __shared__ int held_rows[];  // [n] rows, [n] weights
   __shared__ int ahead[kMaxOutputs], count[kMaxOutputs], first[kMaxOutputs], wave_rows[16], wave_tiles[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, routed = experts - always, per_token = top + always, n = rows * per_token;
   const int chunks = (n - 1) / kPlanChunk + 1, per_group = (chunks + gridDim.x - 1) / gridDim.x;
@@ -191,13 +194,26 @@ __global__ __launch_bounds__(kPlanChunk) void route_plan_kernel(nf_routing r, in
       int at = -1;
       if (k >= top) at = first[routed + k - top] + t;
       else if (own < routed) at = atomicAdd(&first[own], 1);
-      if (at >= 0) {
+      if (at >= 0 && held) {
+        held_rows[at] = t;
+        held_rows[n + at] = (int)__float_as_uint(weight);
+      } else if (at >= 0) {
         r.row_of[at] = t;
         if (r.row_weight) r.row_weight[at] = weight;
       }
       r.place[i] = at;
     }
     if (c + 1 < c1) read_own(c + 1);
+  }
+  if (held) {
+    __syncthreads();
+    int sorted = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) sorted += wave_rows[w];
+    for (int i = tid; i < sorted; i += kPlanChunk) {
+      r.row_of[i] = held_rows[i];
+      if (r.row_weight) r.row_weight[i] = __uint_as_float((uint32_t)held_rows[n + i]);
+    }
   }
 }
 
@@ -238,8 +254,26 @@ int nf_route(const nf_route_args* args, const nf_routing* routing, nf_stream_t s
   const int per = (a.outputs + 63) / 64;
   const int rc = per <= 1 ? go(ic<1>{}) : per <= 2 ? go(ic<2>{}) : per <= 4 ? go(ic<4>{}) : per <= 8 ? go(ic<8>{}) : go(ic<16>{});
   if (rc) return rc;
-  const long long chunks = ((long long)a.rows * per_token + kPlanChunk - 1) / kPlanChunk;
-  route_plan_kernel<<<(unsigned)std::min<long long>(chunks, kPlanGroups), kPlanChunk, 0, s>>>(r, a.rows, a.top, a.always, a.experts + a.always);
+  const size_t n = (size_t)a.rows * per_token;
+  const long long chunks = (long long)(n + kPlanChunk - 1) / kPlanChunk;
+  auto shares = [&](const void* out) {  // memory with what the plan reads
+    auto over = [&](const void* in) { return out && (uintptr_t)out < (uintptr_t)in + n * 4 && (uintptr_t)in < (uintptr_t)out + n * 4; };
+    return over(r.choice) || over(r.weight);
+  };
+  const bool alone = shares(r.place) || shares(r.row_of) || shares(r.row_weight), held = alone && n <= kHeldEntries;
+  if (held) {
+    static bool attr_set = false;  // benign race: the call is idempotent
+    if (!attr_set) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(route_plan_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kHeldEntries * 8);
+      if (e != hipSuccess) {
+        set_error("%s: cannot reserve %d bytes of LDS: %s", who, kHeldEntries * 8, hipGetErrorString(e));
+        return NF_ERR_RUNTIME;
+      }
+      attr_set = true;
+    }
+  }
+  route_plan_kernel<<<alone ? 1u : (unsigned)std::min<long long>(chunks, kPlanGroups), kPlanChunk, held ? n * 8 : 0, s>>>(r, a.rows, a.top, a.always,
+                                                                                                                        a.experts + a.always, held);
   return check_launch("nf_route (plan)");
 }
 
