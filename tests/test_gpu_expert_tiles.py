@@ -29,6 +29,18 @@ def routing(K, counts, tile, rows, rng):
 @pytest.mark.parametrize("counts", [FEW, MANY], ids=["lists of 64", "lists of 128"])
 @pytest.mark.parametrize("N,Kd", [(8, 64), (136, 72), (256, 128), (264, 200), (520, 1000), (1032, 2048), (2048, 2056), (1024, 2112), (1048, 2184), (512, 3000), (2192, 2048)])
 def test_whole_numbers(counts, N, Kd):
+    check(counts, N, Kd, torch.full((len(counts),), 7.0))
+
+
+@pytest.mark.parametrize("N,Kd", [(8192, 2112), (12288, 2184), (16384, 2112), (8192, 2048), (12240, 2048)])
+def test_workgroups_that_go_from_tile_to_tile(N, Kd):
+    """Two to four tiles a workgroup, of other experts, heights and first slabs, the last one cut in its columns or its contraction."""
+    tiles = sum((n + 127) // 128 for n in MANY) * ((N + 255) // 256)
+    assert tiles >= 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    check(MANY, N, Kd, torch.linspace(0.5, 4.0, len(MANY)))
+
+
+def check(counts, N, Kd, limits):
     from nanoflow_amd import kernels as K
     rng = np.random.default_rng(N + Kd)
     counts = np.array(counts)
@@ -53,16 +65,17 @@ def test_whole_numbers(counts, N, Kd):
     assert torch.equal(run(K.ACT_NONE, given, N), bf16(product))
     assert torch.equal(run(K.ACT_SQUARED_RELU, gather, N), bf16(product.clamp(min=0).float().square()))
     assert torch.equal(run(K.ACT_NONE, given, N, weigh=True), bf16(product * torch.from_numpy(weight).cuda()[:, None].double()))
-    # gate and up, weighed first: the sigmoid's rounding and one to bf16
+    # gate and up, weighed first: all exact but the sigmoid (some 2^-20) and one rounding to bf16 (2^-9)
     x = product * torch.from_numpy(weight).cuda()[:, None].double() / 64
-    limits = torch.full((e,), 7.0, device="cuda")
+    limits = limits.cuda()
     scaled = (w.float() / 64).bfloat16()
     d = torch.full((slots, N // 2), 9.0, dtype=torch.bfloat16, device="cuda")
     if N // 2 % 8 == 0:
         K.gemm_grouped_experts(gather, scaled, d, r, slots, True, K.ACT_GATED, weigh=True, gated=(1.702, 1.0, limits))
-        g, u = x[:, 0::2].clamp(max=7.0), x[:, 1::2].clamp(-7.0, 7.0)
+        most = limits[torch.from_numpy(group).cuda()][:, None].double()
+        g, u = x[:, 0::2].minimum(most), x[:, 1::2].clamp(-most, most)
         ref = g * torch.sigmoid(1.702 * g) * (u + 1.0)
-        assert (d.double() - ref).abs().max() <= 2 ** -8 * ref.abs().max()
+        assert ((d.double() - ref).abs() <= 2 ** -8 * ref.abs()).all()
 
 
 @pytest.mark.parametrize("counts,N,Kd", [((65, 96, 70, 80), 1536, 2048), ((72, 65, 90, 66), 256, 4096), ((300, 129, 65, 140), 520, 6144),
