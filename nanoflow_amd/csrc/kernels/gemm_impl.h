@@ -1019,19 +1019,6 @@ static int launch_hybrid(const uint16_t* A, const uint16_t* B0, const uint16_t* 
   return check_launch("gemm launch");
 }
 
-// Compute units of the current device (256 on MI355X); one workgroup of these kernels fills one.
-static int cu_count() {
-  static int n = 0;  // benign race: every caller computes the same value
-  if (n == 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-      v = 256;
-    n = v;
-  }
-  return n;
-}
-
 static bool in_a_gap(int N, int K);  // gemm_rows.h
 static bool rows_pay_dual(int M, int N, int row_bytes, bool f8);
 

@@ -1131,7 +1131,7 @@ static int launch_tile_of(const nf_window_attention_args& a, hipStream_t s) {
     attr_set = true;
   }
   const unsigned tiles = (unsigned)(a.max_rows / tile_tokens + a.req_num);
-  kern<<<dim3((unsigned)(a.kv.kv_heads * chunks), tiles), 256, lds, s>>>(a, gs, chunks, tile_tokens, (long long)tiles * a.kv.kv_heads * chunks <= 2 * 256 + 64);
+  kern<<<dim3((unsigned)(a.kv.kv_heads * chunks), tiles), 256, lds, s>>>(a, gs, chunks, tile_tokens, (long long)tiles * a.kv.kv_heads * chunks <= 2 * cu_count() + 64);
   return check_launch("nf_window_attention (tiles)");
 }
 
@@ -1145,7 +1145,7 @@ static int launch_tile(const nf_window_attention_args& a, hipStream_t s) {
   if constexpr (kMaps == 1) {
     const int group = a.kv.heads / a.kv.kv_heads, chunks = (group + 15) / 16, gs = (group + chunks - 1) / chunks;
     const long long groups = ((long long)a.max_rows / (4 * (16 / gs)) + a.req_num) * a.kv.kv_heads * chunks;
-    if (groups > 3 * 256) return launch_tile_of<KD, VD, 1, 2>(a, s);
+    if (groups > 3 * cu_count()) return launch_tile_of<KD, VD, 1, 2>(a, s);
   }
   return launch_tile_of<KD, VD, kMaps, 1>(a, s);
 }
