@@ -11,8 +11,9 @@
 //   - A workgroup's next tile is on its way while the last slabs of one are multiplied, and its sums leave the registers as 16-byte
 //     stores without LDS: a tile's start and end (6 us of 40 at 2048 deep) are hidden or gone.
 //   - An expert's rows are shared out evenly over its tiles, in steps of 32, and only live rows are multiplied.
-// us, against two workgroups of 128 x 128 a CU (2048 deep) or a 128 x 256 one (3584): 1946 rows, gated 4096 x 2048 and a 33rd expert for all 229 -> 210,
-// 2048 x 2048 back 125 -> 118; 2047 rows, 2048 x 2048 with GELU 123 -> 117; 2048 rows of 4096 x 3584 341 -> 317.
+// us, without a profiler and against what would run instead, two workgroups of 128 x 128 a CU (2048 deep) or a 128 x 256 one on eight wavefronts (3584), turned
+// as well: 1946 rows, gated 4096 x 2048 and a 33rd expert for all 231 -> 211, 2048 x 2048 back 118 -> 114; 2047 rows and identities among the choices, 2048 x
+// 2048 with GELU 115 -> 114, back 111 -> 109 (their layer 461 -> 451); 2048 rows of 4096 x 3584 324 -> 315.  Under a profiler's clocks the third and fourth lose 2 to 7 %.
 // Measured and left: 256 x 256 tiles of as many wavefronts (200 of the 210, but 108 us for 79 where experts have a little more than 256 rows), four
 // wavefronts (the compiler moves 128 sums between register files at every branch), rings of four stages (240 for 215: they fill the memory's queues), the
 // non-temporal hint on weights that two tiles share, a wavefront that asks for lines ahead of the loads (249 -> 311).

@@ -547,7 +547,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_f8_kernel(
 }
 
 // The pair on tiles of two heights in one launch, as gemm_f16_hybrid_kernel: a last round that 256-row tiles fill at most half takes half its time on 128-row ones (1973 x
-// 14336 x 4096, 896 tiles: 768 + 2 x 128; 197 -> 190 us).
+// 14336 x 4096, 896 tiles: 768 + 2 x 128; 197 -> 190 us; 51 launches of 272 to 1048 tiles, 512 to 2048 rows, 1024 to 14336 deep 0.83 to 0.96 of the time).
 __global__ __launch_bounds__(256) void gemm_f8_pair_hybrid_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ B1,
                                                                   const float* __restrict__ sa, const float* __restrict__ sb,
                                                                   const float* __restrict__ sb1, uint16_t* D, int M, int N, int K, int tiles_m,

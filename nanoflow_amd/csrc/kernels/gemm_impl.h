@@ -9,10 +9,10 @@
 // Workgroup = 4 or 8 wavefronts in a WM x WN grid; each wavefront owns a
 // (BM/WM) x (BN/WN) block of 16x16 (or 32x32) MFMA tiles.  K is walked in slabs of 64 through a
 // ring of two to four LDS stages (as many as fit 144 KB).
-// Tiles of 128 rows run on eight: their sub-steps are too short for a wavefront alone on its SIMD to wait out an LDS read in, and a tile's start
+// Tiles of 128 rows run on eight, but the lower halves of launches of two heights and the experts' two workgroups a CU: their sub-steps are too short for a wavefront alone on its SIMD to wait out an LDS read in, and a tile's start
 // and end halve (us, four -> eight: 2046 x 4096 x 4096 63.3 -> 60.1, 2048 deep 37.8 -> 33.6; 2019 x 2048 x 512 9.8 -> 7.9, 8192 deep 67.6 and 67.7; split
-// 128 x 4096 x 4096 18.0 -> 16.6; fp32 sums of 748 x 2048 x 2048 13.7 -> 12.2; pair 128 x 4096 x 4096 27.8 -> 25.3).  Those of 256 rows on four where
-// the contraction is long (dispatch_plain).
+// 128 x 4096 x 4096 18.0 -> 16.6; fp32 sums of 748 x 2048 x 2048 13.7 -> 12.2; pair 128 x 4096 x 4096 27.8 -> 25.3).  Those of 256 rows by the
+// contraction and the rounds (dispatch_plain).
 //
 // Operands go from global memory STRAIGHT INTO LDS (buffer_load_dwordx4 ... lds): a CU moves
 // about 38 GB/s through the load-to-register path but well over 100 GB/s through this one, and
@@ -1188,8 +1188,9 @@ static int dispatch_plain(const uint16_t* A, const uint16_t* B, const uint16_t* 
   if (best == c256 && two_heights)
     return launch_hybrid<E, 256, false, kBCol>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, (int)(t256 - rest256), s);
   // One row of tiles: no higher than its rows need, for the padding is multiplied at the power cap's price (us against 256 x 256, x 128256 x 4096:
-  // 140 rows 238 -> 199, 180 rows 249 -> 222, 192 rows 250 -> 227, 200 rows 253 -> 240; from 225 rows on it is the same tile).  Wavefronts
-  // beside each other, since 224 and 160 rows are no two blocks of whole passes.
+  // 140 rows 238 -> 199, 180 rows 249 -> 222, 192 rows 250 -> 227, 200 rows 253 -> 240; from 225 rows on it is the same tile; 160 launches of 130 to 224 rows,
+  // 32000 to 128256 columns, 512 to 8192 deep 0.75 to 1.02 of the time).  Wavefronts beside each other, since 224 and 160 rows are no two blocks of
+  // whole passes.  The choice above goes by 256 rows all the same: two heights or 256 x 192, where they win, keep the padding (140 x 151936 x 4096).
   if constexpr (kBCol)
     if (best == c256 && M <= 224) {
       if (M <= 160) return launch_gemm<E, 160, 256, 1, 4, false, true>(A, B, nullptr, C, D, M, N, K, alpha, beta, ldc, s);
