@@ -986,8 +986,12 @@ static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1
   // One row of tiles reads the weights once: with the non-temporal hint (three turns on one card: 256 x 128256 x 4096 258 -> 238 us, 66 x
   // 28672 x 8192 103 -> 91, pairs of it 176 -> 158; 200 x 128256 x 4096 between 224 and 263 either way).  Several rows of tiles share them through the caches, which the hint defeats, and shares of a
   // split read runs of a row too short for it (128 x 4096 x 4096 in 8: 19 us, 24 with it).
-  if constexpr (kBCol && BM % 128 != 0 && BM > 128) {
-    return go(std::true_type{});  // heights of one row of tiles
+  if constexpr (kBCol && BM % 128 != 0 && BM > 128) {  // heights that are launched for one row of tiles only
+    if (tiles_m != 1) {
+      set_error("gemm: %d rows on a tile for at most %d", M, BM);
+      return NF_ERR_INVALID_ARGUMENT;
+    }
+    return go(std::true_type{});
   } else {
     if constexpr (kBCol)
       if (tiles_m == 1) return go(std::true_type{});
