@@ -223,6 +223,17 @@ __device__ __forceinline__ void load16_to_lds(rsrc_t r, uint32_t byte_off, uint3
     asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                  :: "s"(lds_base), "v"(byte_off), "s"(r), "n"(kLdsOffset) : "memory", "scc", "m0");
 }
+// The same with a wavefront-uniform part of the address (soff) beside the lane's, which alone is sure to be range-checked: a lane that is to
+// read zeros has to be out of range without it.
+template <int kLdsOffset, bool kOnce = false>
+__device__ __forceinline__ void load16_to_lds_from(rsrc_t r, uint32_t byte_off, uint32_t soff, uint32_t lds_base) {
+  if constexpr (kOnce)
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %4 offen nt lds"
+                 :: "s"(lds_base), "v"(byte_off), "s"(r), "n"(kLdsOffset), "s"(soff) : "memory", "scc", "m0");
+  else
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %4 offen lds"
+                 :: "s"(lds_base), "v"(byte_off), "s"(r), "n"(kLdsOffset), "s"(soff) : "memory", "scc", "m0");
+}
 __device__ __forceinline__ short4_t lds_read_tr16(const uint8_t* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)p);
 }

@@ -186,7 +186,7 @@ __device__ __forceinline__ void gemm_tile(
     const GroupEpilogue& group = {}, const int first_class = 0, const int n_classes = 1, const int turn = 0) {
   static_assert(kClasses == 0 || (!kBCol && WM * WN == 4 && !GemmSmem<BM, BN, kDual ? 2 : 1, kCap>::split), "classes: [K][N] weights, one ring, 16 x 16 MFMAs");
   static_assert(!kGroup || (kBCol && !kDual && !kPartial), "grouped products: plain, k-contiguous weights");
-  static_assert(!kTurn || kGroup, "turned contractions: grouped products");
+  static_assert(!kTurn || kBCol, "turned contractions: k-contiguous weights");
   const int ldb = kGroup ? group_ldb : lda, ldd = kGroup ? group_ldd : N;
   constexpr int NB = kDual ? 2 : 1;
   using SM = GemmSmem<BM, BN, NB, kCap>;
@@ -260,7 +260,7 @@ __device__ __forceinline__ void gemm_tile(
     if constexpr (kGroup) {
       // rows past the group's last one start at the end of the buffer and read as zero
       const size_t row = a_rows ? (size_t)a_rows[gm < M ? gm : 0] : (size_t)gm;
-      a_off[t] = (gm < M ? ((uint32_t)row * (uint32_t)lda + a_kc) * 2u : (uint32_t)((a_extent + 15) & ~(size_t)15)) + (kTurn ? (uint32_t)turn * (BK * 2u) : 0u);
+      a_off[t] = (gm < M ? ((uint32_t)row * (uint32_t)lda + a_kc) * 2u : (uint32_t)((a_extent + 15) & ~(size_t)15));
     } else {
       a_off[t] = ((uint32_t)gm * (uint32_t)lda + a_kc) * 2u;
     }
@@ -272,7 +272,7 @@ __device__ __forceinline__ void gemm_tile(
     uint32_t off;
     if constexpr (kBCol) {
       const int gn = n_base + (t * NW + wave) * 8 + (lane >> 3);
-      off = ((uint32_t)gn * (uint32_t)ldb + a_kc) * 2u + (kTurn ? (uint32_t)turn * (BK * 2u) : 0u);
+      off = ((uint32_t)gn * (uint32_t)ldb + a_kc) * 2u;
     } else {
       const int g = (t * NW + wave) * 64 + lane;  // 16-byte slot of the slab's LDS image
       const int row = g / B_CPR;
@@ -283,10 +283,28 @@ __device__ __forceinline__ void gemm_tile(
     for (int b = 0; b < NB; ++b) b_off[b][t] = off;
   }
 
-  // kTurn: slab s is slab k_slab(s) of K; from the last one the loads go back to the first.
+  // kTurn: slab s is slab s + turn of K, from whose last one the loads go back to the first.  Where it goes round is kept from the compiler: of a
+  // plain selection ahead of the slab loop it makes branches, and permutes the sums at the loop's end (156 moves beside 112 MFMAs).
   const int k_slabs = (K + BK - 1) / BK;
-  auto k_slab = [&](int s) { return !kTurn ? s : s + turn >= k_slabs ? s + turn - k_slabs : s + turn; };
-  auto on_from = [&](int s) { return kTurn && k_slab(s) == k_slabs - 1 ? -(k_slabs - 1) * (BK * 2) : BK * 2; };
+  auto go_round = [&](int k) {
+    if constexpr (kTurn) {
+      int past;
+      asm("s_cmp_ge_i32 %0, %2\n\ts_cselect_b32 %1, %2, 0\n\ts_sub_u32 %0, %0, %1" : "+s"(k), "=&s"(past) : "s"(k_slabs) : "scc");
+    }
+    return k;
+  };
+  auto k_slab = [&](int s) { return kTurn ? go_round(s + turn) : s; };
+  int k_ahead[2];  // kTurn: the two slabs whose loads are next
+  auto look_ahead = [&](int s) {
+    if constexpr (!kTurn) return;
+    k_ahead[0] = k_slab(s);
+    k_ahead[1] = k_slab(s + 1);
+  };
+  auto go_on = [&] {
+    if constexpr (!kTurn) return;
+    k_ahead[0] = k_ahead[1];
+    k_ahead[1] = go_round(k_ahead[0] + 1);
+  };
   // kClasses: slab `u` of K is followed by the next of its class, the class's last by the next class's first.  Every class has as
   // many slabs; those past the end of K read as zero.
   const int class_slabs = (K + 8 * BK - 1) / (8 * BK);
@@ -313,17 +331,23 @@ __device__ __forceinline__ void gemm_tile(
   constexpr int PARTS = NS == 2 ? 3 : 4;         // k-steps the loads of one slab are spread over
   // k_ok: this lane's 16 bytes of the slab's 128-byte rows lie below K.  la / lb: LDS address of
   // the stage the activations / the weights of the slab go to, + wave * 1024.
-  auto load_one = [&](auto t_c, uint32_t la, uint32_t lb, bool k_ok, int by = BK * 2) {
+  auto load_one = [&](auto t_c, uint32_t la, uint32_t lb, bool k_ok, int by = 0) {
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
-      load16_to_lds<t * NW * 1024>(a_rsrc, k_ok ? a_off[t] : kOob, la);
-      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kTurn ? by : BK * 2;
+      if constexpr (kTurn) {
+        load16_to_lds_from<t * NW * 1024>(a_rsrc, k_ok ? a_off[t] : kOob, by, la);
+      } else {
+        load16_to_lds<t * NW * 1024>(a_rsrc, k_ok ? a_off[t] : kOob, la);
+        a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : BK * 2;
+      }
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       constexpr int dst = b * SM::b_bytes + tt * NW * 1024;
-      if constexpr (kBCol) {
+      if constexpr (kTurn) {
+        load16_to_lds_from<dst, kOnce>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, by, lb);
+      } else if constexpr (kBCol) {
         load16_to_lds<dst, kOnce>(b_rsrc[b], k_ok ? b_off[b][tt] : kOob, lb);
-        b_off[b][tt] += kTurn ? by : BK * 2;
+        b_off[b][tt] += BK * 2;
       } else {
         load16_to_lds<dst>(b_rsrc[b], kClasses == 0 || slab_in ? b_off[b][tt] : kOob, lb);
         b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;
@@ -334,29 +358,31 @@ __device__ __forceinline__ void gemm_tile(
   // instructions each: the offset (masked, and advanced for the next slab) first, the M0 write and
   // the load instruction one MFMA later.
   uint32_t pend = 0;
-  auto load_prepare = [&](auto t_c, bool k_ok, int by) {
+  auto load_prepare = [&](auto t_c, bool k_ok) {
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
       pend = k_ok ? a_off[t] : kOob;
-      a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : kTurn ? by : BK * 2;
+      if constexpr (!kTurn) a_off[t] += kClasses > 0 ? (uint32_t)slab_step * (BK * 2) : BK * 2;
     } else {
       constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
       if constexpr (kBCol) {
         pend = k_ok ? b_off[b][tt] : kOob;
-        b_off[b][tt] += kTurn ? by : BK * 2;
+        if constexpr (!kTurn) b_off[b][tt] += BK * 2;
       } else {
         pend = kClasses == 0 || slab_in ? b_off[b][tt] : kOob;
         b_off[b][tt] += kClasses > 0 ? (uint32_t)slab_step * b_slab : b_slab;
       }
     }
   };
-  auto load_issue = [&](auto t_c, uint32_t la, uint32_t lb) {
+  auto load_issue = [&](auto t_c, uint32_t la, uint32_t lb, int by) {
     constexpr int t = decltype(t_c)::value;
     if constexpr (t < A_LOADS) {
-      load16_to_lds<t * NW * 1024>(a_rsrc, pend, la);
+      if constexpr (kTurn) load16_to_lds_from<t * NW * 1024>(a_rsrc, pend, by, la);
+      else load16_to_lds<t * NW * 1024>(a_rsrc, pend, la);
     } else {
-      constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS;
-      load16_to_lds<b * SM::b_bytes + tt * NW * 1024, kOnce>(b_rsrc[b], pend, lb);
+      constexpr int b = (t - A_LOADS) / B_LOADS, tt = (t - A_LOADS) % B_LOADS, dst = b * SM::b_bytes + tt * NW * 1024;
+      if constexpr (kTurn) load16_to_lds_from<dst, kOnce>(b_rsrc[b], pend, by, lb);
+      else load16_to_lds<dst, kOnce>(b_rsrc[b], pend, lb);
     }
   };
   auto load_slab = [&](int stage, int k0, int by) {  // every load of one slab, back to back (one ring for both operands)
@@ -454,8 +480,8 @@ __device__ __forceinline__ void gemm_tile(
           constexpr int NRD = NRB + NRA;
           constexpr int qq = q < NRA ? 2 * NL + NRB + q : q < NRD ? 2 * NL + (q - NRA) : q - NRD;
           if constexpr (qq < 2 * NL) {
-            if constexpr (qq % 2 == 0) load_prepare(ic<L0 + LSTR * (qq / 2)>{}, ld_ok, by);
-            else load_issue(ic<L0 + LSTR * (qq / 2)>{}, la, lb);
+            if constexpr (qq % 2 == 0) load_prepare(ic<L0 + LSTR * (qq / 2)>{}, ld_ok);
+            else load_issue(ic<L0 + LSTR * (qq / 2)>{}, la, lb, by);
           } else if constexpr (qq < 2 * NL + NRB) {
             read_one(ic<TM + HN * CH + (qq - 2 * NL)>{}, ic<K2N>{}, ic<HN>{}, sa, sb);
           } else {
@@ -488,7 +514,8 @@ __device__ __forceinline__ void gemm_tile(
   using F_ = std::false_type;
   const int nslab = kClasses > 0 ? n_classes * class_slabs : (K + BK - 1) / BK;
   // k of slab s, or of slab number u of K
-  auto slab_k = [&](int s, int u) { return (kClasses > 0 ? u : k_slab(s)) * BK; };
+  auto slab_k = [&](int s, int u) { return (kClasses > 0 ? u : s) * BK; };
+  auto place = [](int k) { return kTurn ? k * (BK * 2) : 0; };
 
   if constexpr (SM::split) {
     // ---- two activation stages, three weight stages.  Slab s has its activations in stage s % 2
@@ -509,14 +536,15 @@ __device__ __forceinline__ void gemm_tile(
     };
     auto a_ptr = [&](int stage) { return smem + stage * SM::a_bytes; };
     auto b_ptr = [&](int stage) { return smem + SM::b_ring + stage * NB * SM::b_bytes; };
-    auto k_ok_of = [&](int slab_idx) { return k_slab(slab_idx) * BK + a_kc < K; };
+    auto k_ok_of = [&](int k) { return k * BK + a_kc < K; };
+    auto place = [](int k) { return kTurn ? k * (BK * 2) : 0; };
     // prologue: activations and weights of slab 0, weights of slab 1
     {
       const uint32_t la = a_lds(0), lb0 = b_lds(0), lb1 = b_lds(1);
-      static_for<A_LOADS>([&](auto t_c) { load_one(t_c, la, lb0, k_ok_of(0), on_from(0)); });
-      static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb0, k_ok_of(0), on_from(0)); });
+      static_for<A_LOADS>([&](auto t_c) { load_one(t_c, la, lb0, k_ok_of(k_slab(0)), place(k_slab(0))); });
+      static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb0, k_ok_of(k_slab(0)), place(k_slab(0))); });
       if (nslab > 1) {
-        static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb1, k_ok_of(1), on_from(1)); });
+        static_for<BL>([&](auto t_c) { load_one(ic<A_LOADS + decltype(t_c)::value>{}, la, lb1, k_ok_of(k_slab(1)), place(k_slab(1))); });
         __builtin_amdgcn_s_waitcnt(wait_but_b);
       } else {
         __builtin_amdgcn_s_waitcnt(0x0070);
@@ -526,7 +554,7 @@ __device__ __forceinline__ void gemm_tile(
     static_for<(kM16 ? TM + CH : READS)>([&](auto q_c) { read_one(q_c, ic<0>{}, ic<0>{}, a_ptr(0), b_ptr(0)); });
     if (nslab > 1) {  // what k-step 3 of a slab before slab 0 would have issued
       const uint32_t la = a_lds(1);
-      static_for<HA>([&](auto t_c) { load_one(t_c, la, la, k_ok_of(1), on_from(1)); });
+      static_for<HA>([&](auto t_c) { load_one(t_c, la, la, k_ok_of(k_slab(1)), place(k_slab(1))); });
     }
     // H1: slab s+1 exists, H2: slab s+2 exists
     auto slab2 = [&](auto h1_c, auto h2_c, int s, int bs) {
@@ -534,17 +562,20 @@ __device__ __forceinline__ void gemm_tile(
       const uint8_t *sa = a_ptr(s & 1), *sb = b_ptr(bs);
       const int bs1 = bs == 2 ? 0 : bs + 1, bs2 = bs1 == 2 ? 0 : bs1 + 1;
       const uint32_t la1 = a_lds((s + 1) & 1), lb2 = b_lds(bs2);
-      step(ic<0>{}, ic<HA>{}, ic<1>{}, ic<H1 ? A_LOADS - HA : 0>{}, ic<1>{}, la1, la1, k_ok_of(s + 1), on_from(s + 1), sa, sb);
-      step(ic<1>{}, ic<A_LOADS>{}, ic<1>{}, ic<H2 ? HB : 0>{}, ic<2>{}, lb2, lb2, k_ok_of(s + 2), on_from(s + 2), sa, sb);
-      step(ic<2>{}, ic<A_LOADS + HB>{}, ic<1>{}, ic<H2 ? BL - HB : 0>{}, ic<3>{}, lb2, lb2, k_ok_of(s + 2), on_from(s + 2), sa, sb);
+      const int k1 = kTurn ? k_ahead[0] : s + 1, k2 = kTurn ? k_ahead[1] : s + 2;
+      step(ic<0>{}, ic<HA>{}, ic<1>{}, ic<H1 ? A_LOADS - HA : 0>{}, ic<1>{}, la1, la1, k_ok_of(k1), place(k1), sa, sb);
+      step(ic<1>{}, ic<A_LOADS>{}, ic<1>{}, ic<H2 ? HB : 0>{}, ic<2>{}, lb2, lb2, k_ok_of(k2), place(k2), sa, sb);
+      step(ic<2>{}, ic<A_LOADS + HB>{}, ic<1>{}, ic<H2 ? BL - HB : 0>{}, ic<3>{}, lb2, lb2, k_ok_of(k2), place(k2), sa, sb);
       if constexpr (H1) {
         __builtin_amdgcn_s_waitcnt(H2 ? wait_but_b : 0x0070);
         __syncthreads();
       }
       const uint32_t la2 = a_lds(s & 1);  // slab s+2's activations reuse this slab's stage
-      step(ic<3>{}, ic<0>{}, ic<1>{}, ic<H2 ? HA : 0>{}, ic<H1 ? 0 : -1>{}, la2, la2, k_ok_of(s + 2), on_from(s + 2), a_ptr((s + 1) & 1),
+      step(ic<3>{}, ic<0>{}, ic<1>{}, ic<H2 ? HA : 0>{}, ic<H1 ? 0 : -1>{}, la2, la2, k_ok_of(k2), place(k2), a_ptr((s + 1) & 1),
            b_ptr(bs1));
+      go_on();
     };
+    look_ahead(1);
     int s = 0, bs = 0;
     for (; s + 2 < nslab; ++s) {
       slab2(T_{}, T_{}, s, bs);
@@ -608,10 +639,11 @@ __device__ __forceinline__ void gemm_tile(
     const uint8_t* sb = st + SM::a_bytes;
     const uint32_t ld_a = __builtin_amdgcn_readfirstlane(smem_lds + ls * SM::stage_bytes + wave * 1024);
     if constexpr (kClasses > 0) fetch(u_ahead);
-    const bool ok_a = slab_k(s + NS - 1, u_ahead) + a_kc < K;
-    step(ic<0>{}, ic<1>{}, ic<PARTS>{}, ic<(IA && PARTS > 1) ? nl(1) : 0>{}, ic<1>{}, ld_a, ld_a + SM::a_bytes, ok_a, on_from(s + NS - 1), st, sb);
-    step(ic<1>{}, ic<2>{}, ic<PARTS>{}, ic<(IA && PARTS > 2) ? nl(2) : 0>{}, ic<2>{}, ld_a, ld_a + SM::a_bytes, ok_a, on_from(s + NS - 1), st, sb);
-    step(ic<2>{}, ic<3>{}, ic<PARTS>{}, ic<(IA && PARTS > 3) ? nl(3) : 0>{}, ic<3>{}, ld_a, ld_a + SM::a_bytes, ok_a, on_from(s + NS - 1), st, sb);
+    const int k0 = kTurn ? k_ahead[0] : s + NS - 1, k1 = kTurn ? k_ahead[1] : s + NS;
+    const bool ok_a = slab_k(k0, u_ahead) + a_kc < K;
+    step(ic<0>{}, ic<1>{}, ic<PARTS>{}, ic<(IA && PARTS > 1) ? nl(1) : 0>{}, ic<1>{}, ld_a, ld_a + SM::a_bytes, ok_a, place(k0), st, sb);
+    step(ic<1>{}, ic<2>{}, ic<PARTS>{}, ic<(IA && PARTS > 2) ? nl(2) : 0>{}, ic<2>{}, ld_a, ld_a + SM::a_bytes, ok_a, place(k0), st, sb);
+    step(ic<2>{}, ic<3>{}, ic<PARTS>{}, ic<(IA && PARTS > 3) ? nl(3) : 0>{}, ic<3>{}, ld_a, ld_a + SM::a_bytes, ok_a, place(k0), st, sb);
     if constexpr (!LAST) {
       wait_loads(IA ? 1 : 0);
       __syncthreads();
@@ -623,17 +655,18 @@ __device__ __forceinline__ void gemm_tile(
       fetch(u_ahead);
     }
     step(ic<3>{}, ic<0>{}, ic<PARTS>{}, ic<IB ? nl(0) : 0>{}, ic<LAST ? -1 : 0>{}, ld_b, ld_b + SM::a_bytes,
-         slab_k(s + NS, u_ahead) + a_kc < K, on_from(s + NS), nst, nst + SM::a_bytes);
+         slab_k(k1, u_ahead) + a_kc < K, place(k1), nst, nst + SM::a_bytes);
     if constexpr (kClasses > 0) {
       if (u_now >= 8 * (class_slabs - 1)) end_class((u_now & 7) - first_class);
       u_now = after(u_now);
     }
+    go_on();
   };
 
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p) {
     if constexpr (kClasses > 0) fetch(u_ahead);
-    if (p < nslab) load_slab(p, slab_k(p, u_ahead), on_from(p));
+    if (p < nslab) load_slab(p, slab_k(k_slab(p), u_ahead), place(k_slab(p)));
     if constexpr (kClasses > 0) u_ahead = after(u_ahead);
   }
   // slab 0 must have landed; later prologue loads may still be in flight (exact count only
@@ -644,9 +677,10 @@ __device__ __forceinline__ void gemm_tile(
   if (NS - 1 < nslab) {  // the share of slab NS-1 that a slab's k-step 3 would have issued
     const uint32_t st = __builtin_amdgcn_readfirstlane(smem_lds + (NS - 1) * SM::stage_bytes + wave * 1024);
     if constexpr (kClasses > 0) fetch(u_ahead);
-    const bool k_ok = slab_k(NS - 1, u_ahead) + a_kc < K;
-    static_for<(LOADS + PARTS - 1) / PARTS>([&](auto q_c) { load_one(ic<PARTS * decltype(q_c)::value>{}, st, st + SM::a_bytes, k_ok, on_from(NS - 1)); });
+    const bool k_ok = slab_k(k_slab(NS - 1), u_ahead) + a_kc < K;
+    static_for<(LOADS + PARTS - 1) / PARTS>([&](auto q_c) { load_one(ic<PARTS * decltype(q_c)::value>{}, st, st + SM::a_bytes, k_ok, place(k_slab(NS - 1))); });
   }
+  look_ahead(NS - 1);
   int cs = 0, ls = NS - 1, s = 0;
   for (; s + NS < nslab; ++s) {  // steady state
     slab(T_{}, T_{}, F_{}, s, cs, ls);
@@ -832,15 +866,15 @@ __device__ __forceinline__ bool xcd_tile(int bid, int tiles_m, int tiles_n, int*
   return true;
 }
 
-template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kOnce = false, int kClasses = 0>
+template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, bool kOnce = false, int kClasses = 0, bool kTurn = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_f16_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0,
     const uint16_t* __restrict__ B1, const uint16_t* C, uint16_t* D,
     int M, int N, int K, float alpha, float beta, int ldc, int tiles_m, int tiles_n) {
   int tm, tn;
   if (!xcd_tile(blockIdx.x, tiles_m, tiles_n, &tm, &tn)) return;
-  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, false, false, kWholeCu, kOnce, kClasses>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tm * BM, tn * BN, K, 0,
-                                                                                      0, nullptr, 0, {}, 0, 1 << kClasses);
+  gemm_tile<E, BM, BN, WM, WN, kDual, kBCol, false, false, kWholeCu, kOnce, kClasses, kTurn>(A, B0, B1, C, D, M, N, K, alpha, beta, ldc, tm * BM, tn * BN, K, 0,
+                                                                                      0, nullptr, 0, {}, 0, 1 << kClasses, kTurn ? tn % ((K + BK - 1) / BK) : 0);
 }
 
 // Two tile heights in one launch, for shapes whose 256-row tiles fill the 256 CUs a whole number
@@ -960,6 +994,21 @@ static int launch_splitk(const uint16_t* A, const uint16_t* B, const uint16_t* C
   return check_launch("gemm split-K reduction launch");
 }
 
+// One row of tiles of more than 64 rows, whose column tiles start the contraction at slabs of their own and go round: where rows of weights are whole
+// multiples of 4 KB apart, workgroups that walk K in step ask a few of the memory's channels at a time.  Time turned over straight, weights streamed
+// (a pair by the size of one matrix):
+//   65 to 128 rows, 64 MB and more   0.72 to 1.01 over 80 launches (128 x 65536 x 4096 120 -> 91 us, 66 x 32768 x 4096 58 -> 47, 66 x 128256 x 4096 the same; pair of
+//                                    128 x 28672 x 4096 91 -> 80); 59 MB 0.99 to 1.01
+//   129 to 192 rows                  beyond 128 columns a CU and below 8192 deep 0.75 to 1.00 (130 x 65536 x 2048 68 -> 53); fewer columns are half a round or two
+//                                    heights, 0.97 to 1.03; 8192 deep 0.95 to 1.02
+//   193 to 256 rows                  2048 deep from 192 columns a CU on 0.87 to 0.99 (200 x 128256 x 2048 136 -> 121), 4096 deep 0.94 to 1.06
+// Where K is no multiple of 2048 0.97 to 1.03 in any of them.  Up to 64 rows the order of sums is that of the weight stream, for both layouts.
+static bool turn_pays(int M, int N, int K) {
+  if (M <= 64 || K % 2048 != 0 || (size_t)N * K * 2 < (size_t)64 << 20) return false;
+  if (M <= 128) return true;
+  return M <= 192 ? N > 128 * cu_count() && K < 8192 : N >= 192 * cu_count() && K <= 2048;
+}
+
 template <class E, int BM, int BN, int WM, int WN, bool kDual, bool kBCol, int kClasses = 0>
 static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1, const uint16_t* C,
                        uint16_t* D, int M, int N, int K, float alpha, float beta, int ldc,
@@ -968,8 +1017,8 @@ static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int ntiles = tiles_m * tiles_n;
   const int grid = ((ntiles + 7) / 8) * 8;
-  auto go = [&](auto once_c) {
-    auto kern = gemm_f16_kernel<E, BM, BN, WM, WN, kDual, kBCol, decltype(once_c)::value, kClasses>;
+  auto go = [&](auto once_c, auto turn_c) {
+    auto kern = gemm_f16_kernel<E, BM, BN, WM, WN, kDual, kBCol, decltype(once_c)::value, kClasses, decltype(turn_c)::value>;
     static bool attr_set = false;  // benign race: the call is idempotent
     if (!attr_set) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -986,16 +1035,21 @@ static int launch_gemm(const uint16_t* A, const uint16_t* B0, const uint16_t* B1
   // One row of tiles reads the weights once: with the non-temporal hint (three turns on one card: 256 x 128256 x 4096 258 -> 238 us, 66 x
   // 28672 x 8192 103 -> 91, pairs of it 176 -> 158; 200 x 128256 x 4096 between 224 and 263 either way).  Several rows of tiles share them through the caches, which the hint defeats, and shares of a
   // split read runs of a row too short for it (128 x 4096 x 4096 in 8: 19 us, 24 with it).
+  const bool turned = turn_pays(M, N, K);
   if constexpr (kBCol && BM % 128 != 0 && BM > 128) {  // heights that are launched for one row of tiles only
     if (tiles_m != 1) {
       set_error("gemm: %d rows on a tile for at most %d", M, BM);
       return NF_ERR_INVALID_ARGUMENT;
     }
-    return go(std::true_type{});
+    return turned ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
   } else {
     if constexpr (kBCol)
-      if (tiles_m == 1) return go(std::true_type{});
-    return go(std::false_type{});
+      if (tiles_m == 1) {
+        if constexpr (BM >= 128)
+          if (turned) return go(std::true_type{}, std::true_type{});
+        return go(std::true_type{}, std::false_type{});
+      }
+    return go(std::false_type{}, std::false_type{});
   }
 }
 

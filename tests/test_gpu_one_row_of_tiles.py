@@ -39,3 +39,22 @@ def test_eight_wavefronts(nk, M, N, Kd):
     if nk:
         sums = K.gemm_nk_sums(a.bfloat16(), b.bfloat16(), 16)
         assert torch.equal(sums.double().sum(0), want)
+
+
+@pytest.mark.parametrize("M,N,Kd", [(65, 16392, 2048), (128, 16392, 4096), (129, 32776, 2048), (192, 32776, 2048), (193, 49160, 2048), (256, 49152, 2048)])
+def test_contractions_that_go_round(M, N, Kd):
+    """Column tiles that start K at slabs of their own: every first slab there is, a last column tile that is cut, and the pair."""
+    from nanoflow_amd import kernels as K
+    assert N * Kd * 2 >= 64 << 20 and (N + 255) // 256 >= Kd // 64
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    whole = lambda *shape: torch.randint(-1, 2, shape, generator=gen, device="cuda", dtype=torch.int8)
+    a, b = whole(M, Kd), whole(N, Kd)
+    a16, b16 = a.half(), b.half()
+    want = a16.float() @ b16.float().t()
+    assert want.abs().max() <= 2048
+    guard = torch.full((M + 1, N), 77.0, dtype=torch.float16, device="cuda")
+    K.gemm(a16, b16, b_col_major=True, out=guard[:M])
+    assert torch.equal(guard[:M].float(), want) and (guard[M] == 77.0).all()
+    if M <= 128:
+        u16 = whole(N, Kd).half()
+        assert torch.equal(K.dual_swiglu(a16, b16, u16, b_col_major=True), K.dual_swiglu(a16, b16.t().contiguous(), u16.t().contiguous()))
