@@ -18,7 +18,10 @@ struct TilePlace {
 // kSpread: every XCD takes an eighth of every group's panels instead of its own run of the launch's tiles, for launches whose tiles
 // cost very unlike: the last XCD would have all of an expert that every token goes to (256 rows, 32 experts of 2048 x 2048 and
 // such a one: 92 -> 75 us).  An eighth is a run of neighbours: every eighth panel is 25 % slower (64 rows of 3584 x 4096: 182 us,
-// 139).
+// 139).  And the last expert's panels come first where there are at most 30 rows an expert: an expert that every token goes to follows the
+// others, and its tiles of 128 x 32 are a launch's longest (4 of 32 of 2048 x 2048 beside such a one, us, first expert first -> last first: 24 tokens
+// 47.5 -> 44.4, 49 58.5 -> 49.1, 80 55.8 -> 47.6, 128 53.8 -> 51.5, 200 59.1 -> 58.5; of more rows they take the CUs' intake from the streams: 230 60.9 and 61.9,
+// 256 63.1 and 66.0; without such a one 47.1 to 51.7 and 47.2 to 52.0).
 template <int BM, bool kSpread = false>
 __device__ __forceinline__ TilePlace find_tile(const nf_grouped_gemm_args& a, int bid, int tiles_n) {
   const int tiles_m = (a.M + BM - 1) / BM;
@@ -28,8 +31,10 @@ __device__ __forceinline__ TilePlace find_tile(const nf_grouped_gemm_args& a, in
     if (tiles_n <= 0) return {-1, 0, 0, 0, 0};
   }
   const int m_tiles = a.routing.n_tiles ? *a.routing.n_tiles : tiles_m * a.groups;
-  const int total = m_tiles * tiles_n, logical = kSpread ? bid / 8 : xcd_order(bid, total);
-  if ((!kSpread && bid / 8 >= (total + 7) / 8) || logical >= total) return {-1, 0, 0, 0, 0};
+  const int total = m_tiles * tiles_n;
+  if (bid / 8 >= (kSpread ? total : (total + 7) / 8)) return {-1, 0, 0, 0, 0};
+  const int logical = !kSpread ? xcd_order(bid, total) : a.max_rows <= 30 * a.groups ? total - 1 - bid / 8 : bid / 8;
+  if (logical >= total) return {-1, 0, 0, 0, 0};
   const int mt = logical / tiles_n, n_tile = logical % tiles_n;
   if (a.routing.n_tiles) {
     const int g = a.routing.tile_group[mt], row0 = a.routing.offsets[g], rows = a.routing.offsets[g + 1] - row0;

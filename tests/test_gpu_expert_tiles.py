@@ -40,6 +40,14 @@ def test_workgroups_that_go_from_tile_to_tile(N, Kd):
     check(MANY, N, Kd, torch.linspace(0.5, 4.0, len(MANY)))
 
 
+@pytest.mark.parametrize("counts", [(0, 1, 16, 33, 49, 10, 65), (3, 0, 65, 0), (0, 0, 0, 5)], ids=str)
+@pytest.mark.parametrize("N,Kd", [(520, 1600), (1032, 2048), (2048, 1544)])
+def test_last_expert_first(counts, N, Kd):
+    """At most 30 rows an expert: the weight stream goes through the experts from the last one on."""
+    assert sum(counts) <= 30 * len(counts)
+    check(counts, N, Kd, torch.full((len(counts),), 7.0))
+
+
 def check(counts, N, Kd, limits):
     from nanoflow_amd import kernels as K
     rng = np.random.default_rng(N + Kd)
