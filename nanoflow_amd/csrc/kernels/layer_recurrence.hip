@@ -219,6 +219,12 @@ __device__ __forceinline__ ChunkSpan find_chunk(const nf_recurrence_args& a, int
   return {-1, 0, 0, slot};
 }
 
+}  // namespace nf
+
+#include "recurrence_fixed.h"
+
+namespace nf {
+
 template <int KIND, int NKT, int NVT>
 struct ChunkShape {
   static constexpr int KP = NKT * 16, VP = 4 * NVT * 16;
@@ -509,7 +515,8 @@ __global__ __launch_bounds__(256, 2) void recur_chunk_state_kernel(nf_recurrence
     if ((int)threadIdx.x < pd.kp) chunk_factors(a, pd, max_chunks, ch.slot, h)[threadIdx.x] = exp2f(log2_all);
 }
 
-template <int KIND>
+// kFixedForm: the states lie as recurrence_fixed.h has them
+template <int KIND, bool kFixedForm = false>
 __global__ __launch_bounds__(256) void recur_chunk_scan_kernel(nf_recurrence_args a, int len, int max_chunks) {
   const RecurrenceDims pd = padded(a.dim, a.vdim);
   const int req = a.req_begin + blockIdx.x, h = blockIdx.y;
@@ -521,7 +528,8 @@ __global__ __launch_bounds__(256) void recur_chunk_scan_kernel(nf_recurrence_arg
   const int f4 = blockIdx.z * 256 + threadIdx.x, e = f4 * 4;  // four rows of a column, in fragment order
   if (e < pd.kp * pd.vp) {
     const int v_tiles = pd.vp / 16, lane = f4 & 63, tile = f4 >> 6;
-    const int k = tile / v_tiles * 16 + (lane >> 4) * 4, c = tile % v_tiles * 16 + (lane & 15);
+    int k = tile / v_tiles * 16 + (lane >> 4) * 4, c = tile % v_tiles * 16 + (lane & 15);
+    if constexpr (kFixedForm) fixed_place(f4, &k, &c);
     float* state = a.state + ((size_t)state_slot * a.heads + h) * pd.kp * pd.vp + (size_t)k * pd.vp + c;
     const float ld2 = KIND == NF_RECURRENCE_FIXED_DECAY ? a.log2_decay[h] : 0.f;
     float4_t cur{0.f, 0.f, 0.f, 0.f};
@@ -730,11 +738,49 @@ static int launch_chunks(const nf_recurrence_args& a, const ChunkPlan& p, hipStr
   return check_launch("nf_linear_recurrence (chunk outputs)");
 }
 
+// Fixed decays on the 16-bit matrix instructions (recurrence_fixed.h): heads of 128 x 128 in bf16, neither rotated nor gated, rows read and written 16 bytes at
+// a time; wherever the fp32 form takes chunks, for it is slower at every size (16 heads, us, fp32 form and this: 40 rows 25.8, 14.6; 500 rows 42, 24; 2047
+// 67, 38; 8000 195, 113; 8 requests of 256 72, 49).  Halves of a chunk where requests hardly fill one and the CUs are not all taken: 128 rows 20.1 -> 16.9 us,
+// but 2 x 300 25.7 -> 27.0.
+static ChunkPlan fixed_plan(const nf_recurrence_args& a) {
+  if (a.dtype != NF_BF16 || a.kind != NF_RECURRENCE_FIXED_DECAY || a.dim != kFixedDim || a.vdim != kFixedDim || a.rot.dims != 0 || a.g) return {0, 0};
+  if ((a.q_ld | a.k_ld | a.v_ld | a.out_ld | a.out_col) % 8 || ((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out) % 16) return {0, 0};
+  const bool brief = a.rows <= 160ll * a.req_num && ((long long)a.rows / kFixedChunk + a.req_num) * a.heads <= cu_count();
+  const int len = brief ? kFixedChunk / 2 : kFixedChunk, chunks = a.rows / len + a.req_num;
+  if ((size_t)chunks * chunk_bytes(a.heads, a.dim, a.vdim) > a.workspace_bytes) return {0, 0};
+  return {len, chunks};
+}
+static int launch_fixed(const nf_recurrence_args& a, const ChunkPlan& p, hipStream_t s) {
+  static bool attr_set = false;  // benign race: the call is idempotent
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(recur_fixed_state_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * FixedTile::bytes);
+    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void*>(recur_fixed_out_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kFixedOutLds);
+    if (e != hipSuccess) {
+      set_error("nf_linear_recurrence: cannot reserve %d bytes of LDS: %s", kFixedOutLds, hipGetErrorString(e));
+      return NF_ERR_RUNTIME;
+    }
+    attr_set = true;
+  }
+  const dim3 grid((unsigned)p.chunks, (unsigned)a.heads);
+  recur_fixed_state_kernel<<<grid, 512, 2 * FixedTile::bytes, s>>>(a, p.len);
+  int rc = check_launch("nf_linear_recurrence (chunk states)");
+  if (rc) return rc;
+  recur_chunk_scan_kernel<NF_RECURRENCE_FIXED_DECAY, true><<<dim3((unsigned)a.req_num, (unsigned)a.heads, kFixedDim * kFixedDim / 1024), 256, 0, s>>>(a, p.len, p.chunks);
+  rc = check_launch("nf_linear_recurrence (chunk scan)");
+  if (rc) return rc;
+  recur_fixed_out_kernel<<<grid, 512, kFixedOutLds, s>>>(a, p.len);
+  return check_launch("nf_linear_recurrence (chunk outputs)");
+}
+
 template <class T, int KIND>
 static int launch_recurrence(nf_recurrence_args a, hipStream_t s) {
   if (KIND == NF_RECURRENCE_TOKEN_DECAY) a.k_scale = 1.f;
   const ChunkPlan p = chunk_plan(a);
   if (p.chunks == 0) return launch_seq<T, KIND>(a, s);
+  if constexpr (std::is_same_v<T, bf16_t> && KIND == NF_RECURRENCE_FIXED_DECAY) {
+    const ChunkPlan f = fixed_plan(a);
+    if (f.chunks > 0) return launch_fixed(a, f, s);
+  }
   const RecurrenceDims pd = padded(a.dim, a.vdim);
   const bool wide = pd.vp > 64;
   if (pd.kp <= 32) return wide ? launch_chunks<T, KIND, 2, 2>(a, p, s) : launch_chunks<T, KIND, 2, 1>(a, p, s);
