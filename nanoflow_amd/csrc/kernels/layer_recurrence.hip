@@ -58,7 +58,7 @@ __device__ __forceinline__ float token_log2_decay(const nf_recurrence_args& a, i
 }
 
 template <class T, int NP, int KIND>
-__global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, int tb) {
+__global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, int tb, bool through) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const RecurrenceDims pd = padded(a.dim, a.vdim);
   const int req = a.req_begin + blockIdx.x, h = blockIdx.y;
@@ -139,6 +139,16 @@ __global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, i
       }
       if (lane < 16) *reinterpret_cast<float4_t*>(sp + (t * 4 + swave) * vw + col) = o;
     }
+    if (r0 + tb >= row1) {  // on its way while the rows are normed
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const int k = krow + 16 * i;
+        if (k >= pd.kp || col >= pd.vp) continue;
+        float* to = state + (size_t)k * pd.vp + col;
+        if (through) store_through(to, S[i]);
+        else *reinterpret_cast<float4_t*>(to) = S[i];
+      }
+    }
     __syncthreads();
     // per row: the four partial sums, the current token's own term, norm, gate
     for (int t = wave; t < n; t += n_waves) {
@@ -168,11 +178,6 @@ __global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, i
     }
     __syncthreads();
   }
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int k = krow + 16 * i;
-    if (k < pd.kp && col < pd.vp) *reinterpret_cast<float4_t*>(state + (size_t)k * pd.vp + col) = S[i];
-  }
   if (a.shift_x && h == 0)
     for (int c = tid * 4; c < a.shift_ld; c += blockDim.x * 4)
       *reinterpret_cast<float4_t*>(a.shift_state + (size_t)slot * a.shift_ld + c) =
@@ -190,8 +195,11 @@ static int launch_seq(const nf_recurrence_args& a, hipStream_t s) {
   int tb = a.rows == a.req_num ? 1 : 8;
   while (tb > 1 && lds_of(tb) > 64 * 1024) tb /= 2;
   const dim3 grid((unsigned)a.req_num, (unsigned)a.heads);
+  // More than 4 MB of states go through the caches (one row a request, us, before and so: 16 requests of 32 heads of 64 x 64, 8 MB, 7.6 -> 6.5, 64 18.1 -> 14.8,
+  // 256 63 -> 60, 16 of 16 heads of 128 x 128 10.7 -> 8.6; 4 MB 5.9 either way, 0.5 MB 5.3 and 5.6).
+  const bool through = (size_t)a.req_num * a.heads * pd.kp * pd.vp * sizeof(float) > (size_t)4 << 20;
   auto go = [&](auto np) {
-    recur_seq_kernel<T, decltype(np)::value, KIND><<<grid, ns * 256, lds_of(tb), s>>>(a, tb);
+    recur_seq_kernel<T, decltype(np)::value, KIND><<<grid, ns * 256, lds_of(tb), s>>>(a, tb, through);
     return check_launch("nf_linear_recurrence");
   };
   const int np = pd.kp / 16;
