@@ -252,8 +252,13 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // A 16-byte store that goes through the XCD's L2 to memory at once (sc1).  A kernel's end waits until what it left in the L2s is written back: 16 MB of ordinary
 // stores take 5.0 us in a launch of nothing else, 3.8 so, 4 MB 2.7 and 2.3.  For megabytes that no kernel reads soon; what the next one reads is better
-// left in the caches.
-__device__ __forceinline__ void store_through(float* p, float4_t v) { asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory"); }
+// left in the caches.  `base` is the same for the whole wavefront, `bytes` of it are there.  A builtin, so that the compiler knows when it reads v: straight after an
+// MFMA that writes v, or before an instruction that does, a store in inline assembly would need waits that nothing puts there.
+__device__ __forceinline__ void store_through(float* base, uint32_t bytes, uint32_t offset, float4_t v) {
+  typedef uint32_t words_t __attribute__((ext_vector_type(4)));
+  constexpr int kSc1 = 16;
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(words_t, v), __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00020000), (int)offset, 0, kSc1);
+}
 
 // Compute units of the current device (256 on MI355X).
 inline int cu_count() {

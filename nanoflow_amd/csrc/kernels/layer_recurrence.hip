@@ -8,7 +8,8 @@
 //
 // recur_seq_kernel: one workgroup per (request, head) holds the head's state in registers and walks
 // the request's rows, a few at a time through LDS.  Decode (one row): the state is streamed in, used,
-// and streamed out once.
+// and streamed out once, through the caches (us, ordinary stores and these: 16 requests of 32 heads of 64 x 64, 8 MB, 7.4 -> 5.7, 64 17.0 -> 14.2, 256 60.5 ->
+// 58.5, 16 of 16 heads of 128 x 128 10.0 -> 7.8; 0.5 to 4 MB 5.0 to 5.5 and 5.0 to 5.2).
 //
 // Portions of prompts are cut into chunks that are computed side by side, in three launches:
 //   recur_chunk_state_kernel  what every chunk adds to a state that enters it as zero, and the factor the
@@ -58,7 +59,7 @@ __device__ __forceinline__ float token_log2_decay(const nf_recurrence_args& a, i
 }
 
 template <class T, int NP, int KIND>
-__global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, int tb, bool through) {
+__global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, int tb) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const RecurrenceDims pd = padded(a.dim, a.vdim);
   const int req = a.req_begin + blockIdx.x, h = blockIdx.y;
@@ -140,13 +141,13 @@ __global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, i
       if (lane < 16) *reinterpret_cast<float4_t*>(sp + (t * 4 + swave) * vw + col) = o;
     }
     if (r0 + tb >= row1) {  // on its way while the rows are normed
+      // The state has long been there; said once, ahead of the branches, it spares a wait for each store ahead of the next.
+      __builtin_amdgcn_s_waitcnt(0x0F70);
 #pragma unroll
       for (int i = 0; i < NP; ++i) {
         const int k = krow + 16 * i;
         if (k >= pd.kp || col >= pd.vp) continue;
-        float* to = state + (size_t)k * pd.vp + col;
-        if (through) store_through(to, S[i]);
-        else *reinterpret_cast<float4_t*>(to) = S[i];
+        store_through(state, (uint32_t)(pd.kp * pd.vp * sizeof(float)), (uint32_t)((k * pd.vp + col) * sizeof(float)), S[i]);
       }
     }
     __syncthreads();
@@ -195,11 +196,8 @@ static int launch_seq(const nf_recurrence_args& a, hipStream_t s) {
   int tb = a.rows == a.req_num ? 1 : 8;
   while (tb > 1 && lds_of(tb) > 64 * 1024) tb /= 2;
   const dim3 grid((unsigned)a.req_num, (unsigned)a.heads);
-  // More than 4 MB of states go through the caches (one row a request, us, before and so: 16 requests of 32 heads of 64 x 64, 8 MB, 7.6 -> 6.5, 64 18.1 -> 14.8,
-  // 256 63 -> 60, 16 of 16 heads of 128 x 128 10.7 -> 8.6; 4 MB 5.9 either way, 0.5 MB 5.3 and 5.6).
-  const bool through = (size_t)a.req_num * a.heads * pd.kp * pd.vp * sizeof(float) > (size_t)4 << 20;
   auto go = [&](auto np) {
-    recur_seq_kernel<T, decltype(np)::value, KIND><<<grid, ns * 256, lds_of(tb), s>>>(a, tb, through);
+    recur_seq_kernel<T, decltype(np)::value, KIND><<<grid, ns * 256, lds_of(tb), s>>>(a, tb);
     return check_launch("nf_linear_recurrence");
   };
   const int np = pd.kp / 16;
