@@ -228,6 +228,7 @@ __device__ __forceinline__ ChunkSpan find_chunk(const nf_recurrence_args& a, int
 }  // namespace nf
 
 #include "recurrence_fixed.h"
+#include "recurrence_token.h"
 
 namespace nf {
 
@@ -521,8 +522,8 @@ __global__ __launch_bounds__(256, 2) void recur_chunk_state_kernel(nf_recurrence
     if ((int)threadIdx.x < pd.kp) chunk_factors(a, pd, max_chunks, ch.slot, h)[threadIdx.x] = exp2f(log2_all);
 }
 
-// kFixedForm: the states lie as recurrence_fixed.h has them
-template <int KIND, bool kFixedForm = false>
+// kForm: the states lie as recurrence_fixed.h or recurrence_token.h, of the kind, has them
+template <int KIND, bool kForm = false>
 __global__ __launch_bounds__(256) void recur_chunk_scan_kernel(nf_recurrence_args a, int len, int max_chunks) {
   const RecurrenceDims pd = padded(a.dim, a.vdim);
   const int req = a.req_begin + blockIdx.x, h = blockIdx.y;
@@ -535,7 +536,7 @@ __global__ __launch_bounds__(256) void recur_chunk_scan_kernel(nf_recurrence_arg
   if (e < pd.kp * pd.vp) {
     const int v_tiles = pd.vp / 16, lane = f4 & 63, tile = f4 >> 6;
     int k = tile / v_tiles * 16 + (lane >> 4) * 4, c = tile % v_tiles * 16 + (lane & 15);
-    if constexpr (kFixedForm) fixed_place(f4, &k, &c);
+    if constexpr (kForm) KIND == NF_RECURRENCE_FIXED_DECAY ? fixed_place(f4, &k, &c) : token_place(f4, &k, &c);
     float* state = a.state + ((size_t)state_slot * a.heads + h) * pd.kp * pd.vp + (size_t)k * pd.vp + c;
     const float ld2 = KIND == NF_RECURRENCE_FIXED_DECAY ? a.log2_decay[h] : 0.f;
     float4_t cur{0.f, 0.f, 0.f, 0.f};
@@ -751,6 +752,7 @@ static int launch_chunks(const nf_recurrence_args& a, const ChunkPlan& p, hipStr
 static ChunkPlan fixed_plan(const nf_recurrence_args& a) {
   if (a.dtype != NF_BF16 || a.kind != NF_RECURRENCE_FIXED_DECAY || a.dim != kFixedDim || a.vdim != kFixedDim || a.rot.dims != 0 || a.g) return {0, 0};
   if ((a.q_ld | a.k_ld | a.v_ld | a.out_ld | a.out_col) % 8 || ((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out) % 16) return {0, 0};
+  if (std::max(std::max(a.q_ld, a.k_ld), a.v_ld) >= 1 << 24) return {0, 0};  // a chunk's rows within 32-bit offsets
   const bool brief = a.rows <= 160ll * a.req_num && ((long long)a.rows / kFixedChunk + a.req_num) * a.heads <= cu_count();
   const int len = brief ? kFixedChunk / 2 : kFixedChunk, chunks = a.rows / len + a.req_num;
   if ((size_t)chunks * chunk_bytes(a.heads, a.dim, a.vdim) > a.workspace_bytes) return {0, 0};
@@ -778,6 +780,31 @@ static int launch_fixed(const nf_recurrence_args& a, const ChunkPlan& p, hipStre
   return check_launch("nf_linear_recurrence (chunk outputs)");
 }
 
+// Decays of every token, 64 tokens at a time (recurrence_token.h): heads of 64 x 64 in bf16, rows read and written 16 bytes at a time; wherever the general form
+// takes chunks, for it is slower at every size (32 heads, us, general form and this: 40 rows 21.1, 14.1; 129 rows 28.0, 16.3; 500 rows 32, 20; 3000 85, 60;
+// 8000, in its chunks of 256, 173, 135; 8 requests of 256 61, 48; 2047 rows of which most blocks decay below 2^-100, its steps then of four tokens or one, 597, 72).
+static ChunkPlan token_plan(const nf_recurrence_args& a) {
+  if (a.dtype != NF_BF16 || a.kind != NF_RECURRENCE_TOKEN_DECAY || a.dim != kTokenDim || a.vdim != kTokenDim) return {0, 0};
+  if ((a.q_ld | a.k_ld | a.v_ld | (a.g ? a.g_ld : 0) | a.out_ld | a.out_col) % 8 || a.z_ld % 4 ||
+      ((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.g | (uintptr_t)a.out | (uintptr_t)a.z | (uintptr_t)a.w0 | (uintptr_t)a.u) % 16)
+    return {0, 0};
+  if (std::max(a.k_ld, a.v_ld) >= 1 << 24) return {0, 0};  // a chunk's rows within 32-bit offsets
+  const int chunks = a.rows / kTokenChunk + a.req_num;
+  if ((size_t)chunks * chunk_bytes(a.heads, a.dim, a.vdim) > a.workspace_bytes) return {0, 0};
+  return {kTokenChunk, chunks};
+}
+static int launch_token(const nf_recurrence_args& a, const ChunkPlan& p, hipStream_t s) {
+  const dim3 grid((unsigned)p.chunks, (unsigned)a.heads);
+  recur_token_state_kernel<<<grid, 4 * kTokenChunk, 0, s>>>(a, p.chunks);
+  int rc = check_launch("nf_linear_recurrence (chunk states)");
+  if (rc) return rc;
+  recur_chunk_scan_kernel<NF_RECURRENCE_TOKEN_DECAY, true><<<dim3((unsigned)a.req_num, (unsigned)a.heads, kTokenDim * kTokenDim / 1024), 256, 0, s>>>(a, p.len, p.chunks);
+  rc = check_launch("nf_linear_recurrence (chunk scan)");
+  if (rc) return rc;
+  recur_token_out_kernel<<<grid, 4 * kTokenChunk, 0, s>>>(a);
+  return check_launch("nf_linear_recurrence (chunk outputs)");
+}
+
 template <class T, int KIND>
 static int launch_recurrence(nf_recurrence_args a, hipStream_t s) {
   if (KIND == NF_RECURRENCE_TOKEN_DECAY) a.k_scale = 1.f;
@@ -786,6 +813,10 @@ static int launch_recurrence(nf_recurrence_args a, hipStream_t s) {
   if constexpr (std::is_same_v<T, bf16_t> && KIND == NF_RECURRENCE_FIXED_DECAY) {
     const ChunkPlan f = fixed_plan(a);
     if (f.chunks > 0) return launch_fixed(a, f, s);
+  }
+  if constexpr (std::is_same_v<T, bf16_t> && KIND == NF_RECURRENCE_TOKEN_DECAY) {
+    const ChunkPlan f = token_plan(a);
+    if (f.chunks > 0) return launch_token(a, f, s);
   }
   const RecurrenceDims pd = padded(a.dim, a.vdim);
   const bool wide = pd.vp > 64;
