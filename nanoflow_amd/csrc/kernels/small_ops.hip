@@ -165,6 +165,9 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(u32x4* __restrict__ out,
     return yv;
   };
   if constexpr (kHeld) {
+    // The loads; said once, ahead of the branches, it spares a wait for each store ahead of the next (us, 1 row of 4096 2.38 -> 2.26, quantised 3.36 -> 3.13,
+    // 64 rows 2.66 -> 2.54, 3.75 -> 3.50, 2048 rows 6.72 -> 6.60; 64 rows of 8192 3.31 -> 2.91).
+    __builtin_amdgcn_s_waitcnt(0x0F70);
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       if ((int)threadIdx.x + k * 256 < vec_per_row) {
