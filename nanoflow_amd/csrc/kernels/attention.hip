@@ -356,8 +356,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
             s[blk][r] *= scale_log2;
             if (ok[blk][r]) mx = fmaxf(mx, s[blk][r]);
           }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = max_over_lane_groups(mx);
         const float m_new = fmaxf(m_run, mx);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         m_run = m_new;
@@ -395,8 +394,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_decode_kernel(
           dma_v(pp + 2 * NW, buf);
         }
       }
-      l_run += __shfl_xor(l_run, 16, 64);
-      l_run += __shfl_xor(l_run, 32, 64);
+      l_run = sum_over_near_lane_groups(l_run);
 
       // ---- merge the wavefronts.  oacc[i][r] = O[column c16][feature 16i + 4g + r].  Each
       // wavefront parks its partial result in its own LDS region (its streaming is over).

@@ -71,8 +71,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_e4m3_kernel(const uint
     for (int c = tid; c < chunks; c += kThreads) chunk_max(src[c]);
   }
   float amax = fmaxf((float)top[0], (float)top[1]);
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+  amax = wave_max(amax);
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
   amax = red[0];

@@ -337,8 +337,7 @@ __global__ __launch_bounds__(256, kVec <= 2 ? 8 : 5) void qkv_append4_kernel(nf_
         for (int i = 0; i < kVec; ++i)
 #pragma unroll
           for (int e = 0; e < 4; ++e) sq += v[i][u][e] * v[i][u][e];
-#pragma unroll
-        for (int m = 8; m > 0; m >>= 1) sq += __shfl_xor(sq, m, 64);
+        sq = sum_of_16(sq);
         const float inv = 1.f / sqrtf(sq / (float)dim + eps);
         if (w) {
 #pragma unroll
@@ -412,8 +411,7 @@ __global__ __launch_bounds__(256, kVec <= 2 ? 8 : 5) void qkv_append4_kernel(nf_
       const float4_t v = row.four(v_col + head * kv.vdim + c, false);
       sq += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
     }
-#pragma unroll
-    for (int m = 8; m > 0; m >>= 1) sq += __shfl_xor(sq, m, 64);
+    sq = sum_of_16(sq);
     inv = 1.f / sqrtf(sq / (float)kv.vdim + eps);
   }
   for (int c = (tid & 15) * 4; c < kv.v_pad; c += 64) {
@@ -523,9 +521,7 @@ __global__ __launch_bounds__(64) void attn_rows_kernel(nf_window_attention_args 
         s = dot * a.scale;
         if (a.softcap > 0.f) s = a.softcap * tanhf(s / a.softcap);
       }
-      float mx = s;
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+      const float mx = wave_max(s);
       const float m_new = fmaxf(m, mx), alpha = expf(m - m_new);
       const float w = see ? expf(s - m_new) : 0.f;
       m = m_new;
@@ -775,8 +771,7 @@ __global__ __launch_bounds__(window_threads(kMaps, VD)) void attn_window_kernel(
           mx = fmaxf(mx, s[n][b][r]);
         }
       mx = mx > -1e30f ? mx * scale2 : mx;
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_over_lane_groups(mx);
       // brought to a new maximum only when it has grown by 2^8: weights up to 256 cost nothing in fp32
       if (__any(mx > m[n] + 8.f)) {
         const float m_new = fmaxf(m[n], mx), alpha = __builtin_amdgcn_exp2f(m[n] - m_new);
@@ -808,10 +803,7 @@ __global__ __launch_bounds__(window_threads(kMaps, VD)) void attn_window_kernel(
 
   bf16_t* out = (bf16_t*)a.out;
 #pragma unroll
-  for (int n = 0; n < NC; ++n) {
-    l[n] += __shfl_xor(l[n], 16, 64);
-    l[n] += __shfl_xor(l[n], 32, 64);
-  }
+  for (int n = 0; n < NC; ++n) l[n] = sum_over_near_lane_groups(l[n]);
   if constexpr (kDecode) {
     // merge the wavefronts: m and l of [wave][map][16 columns], O of [wave][map][heads][v_pad]
     float* sm = merge_lds;

@@ -202,9 +202,7 @@ __global__ __launch_bounds__(64) void latent_rows_kernel(nf_latent_attention_arg
       }
       s = dot * a.scale;
     }
-    float mx = s;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+    const float mx = wave_max(s);
     const float m_new = fmaxf(m, mx), alpha = expf(m - m_new), w = see ? expf(s - m_new) : 0.f;
     m = m_new;
     l = l * alpha + w;
@@ -496,9 +494,7 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(nf_latent_attention_a
   const int R = a.layout.rank_pad, at = lane < p.splits ? lane : 0;
   const float* ml = p.part_ml + (size_t)pair * p.splits * 2;
   const float m = lane < p.splits ? ml[2 * at] : -1e30f, l = lane < p.splits ? ml[2 * at + 1] : 0.f;
-  float mm = m;
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) mm = fmaxf(mm, __shfl_xor(mm, d, 64));
+  const float mm = wave_max(m);
   const float den = wave_sum(l * __builtin_amdgcn_exp2f(m - mm));
   const float f = l > 0.f ? __builtin_amdgcn_exp2f(m - mm) / den : 0.f;  // 0: a share whose keys are all unseen
   bf16_t* dst = (bf16_t*)a.out + ((size_t)a.row_begin * a.layout.heads + pair) * R;

@@ -134,10 +134,7 @@ __global__ __launch_bounds__(1024) void recur_seq_kernel(nf_recurrence_args a, i
         S[i] = S[i] * w + v * sk[t * pd.kp + k];
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        o[e] += __shfl_xor(o[e], 16, 64);
-        o[e] += __shfl_xor(o[e], 32, 64);
-      }
+      for (int e = 0; e < 4; ++e) o[e] = sum_over_near_lane_groups(o[e]);
       if (lane < 16) *reinterpret_cast<float4_t*>(sp + (t * 4 + swave) * vw + col) = o;
     }
     if (r0 + tb >= row1) {  // on its way while the rows are normed
@@ -372,8 +369,7 @@ __device__ __forceinline__ void decay_sums(const nf_recurrence_args& a, ChunkLds
     const int t = threadIdx.x >> 4, l = threadIdx.x & 15;
     float b = 0.f;
     for (int e = l; e < a.dim; e += 16) b += s.q[t * C::kPitch + e] * s.k[t * C::kPitch + e] * a.u[(size_t)h * a.dim + e];
-#pragma unroll
-    for (int m = 8; m > 0; m >>= 1) b += __shfl_xor(b, m, 64);
+    b = sum_of_16(b);
     if (l == 0) s.bonus[t] = b;
   }
 }
@@ -681,8 +677,7 @@ __global__ __launch_bounds__(256, 2) void recur_chunk_out_kernel(nf_recurrence_a
         ss += o[vt][r] * o[vt][r];
         s.o[(4 * g + r) * C::vPitch + (wave * NVT + vt) * 16 + l16] = o[vt][r];
       }
-#pragma unroll
-      for (int m = 8; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
+      ss = sum_of_16(ss);
       if (l16 == 0) s.ss[4 * g + r][wave] = ss;
     }
     __syncthreads();

@@ -39,8 +39,7 @@ __global__ __launch_bounds__(256) void route_rows_kernel(nf_route_args a, int32_
     }
     mx = fmaxf(mx, s[i]);
   }
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+  mx = wave_max(mx);
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {

@@ -209,8 +209,7 @@ __global__ __launch_bounds__(kTokenChunk * 4, 3) void recur_token_out_kernel(nf_
       through[c] = to;
       low |= to < kMinStepLog2;
     }
-    bonus += __shfl_xor(bonus, 16, 64);
-    bonus += __shfl_xor(bonus, 32, 64);
+    bonus = sum_over_near_lane_groups(bonus);
     if (blk + 1 < kBlocks) {
 #pragma unroll
       for (int c = 0; c < 16; ++c) {
@@ -242,8 +241,7 @@ __global__ __launch_bounds__(kTokenChunk * 4, 3) void recur_token_out_kernel(nf_
           const float l = __shfl(lw[c], from, 64);
           between[c] += d <= l16 ? l : 0.f;
         }
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
+        s = sum_over_near_lane_groups(s);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (4 * g + r == l16 - d) own[r] = s;
@@ -335,8 +333,7 @@ __global__ __launch_bounds__(kTokenChunk * 4, 3) void recur_token_out_kernel(nf_
   for (int c = 0; c < 4; ++c)
 #pragma unroll
     for (int r = 0; r < 4; ++r) ss += o[c][r] * o[c][r];
-  ss += __shfl_xor(ss, 16, 64);
-  ss += __shfl_xor(ss, 32, 64);
+  ss = sum_over_near_lane_groups(ss);
   const float inv = a.g ? a.out_scale / sqrtf(ss / (float)kTokenDim + a.eps) : a.out_scale;
   float4_t y[4];
 #pragma unroll

@@ -178,8 +178,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(u32x4* __restrict__ out,
     for (int i = threadIdx.x; i < vec_per_row; i += 256) normalise(i, x[i], w[i]);
   }
   if constexpr (kQuant) {
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+    amax = wave_max(amax);
     if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
@@ -270,13 +269,11 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const uint16_t* __restrict
 #pragma unroll
     for (int m = 32; m > 0; m >>= 1) take(__shfl_xor(best, m, 64), (uint32_t)__shfl_xor((int)key, m, 64));
   } else {
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) best = fmaxf(best, __shfl_xor(best, m, 64));
+    best = wave_max(best);
     if ((tid & 63) == 0) s_v[tid >> 6] = best;
     __syncthreads();
     best = s_v[tid & 15];
-#pragma unroll
-    for (int m = 8; m > 0; m >>= 1) best = fmaxf(best, __shfl_xor(best, m, 64));
+    best = max_of_16(best);
     if (mine == best && best > -10000.f) find();
 #pragma unroll
     for (int m = 32; m > 0; m >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, m, 64));
