@@ -1,8 +1,10 @@
 // Routing of a mixture of experts: scores, choice, and the order of the chosen rows by expert.
 //
 // route_rows_kernel: one wavefront per token, its scores in registers (fp32 softmax over all outputs, or a sigmoid of each), groups of
-//   outputs closed by the rank of their largest entry, the `top` largest taken one after the other, then the
-//   experts that every token has.
+//   outputs closed by the rank of their largest entry, the `top` largest taken one after the other (up to 64 outputs: all at once, by rank), then the
+//   experts that every token has.  What bounds it is a chain of dependent steps: loads that are all on their way before the first is waited for, and lanes that
+//   meet without LDS, took both launches from 11.6 to 9.1 us (256 rows of 32 outputs in 8 groups, 4 a token, 16 shares), 11.9 to 9.9 (2047 rows of 40, 5 a
+//   token), 8.2 to 6.5 (one row).
 // route_plan_kernel: counts the rows of every expert, places them (an expert's rows consecutive)
 //   and lists the m tiles of the grouped product.  The place of a row inside its expert's run
 //   depends on the order of LDS atomics; nothing computed from it does.
@@ -15,28 +17,35 @@ namespace nf {
 
 constexpr int kMaxOutputs = 1024, kMaxTop = 64;
 
+__device__ __forceinline__ float lane_value(float x, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane)); }
+
 template <int kPer>  // outputs per lane
 __global__ __launch_bounds__(256) void route_rows_kernel(nf_route_args a, int32_t* __restrict__ choice, float* __restrict__ weight) {
-  __shared__ float entry[4][kPer * 64], best_of[4][kPer * 64];
+  __shared__ float entry[4][kPer > 1 ? kPer * 64 : 1], best_of[4][kPer > 1 ? kPer * 64 : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
   const bool live = t < a.rows;
   const float* __restrict__ z = a.z + (size_t)(live ? t : 0) * a.ld;
   const int shares = a.shares, outputs = a.outputs, per_token = a.top + a.always;
   const size_t slice = (size_t)a.rows * a.ld;
   float s[kPer], c[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) c[i] = a.correction ? a.correction[min(i * 64 + lane, outputs - 1)] : 0.f;
+  // lane p: share p of the score of the experts that every token has
+  const float gate_share = a.always > 0 && !a.always_plain && lane < shares ? z[lane * slice + outputs] : 0.f;
   float mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int o = i * 64 + lane;
-    s[i] = -INFINITY;
-    if (o < outputs) {
-      float part[kMaxShares];  // in flight together
+    const float* at = z + min(o, outputs - 1);
+    float sum = at[0];
+    if (shares > 1) {
+      float part[kMaxShares];  // in flight together: with a branch around each the compiler lets them wait for each other
 #pragma unroll
-      for (int p = 0; p < kMaxShares; ++p) part[p] = p < shares ? z[p * slice + o] : 0.f;
-      s[i] = part[0];
+      for (int p = 1; p < kMaxShares; ++p) part[p] = at[(size_t)min(p, shares - 1) * slice];
 #pragma unroll
-      for (int p = 1; p < kMaxShares; ++p) s[i] += part[p];
+      for (int p = 1; p < kMaxShares; ++p) sum += p < shares ? part[p] : 0.f;
     }
+    s[i] = o < outputs ? sum : -INFINITY;
     mx = fmaxf(mx, s[i]);
   }
   mx = wave_max(mx);
@@ -53,69 +62,117 @@ __global__ __launch_bounds__(256) void route_rows_kernel(nf_route_args a, int32_
   for (int i = 0; i < kPer; ++i) {
     const int o = i * 64 + lane;
     s[i] /= sum;
-    c[i] = o < outputs ? s[i] + (a.correction ? a.correction[o] : 0.f) : -INFINITY;
+    c[i] = o < outputs ? s[i] + c[i] : -INFINITY;
   }
-  if (a.groups > 1) {  // the same for every wavefront: the barriers are met by all
-    const int size = outputs / a.groups;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) entry[wave][i * 64 + lane] = c[i];
-    __syncthreads();
-    for (int g = lane; g < a.groups; g += 64) {
-      float b = entry[wave][g * size];
-      for (int e = 1; e < size; ++e) b = fmaxf(b, entry[wave][g * size + e]);
-      best_of[wave][g] = b;
-    }
-    __syncthreads();
-    for (int g = lane; g < a.groups; g += 64) {
-      const float b = best_of[wave][g];
+  if constexpr (kPer == 1) {
+    // An output a lane: its rank is the number of those ahead of it, read lane by lane into scalar registers, and the wavefront needs neither LDS nor a chain of
+    // `top` maxima.
+    float mine = c[0] > -INFINITY ? c[0] : -INFINITY;  // what is no number is not chosen
+    const int even = (outputs + 7) / 8 * 8;            // the lanes past the outputs are ahead of no one
+    if (a.groups > 1) {
+      const int size = outputs / a.groups, group = lane / size;
+      float best = -INFINITY;
+#pragma unroll 8
+      for (int o = 0; o < even; ++o) {
+        const float x = lane_value(mine, o);
+        best = o >= group * size && o < group * size + size ? fmaxf(best, x) : best;
+      }
       int ahead = 0;  // groups with a larger entry, or as large and before it
-      for (int o = 0; o < a.groups; ++o) ahead += best_of[wave][o] > b || (best_of[wave][o] == b && o < g);
-      entry[wave][g] = ahead < a.keep_groups ? 1.f : 0.f;
+      for (int g = 0; g < a.groups; ++g) {
+        const float x = lane_value(best, g * size);
+        ahead += x > best || (x == best && g < group);
+      }
+      if (ahead >= a.keep_groups) mine = -INFINITY;
     }
-    __syncthreads();
+    if (!live) return;
+    int ahead = 0;  // larger scores, and as large ones before it
+#pragma unroll 8
+    for (int o = 0; o < even; ++o) {
+      const float x = lane_value(mine, o);
+      ahead += x > mine || (x == mine && o < lane);
+    }
+    const bool some = mine > -INFINITY;
+    const int chosen = (int)__popcll(__ballot(some));
+    if (some && ahead < a.top) {
+      choice[(size_t)t * per_token + ahead] = lane;
+      weight[(size_t)t * per_token + ahead] = s[0] * a.scale;
+    }
+    if (lane >= chosen && lane < a.top) {  // scores that are no numbers: a valid index all the same
+      choice[(size_t)t * per_token + lane] = 0;
+      weight[(size_t)t * per_token + lane] = 0.f * a.scale;
+    }
+  } else {
+    if (a.groups > 1) {  // the same for every wavefront: the barriers are met by all
+      const int size = outputs / a.groups;
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int o = i * 64 + lane;
-      if (o < outputs && entry[wave][o / size] == 0.f) c[i] = -INFINITY;
+      for (int i = 0; i < kPer; ++i) entry[wave][i * 64 + lane] = c[i];
+      __syncthreads();
+      for (int g = lane; g < a.groups; g += 64) {
+        float b = entry[wave][g * size];
+        for (int e = 1; e < size; ++e) b = fmaxf(b, entry[wave][g * size + e]);
+        best_of[wave][g] = b;
+      }
+      __syncthreads();
+      for (int g = lane; g < a.groups; g += 64) {
+        const float b = best_of[wave][g];
+        int ahead = 0;  // groups with a larger entry, or as large and before it
+        for (int o = 0; o < a.groups; ++o) ahead += best_of[wave][o] > b || (best_of[wave][o] == b && o < g);
+        entry[wave][g] = ahead < a.keep_groups ? 1.f : 0.f;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int o = i * 64 + lane;
+        if (o < outputs && entry[wave][o / size] == 0.f) c[i] = -INFINITY;
+      }
+    }
+    if (!live) return;
+    for (int k = 0; k < a.top; ++k) {
+      float best = -INFINITY, w = 0.f;
+      int at = 0x7fffffff;
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        if (c[i] > best) {  // the smallest of equal ones: i ascends
+          best = c[i];
+          at = i * 64 + lane;
+          w = s[i];
+        }
+#pragma unroll
+      for (int m = 32; m > 0; m >>= 1) {
+        const float b2 = __shfl_xor(best, m, 64), w2 = __shfl_xor(w, m, 64);
+        const int a2 = __shfl_xor(at, m, 64);
+        if (b2 > best || (b2 == best && a2 < at)) {
+          best = b2;
+          at = a2;
+          w = w2;
+        }
+      }
+      if (at >= outputs) at = 0, w = 0.f;  // scores that are no numbers: a valid index all the same
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        if (i * 64 + lane == at) c[i] = -INFINITY;
+      if (lane == 0) {
+        choice[(size_t)t * per_token + k] = at;
+        weight[(size_t)t * per_token + k] = w * a.scale;
+      }
     }
   }
-  if (!live) return;
-  for (int k = 0; k < a.top; ++k) {
-    float best = -INFINITY, w = 0.f;
-    int at = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i)
-      if (c[i] > best) {  // the smallest of equal ones: i ascends
-        best = c[i];
-        at = i * 64 + lane;
-        w = s[i];
-      }
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-      const float b2 = __shfl_xor(best, m, 64), w2 = __shfl_xor(w, m, 64);
-      const int a2 = __shfl_xor(at, m, 64);
-      if (b2 > best || (b2 == best && a2 < at)) {
-        best = b2;
-        at = a2;
-        w = w2;
-      }
-    }
-    if (at >= outputs) at = 0, w = 0.f;  // scores that are no numbers: a valid index all the same
-#pragma unroll
-    for (int i = 0; i < kPer; ++i)
-      if (i * 64 + lane == at) c[i] = -INFINITY;
-    if (lane == 0) {
-      choice[(size_t)t * per_token + k] = at;
-      weight[(size_t)t * per_token + k] = w * a.scale;
-    }
-  }
+  float g = 0.f;
+  for (int p = 0; p < shares; ++p) g += lane_value(gate_share, p);
   if (lane < a.always) {
-    float g = 0.f;
-    if (!a.always_plain)
-      for (int p = 0; p < shares; ++p) g += z[p * slice + outputs];
     choice[(size_t)t * per_token + a.top + lane] = outputs + lane;
     weight[(size_t)t * per_token + a.top + lane] = a.always_plain ? 1.f : 1.f / (1.f + expf(-g));
   }
+}
+
+// The sum over a wavefront's lanes up to this one: within 16 lanes, then the last of 16 to the next 16, then the last of 32 to the next 32.
+__device__ __forceinline__ int sum_to_lane(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  return x + __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
 }
 
 // experts: of the grouped product, the last `always` of which have every token's row, in the tokens' order.
@@ -156,24 +213,17 @@ __global__ __launch_bounds__(kPlanChunk) void route_plan_kernel(nf_routing r, in
   __syncthreads();
   // exclusive sums over the experts: rows, tiles
   const int before = ahead[tid], c = count[tid] + before, tiles = (c + r.tile_rows - 1) / r.tile_rows;
-  int rows_to = c, tiles_to = tiles;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int a = __shfl_up(rows_to, d, 64), b = __shfl_up(tiles_to, d, 64);
-    if (lane >= d) {
-      rows_to += a;
-      tiles_to += b;
-    }
-  }
+  int rows_to = sum_to_lane(c), tiles_to = sum_to_lane(tiles);
   if (lane == 63) {
     wave_rows[wave] = rows_to;
     wave_tiles[wave] = tiles_to;
   }
   __syncthreads();
-  for (int w = 0; w < wave; ++w) {
-    rows_to += wave_rows[w];
-    tiles_to += wave_tiles[w];
-  }
+  if (wave * 64 < experts)  // no one reads what the others have
+    for (int w = 0; w < wave; ++w) {
+      rows_to += wave_rows[w];
+      tiles_to += wave_tiles[w];
+    }
   first[tid] = rows_to - c + before;  // nobody's entries are ahead of another's at the experts of every token
   if (blockIdx.x == 0 && tid < experts) {
     const int tile0 = tiles_to - tiles;
