@@ -17,7 +17,8 @@
 //   recur_chunk_scan_kernel   the state that enters each chunk (one pass over the chunks per element), and
 //                             the state the request leaves behind;
 //   recur_chunk_out_kernel    every chunk's outputs from its entering state.
-// Inside a chunk the state lives in MFMA accumulators (v_mfma_f32_16x16x4_f32: products and sums in fp32)
+// Heads of 128 x 128 under fixed decays and of 64 x 64 under decays of the token have forms of their own in bf16 (recurrence_fixed.h, recurrence_token.h); in this one,
+// the general one, inside a chunk the state lives in MFMA accumulators (v_mfma_f32_16x16x4_f32: products and sums in fp32)
 // and 16 tokens are taken at a time:  o = (decayed q) S + A v,  S <- decays * S + (decayed k)^T v,  A[i][j] =
 // q_i . k_j times the decay between the two.  An accumulator's rows 4g + r are the k index g of the r-th
 // MFMA that multiplies by it, so S and A are operands where they lie.  A token's own decays enter as
