@@ -691,6 +691,18 @@ def _call(name, *args):
     _check(getattr(lib(), name)(*args), name)
 
 
+def _typed(dtype, **tensors):
+    """The kernel is told one element type for all of these (None: not given): of another it would read or write past a tensor's end."""
+    for name, t in tensors.items():
+        if t is not None and t.dtype != dtype:
+            raise TypeError(f"{name} is {t.dtype}, not {dtype}")
+
+
+def _of(layout):
+    """The element type of a layout, for _typed."""
+    return torch.bfloat16 if layout.dtype == BF16 else torch.float32
+
+
 ACT_NONE, ACT_SQUARED_RELU, ACT_SILU, ACT_GELU, ACT_GATED = 0, 1, 2, 3, 4
 SCORES_SOFTMAX, SCORES_SIGMOID = 0, 1
 NORM_NONE, NORM_RMS, NORM_LAYER = 0, 1, 2
@@ -699,6 +711,7 @@ NORM_NONE, NORM_RMS, NORM_LAYER = 0, 1, 2
 def gemm_nk(a, b, squared_relu=False, workspace=None, act=None, bias=None):
     """act(a . b^T + bias), b [N, K], in the type of a (bf16: an activation or a bias, not both)."""
     act = act or (ACT_SQUARED_RELU if squared_relu else ACT_NONE)
+    _typed(a.dtype, b=b, bias=bias)
     M, K = a.shape
     N = b.shape[0]
     d = torch.empty((M, N), dtype=a.dtype, device=a.device)
@@ -718,6 +731,7 @@ def gemm_nk(a, b, squared_relu=False, workspace=None, act=None, bias=None):
 
 def gemm_nk_sums(a, b, max_shares=1):
     """fp32 sums [shares, M, N] of a . b^T (bf16 operands)."""
+    _typed(torch.bfloat16, a=a, b=b)
     M, K = a.shape
     N = b.shape[0]
     shares = lib().nf_gemm_nk_sums_shares(M, N, K, max_shares)
@@ -728,6 +742,7 @@ def gemm_nk_sums(a, b, max_shares=1):
 
 def embed_rows(tokens, positions, embed, pos, scale=1.0):
     """(fp32 rows, rows in the tables' type); the embedding is multiplied by scale"""
+    _typed(embed.dtype, pos=pos)
     T, ld = tokens.numel(), embed.shape[1]
     x = torch.empty((T, ld), dtype=torch.float32, device=embed.device)
     act = torch.empty((T, ld), dtype=embed.dtype, device=embed.device)
@@ -736,6 +751,7 @@ def embed_rows(tokens, positions, embed, pos, scale=1.0):
 
 
 def norm(kind, weight=None, bias=None, eps=0.0) -> Norm:
+    _typed(torch.float32, weight=weight, bias=bias)
     n = Norm(kind, _p(weight), _p(bias), eps)
     n.tensors = (weight, bias)      # the struct holds addresses only
     return n
@@ -743,11 +759,15 @@ def norm(kind, weight=None, bias=None, eps=0.0) -> Norm:
 
 def residual_rows(y, x, act, width, y_norm=None, next_norm=None, y_scale=1.0, add=None, table=None, tokens=None, table_scale=1.0):
     """x += y_scale * y_norm(y) in place; y [shares, T, ld] fp32 or [T, ld] bf16 (or None); then x += add + table_scale * table[tokens];
-    act (or None) receives next_norm(x) in its type."""
+    act (or None) receives next_norm(x) in its type, which is the table's too."""
+    _typed(torch.float32, x=x, add=add)
+    kind = act if act is not None else table
+    if kind is not None:
+        _typed(kind.dtype, table=table)
     shares = y.shape[0] if y is not None and y.dim() == 3 else 1
     T, ld = x.shape
     a = ResidualArgs(rows=T, width=width, ld=ld, y_dtype=F32 if y is None else _dt(y), shares=shares, y=_p(y), y_norm=y_norm or Norm(),
-                     next=next_norm or Norm(), y_scale=y_scale, x=_p(x), dtype=_dt(act) if act is not None else F32, act=_p(act), add=_p(add),
+                     next=next_norm or Norm(), y_scale=y_scale, x=_p(x), dtype=_dt(kind) if kind is not None else F32, act=_p(act), add=_p(add),
                      table=_p(table), tokens=_p(tokens), table_scale=table_scale)
     _call("nf_residual_rows", C.byref(a), _stream())
 
@@ -755,6 +775,8 @@ def residual_rows(y, x, act, width, y_norm=None, next_norm=None, y_scale=1.0, ad
 def mixture_rows(y, routing, top, identity, x, act, width, next_norm=None, y_scale=1.0, y_norm=None, plain=False):
     """x += y_scale * y_norm of the weighted sum (plain: the sum) of every token's sorted rows of y [sorted, ld] and of identity
     [T, ld] (or None)."""
+    _typed(torch.float32, x=x)
+    _typed(y.dtype, identity=identity, act=act)
     T, ld = x.shape
     if plain:
         routing = Routing.from_buffer_copy(routing)
@@ -765,6 +787,7 @@ def mixture_rows(y, routing, top, identity, x, act, width, next_norm=None, y_sca
 
 
 def norm_rows(x, index, n, width, dtype):
+    _typed(torch.float32, x=x)
     out = torch.empty((x.shape[0] if index is None else index.numel(), x.shape[1]), dtype=dtype, device=x.device)
     _call("nf_norm_rows", _dt(out), _p(x), _p(index), C.byref(n), _p(out), out.shape[0], width, x.shape[1], _stream())
     return out
@@ -781,10 +804,13 @@ def gather_norm_rows(x, index, weight, width, eps, dtype):
 
 def gated_norm_rows(o, g, weight, width, eps):
     """RMS norm of the rows of o, times weight and sigmoid(g), in place."""
+    _typed(o.dtype, g=g)
+    _typed(torch.float32, weight=weight)
     _call("nf_gated_norm_rows", _dt(o), _p(o), o.shape[1], _p(g), g.shape[1], _p(weight), o.shape[0], width, eps, _stream())
 
 
 def token_gate_rows(sums, tokens, table, col0, dim):
+    _typed(torch.float32, sums=sums)
     out = torch.empty(sums.shape[1:], dtype=table.dtype, device=sums.device)
     _call("nf_token_gate_rows", _dt(table), _p(sums), sums.shape[0], _p(tokens), _p(table), table.shape[1], col0, dim, _p(out),
           sums.shape[1], sums.shape[2], _stream())
@@ -794,6 +820,7 @@ def token_gate_rows(sums, tokens, table, col0, dim):
 def route(z, outputs, experts, top, correction, scale, tile_rows, groups=1, keep_groups=1, always=0, scores=SCORES_SOFTMAX, always_plain=False):
     """(Routing, dict of its tensors) of router outputs z [shares, T, ld] fp32; always: experts of every token behind the chosen
     ones, weighed by the column after the outputs (always_plain: by 1)."""
+    _typed(torch.float32, z=z, correction=correction)
     shares, T, ld = z.shape
     n, e = T * (top + always), experts + always
     i32 = lambda k: torch.full((k,), -7, dtype=torch.int32, device=z.device)
@@ -810,6 +837,7 @@ def route(z, outputs, experts, top, correction, scale, tile_rows, groups=1, keep
 
 def gemm_grouped_heads(a, b, d, a_group, d_group):
     """D_g = A_g . B_g^T for b [groups, N, K]: all rows of a, columns from g * a_group, to d's from g * d_group."""
+    _typed(a.dtype, b=b, d=d)
     g, N, Kd = b.shape
     args = GroupedGemmArgs(dtype=_dt(a), groups=g, M=a.shape[0], N=N, K=Kd, a=_p(a), lda=a.shape[1], a_group=a_group, b=_p(b), d=_p(d),
                            ldd=d.shape[1], d_group=d_group)
@@ -820,6 +848,8 @@ def gemm_grouped_heads(a, b, d, a_group, d_group):
 def gemm_grouped_experts(a, b, d, routing, max_rows, gather, act=ACT_NONE, weigh=False, gated=(1.0, 0.0, None)):
     """Sorted rows d = act(A . B_e^T): a holds tokens (gather) or sorted rows.  weigh: the product's rows are multiplied by their
     weights first; gated: slope, shift and limits per expert of ACT_GATED."""
+    _typed(a.dtype, b=b, d=d)
+    _typed(torch.float32, limits=gated[2])
     e, N, Kd = b.shape
     args = GroupedGemmArgs(dtype=_dt(a), act=act, groups=e, M=a.shape[0], N=N, K=Kd, a=_p(a), lda=a.shape[1], b=_p(b), d=_p(d),
                            ldd=d.shape[1], routing=routing, gather=int(gather), max_rows=max_rows, weigh=int(weigh),
@@ -829,6 +859,7 @@ def gemm_grouped_experts(a, b, d, routing, max_rows, gather, act=ACT_NONE, weigh
 
 
 def token_shift(x, shift_state, mu, input_indptr, rev_input_indptr, positions, state_slots, dtype):
+    _typed(torch.float32, x=x, shift_state=shift_state, mu=mu)
     T, ld = x.shape
     out = torch.empty((mu.shape[0], T, ld), dtype=dtype, device=x.device)
     _call("nf_token_shift", _dt(out), _p(x), _p(shift_state), _p(mu), _p(out), mu.shape[0], _p(input_indptr),
@@ -837,12 +868,14 @@ def token_shift(x, shift_state, mu, input_indptr, rev_input_indptr, positions, s
 
 
 def tanh_rows(sums, dtype):
+    _typed(torch.float32, sums=sums)
     out = torch.empty(sums.shape[1:], dtype=dtype, device=sums.device)
     _call("nf_tanh_rows", _dt(out), _p(sums), sums.shape[0], _p(out), sums.shape[1], sums.shape[2], _stream())
     return out
 
 
 def argmax_f32(logits, cols=None):
+    _typed(torch.float32, logits=logits)
     out = torch.empty((logits.shape[0],), dtype=torch.int32, device=logits.device)
     _call("nf_argmax_f32", _p(logits), _p(out), logits.shape[0], cols or logits.shape[1], logits.shape[1], _stream())
     return out
@@ -860,6 +893,7 @@ def kv_pool(layout: KVLayout, pages, device="cuda"):
 
 def rotation(table=None, dims=0, interleaved=False) -> Rotation:
     """table: fp32 [positions, dims / 2, 2] of (cos, sin)."""
+    _typed(torch.float32, table=table)
     r = Rotation(_p(table) if table is not None else None, dims, int(interleaved))
     r.tensors = (table,)            # the struct holds addresses only
     return r
@@ -867,6 +901,7 @@ def rotation(table=None, dims=0, interleaved=False) -> Rotation:
 
 def short_conv(weight, state, input_indptr, state_slots) -> ShortConv:
     """weight [taps, columns], state [slots, taps - 1, columns] in the type of the projected rows."""
+    _typed(weight.dtype, state=state)
     c = ShortConv(weight.shape[0], _p(weight), _p(state), _p(input_indptr), _p(state_slots))
     c.tensors = (weight, state, input_indptr, state_slots)      # the struct holds addresses only
     return c
@@ -876,6 +911,8 @@ def qkv_append(layout, proj, cols, q_norm, k_norm, eps, rot, pool, kv_indptr, kv
                value_norm=False, value_rot=None):
     """Returns the normed, rotated queries [T, heads * maps, k_pad]; keys and values go to the pool's pages, what a convolution
     needs of these rows to its state."""
+    _typed(_of(layout), proj=proj, pool=pool, conv_weight=getattr(conv, "tensors", (None,))[0])
+    _typed(torch.float32, q_norm=q_norm, k_norm=k_norm)
     T = proj.shape[0]
     q = torch.empty((T, layout.heads * layout.maps, layout.k_pad), dtype=proj.dtype, device=proj.device)
     _call("nf_qkv_append", C.byref(layout), _p(proj), proj.shape[1], *cols, _p(q_norm), _p(k_norm), eps, C.byref(rot),
@@ -891,6 +928,8 @@ def window_attention(layout, q, pool, batch, *, window, keep_first, scale, sink=
                      map_weight=0.0, head_eps=None, chunk=0, out_rot=None):
     """batch: dict of device arrays input_indptr, kv_indptr, kv_indices, rev_input_indptr, positions; the first
     `decode` requests have one row each.  Returns [T, heads * vdim]."""
+    _typed(_of(layout), q=q, pool=pool, gate=gate)
+    _typed(torch.float32, sink=sink)
     T = q.shape[0]
     out = torch.zeros((T, layout.heads * layout.vdim), dtype=q.dtype, device=q.device)
     n_req = batch["input_indptr"].numel() - 1
@@ -918,6 +957,8 @@ def latent_pool(layout: LatentLayout, pages, device="cuda"):
 
 def latent_append(layout, proj, cols, weight, eps, rot, q, pool, batch):
     """cols: (rotated query parts, latent); q [T, heads, row_ld] receives its columns from rank_pad on."""
+    _typed(_of(layout), proj=proj, q=q, pool=pool)
+    _typed(torch.float32, weight=weight)
     _call("nf_latent_append", C.byref(layout), _p(proj), proj.shape[1], *cols, _p(weight), eps, C.byref(rot), _p(q), _p(pool),
           *(_p(batch[n]) for n in ("kv_indptr", "kv_indices", "rev_input_indptr", "positions")), proj.shape[0], proj.shape[0], _stream())
 
@@ -925,6 +966,7 @@ def latent_append(layout, proj, cols, weight, eps, rot, q, pool, batch):
 def latent_expand(layout, dim_pad, vdim_pad, weight, pool, batch, req_begin, req_end, max_pages):
     """Keys and values of all heads of the requests' positions: (KVLayout, pages, page_ids); weight [heads * (dim_pad + vdim_pad),
     rank_pad], keys first."""
+    _typed(_of(layout), pool=pool, weight=weight)
     H = layout.heads
     kv = kv_layout(pool.dtype, H, H, dim_pad + layout.rot_dim, vdim_pad)
     new = lambda *shape: torch.full(shape, 3.0, dtype=pool.dtype, device=pool.device)
@@ -941,6 +983,7 @@ def latent_expand(layout, dim_pad, vdim_pad, weight, pool, batch, req_begin, req
 
 
 def latent_queries(kv, dim_pad, proj, q_col, rot_dim, rot, positions, row_begin, rows):
+    _typed(_of(kv), proj=proj)
     q = torch.zeros((proj.shape[0], kv.heads, kv.k_pad), dtype=proj.dtype, device=proj.device)
     _call("nf_latent_queries", C.byref(kv), dim_pad, _p(proj), proj.shape[1], q_col, rot_dim, C.byref(rot), _p(positions), _p(q), row_begin, rows,
           _stream())
@@ -949,6 +992,7 @@ def latent_queries(kv, dim_pad, proj, q_col, rot_dim, rot, positions, row_begin,
 
 def latent_attention(layout, q, pool, batch, *, scale, decode=0, workspace=True, window=0):
     """q [T, heads, row_ld]; returns [T, heads, rank_pad]."""
+    _typed(_of(layout), q=q, pool=pool)
     T = q.shape[0]
     out = torch.zeros((T, layout.heads, layout.rank_pad), dtype=q.dtype, device=q.device)
     n_req = batch["input_indptr"].numel() - 1
@@ -969,6 +1013,8 @@ def linear_recurrence(kind, q, k, v, g, heads, dim, vdim, state, batch, *, eps, 
                       shift_state=None):
     """q, k, v, g: 2-d tensors of rows; batch: device arrays input_indptr, positions, state_slots.  Returns
     [T, heads * vdim]; the state is updated in place."""
+    _typed(q.dtype, k=k, v=v, g=g)
+    _typed(torch.float32, state=state, log2_decay=log2_decay, z=z, w0=w0, u=u, norm_weight=norm_weight, shift_x=shift_x, shift_state=shift_state)
     T = q.shape[0]
     out = torch.zeros((T, heads * vdim), dtype=q.dtype, device=q.device)
     n_req = batch["input_indptr"].numel() - 1
