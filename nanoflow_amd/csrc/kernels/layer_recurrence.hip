@@ -539,7 +539,10 @@ __global__ __launch_bounds__(256) void recur_chunk_scan_kernel(nf_recurrence_arg
     float4_t cur{0.f, 0.f, 0.f, 0.f};
     if (a.positions[row0] != 0)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) cur[r] = state[(size_t)r * pd.vp];
+      for (int r = 0; r < 4; ++r) {
+        cur[r] = state[(size_t)r * pd.vp];
+        if constexpr (kForm && KIND == NF_RECURRENCE_FIXED_DECAY) cur[r] = __builtin_canonicalizef(cur[r]);  // NaN shows in the upper half, all that `split` has of it
+      }
     constexpr int kAhead = 4;  // loads do not depend on the running state
     for (int c0 = 0; c0 < chunks; c0 += kAhead) {
       float4_t add[kAhead], f[kAhead];

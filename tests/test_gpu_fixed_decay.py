@@ -90,3 +90,10 @@ def test_what_is_not_finite_stays_with_its_tokens(bad, row):
     qkv[:, 0] = qkv[:, 0].abs() + 1
     got, _ = run(qkv, state, [(4, 200)], [0.9], 1.0, 1.0, 0)
     assert bool((got[:, 0, 5].isnan() if bad != bad else got[:, 0, 5] == bad).all()) and got[:, 0, :5].isfinite().all()
+
+
+def test_a_nan_of_its_lowest_bit_is_no_infinity():
+    qkv, state = operands([(4, 40)], 1)
+    state.view(torch.int32)[0, 0, 3, 5] = 0x7f800001
+    got, st = run(qkv, state, [(4, 40)], [0.9], 1.0, 1.0, 0)
+    assert got[:, 0, 5].isnan().all() and st[0, 0, 3, 5].isnan() and got[:, 0, :5].isfinite().all()
