@@ -9,7 +9,9 @@
 // eight bits whose sum it is (`split`), so their products are exact as well and the sums are fp32, as they were: three MFMAs for one, at an eighth of its cost
 // per token.  2047 tokens of 16 heads (us, fp32 form -> this): chunk states 18.8 -> 11.1, scan 13.5 -> 9.5 over half as many states, outputs 35.5 -> 17.0; the
 // states' error against 64 bits 9.6e-8 -> 7.0e-8.
-// A token's infinities and NaN reach the tokens of its 16 and later ones, as in the fp32 form.
+// A token's infinities and NaN reach the tokens of its 16 and later ones, as in the fp32 form.  But an infinity against a number of which eight bits are the whole
+// meets zeros as that number's other parts, and tokens of a whole chunk meet one by one: so a wavefront whose sums are not all finite takes the others again 16 tokens
+// at a time in fp32 (`fixed_steps`), as the fp32 form does.  (The figures are without that check, 40 vector instructions a wavefront and phase.)
 
 namespace nf {
 
@@ -50,6 +52,21 @@ __device__ __forceinline__ float4_t mfma_bf16(const A& a, const B& b, float4_t c
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+// Whether all sums of the wavefront are finite; and x with what is not as y has it.
+template <int n>
+__device__ __forceinline__ bool all_finite(const float4_t (&x)[n]) {
+  float4_t zero{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < n; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) zero[r] = __builtin_fmaf(x[i][r], 0.f, zero[r]);
+  return !__any(zero[0] + zero[1] + (zero[2] + zero[3]) != 0.f);  // true of a NaN
+}
+__device__ __forceinline__ void mend(float4_t& x, const float4_t& y) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) x[r] = fabsf(x[r]) < INFINITY ? x[r] : y[r];
+}
+
 // Rows of 128 bf16 in LDS, 16 chunks of 16 bytes permuted within a row by its number in 16: a chunk of 16 neighbouring rows, and 32 bytes of 16 rows
 // that a transposing read takes, lie in different banks.
 struct FixedTile {
@@ -66,6 +83,9 @@ struct FixedTile {
       load16_to_lds(r, row < n ? off : kOob, __builtin_amdgcn_readfirstlane(lds + (i * 8 + wave) * 1024));
     }
   }
+  static __device__ __forceinline__ float one(const uint8_t* tile, int row, int col) {
+    return bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(tile + chunk(row, col >> 3) + (col & 7) * 2));
+  }
   // What an MFMA operand of four tokens each is made of: tokens first .. first + 3 of the lane's column of 16-column unit u; the lane group's
   // lanes read four rows of 32 bytes between them.
   static __device__ __forceinline__ short4_t column(const uint8_t* tile, int first, int u, int i16) {
@@ -81,6 +101,28 @@ __device__ __forceinline__ void fixed_place(int f4, int* k, int* c) {
   const int lane = (f4 >> 1) & 63, tile = f4 >> 7;
   *k = (tile & 3) * 32 + (f4 & 1) * 16 + (lane >> 4) * 4;
   *c = (tile >> 2) * 16 + (lane & 15);
+}
+
+// A chunk as the fp32 form takes it, for 16 columns of v from `col` on: S [row of k 16 kt + 4 lq + r][column l16] before the 16 tokens from t0 on, and after
+// them; outputs(t0, S) has the former.
+template <class F>
+__device__ __forceinline__ void fixed_steps(const nf_recurrence_args& a, const uint8_t* kt, const uint8_t* vt, float ld2, int n, int col, int l16, int lq, float4_t (&S)[8],
+                                            F&& outputs) {
+#pragma unroll 1
+  for (int t0 = 0; t0 < n; t0 += 16) {
+    outputs(t0, S);
+    const int some = min(16, n - t0);
+    const float keep = __builtin_amdgcn_exp2f((float)some * ld2);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) S[i] *= keep;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 4 * lq + r;
+      const float v = FixedTile::one(vt, t0 + t, col + l16), f = t < some ? __builtin_amdgcn_exp2f((float)(some - 1 - t) * ld2) : 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(FixedTile::one(kt, t0 + t, i * 16 + l16) * a.k_scale * f, v, S[i], 0, 0, 0);
+    }
+  }
 }
 
 // What a chunk adds to the state.  A wavefront has 16 columns of v, all rows of k.
@@ -117,6 +159,14 @@ __global__ __launch_bounds__(512) void recur_fixed_state_kernel(nf_recurrence_ar
       for (int p = 2; p >= 0; --p) S[i] = mfma_bf16(k8, w.part[p], S[i]);
     }
   }
+  if (!all_finite(S)) {
+    float4_t again[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) again[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+    fixed_steps(a, kt, vt, ld2, ch.n, wave * 16, l16, lq, again, [](int, const float4_t (&)[8]) {});
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mend(S[i], again[i]);
+  }
   float* dst = (float*)a.workspace + ((size_t)ch.slot * a.heads + h) * kFixedDim * kFixedDim;
 #pragma unroll
   for (int i = 0; i < 8; ++i) *reinterpret_cast<float4_t*>(dst + ((size_t)(wave * 4 + i / 2) * 64 + lane) * 8 + (i & 1) * 4) = S[i];
@@ -141,13 +191,14 @@ __global__ __launch_bounds__(512) void recur_fixed_out_kernel(nf_recurrence_args
   FixedTile::load((const uint16_t*)a.v + (size_t)ch.row0 * a.v_ld + h * kFixedDim, a.v_ld, ch.n, lds0 + 2 * FixedTile::bytes, wave, lane);
   const float ld2 = a.log2_decay[h];
   const float* src = (const float*)a.workspace + ((size_t)ch.slot * a.heads + h) * kFixedDim * kFixedDim;
+  auto raw_at = [&](int c, int b, int e) { return *reinterpret_cast<const float4_t*>(src + ((size_t)((w4 * 2 + c) * 4 + b) * 64 + lane) * 8 + e * 4); };
   float4_t raw[2][4][2];
 #pragma unroll
   for (int c = 0; c < 2; ++c)
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int e = 0; e < 2; ++e) raw[c][b][e] = *reinterpret_cast<const float4_t*>(src + ((size_t)((w4 * 2 + c) * 4 + b) * 64 + lane) * 8 + e * 4);
+      for (int e = 0; e < 2; ++e) raw[c][b][e] = raw_at(c, b, e);
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
   const bool some = group * 64 < ch.n;  // this group has tokens
@@ -241,8 +292,41 @@ __global__ __launch_bounds__(512) void recur_fixed_out_kernel(nf_recurrence_args
         }
       }
     }
-    __syncthreads();
+    if (jb == 0) __syncthreads();
   }
+  if (some)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      if (all_finite(o[c])) continue;
+      const int col = (w4 * 2 + c) * 16;
+      float4_t S[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) S[i] = raw_at(c, i >> 1, i & 1);
+      fixed_steps(a, kt, vt, ld2, min(ch.n, group * 64 + 64), col, l16, lq, S, [&](int t0, const float4_t (&S)[8]) {
+        if (t0 < group * 64) return;
+        const int n = min(16, ch.n - t0);
+        float4_t at{0.f, 0.f, 0.f, 0.f}, y{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float q = FixedTile::one(qt, t0 + l16, i * 16 + 4 * lq + r);
+            at = __builtin_amdgcn_mfma_f32_16x16x4f32(FixedTile::one(kt, t0 + l16, i * 16 + 4 * lq + r) * a.k_scale, q, at, 0, 0, 0);
+            y = __builtin_amdgcn_mfma_f32_16x16x4f32(S[i][r], q, y, 0, 0, 0);
+          }
+        y *= __builtin_amdgcn_exp2f((float)(l16 + 1) * ld2);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = 4 * lq + r;
+          const float x = j <= l16 && l16 < n ? at[r] * __builtin_amdgcn_exp2f((float)(l16 - j) * ld2) : 0.f;
+          y = __builtin_amdgcn_mfma_f32_16x16x4f32(FixedTile::one(vt, t0 + j, col + l16), x, y, 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (t == (t0 >> 4 & 3)) mend(o[c][t], y);
+      });
+    }
+  __syncthreads();
 
   // ---- through LDS, where q was: a token's 128 columns are written together
 #pragma unroll

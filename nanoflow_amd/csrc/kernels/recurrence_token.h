@@ -7,7 +7,10 @@
 // L, the sums of log2 decays, are scans over the lanes of a wavefront.  Within a block the scores are products of q 2^(L before i) and k 2^-(L through j), both from the
 // block's start, or, where some channel's L is below -100, worked out one by one.  Between blocks no factor is above 1: k has decayed to the end of its own block,
 // q from the start of its own, and the blocks between the two multiply q.  Scores and the state's part are MFMAs in fp32; the values are exact in bf16, so scores and
-// decayed keys are taken apart into three bf16 numbers each (recurrence_fixed.h) where they meet them, and nothing is rounded that was not.
+// decayed keys are taken apart into three bf16 numbers each (recurrence_fixed.h) where they meet them, and nothing is rounded that was not.  Sums that are not
+// finite are taken again block after block in fp32, for the reasons given there: they are then what the general form's steps of 16 tokens leave.  (Its outputs take fewer
+// where a channel decays below 2^-100 over 16; an infinity that it still has there is NaN in its states from the next chunk on.  The
+// figures below are without the check, 20 vector instructions a wavefront.)
 // 2019 tokens of 32 heads in two requests (us, general form -> this): chunk states 15.2 -> 11.3, scan 8.4 (bytes), outputs 35.8 -> 23.5; the states' error against
 // 64 bits 7.3e-8 -> 6.2e-8.  The outputs are bound by what their wavefronts issue (1250 vector and 112 matrix instructions for 16 tokens), little of it side
 // by side; the same on 8 wavefronts and chunks of 128 took 32: the last block has seven before it.
@@ -51,6 +54,10 @@ struct TokenTile {
   // results give every lane 16 columns beside each other.
   static __device__ __forceinline__ short4_t column(const uint8_t* tile, int first, int u, int i16) {
     return lds_read_tr16(tile + piece(first + (i16 >> 2), 2 * u + ((i16 & 3) >> 1)) + (i16 & 1) * 8);
+  }
+  static __device__ __forceinline__ int spread_column(int u, int i16) { return 16 * (i16 >> 2) + 4 * u + (i16 & 3); }
+  static __device__ __forceinline__ float one(const uint8_t* tile, int row, int col) {
+    return bf16_bits_to_f32(*reinterpret_cast<const uint16_t*>(tile + piece(row, col >> 3) + (col & 7) * 2));
   }
   static __device__ __forceinline__ short4_t spread(const uint8_t* tile, int first, int u, int i16) {
     return lds_read_tr16(tile + piece(first + (i16 >> 2), 2 * (i16 & 3) + (u >> 1)) + (u & 1) * 8);
@@ -122,6 +129,36 @@ __global__ __launch_bounds__(kTokenChunk * 4, 4) void recur_token_state_kernel(n
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int c = 0; c < 4; ++c) S[c] = mfma_bf16(w[s].part[p], v8[s][c], S[c]);
+  if (!all_finite(S)) {
+    // Token after token, its decay worked out again: what is kept in registers for this would cost every launch a workgroup a CU.
+    float4_t again[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) again[c] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int blk = 0; blk < kBlocks; ++blk) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float keep = __builtin_amdgcn_exp2f(__shfl(sum, blk * 16 + 4 * g + r, 64));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) again[c][r] *= keep;
+      }
+      float later = 0.f;
+#pragma unroll 1
+      for (int i = 15; i >= 0; --i) {  // the lanes of a group have its block's tokens
+        const int t = g * 16 + i;
+        const size_t row = ch.row0 + min(t, ch.n - 1);
+        float z = a.z[row * a.z_ld + h * kTokenDim + channel];
+        for (int s = 1; s < a.z_shares; ++s) z += a.z[((size_t)s * a.total_rows + row) * a.z_ld + h * kTokenDim + channel];
+        const float k = TokenTile::one(kt, t, channel) * __builtin_amdgcn_exp2f(later);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          again[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(g == blk ? k : 0.f, g == blk ? TokenTile::one(vt, t, TokenTile::spread_column(c, l16)) : 0.f, again[c], 0, 0, 0);
+        later += t < ch.n ? log2_decay_of(z, a.w0[h * kTokenDim + channel]) : 0.f;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) mend(S[c], again[c]);
+  }
   float* dst = (float*)a.workspace + ((size_t)ch.slot * a.heads + h) * kTokenDim * kTokenDim;
 #pragma unroll
   for (int c = 0; c < 4; ++c) *reinterpret_cast<float4_t*>(dst + ((size_t)(c * 4 + g) * 64 + wave * 16 + l16) * 4) = S[c];
@@ -325,6 +362,38 @@ __global__ __launch_bounds__(kTokenChunk * 4, 3) void recur_token_out_kernel(nf_
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int c = 0; c < 4; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[c][r], now[4 * b + r], o[c], 0, 0, 0);
+  }
+
+  if (!all_finite(o)) {
+#pragma unroll 1
+    for (int c = 0; c < 4; ++c) {
+      const int col_v = TokenTile::spread_column(c, l16);
+      float4_t s[4], y{0.f, 0.f, 0.f, 0.f};  // s: rows 16 g + 4 kt + r of k, column col_v; y: columns 16 g + 4 c + r of the token l16
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) s[kt] = *reinterpret_cast<const float4_t*>(lds + L::state + (c * 4 + kt) * 1024 + lane * 16);
+#pragma unroll 1
+      for (int b = 0; b < blk; ++b)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+          const float4_t total = *reinterpret_cast<const float4_t*>(lds + L::totals + b * 256 + g * 64 + kt * 16);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[kt][r] *= __builtin_amdgcn_exp2f(total[r]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float k = *reinterpret_cast<const float*>(lds + L::keys + (b * 4 + kt) * 1024 + ((l16 >> 2) * 16 + 4 * g + r) * 16 + (l16 & 3) * 4);
+            s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, TokenTile::one(lds, b * 16 + 4 * g + r, col_v), s[kt], 0, 0, 0);
+          }
+        }
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y = __builtin_amdgcn_mfma_f32_16x16x4f32(s[kt][r], q[4 * kt + r], y, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y = __builtin_amdgcn_mfma_f32_16x16x4f32(TokenTile::one(lds, blk * 16 + 4 * g + r, col_v), own[r], y, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i == c) mend(o[i], y);
+    }
   }
 
   // ---- norm over the head's columns, gate

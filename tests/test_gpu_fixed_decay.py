@@ -92,6 +92,28 @@ def test_what_is_not_finite_stays_with_its_tokens(bad, row):
     assert bool((got[:, 0, 5].isnan() if bad != bad else got[:, 0, 5] == bad).all()) and got[:, 0, :5].isfinite().all()
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf")])
+@pytest.mark.parametrize("row", [0, 16, 50, 96, 127, 130, 199])      # 16, 96: the first of sixteen; 127, 199: a chunk's last, whose key the state takes undecayed
+@pytest.mark.parametrize("what", ["q", "k", "v", "state"])
+@pytest.mark.parametrize("k_scale", [1.0, 0.31])
+def test_infinities_are_those_of_the_general_form(what, row, bad, k_scale):
+    """Operands of eight significant bits or fewer beside them: all of q, k and v, and every fourth column of the state."""
+    reqs, heads = [(4, 200)], 2
+    qkv, state = operands(reqs, heads)
+    state[:, :, :, ::4] = state[:, :, :, ::4].bfloat16().float()
+    if what == "state":
+        state[0, 1, row % D, 5] = bad
+    else:
+        qkv[row, "qkv".index(what), 1, 5] = bad
+    got, st = run(qkv, state, reqs, [0.9, 0.97], k_scale, 0.5, 0)
+    want, left = run(qkv, state, reqs, [0.9, 0.97], k_scale, 0.5, 4)
+    assert not want.isfinite().all()
+    for x, y, off in ((got, want, 2.0 ** -7), (st, left, 0.0)):
+        assert torch.equal(x[y.isinf()], y[y.isinf()]) and torch.equal(x.isfinite(), y.isfinite())
+        ok = y.isfinite()
+        assert bool(((x[ok] - y[ok]).abs() <= off * y[ok].abs() + 8e-6 * y[ok].abs().max()).all())
+
+
 def test_a_nan_of_its_lowest_bit_is_no_infinity():
     qkv, state = operands([(4, 40)], 1)
     state.view(torch.int32)[0, 0, 3, 5] = 0x7f800001

@@ -89,3 +89,25 @@ def test_what_is_not_finite_stays_with_its_tokens(bad, row):
     want, left = run(s, reqs, False, 4)
     assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 4e-5 * want.abs().max()).all())
     assert float((st - left).abs().max() / left.abs().max()) < 4e-6
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf")])
+@pytest.mark.parametrize("row", [0, 16, 40, 48, 63, 70, 99])      # 16, 48: the first of sixteen; 63, 99: a chunk's last, whose key the state takes undecayed
+@pytest.mark.parametrize("what", ["q", "k", "v", "state"])
+@pytest.mark.parametrize("gate", [False, True])
+def test_infinities_are_those_of_the_general_form(gate, what, row, bad):
+    """Operands of eight significant bits or fewer beside them: all of q, k and v, and every fourth column of the state."""
+    reqs = [(4, 100)]
+    s = operands(reqs, 2, -2.0)
+    s["state"][:, :, :, ::4] = s["state"][:, :, :, ::4].bfloat16().float()
+    if what == "state":
+        s["state"][0, 1, row % D, 5] = bad
+    else:
+        s["rkvg"]["qkv".index(what), row, 1, 5] = bad
+    got, st = run(s, reqs, gate, 0)
+    want, left = run(s, reqs, gate, 4)
+    assert not want.isfinite().all()
+    for x, y, off in ((got, want, 2.0 ** -7), (st, left, 0.0)):
+        assert torch.equal(x[y.isinf()], y[y.isinf()]) and torch.equal(x.isfinite(), y.isfinite())
+        ok = y.isfinite()
+        assert bool(((x[ok] - y[ok]).abs() <= off * y[ok].abs() + 4e-5 * y[ok].abs().max()).all())
