@@ -41,20 +41,35 @@ def test_eight_wavefronts(nk, M, N, Kd):
         assert torch.equal(sums.double().sum(0), want)
 
 
-@pytest.mark.parametrize("M,N,Kd", [(65, 16392, 2048), (128, 16392, 4096), (129, 32776, 2048), (192, 32776, 2048), (193, 49160, 2048), (256, 49152, 2048)])
-def test_contractions_that_go_round(M, N, Kd):
-    """Column tiles that start K at slabs of their own: every first slab there is, a last column tile that is cut, and the pair."""
+# by the tiles they are computed in on 256 CUs
+ROUND = {"128 x 128": [(65, 16392, 2048), (128, 16392, 4096)], "128 x 256": [(66, 33608, 2048), (128, 65400, 2048)], "160 x 256": [(129, 49864, 2048), (160, 65400, 2048)],
+         "192 x 256": [(161, 49864, 2048), (192, 65400, 2048)], "224 x 256": [(193, 49160, 2048), (224, 65400, 2048)], "256 x 256": [(225, 49864, 2048), (256, 65400, 2048)],
+         "256 x 192": [(129, 32776, 2048), (192, 32776, 4096), (256, 49152, 2048)]}
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M,N,Kd", [s for shapes in ROUND.values() for s in shapes])
+def test_contractions_that_go_round(M, N, Kd, dtype):
+    """Column tiles that start K at slabs of their own: every first slab there is, and a last column tile that is cut."""
     from nanoflow_amd import kernels as K
     assert N * Kd * 2 >= 64 << 20 and (N + 255) // 256 >= Kd // 64
     gen = torch.Generator(device="cuda").manual_seed(M)
-    whole = lambda *shape: torch.randint(-1, 2, shape, generator=gen, device="cuda", dtype=torch.int8)
-    a, b = whole(M, Kd), whole(N, Kd)
-    a16, b16 = a.half(), b.half()
-    want = a16.float() @ b16.float().t()
-    assert want.abs().max() <= 2048
-    guard = torch.full((M + 1, N), 77.0, dtype=torch.float16, device="cuda")
-    K.gemm(a16, b16, b_col_major=True, out=guard[:M])
-    assert torch.equal(guard[:M].float(), want) and (guard[M] == 77.0).all()
-    if M <= 128:
-        u16 = whole(N, Kd).half()
-        assert torch.equal(K.dual_swiglu(a16, b16, u16, b_col_major=True), K.dual_swiglu(a16, b16.t().contiguous(), u16.t().contiguous()))
+    whole = lambda *shape, top=1: torch.randint(-top, top + 1, shape, generator=gen, device="cuda", dtype=torch.int8)
+    cast = lambda t: t.to(getattr(torch, dtype))
+    a, b, c = whole(M, Kd), whole(N, Kd), whole(M, N, top=8)
+    want = a.float() @ b.float().t()
+    assert want.abs().max() <= 1024
+    guard = torch.full((M + 1, N), 77.0, dtype=getattr(torch, dtype), device="cuda")
+    K.gemm(cast(a), cast(b), b_col_major=True, out=guard[:M])
+    assert torch.equal(guard[:M], cast(want)) and (guard[M] == 77.0).all()
+    K.gemm(cast(a), cast(b), Cmat=cast(c), beta=1.0, b_col_major=True, out=guard[:M])
+    assert torch.equal(guard[:M], cast(want + c)) and (guard[M] == 77.0).all()
+
+
+# 128 x 128, and 256 x 128, of both matrices
+@pytest.mark.parametrize("M,N,Kd", [(65, 16392, 2048), (128, 16392, 4096), (129, 49864, 2048), (180, 49864, 2048), (256, 49864, 2048)])
+def test_pairs_that_go_round(M, N, Kd):
+    from nanoflow_amd import kernels as K
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    a, g, u = (torch.randint(-1, 2, shape, generator=gen, device="cuda", dtype=torch.int8).half() for shape in ((M, Kd), (N, Kd), (N, Kd)))
+    assert torch.equal(K.dual_swiglu(a, g, u, b_col_major=True), K.dual_swiglu(a, g.t().contiguous(), u.t().contiguous()))
