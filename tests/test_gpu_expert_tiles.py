@@ -40,12 +40,18 @@ def test_workgroups_that_go_from_tile_to_tile(N, Kd):
     check(MANY, N, Kd, torch.linspace(0.5, 4.0, len(MANY)))
 
 
-@pytest.mark.parametrize("counts", [(0, 1, 16, 33, 49, 10, 65), (3, 0, 65, 0), (0, 0, 0, 5)], ids=str)
+@pytest.mark.parametrize("counts", [(0, 1, 16, 20, 0, 10, 65), (3, 0, 65, 0, 0), (0, 0, 0, 5)], ids=str)
 @pytest.mark.parametrize("N,Kd", [(520, 1600), (1032, 2048), (2048, 1544)])
 def test_last_expert_first(counts, N, Kd):
-    """At most 30 rows an expert: the weight stream goes through the experts from the last one on."""
-    assert sum(counts) <= 30 * len(counts)
+    """Few rows an expert, for this depth, and at most 30: the weight stream goes through the experts from the last one on."""
+    assert N >= 512 and sum(counts) <= min(30, 16 + (Kd - 1536) * 24 // 512) * len(counts)
     check(counts, N, Kd, torch.full((len(counts),), 7.0))
+
+
+@pytest.mark.parametrize("counts", [(64, 65, 1, 0, 20), (64, 65, 2, 0, 20)], ids=["30 rows an expert", "more"])
+def test_either_order_of_experts(counts):
+    """The most rows of which the last expert comes first, and a row more, of which the first one does."""
+    check(counts, 1032, 2048, torch.full((len(counts),), 7.0))
 
 
 def check(counts, N, Kd, limits):
