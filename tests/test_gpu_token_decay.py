@@ -11,11 +11,11 @@ pytestmark = pytest.mark.gpu
 D = 64
 
 
-def operands(reqs, heads, mean, seed=0):
+def operands(reqs, heads, mean, seed=0, shares=2):
     g = torch.Generator(device="cuda").manual_seed(seed)
     T = sum(n for _, n in reqs)
     rn = lambda *s: torch.randn(s, generator=g, device="cuda")
-    return dict(rkvg=rn(4, T, heads, D).bfloat16(), z=rn(2, T, heads, D) * 0.7, w0=rn(heads, D) * 0.3 + mean, u=rn(heads, D), norm=rn(heads, D) * 0.1 + 1,
+    return dict(rkvg=rn(4, T, heads, D).bfloat16(), z=rn(shares, T, heads, D) * 0.7, w0=rn(heads, D) * 0.3 + mean, u=rn(heads, D), norm=rn(heads, D) * 0.1 + 1,
                 state=rn(len(reqs), heads, D, D))
 
 
@@ -35,7 +35,7 @@ def run(s, reqs, gate, pad):
     a = K.RecurrenceArgs(dtype=K.BF16, kind=K.TOKEN_DECAY, heads=heads, dim=D, vdim=D, eps=1e-5, state=st.data_ptr(), out=out.data_ptr(), out_ld=out.shape[1],
                          out_col=8, input_indptr=indptr.data_ptr(), positions=pos.data_ptr(), state_slots=slots.data_ptr(), total_rows=T,
                          workspace=ws.data_ptr(), workspace_bytes=need, q=at[0], k=at[1], v=at[2], g=at[3] if gate else None, q_ld=ld, k_ld=ld, v_ld=ld, g_ld=ld,
-                         z=s["z"].data_ptr(), z_ld=ld, z_shares=2, w0=s["w0"].data_ptr(), u=s["u"].data_ptr(),
+                         z=s["z"].data_ptr(), z_ld=ld, z_shares=len(s["z"]), w0=s["w0"].data_ptr(), u=s["u"].data_ptr(),
                          norm_weight=s["norm"].data_ptr() if gate else None, out_scale=0.5, req_begin=0, req_num=len(reqs), row_begin=0, rows=T)
     assert K.lib().nf_linear_recurrence(C.byref(a), torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
@@ -68,6 +68,18 @@ def test_against_float64_and_the_general_form(reqs, heads, mean, gate):
     want, left = wanted(s, reqs, gate)
     for pad in (0, 4):
         got, st = run(s, reqs, gate, pad)
+        assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 4e-5 * want.abs().max()).all()), pad
+        assert float((st.double() - left).abs().max() / left.abs().max()) < 4e-6, pad
+
+
+# more chunks than the scan requests at once, with a remainder, ahead of another request; the shares of the decays
+@pytest.mark.parametrize("reqs", [[(0, 449), (7, 322)], [(5, 321), (0, 24), (64, 257)]], ids=str)
+@pytest.mark.parametrize("shares", [1, 3])
+def test_many_chunks(reqs, shares):
+    s = operands(reqs, 2, -3.0, shares=shares)
+    want, left = wanted(s, reqs, True)
+    for pad in (0, 4):
+        got, st = run(s, reqs, True, pad)
         assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 4e-5 * want.abs().max()).all()), pad
         assert float((st.double() - left).abs().max() / left.abs().max()) < 4e-6, pad
 
