@@ -537,7 +537,6 @@ __device__ __forceinline__ void gemm_tile(
     auto a_ptr = [&](int stage) { return smem + stage * SM::a_bytes; };
     auto b_ptr = [&](int stage) { return smem + SM::b_ring + stage * NB * SM::b_bytes; };
     auto k_ok_of = [&](int k) { return k * BK + a_kc < K; };
-    auto place = [](int k) { return kTurn ? k * (BK * 2) : 0; };
     // prologue: activations and weights of slab 0, weights of slab 1
     {
       const uint32_t la = a_lds(0), lb0 = b_lds(0), lb1 = b_lds(1);

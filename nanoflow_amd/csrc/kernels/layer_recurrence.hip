@@ -223,6 +223,15 @@ __device__ __forceinline__ ChunkSpan find_chunk(const nf_recurrence_args& a, int
   return {-1, 0, 0, slot};
 }
 
+// Workspace: [chunks][heads] states in fragment order -- tile (kt, vt) of 16 x 16, lane, four rows -- then
+// (TOKEN_DECAY) [chunks][heads][kp] factors.
+__device__ __forceinline__ float* chunk_states(const nf_recurrence_args& a, const RecurrenceDims& pd, int slot, int h) {
+  return (float*)a.workspace + ((size_t)slot * a.heads + h) * pd.kp * pd.vp;
+}
+__device__ __forceinline__ float* chunk_factors(const nf_recurrence_args& a, const RecurrenceDims& pd, int max_chunks, int slot, int h) {
+  return (float*)a.workspace + (size_t)max_chunks * a.heads * pd.kp * pd.vp + ((size_t)slot * a.heads + h) * pd.kp;
+}
+
 }  // namespace nf
 
 #include "recurrence_fixed.h"
@@ -448,15 +457,6 @@ __device__ __forceinline__ void update_state(float4_t (&S)[NKT][NVT], const Chun
       for (int r = 0; r < 4; ++r) S[kt][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[r], vr[vt][r], S[kt][vt], 0, 0, 0);
     }
   }
-}
-
-// Workspace: [chunks][heads] states in fragment order -- tile (kt, vt) of 16 x 16, lane, four rows -- then
-// (TOKEN_DECAY) [chunks][heads][kp] factors.
-__device__ __forceinline__ float* chunk_states(const nf_recurrence_args& a, const RecurrenceDims& pd, int slot, int h) {
-  return (float*)a.workspace + ((size_t)slot * a.heads + h) * pd.kp * pd.vp;
-}
-__device__ __forceinline__ float* chunk_factors(const nf_recurrence_args& a, const RecurrenceDims& pd, int max_chunks, int slot, int h) {
-  return (float*)a.workspace + (size_t)max_chunks * a.heads * pd.kp * pd.vp + ((size_t)slot * a.heads + h) * pd.kp;
 }
 
 // The bound of two workgroups a CU keeps the state in VGPRs: with more room the compiler moves it to accumulation

@@ -167,7 +167,7 @@ __global__ __launch_bounds__(512) void recur_fixed_state_kernel(nf_recurrence_ar
 #pragma unroll
     for (int i = 0; i < 8; ++i) mend(S[i], again[i]);
   }
-  float* dst = (float*)a.workspace + ((size_t)ch.slot * a.heads + h) * kFixedDim * kFixedDim;
+  float* dst = chunk_states(a, {kFixedDim, kFixedDim}, ch.slot, h);
 #pragma unroll
   for (int i = 0; i < 8; ++i) *reinterpret_cast<float4_t*>(dst + ((size_t)(wave * 4 + i / 2) * 64 + lane) * 8 + (i & 1) * 4) = S[i];
 }
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(512) void recur_fixed_out_kernel(nf_recurrence_args
   FixedTile::load((const uint16_t*)a.k + (size_t)ch.row0 * a.k_ld + h * kFixedDim, a.k_ld, ch.n, lds0 + FixedTile::bytes, wave, lane);
   FixedTile::load((const uint16_t*)a.v + (size_t)ch.row0 * a.v_ld + h * kFixedDim, a.v_ld, ch.n, lds0 + 2 * FixedTile::bytes, wave, lane);
   const float ld2 = a.log2_decay[h];
-  const float* src = (const float*)a.workspace + ((size_t)ch.slot * a.heads + h) * kFixedDim * kFixedDim;
+  const float* src = chunk_states(a, {kFixedDim, kFixedDim}, ch.slot, h);
   auto raw_at = [&](int c, int b, int e) { return *reinterpret_cast<const float4_t*>(src + ((size_t)((w4 * 2 + c) * 4 + b) * 64 + lane) * 8 + e * 4); };
   float4_t raw[2][4][2];
 #pragma unroll

@@ -101,10 +101,8 @@ __global__ __launch_bounds__(kTokenChunk * 4, 4) void recur_token_state_kernel(n
   }
   const float beside = __shfl_xor(sum, 16, 64), pair = (g & 1) ? beside + sum : sum + beside, other = __shfl_xor(pair, 32, 64);
   const float after = ((g & 1) ? 0.f : beside) + (g < 2 ? other : 0.f);
-  if (g == 0) {
-    const RecurrenceDims pd{kTokenDim, kTokenDim};
-    ((float*)a.workspace + (size_t)max_chunks * a.heads * pd.kp * pd.vp + ((size_t)ch.slot * a.heads + h) * pd.kp)[channel] = exp2f(pair + other);
-  }
+  const RecurrenceDims pd{kTokenDim, kTokenDim};
+  if (g == 0) chunk_factors(a, pd, max_chunks, ch.slot, h)[channel] = exp2f(pair + other);
   float4_t S[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) S[c] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -159,7 +157,7 @@ __global__ __launch_bounds__(kTokenChunk * 4, 4) void recur_token_state_kernel(n
 #pragma unroll
     for (int c = 0; c < 4; ++c) mend(S[c], again[c]);
   }
-  float* dst = (float*)a.workspace + ((size_t)ch.slot * a.heads + h) * kTokenDim * kTokenDim;
+  float* dst = chunk_states(a, pd, ch.slot, h);
 #pragma unroll
   for (int c = 0; c < 4; ++c) *reinterpret_cast<float4_t*>(dst + ((size_t)(c * 4 + g) * 64 + wave * 16 + l16) * 4) = S[c];
 }
@@ -201,7 +199,7 @@ __global__ __launch_bounds__(kTokenChunk * 4, 3) void recur_token_out_kernel(nf_
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
   TokenTile::load((const uint16_t*)a.v + (size_t)ch.row0 * a.v_ld + h * kTokenDim, a.v_ld, ch.n, lds0, wave, lane);
-  const rsrc_t state = make_rsrc((const float*)a.workspace + ((size_t)ch.slot * a.heads + h) * kTokenDim * kTokenDim, kTokenDim * kTokenDim * 4);
+  const rsrc_t state = make_rsrc(chunk_states(a, {kTokenDim, kTokenDim}, ch.slot, h), kTokenDim * kTokenDim * 4);
 #pragma unroll
   for (int i = 0; i < 16 / kBlocks; ++i) {
     const int at = (i * kBlocks + wave) * 1024;
