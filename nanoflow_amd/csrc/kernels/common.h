@@ -73,8 +73,8 @@ __device__ __forceinline__ float sum_over_near_lane_groups(float v) {
 
 // Over the 16 lanes of a group, and over a wavefront: the pairs of lanes that differ in one bit, the highest first.  Once lanes that differ in bit 3 agree, a rotation by
 // 4 within the 16 meets the lane that differs in bit 2, and so on: data paths of the vector unit (DPP), where a shuffle is a round trip through LDS.
-// A step of decode attention has two round trips less in its chain, a row norm six (layers of few rows, us: 1 request 103.2 -> 101.6, 16 under e4m3 93.0 -> 90.6,
-// 64 of a parallel layer 141.5 -> 137.7).
+// A step of decode attention has two round trips less in its chain, a row norm six (64 requests of a parallel layer, us, 141.5 -> 137.7; layers of one and of 16 requests
+// were timed only together with the RMS norm's stores: 103.3 -> 101.6, 93.0 -> 90.6).
 template <int n>
 __device__ __forceinline__ float rotated_in_16(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + n, 0xf, 0xf, true));

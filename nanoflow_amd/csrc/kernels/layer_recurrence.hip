@@ -745,8 +745,8 @@ static int launch_chunks(const nf_recurrence_args& a, const ChunkPlan& p, hipStr
 }
 
 // Fixed decays on the 16-bit matrix instructions (recurrence_fixed.h): heads of 128 x 128 in bf16, neither rotated nor gated, rows read and written 16 bytes at
-// a time; wherever the fp32 form takes chunks, for it is slower at every size (16 heads, us, fp32 form and this: 40 rows 25.8, 14.6; 500 rows 42, 24; 2047
-// 67, 38; 8000 195, 113; 8 requests of 256 72, 49).  Halves of a chunk where requests hardly fill one and the CUs are not all taken: 128 rows 20.1 -> 16.9 us,
+// a time; wherever the fp32 form takes chunks, for it was slower at every number of rows (all of 16 heads, us, fp32 form and this: 40 rows 25.8, 14.6; 500 rows 42, 24; 2047
+// 67, 38; 8000 195, 113; 8 requests of 256 72, 49; fewer heads were not timed: of a long prompt they leave CUs idle in either form).  Halves of a chunk where requests hardly fill one and the CUs are not all taken: 128 rows 20.1 -> 16.9 us,
 // but 2 x 300 25.7 -> 27.0.
 static ChunkPlan fixed_plan(const nf_recurrence_args& a) {
   if (a.dtype != NF_BF16 || a.kind != NF_RECURRENCE_FIXED_DECAY || a.dim != kFixedDim || a.vdim != kFixedDim || a.rot.dims != 0 || a.g) return {0, 0};
@@ -780,7 +780,7 @@ static int launch_fixed(const nf_recurrence_args& a, const ChunkPlan& p, hipStre
 }
 
 // Decays of every token, 64 tokens at a time (recurrence_token.h): heads of 64 x 64 in bf16, rows read and written 16 bytes at a time; wherever the general form
-// takes chunks, for it is slower at every size (32 heads, us, general form and this: 40 rows 21.1, 14.1; 129 rows 28.0, 16.3; 500 rows 32, 20; 3000 85, 60;
+// takes chunks, for it was slower at every number of rows (all of 32 heads, us, general form and this: 40 rows 21.1, 14.1; 129 rows 28.0, 16.3; 500 rows 32, 20; 3000 85, 60;
 // 8000, in its chunks of 256, 173, 135; 8 requests of 256 61, 48; 2047 rows of which most blocks decay below 2^-100, its steps then of four tokens or one, 597, 72).
 static ChunkPlan token_plan(const nf_recurrence_args& a) {
   if (a.dtype != NF_BF16 || a.kind != NF_RECURRENCE_TOKEN_DECAY || a.dim != kTokenDim || a.vdim != kTokenDim) return {0, 0};

@@ -4,7 +4,8 @@
 //   outputs closed by the rank of their largest entry, the `top` largest taken one after the other (up to 64 outputs: all at once, by rank), then the
 //   experts that every token has.  What bounds it is a chain of dependent steps: loads that are all on their way before the first is waited for, and lanes that
 //   meet without LDS, took both launches from 11.6 to 9.1 us (256 rows of 32 outputs in 8 groups, 4 a token, 16 shares), 11.9 to 9.9 (2047 rows of 40, 5 a
-//   token), 8.2 to 6.5 (one row).
+//   token), 8.2 to 6.5 (one row).  (Timed of 1, 4 and 16 shares.  All but the first are requested kMaxShares - 1 at a time, those past the last as the last again, from
+//   the caches.)
 // route_plan_kernel: counts the rows of every expert, places them (an expert's rows consecutive)
 //   and lists the m tiles of the grouped product.  The place of a row inside its expert's run
 //   depends on the order of LDS atomics; nothing computed from it does.

@@ -12,7 +12,7 @@
 // where a channel decays below 2^-100 over 16; an infinity that it still has there is NaN in its states from the next chunk on.  The
 // figures below are without the check, 20 vector instructions a wavefront.)
 // 2019 tokens of 32 heads in two requests (us, general form -> this): chunk states 15.2 -> 11.3, scan 8.4 (bytes), outputs 35.8 -> 23.5; the states' error against
-// 64 bits 7.3e-8 -> 6.2e-8.  The outputs are bound by what their wavefronts issue (1250 vector and 112 matrix instructions for 16 tokens), little of it side
+// 64 bits 7.3e-8 -> 6.2e-8.  The outputs are bound by what their wavefronts issue (some 1250 vector instructions for 16 tokens, and 92 to 152 matrix ones, 122 on average), little of it side
 // by side; the same on 8 wavefronts and chunks of 128 took 32: the last block has seven before it.
 
 namespace nf {
