@@ -97,7 +97,8 @@ def test_what_is_not_finite_stays_with_its_tokens(bad, row):
 @pytest.mark.parametrize("what", ["q", "k", "v", "state"])
 @pytest.mark.parametrize("k_scale", [1.0, 0.31])
 def test_infinities_are_those_of_the_general_form(what, row, bad, k_scale):
-    """Operands of eight significant bits or fewer beside them: all of q, k and v, and every fourth column of the state."""
+    """Operands of eight significant bits or fewer beside them: all of q, k and v, and every fourth column of the state.  What is finite may differ by the bounds of
+    both forms."""
     reqs, heads = [(4, 200)], 2
     qkv, state = operands(reqs, heads)
     state[:, :, :, ::4] = state[:, :, :, ::4].bfloat16().float()

@@ -108,7 +108,8 @@ def test_what_is_not_finite_stays_with_its_tokens(bad, row):
 @pytest.mark.parametrize("what", ["q", "k", "v", "state"])
 @pytest.mark.parametrize("gate", [False, True])
 def test_infinities_are_those_of_the_general_form(gate, what, row, bad):
-    """Operands of eight significant bits or fewer beside them: all of q, k and v, and every fourth column of the state."""
+    """Operands of eight significant bits or fewer beside them: all of q, k and v, and every fourth column of the state.  What is finite may differ by the bounds of
+    both forms."""
     reqs = [(4, 100)]
     s = operands(reqs, 2, -2.0)
     s["state"][:, :, :, ::4] = s["state"][:, :, :, ::4].bfloat16().float()
@@ -122,4 +123,4 @@ def test_infinities_are_those_of_the_general_form(gate, what, row, bad):
     for x, y, off in ((got, want, 2.0 ** -7), (st, left, 0.0)):
         assert torch.equal(x[y.isinf()], y[y.isinf()]) and torch.equal(x.isfinite(), y.isfinite())
         ok = y.isfinite()
-        assert bool(((x[ok] - y[ok]).abs() <= off * y[ok].abs() + 4e-5 * y[ok].abs().max()).all())
+        assert bool(((x[ok] - y[ok]).abs() <= off * y[ok].abs() + 8e-5 * y[ok].abs().max()).all())
